@@ -23,7 +23,9 @@
  *  - threads: every entry point may be called from several host threads at
  *    once (the reference is driven from one thread).  The library's only
  *    shared state is the profiling sums of vl_beam_profile (mutex), the launch
- *    counter of vl_beam_launches (atomic) and the thread-local error text.  A workspace belongs to ONE call at a time: the
+ *    counter of vl_beam_launches (atomic), the page of pinned host memory that
+ *    progress checks are reported in (each call borrows a slot of it, mutex)
+ *    and the thread-local error text.  A workspace belongs to ONE call at a time: the
  *    beam-search loop keeps its control block, visit queues and visited lists
  *    in it, so two vl_closest_vectors calls in flight need two workspaces;
  *  - return value 0 is success; a negative value is an error whose text
@@ -224,8 +226,10 @@ int64_t vl_beam_workspace_bytes(const vl_beam_params *p);
 
 /* Runs the whole loop of closest_vectors on the search queue in place and
  * returns the number of iterations (a multiple of speculative_readahead) or
- * a negative error.  Synchronises the stream every speculative_readahead
- * iterations to read the batch-wide "any row changed" flag, as the
+ * a negative error.  Waits every speculative_readahead iterations for the
+ * batch-wide "any row changed" flag, which the GPU writes to pinned host memory
+ * of the library (one page per process) while it goes on with the next
+ * iteration, and for the stream before it returns; the cadence is the one the
  * reference does (ann.py:90-91).  Rows of the search queue are exact on
  * [:, :queue_length]; slots beyond are unspecified. */
 int64_t vl_closest_vectors(const vl_beam_params *p,

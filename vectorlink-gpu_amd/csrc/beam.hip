@@ -66,6 +66,66 @@ struct EventSet {
     }
 };
 
+// Pinned host memory for the reports of the progress checks: one page of slots for the whole process, made with the
+// first call and kept; a call borrows a slot.  With every slot lent out (64 calls at once) or no page to be had, a call
+// waits for its stream at every check and fetches the flags instead.
+class ReportSlot {
+public:
+    ReportSlot() {
+        std::lock_guard<std::mutex> hold(mutex_);
+        if (!page_ && !refused_) {
+            void *p = nullptr;
+            if (hipHostMalloc(&p, kSlots * sizeof(Slot), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess)
+                page_ = static_cast<Slot *>(p);
+            else {
+                refused_ = true;
+                (void)hipGetLastError();
+            }
+        }
+        for (int i = 0; page_ && i < kSlots; ++i)
+            if (!((lent_ >> i) & 1)) {
+                lent_ |= 1ull << i;
+                index_ = i;
+                page_[i].report.check = 0;
+                break;
+            }
+    }
+    ~ReportSlot() {
+        if (index_ < 0) return;
+        std::lock_guard<std::mutex> hold(mutex_);
+        lent_ &= ~(1ull << index_);
+    }
+    ReportSlot(const ReportSlot &) = delete;
+    ReportSlot &operator=(const ReportSlot &) = delete;
+    BeamReport *get() const { return index_ < 0 ? nullptr : &page_[index_].report; }
+
+private:
+    static constexpr int kSlots = 64;
+    struct alignas(64) Slot { BeamReport report; };
+    static inline std::mutex mutex_;
+    static inline Slot *page_ = nullptr;
+    static inline bool refused_ = false;
+    static inline uint64_t lent_ = 0;
+    int index_ = -1;
+};
+
+// Waits until the launch behind the check after iteration t has reported.  The stream is asked now and then, so that a
+// launch that failed ends the wait.
+int wait_for_report(const BeamReport *r, int t, hipStream_t st) {
+    for (unsigned spins = 1;; ++spins) {
+        if (__atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t) return VL_OK;
+        if ((spins & 0xffff) == 0) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) continue;
+            VL_HIP(e);
+            if (__atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t) return VL_OK;
+            vl_set_error("the progress check after iteration %d was not reported", t);
+            return VL_ERR_HIP;
+        }
+        __builtin_ia32_pause();
+    }
+}
+
 struct MergeArgs {
     BeamCtrl *ctrl;
     int iter;
@@ -771,6 +831,7 @@ struct StepArgs {
     int64_t rounded_query_bytes;
     int window;     // beam_window_kernel: iterations m.iter ... m.iter + window - 1 in this launch
     int lds_slots;  // beam_window_kernel: entries of the row's distance table in LDS (a power of two, or 0)
+    BeamReport *report;  // pinned host memory that hears of the progress checks, or null
 };
 
 // A probe of the distance cache is a random 8-byte read and every evaluated distance a random 8-byte
@@ -840,7 +901,7 @@ __device__ __forceinline__ void beam_step_body(const StepArgs &s) {
     int32_t my_excl = VL_MAXINT;
     if (a.excl && tid < a.excl_cols) my_excl = a.excl[row * a.excl_cols + tid];
 
-    const int gate = beam_gate(c, t, a.readahead, a.E, blockIdx.x == 0 && tid == 0);
+    const int gate = beam_gate(c, t, a.readahead, a.E, blockIdx.x == 0 && tid == 0, s.report);
     if (gate == 2) return;
     if (!beam_row_state_ok(c, pre.cnt, seen_bound, tid == 0)) return;
     if (gate == 1 || (a.row_quiet && quiet >= a.readahead)) {
@@ -1238,7 +1299,7 @@ __device__ __forceinline__ void beam_window_body(const StepArgs &s) {
 
     // (the visited lists cannot be full in these iterations; the slots of `first` are not read here, because rows
     // of this very launch that finish early write the one the next launch reads)
-    const int gate = beam_gate(c, t0, a.readahead, a.E, blockIdx.x == 0 && tid == 0, false);
+    const int gate = beam_gate(c, t0, a.readahead, a.E, blockIdx.x == 0 && tid == 0, s.report, false);
     if (gate == 2) return;
     if (!beam_row_state_ok(c, cnt, seen_bound, tid == 0)) return;
     int *first_after = &c->first[(t0 + W) % 3];  // what the launch of iteration t0 + W reads
@@ -1950,6 +2011,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     step.sketch_chunks = (int)sketch_data_chunks(p->dim);
     step.window = 0;
     step.lds_slots = 0;
+    step.report = nullptr;
     step.memo_shift = 32;
     if (step.memo) {
         int lg = 0;
@@ -2045,41 +2107,43 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     const uint8_t *sketch_table = step.sketch;
     int sketch_rows = sketch_from_start ? (int)p->n_rows : 0;
     int64_t t = 0;
+    // A call that is not profiled keeps the GPU busy across its progress checks: the launch after a checking iteration
+    // is enqueued before the host knows what the check found - it does nothing if the check ended the loop (beam_gate)
+    // - and reports it from its first workgroup.
+    ReportSlot slot;
+    const bool ahead = use_fused && !prof && slot.get() != nullptr;
+    step.report = ahead ? slot.get() : nullptr;
+    auto launch_next = [&]() -> int {  // the fused launch that follows iteration t; moves t on
+        const bool windowed = window_fits(t + 1) && t % R == 0;
+        a.iter = (int)(t + 1);
+        step.m = a;
+        // (the sketch kernel also for a first window: its rows leave the sketch alone in iteration 1)
+        step.sketch = ((windowed || t > 0) && 2 * (int64_t)sketch_rows >= p->n_rows) ? sketch_table : nullptr;
+        step.window = windowed ? R : 0;
+        step.lds_slots = windowed ? lds_slots : 0;
+        const int e = launch_step_by_dim(step, aligned, step_threads, windowed ? smem_window : smem, st);
+        t += windowed ? R : 1;
+        return e;
+    };
+    int64_t checked = 0;  // iterations up to the last progress check
     for (;;) {
         int launches = 0;  // of this stretch between two progress checks
-        if (window_fits(t + 1)) {
-            // the sketch kernel also for the first window: its rows leave the sketch alone in iteration 1
-            if (prof) VL_HIP(hipEventRecord(ev[0], st));
-            a.iter = (int)(t + 1);
-            step.m = a;
-            step.sketch = (2 * (int64_t)sketch_rows >= p->n_rows) ? sketch_table : nullptr;
-            step.window = R;
-            step.lds_slots = lds_slots;
-            rc = launch_step_by_dim(step, aligned, step_threads, smem_window, st);
-            if (rc < 0) return rc;
-            if (prof) VL_HIP(hipEventRecord(ev[1], st));
-            step.window = 0;
-            step.lds_slots = 0;
-            t += R;
-            launches = 1;
-        }
-        for (int r = 0; r < R && !launches; ++r) {
-            ++t;
-            if (prof) VL_HIP(hipEventRecord(ev[3 * r], st));
-            a.iter = (int)t;
+        checked += R;
+        while (t < checked) {
+            const int at = launches++;
+            if (prof) VL_HIP(hipEventRecord(ev[3 * at], st));
             if (use_fused) {
-                step.m = a;
-                step.sketch = (t > 1 && 2 * (int64_t)sketch_rows >= p->n_rows) ? sketch_table : nullptr;
-                rc = launch_step_by_dim(step, aligned, step_threads, smem, st);
+                rc = launch_next();
                 if (rc < 0) return rc;
-                if (prof) VL_HIP(hipEventRecord(ev[3 * r + 1], st));
+                if (prof) VL_HIP(hipEventRecord(ev[3 * at + 1], st));
                 continue;
             }
+            a.iter = (int)++t;
             rc = vl_launch_expand(queries, p->n_rows, vectors, p->n_vectors, p->dim, nullptr, v_ids, l.Vt, beams,
                                   p->n_vectors, p->width, l.m, cand_ids, cand_d, ctrl, (int)t, R, (int)l.E, l.VL,
                                   prof ? 1 : 0, memo, l.memo_slots, (int)p->metric, st);
             if (rc < 0) return rc;
-            if (prof) VL_HIP(hipEventRecord(ev[3 * r + 1], st));
+            if (prof) VL_HIP(hipEventRecord(ev[3 * at + 1], st));
             if (use_sort_merge)
                 hipLaunchKernelGGL(beam_merge_kernel, dim3((unsigned)p->n_rows), dim3(kQueueThreads), smem, st, a);
             else if (merge_threads == 64)
@@ -2089,30 +2153,41 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
             else
                 hipLaunchKernelGGL(beam_merge2_kernel<256>, dim3((unsigned)p->n_rows), dim3(256), smem, st, a);
             VL_LAUNCH_CHECK("beam merge kernel");
-            if (prof) VL_HIP(hipEventRecord(ev[3 * r + 2], st));
+            if (prof) VL_HIP(hipEventRecord(ev[3 * at + 2], st));
         }
-        // one copy brings the ring of progress flags and the two words behind it (they are neighbours in the
-        // control block): this check's flag, the rows still using the sketch, the error flag
-        struct {
-            int changed[64];
-            int sketch_rows, error;
-        } seen_by_host;
-        static_assert(offsetof(BeamCtrl, error) - offsetof(BeamCtrl, changed) == 65 * sizeof(int) &&
-                          offsetof(BeamCtrl, sketch_rows) - offsetof(BeamCtrl, changed) == 64 * sizeof(int),
-                      "changed[64], sketch_rows, error follow each other");
-        VL_HIP(hipMemcpyAsync(&seen_by_host, &ctrl->changed[0], sizeof(seen_by_host), hipMemcpyDeviceToHost, st));
-        VL_HIP(hipStreamSynchronize(st));
-        const int changed = seen_by_host.changed[(t / R) & 63];
-        const int state[2] = {seen_by_host.sketch_rows, seen_by_host.error};
-        if (sketch_table) sketch_rows = state[0];
-        if (state[1]) {
+        BeamReport found;
+        if (ahead) {
+            rc = launch_next();
+            if (rc < 0) return rc;
+            rc = wait_for_report(slot.get(), (int)checked, st);
+            if (rc < 0) return rc;
+            found = *slot.get();
+            // the launch that has nothing left to do is waited for: the caller may use the workspace on another stream
+            if (!found.changed || found.error) VL_HIP(hipStreamSynchronize(st));
+        } else {
+            // one copy brings the ring of progress flags and the two words behind it (they are neighbours in the
+            // control block): this check's flag, the rows still using the sketch, the error flag
+            struct {
+                int changed[64];
+                int sketch_rows, error;
+            } seen_by_host;
+            static_assert(offsetof(BeamCtrl, error) - offsetof(BeamCtrl, changed) == 65 * sizeof(int) &&
+                              offsetof(BeamCtrl, sketch_rows) - offsetof(BeamCtrl, changed) == 64 * sizeof(int),
+                          "changed[64], sketch_rows, error follow each other");
+            VL_HIP(hipMemcpyAsync(&seen_by_host, &ctrl->changed[0], sizeof(seen_by_host), hipMemcpyDeviceToHost, st));
+            VL_HIP(hipStreamSynchronize(st));
+            found.changed = seen_by_host.changed[(checked / R) & 63];
+            found.sketch_rows = seen_by_host.sketch_rows;
+            found.error = seen_by_host.error;
+        }
+        if (sketch_table) sketch_rows = found.sketch_rows;
+        if (found.error) {
             vl_set_error("a row's visited list holds more ids than %lld iterations can have put there: the workspace "
-                         "was overwritten while the loop ran - is it shared with a concurrent call?", (long long)t);
+                         "was overwritten while the loop ran - is it shared with a concurrent call?", (long long)checked);
             return VL_ERR_STATE;
         }
         if (prof) {
-            const int timed = launches ? launches : R;
-            for (int r = 0; r < timed; ++r) {
+            for (int r = 0; r < launches; ++r) {
                 float ms = 0;
                 VL_HIP(hipEventElapsedTime(&ms, ev[3 * r], ev[3 * r + 1]));
                 mine.expand_ms += ms;
@@ -2121,14 +2196,14 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
                     mine.merge_ms += ms;
                 }
             }
-            mine.expand_launches += timed;
-            mine.merge_launches += timed;
+            mine.expand_launches += launches;
+            mine.merge_launches += launches;
         }
-        if (!changed) break;  // ann.py:90-91
-        if (t > t_limit) {
+        if (!found.changed) break;  // ann.py:90-91
+        if (checked > t_limit) {
             vl_set_error("beam search still changing after %lld iterations (bound %lld): its workspace was "
                          "overwritten while it ran - is it shared with a concurrent call?",
-                         (long long)t, (long long)t_limit);
+                         (long long)checked, (long long)t_limit);
             return VL_ERR_STATE;
         }
     }
@@ -2148,9 +2223,9 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
         g_prof.expand_launches += mine.expand_launches; g_prof.merge_launches += mine.merge_launches;
         g_prof.evals += mine.evals; g_prof.wanted += mine.wanted; g_prof.sketched += mine.sketched;
         g_prof.rows += p->n_rows;
-        g_prof.iterations += t;
+        g_prof.iterations += checked;
     }
-    return t;
+    return checked;
 }
 
 }  // namespace

@@ -10,6 +10,10 @@
 //   changed[64] - ring of "some row changed" flags, one per checking iteration
 //   sketch_rows - how many rows currently use the 8-bit sketch (they opt in once and may opt out once)
 //   error       - a row found its own state impossible (see beam_row_state_ok)
+// What the host needs to know at a progress check goes to a BeamReport in pinned host memory: the first workgroup of
+// the launch after the checking iteration writes it (beam_gate) and the host, which has already enqueued that launch,
+// polls it.  A copy of the flag and a wait for the stream instead left the GPU idle for 35 - 55 us per check (its five
+// iterations of 256 queries at 4,096 x 128 take 105 us).
 #pragma once
 #include "vl_common.h"
 
@@ -28,6 +32,17 @@ struct BeamCtrl {
     unsigned long long wanted[kBeamStripes];  // candidate distances asked for (fetched or served by the cache)
     unsigned long long sketched[kBeamStripes];  // candidate rows looked at through the 8-bit sketch only
 };
+
+struct BeamReport {
+    int changed, sketch_rows, error;  // as in BeamCtrl, after the checking iteration
+    int check;                        // written last: iterations run up to that check
+};
+__device__ inline void beam_report(const BeamCtrl *c, int t, int R, BeamReport *out) {
+    out->changed = c->changed[(t / R) & 63];
+    out->sketch_rows = c->sketch_rows;
+    out->error = c->error;
+    __hip_atomic_store(&out->check, t, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // A row's visited list holds at most Vt ids per earlier iteration and never more than its E slots.  A
 // count beyond that was not written by this loop (its workspace is shared with another call): the row
@@ -51,9 +66,12 @@ __device__ inline bool beam_row_state_ok(BeamCtrl *c, int cnt, int bound, bool w
 // look_at_fill = false (a launch that takes rows through several iterations, none of which can find a
 // visited list full): state 1 is not looked for - rows of such a launch that finish early raise the slot of
 // `first` that the launch after it reads, which for some lengths is the slot of iteration t - 1 modulo 3.
-__device__ inline int beam_gate(BeamCtrl *c, int t, int R, int E, bool writer, bool look_at_fill = true) {
+// report (may be null): where the launch after a checking iteration tells the host what that check found.
+__device__ inline int beam_gate(BeamCtrl *c, int t, int R, int E, bool writer, BeamReport *report = nullptr,
+                                bool look_at_fill = true) {
     int stop = c->stop;
     const bool after_check = t > 1 && ((t - 1) % R) == 0;
+    if (writer && report && after_check) beam_report(c, t - 1, R, report);
     if (!stop && after_check && c->changed[((t - 1) / R) & 63] == 0) {
         stop = 1;
         if (writer) c->ended_after = t - 1;  // the loop ran t - 1 iterations
