@@ -229,8 +229,8 @@ int64_t vl_beam_workspace_bytes(const vl_beam_params *p);
  * a negative error.  Waits every speculative_readahead iterations for the
  * batch-wide "any row changed" flag, which the GPU writes to pinned host memory
  * of the library (one page per process) while it goes on with the next
- * iteration, and for the stream before it returns; the cadence is the one the
- * reference does (ann.py:90-91).  Rows of the search queue are exact on
+ * iteration, and for the stream before it returns; the cadence is the
+ * reference's (ann.py:90-91).  Rows of the search queue are exact on
  * [:, :queue_length]; slots beyond are unspecified. */
 int64_t vl_closest_vectors(const vl_beam_params *p,
                            const float *queries, const float *vectors,

@@ -410,28 +410,6 @@ __device__ inline void raise_running_max(int *slot, int cnt, int bound) {
     else atomicMax(slot, cnt);
 }
 
-// Smallest 32-bit value over a wavefront, in every lane: halves and rows are folded with the swap instructions
-// and DPP row shifts that fold_group uses (a lane without a source keeps its own value), a few cycles per
-// step where a cross-lane shuffle through the LDS crossbar takes a round trip each.
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
-    {
-        uint32_t lo = x, hi = x;
-        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lo), "+v"(hi));
-        x = lo < hi ? lo : hi;
-    }
-    {
-        uint32_t even = x, odd = x;
-        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(even), "+v"(odd));
-        x = even < odd ? even : odd;
-    }
-    uint32_t y;
-    y = __builtin_amdgcn_update_dpp(x, x, 0x108, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:8
-    y = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:4
-    y = __builtin_amdgcn_update_dpp(x, x, 0x102, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:2
-    y = __builtin_amdgcn_update_dpp(x, x, 0x101, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:1
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
-}
-
 // Smallest value over the workgroup of each thread's `mine` (0xFFFFFFFF = none).
 // red: 2 * kQueueWaves words of LDS, used alternately so one barrier per call suffices.
 __device__ inline uint32_t block_min_u32(uint32_t mine, uint32_t *red, int round) {

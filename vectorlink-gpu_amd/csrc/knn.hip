@@ -12,20 +12,17 @@
 // private sorted list of the k best (distance, id) keys for each of its two
 // query columns.  The Q x N distance matrix never exists in memory.  A second
 // kernel merges the per-lane lists of a query in LDS.
+#include "knn_device.h"
+#include "knn_few.h"
+
 #include <type_traits>
 
-#include "rowsort.h"
 
 namespace {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int KMAX = 16;      // longest list kept per lane and query
 constexpr int TQ = 128;       // queries per workgroup
 constexpr int TV = 128;       // vectors per step
-constexpr int KT = 32;        // floats of the reduction dimension per stage
-constexpr int CH = KT / 4;    // 16-byte chunks per row and stage
-constexpr int TILE = 128 * KT;  // floats of one staged operand tile (16 KB)
 constexpr int LISTS_PER_STRIP = 4;  // two half-waves x two wave rows see the same query
 // workgroups of the tile kernel resident at once: two per compute unit (64 KB of LDS each), 256 CUs on an MI355X;
 // the count is read from the device on first use
@@ -38,65 +35,6 @@ int64_t resident_workgroups() {
         return (int64_t)2 * cus;
     }();
     return n;
-}
-
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void glb_void;
-
-__device__ __align__(16) const float kZeroChunk[4] = {0.f, 0.f, 0.f, 0.f};
-
-// A lane's list of the KK best so far: distances ascending with their ids.  A lane meets its
-// candidates in ascending id order, so one that ties a kept distance belongs behind it: comparing
-// distances alone orders (distance, id) pairs correctly.  The new distance column is a median of
-// three per slot; ids follow the same comparisons.
-template <int KK>
-__device__ __forceinline__ void list_insert(float (&kd)[KK], int32_t (&kid)[KK], float d, int32_t id) {
-#pragma unroll
-    for (int i = KK - 1; i > 0; --i) {
-        const bool before_prev = d < kd[i - 1], before_this = d < kd[i];
-        kid[i] = before_prev ? kid[i - 1] : (before_this ? id : kid[i]);
-        kd[i] = __builtin_amdgcn_fmed3f(kd[i - 1], d, kd[i]);
-    }
-    const bool first = d < kd[0];
-    kid[0] = first ? id : kid[0];
-    kd[0] = first ? d : kd[0];
-}
-
-// Chunk c (16 bytes) of tile row r lives in slot r * CH + (c ^ swz(r)): sixteen consecutive
-// rows read the same chunk index from sixteen different 16-byte bank groups.
-__device__ __forceinline__ int swz(int r) { return (r >> 1) & (CH - 1); }
-
-// Staging: 128 rows x KT floats of an operand go straight from global memory into LDS (no
-// registers in between).  A wavefront instruction fills 1 KB = 8 tile rows and lane i writes
-// slot i of those rows, so it fetches the chunk that belongs there.  Each lane has four such
-// (row, chunk) duties per operand; their source addresses at k = 0 are kept as pointers.
-// Rows past `last` repeat row `last` (their results are discarded later).
-__device__ __forceinline__ void duty_pointers(const float *__restrict__ src, int64_t first, int64_t last, int dim,
-                                              int wave, int lane, const float *(&p)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = 8 * (4 * wave + i) + (lane >> 3);
-        const int c = (lane & (CH - 1)) ^ swz(r);
-        int64_t row = first + r;
-        row = row < last ? row : last;
-        p[i] = src + row * dim + 4 * c;
-    }
-}
-
-// RAGGED: the last stage reaches past `dim`; chunks out there come from a zero chunk.
-template <bool RAGGED>
-__device__ __forceinline__ void stage_operand(const float *const (&p)[4], int kt, int dim, float *tile, int wave,
-                                              int lane) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float *g = p[i] + kt;
-        if constexpr (RAGGED) {
-            const int r = 8 * (4 * wave + i) + (lane >> 3);
-            const int c = (lane & (CH - 1)) ^ swz(r);
-            if (kt + 4 * c >= dim) g = kZeroChunk;
-        }
-        __builtin_amdgcn_global_load_lds((glb_void *)g, (lds_void *)(tile + 8 * (4 * wave + i) * KT), 16, 0, 0);
-    }
 }
 
 // every query's shared bound starts at infinity
@@ -338,11 +276,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     vn[r] = v_norm[v < vlimit ? v : vlimit - 1];
                 }
             }
-            auto distance = [&](int cb, int r) {
-                if constexpr (L2) return fmaxf(fmaf(-2.0f, acc[rb][cb][r], qn[cb] + vn[r]), 0.0f);
-                const float d = (1.0f - acc[rb][cb][r]) * 0.5f;
-                return d < 0.0f ? 0.0f : (d > 1.0f ? 1.0f : d);
-            };
+            auto distance = [&](int cb, int r) { return tile_distance<L2>(acc[rb][cb][r], qn[cb], vn[r]); };
 #pragma unroll
             for (int cb = 0; cb < 2; ++cb) {
                 uint64_t hit[16], any = 0;
@@ -454,6 +388,7 @@ struct KnnPlan {
     int list_len;
     int n_strips;
     int64_t strip_len;
+    bool few;  // the kernel of knn_few.hip takes the call (see vl_knn_exact_metric)
     int n_cand;
     int64_t cand_bytes;  // per-lane candidate lists; the queries' shared bounds and the rows' squared lengths (L2) follow
     int64_t bytes;
@@ -488,6 +423,8 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, KnnPl
     p->strip_len = len;
     p->list_len = list_length(k);
     p->n_cand = (int)(strips * LISTS_PER_STRIP * p->list_len);
+    p->few = n_queries <= kFewQueries;
+    if (p->few) p->n_cand = (int)(vl_knn_few_lists(n_vectors) * p->list_len);
     p->cand_bytes = (n_queries > 0 ? n_queries : 1) * (int64_t)p->n_cand * 8;
     p->bytes = p->cand_bytes + ((2 * n_queries + n_vectors) * 4 + 15) / 16 * 16;
     return VL_OK;
@@ -536,8 +473,6 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     uint32_t *q_bound = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(workspace) + p.cand_bytes);
     float *q_norm = reinterpret_cast<float *>(q_bound + n_queries);
     float *v_norm = q_norm + n_queries;
-    hipLaunchKernelGGL(knn_bound_init_kernel, dim3(vl_grid_for(n_queries, 256)), dim3(256), 0, st, q_bound, n_queries);
-    VL_LAUNCH_CHECK("knn_bound_init_kernel");
     if (l2) {
         VL_REQUIRE((n_vectors + 3) / 4 <= kMaxBlocks * 4, "too many vectors for one call");
         hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, queries,
@@ -546,6 +481,11 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
                            n_vectors, (int)dim, v_norm);
         VL_LAUNCH_CHECK("row_norms_kernel");
     }
+    if (p.few)
+        return vl_knn_few(queries, n_queries, vectors, n_vectors, dim, k, p.list_len, l2, q_norm, v_norm, cand, ids_out,
+                          dists_out, st);
+    hipLaunchKernelGGL(knn_bound_init_kernel, dim3(vl_grid_for(n_queries, 256)), dim3(256), 0, st, q_bound, n_queries);
+    VL_LAUNCH_CHECK("knn_bound_init_kernel");
 #define VL_KNN_LAUNCH(KK)                                                                                     \
     do {                                                                                                      \
         if (l2)                                                                                               \

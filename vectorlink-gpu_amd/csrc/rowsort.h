@@ -46,6 +46,35 @@ __device__ inline void block_bitonic_sort(uint64_t *keys, int P) {
     }
 }
 
+// Smallest 32-bit value over a wavefront, in every lane: halves and rows are folded with the swap instructions
+// and DPP row shifts that fold_group (dist_device.h) uses (a lane without a source keeps its own value), a few cycles per
+// step where a cross-lane shuffle through the LDS crossbar takes a round trip each.
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
+    {
+        uint32_t lo = x, hi = x;
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lo), "+v"(hi));
+        x = lo < hi ? lo : hi;
+    }
+    {
+        uint32_t even = x, odd = x;
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(even), "+v"(odd));
+        x = even < odd ? even : odd;
+    }
+    uint32_t y;
+    y = __builtin_amdgcn_update_dpp(x, x, 0x108, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:8
+    y = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:4
+    y = __builtin_amdgcn_update_dpp(x, x, 0x102, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:2
+    y = __builtin_amdgcn_update_dpp(x, x, 0x101, 0xf, 0xf, false); x = y < x ? y : x;  // row_shl:1
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+}
+
+// Smallest 64-bit key over a wavefront, in every lane.
+__device__ __forceinline__ uint64_t wave_min_u64(uint64_t x) {
+    const uint32_t hi = wave_min_u32((uint32_t)(x >> 32));
+    const uint32_t lo = wave_min_u32((uint32_t)(x >> 32) == hi ? (uint32_t)x : 0xFFFFFFFFu);
+    return ((uint64_t)hi << 32) | lo;
+}
+
 __device__ inline bool same_id_ignoring_flag(int32_t a, int32_t b) {
     return (a & ~VL_DUP_FLAG) == (b & ~VL_DUP_FLAG);  // kernels.py:325-330
 }
