@@ -63,3 +63,52 @@ def test_a_few_queries_among_equal_rows(n, nq):
     (gi, gd) = knn_exact(dev(q), dev(v), 16)
     assert np.array_equal(gi.cpu().numpy(), np.tile(np.arange(16, dtype=np.int32), (nq, 1)))
     assert all(len(set(r)) == 1 for r in gd.cpu().numpy().tolist())
+
+
+# the bfloat16 filter: tiles of 256 x 256 and stages of 64 columns with remainders, an odd number of stages, three more
+# columns for L2, rows of very different lengths, and more than one converted piece of the table (2 GiB of 64 columns)
+@pytest.mark.parametrize("n,dim,nq,k,metric", [
+    (4096, 64, 129, 10, "cosine"), (4097, 4, 256, 16, "cosine"), (5000, 60, 257, 4, "l2"), (6000, 64, 300, 1, "l2"),
+    (40_000, 192, 700, 16, "cosine"), (33_000, 196, 513, 12, "l2"), (17_000_000, 4, 150, 4, "cosine")])
+def test_the_filter_and_a_few_queries_agree(n, dim, nq, k, metric):
+    print(f"filter n={n} dim={dim} nq={nq} k={k} {metric}", flush=True)
+    from vectorlink_gpu.kernels import knn_exact
+
+    gen = torch.Generator(device=DEV).manual_seed(n + dim)
+    v = torch.randn((n, dim), generator=gen, device=DEV)
+    q = torch.randn((nq, dim), generator=gen, device=DEV)
+    if metric == "cosine":
+        v, q = torch.nn.functional.normalize(v, dim=1), torch.nn.functional.normalize(q, dim=1)
+    else:
+        v *= torch.rand((n, 1), generator=gen, device=DEV) * 4
+    v[n - 1] = q[nq - 1]
+    v[n // 3] = v[n - 1]  # a tie that the ids decide
+    (gi, gd) = knn_exact(q, v, k, metric)
+    for s in range(0, nq, 32):
+        (fi, fd) = knn_exact(q[s:s + 32].contiguous(), v, k, metric)
+        assert torch.equal(gi[s:s + 32], fi) and torch.equal(gd[s:s + 32], fd)
+    assert int(gi[nq - 1, 0]) == n // 3
+
+
+@pytest.mark.parametrize("bad", ["equal rows", "an infinite row"])
+def test_what_the_filter_leaves_to_the_tiles(bad):
+    """More rows within the rounding of each other than a query's buffer holds, or no bound at all."""
+    print(f"filter with {bad}", flush=True)
+    from vectorlink_gpu.kernels import knn_exact
+
+    rng = np.random.default_rng(8)
+    v = rows(rng, 9000, 32)
+    if bad == "equal rows":
+        v[:5000] = v[0]
+    q = rows(rng, 300, 32)
+    q[:200] = v[0] + 0.01 * q[:200]
+    gv = dev(v)
+    if bad != "equal rows":
+        gv[4321, 5] = float("inf")
+    gq = dev(q)
+    (gi, gd) = knn_exact(gq, gv, 10)
+    for s in range(0, 300, 32):
+        (fi, fd) = knn_exact(gq[s:s + 32].contiguous(), gv, 10)
+        assert torch.equal(gi[s:s + 32], fi) and torch.equal(gd[s:s + 32], fd)
+    if bad == "equal rows":
+        assert np.array_equal(gi[:200].cpu().numpy(), np.tile(np.arange(10, dtype=np.int32), (200, 1)))

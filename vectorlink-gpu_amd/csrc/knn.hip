@@ -3,6 +3,9 @@
 // vectorlink_gpu/ann.py:235-259); this is the ground truth for recall@k and the
 // only contraction-shaped step of the path.
 //
+// Small batches go to knn_few.hip and most others through knn_filter.hip; this file holds the float32 tiles, which take
+// tables of fewer than 4,096 rows and what the filter cannot decide.  All three give the same bits.
+//
 // One workgroup (4 wavefronts, 2 x 2) owns 128 queries and a strip of the
 // vector set; operand tiles go from global memory straight into LDS
 // (global_load_lds, double-buffered: the next stage lands while this one is
@@ -14,6 +17,7 @@
 // kernel merges the per-lane lists of a query in LDS.
 #include "knn_device.h"
 #include "knn_few.h"
+#include "knn_filter.h"
 
 #include <type_traits>
 
@@ -70,7 +74,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                                       int dim, int64_t strip_len, int n_strips,
                                                       int n_qblocks, int q_group, uint64_t *__restrict__ cand,
                                                       const float *__restrict__ q_norm,
-                                                      const float *__restrict__ v_norm, uint32_t *__restrict__ q_bound) {
+                                                      const float *__restrict__ v_norm, uint32_t *__restrict__ q_bound,
+                                                      const int32_t *__restrict__ wanted) {
     // two buffers per operand as separate arrays: the compiler can then tell that the loads
     // landing in one buffer do not touch the one being read
     __shared__ __align__(16) float sV0[TILE];
@@ -106,6 +111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             q_block = (n_qblocks / q_group) * q_group + (int)(w - (int64_t)strip * rest);
         }
     }
+    if (wanted && wanted[q_block] == 0) return;  // (uniform over the workgroup) answered by the filter
     const int64_t q0 = (int64_t)q_block * TQ;
     const int64_t v_begin = strip * strip_len;
     const int64_t v_end = min(n_vectors, v_begin + strip_len);
@@ -332,9 +338,9 @@ constexpr int kSelectLists = 4;  // lists per lane: 64 strips x 4 lists at most
 
 __global__ __launch_bounds__(256) void knn_select_kernel(const uint64_t *__restrict__ cand, int n_lists, int KK, int k,
                                                          int32_t *__restrict__ ids_out, float *__restrict__ d_out,
-                                                         int64_t n_queries) {
+                                                         int64_t n_queries, const int32_t *__restrict__ wanted) {
     const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (q >= n_queries) return;  // the whole wavefront leaves
+    if (q >= n_queries || (wanted && wanted[q / TQ] == 0)) return;  // the whole wavefront leaves
     const int lane = threadIdx.x & 63;
     const uint64_t *base = cand + q * n_lists * KK;
     uint64_t head[kSelectLists], next[kSelectLists];
@@ -388,13 +394,17 @@ struct KnnPlan {
     int list_len;
     int n_strips;
     int64_t strip_len;
-    bool few;  // the kernel of knn_few.hip takes the call (see vl_knn_exact_metric)
+    bool few;     // the kernel of knn_few.hip takes the call (see vl_knn_exact_metric)
+    bool filter;  // the filter of knn_filter.hip takes it, and the tiles what it leaves
+    KnnFilterPlan fp;
+    int64_t off_flags, off_filter;
     int n_cand;
     int64_t cand_bytes;  // per-lane candidate lists; the queries' shared bounds and the rows' squared lengths (L2) follow
     int64_t bytes;
 };
 
-int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, KnnPlan *p) {
+// l2: the plan of an L2 call; its workspace is never smaller than a cosine call's.
+int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, KnnPlan *p) {
     VL_REQUIRE(n_queries >= 0 && n_vectors > 0 && dim > 0, "bad sizes");
     VL_REQUIRE(k >= 1 && k <= KMAX, "k must be between 1 and %d", KMAX);
     VL_REQUIRE(dim % 4 == 0, "exact kNN tiles need a dimension that is a multiple of 4");
@@ -423,10 +433,16 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, KnnPl
     p->strip_len = len;
     p->list_len = list_length(k);
     p->n_cand = (int)(strips * LISTS_PER_STRIP * p->list_len);
-    p->few = n_queries <= kFewQueries;
+    p->few = vl_knn_is_few(n_queries, n_vectors, dim);
     if (p->few) p->n_cand = (int)(vl_knn_few_lists(n_vectors) * p->list_len);
     p->cand_bytes = (n_queries > 0 ? n_queries : 1) * (int64_t)p->n_cand * 8;
     p->bytes = p->cand_bytes + ((2 * n_queries + n_vectors) * 4 + 15) / 16 * 16;
+    p->filter = !p->few && vl_knn_filter_plan(n_queries, n_vectors, dim, k, l2, &p->fp);
+    if (p->filter) {
+        p->off_flags = (p->bytes + 255) / 256 * 256;
+        p->off_filter = (p->off_flags + q_blocks * 4 + 255) / 256 * 256;
+        p->bytes = p->off_filter + p->fp.bytes + 256;  // (the workspace itself may be 16-byte aligned only)
+    }
     return VL_OK;
 }
 
@@ -434,7 +450,7 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, KnnPl
 
 VL_EXPORT int64_t vl_knn_workspace_bytes(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k) {
     KnnPlan p;
-    int rc = knn_plan(n_queries, n_vectors, dim, k, &p);
+    int rc = knn_plan(n_queries, n_vectors, dim, k, true, &p);  // serves both metrics
     return rc < 0 ? rc : p.bytes;
 }
 
@@ -450,7 +466,8 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
                                   float *dists_out, void *workspace, int64_t workspace_bytes, void *stream) {
     VL_REQUIRE(metric == VL_METRIC_COSINE || metric == VL_METRIC_L2, "unknown metric %d", (int)metric);
     KnnPlan p;
-    int rc = knn_plan(n_queries, n_vectors, dim, k, &p);
+    const bool l2 = metric == VL_METRIC_L2;
+    int rc = knn_plan(n_queries, n_vectors, dim, k, l2, &p);
     if (rc < 0) return rc;
     if (n_queries == 0) return VL_OK;
     VL_REQUIRE(queries && vectors && ids_out && dists_out && workspace, "null pointer");
@@ -469,11 +486,21 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     q_group = q_group < 1 ? 1 : (q_group > 8 ? 8 : q_group);
     const int64_t blocks = (q_blocks * p.n_strips + 7) / 8 * 8;
     VL_REQUIRE(blocks <= kMaxBlocks * 4, "too many tiles for one call");
-    const bool l2 = metric == VL_METRIC_L2;
     uint32_t *q_bound = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(workspace) + p.cand_bytes);
     float *q_norm = reinterpret_cast<float *>(q_bound + n_queries);
     float *v_norm = q_norm + n_queries;
-    if (l2) {
+    // A batch goes to the kernel for a few queries (knn_few.h says where the line lies), else through the bfloat16 filter,
+    // which leaves the query blocks it cannot answer to the float32 tiles below; a table below 4,096 rows to the tiles.
+    const int32_t *wanted = nullptr;
+    char *const ws = (char *)workspace;
+    if (p.filter) {
+        int32_t *flags = (int32_t *)(ws + p.off_flags);
+        char *const filter_ws = (char *)(((uintptr_t)(ws + p.off_filter) + 255) / 256 * 256);
+        rc = vl_knn_filter(p.fp, queries, n_queries, vectors, n_vectors, dim, k, l2, q_norm, v_norm, flags, TQ,
+                           filter_ws, ids_out, dists_out, st);
+        if (rc < 0) return rc;
+        wanted = flags;
+    } else if (l2) {
         VL_REQUIRE((n_vectors + 3) / 4 <= kMaxBlocks * 4, "too many vectors for one call");
         hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, queries,
                            n_queries, (int)dim, q_norm);
@@ -491,11 +518,11 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
         if (l2)                                                                                               \
             hipLaunchKernelGGL((knn_tile_kernel<KK, true>), dim3((unsigned)blocks), dim3(256), 0, st, queries, \
                                n_queries, vectors, n_vectors, (int)dim, p.strip_len, p.n_strips, (int)q_blocks, \
-                               (int)q_group, cand, q_norm, v_norm, q_bound);                                  \
+                               (int)q_group, cand, q_norm, v_norm, q_bound, wanted);                          \
         else                                                                                                  \
             hipLaunchKernelGGL((knn_tile_kernel<KK, false>), dim3((unsigned)blocks), dim3(256), 0, st, queries, \
                                n_queries, vectors, n_vectors, (int)dim, p.strip_len, p.n_strips, (int)q_blocks, \
-                               (int)q_group, cand, nullptr, nullptr, q_bound);                                \
+                               (int)q_group, cand, nullptr, nullptr, q_bound, wanted);                        \
     } while (0)
     switch (p.list_len) {
         case 1: VL_KNN_LAUNCH(1); break;
@@ -510,7 +537,7 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     const int n_lists = p.n_strips * LISTS_PER_STRIP;
     VL_REQUIRE(n_lists <= 64 * kSelectLists, "too many candidate lists per query");
     hipLaunchKernelGGL(knn_select_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, cand, n_lists,
-                       p.list_len, (int)k, ids_out, dists_out, n_queries);
+                       p.list_len, (int)k, ids_out, dists_out, n_queries, wanted);
     VL_LAUNCH_CHECK("knn_select_kernel");
     return VL_OK;
 }

@@ -234,7 +234,7 @@ int64_t vl_knn_few_lists(int64_t n_vectors) { return 2 * (int64_t)few_waves(n_ve
 int vl_knn_few(const float *queries, int64_t n_queries, const float *vectors, int64_t n_vectors, int64_t dim, int64_t k,
                int list_len, bool l2, const float *q_norm, const float *v_norm, uint64_t *cand, int32_t *ids_out,
                float *dists_out, hipStream_t st) {
-    VL_REQUIRE(n_queries >= 1 && n_queries <= kFewQueries, "too many queries for the few-query kernel");
+    VL_REQUIRE(vl_knn_is_few(n_queries, n_vectors, dim), "too many queries for the few-query kernel");
     const int waves = few_waves(n_vectors);
     const dim3 grid((unsigned)((n_queries + 31) / 32), (unsigned)((waves + 3) / 4));
 #define VL_FEW_LAUNCH(KERNEL)                                                                                        \
