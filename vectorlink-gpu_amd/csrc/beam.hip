@@ -17,10 +17,7 @@
 // the host only reads the changed flag every speculative_readahead
 // iterations, the cadence at which the reference tests for progress
 // (ann.py:68,90-91).
-#include "beam_ctrl.h"
-#include "rowsort.h"
-#include "dist_device.h"
-#include "sketch_device.h"
+#include "beam_row.h"
 #include <stddef.h>
 #include <stdlib.h>
 #include <atomic>
@@ -36,8 +33,6 @@ int vl_launch_expand(const float *queries, int64_t n_rows, const float *vectors,
 int vl_launch_sketch_queries(const float *queries, int64_t n_rows, int64_t dim, uint8_t *out_rows, hipStream_t st);
 
 namespace {
-
-constexpr int kMaxVisit = 64;  // parallel_visit_count handled by one wavefront
 
 // Optional per-kernel timing of the loop (off by default): HIP events around
 // every expand and merge launch on the caller's stream, summed per call.
@@ -125,28 +120,6 @@ int wait_for_report(const BeamReport *r, int t, hipStream_t st) {
         __builtin_ia32_pause();
     }
 }
-
-struct MergeArgs {
-    BeamCtrl *ctrl;
-    int iter;
-    int readahead;
-    int64_t n_rows;
-    const int32_t *cand_ids;
-    const float *cand_d;
-    int m;
-    int32_t *q_ids;
-    float *q_d;
-    int cap, L, Ps;
-    const int32_t *excl;
-    int excl_cols;
-    int32_t *v_ids;
-    float *v_d;
-    int VL, Vt, Pv, Pc;
-    int32_t *seen;
-    int32_t *seen_count;
-    int E;
-    int32_t *row_quiet;  // per-query stop only (else null): iterations in a row that left the row's search queue unchanged
-};
 
 __device__ inline bool sorted_contains(const int32_t *a, int n, int32_t v) {
     int lo = 0, hi = n;
@@ -397,19 +370,6 @@ __device__ inline int block_compact(const uint64_t *src, int n, uint64_t *dst, P
     return run;
 }
 
-// Raise the batch-wide running maximum *slot to at least cnt.  Same-address
-// atomics from thousands of workgroups serialise in L2 and were the most
-// expensive part of the merge step, so they are kept for the rare case only:
-// a row that is at the largest fill any row can have (bound) publishes it with
-// a plain store - every such writer stores the same value and no atomicMax of a
-// smaller value can lower it - and any row skips the update when a late read
-// shows the slot is already there.
-__device__ inline void raise_running_max(int *slot, int cnt, int bound) {
-    if (__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= cnt) return;
-    if (cnt >= bound) __hip_atomic_store(slot, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else atomicMax(slot, cnt);
-}
-
 // Smallest value over the workgroup of each thread's `mine` (0xFFFFFFFF = none).
 // red: 2 * kQueueWaves words of LDS, used alternately so one barrier per call suffices.
 __device__ inline uint32_t block_min_u32(uint32_t mine, uint32_t *red, int round) {
@@ -425,79 +385,24 @@ __device__ inline uint32_t block_min_u32(uint32_t mine, uint32_t *red, int round
     return m;
 }
 
-// A candidate's upper bound (a cosine distance, in [0, 1]) and its slot in one 32-bit key, smallest bound first:
-// the bound to 19 bits, rounded down, then the slot (a row has at most kMaxCandidates candidate slots: more would
-// not fit the LDS).  Only used to choose which candidates to look at first - any choice is a valid one there - so
-// the rounding costs nothing but a slightly different pick among near-equal bounds.  Never 0xFFFFFFFF.
-constexpr int kMaxCandidates = 8192;
-__device__ __forceinline__ uint32_t bound_slot_key(float hi, int slot) {
-    return ((uint32_t)(hi * 524286.0f) << 13) | (uint32_t)slot;
-}
-
-// Workgroup-wide scalars shared by the expand and merge phases of a row.
-__shared__ int g_n_ex_s;                  // exclusion ids before the row's first empty one
-__shared__ int32_t g_visit_s[kMaxVisit];  // the ids popped from the visit queue in this iteration
-// The ids the merge phase adds to the visited list (between two of its barriers).  The expand phase and the exact
-// rounds of a sketched row, which run before and after that, use the same 256 bytes as the wavefronts' lists of
-// candidate lanes (wave_sketch, wave_distances_lds: 64 bytes each) - sixteen 128-thread workgroups of the
-// 128-column shape fit a compute unit's LDS with these bytes shared and fifteen without.
-__shared__ int32_t g_new_s[kMaxVisit];
-static_assert(kMaxVisit * 4 >= 256, "one byte per thread of the largest workgroup");
-
-// What the fused step has read of a row before its merge phase starts.
-struct RowState {
-    int cnt;    // fill of the row's visited list
-    int first;  // first visited-list column that is free in every row
-};
-
-// FUSED: the candidates of this row are already in LDS (ids at uk, distances behind them,
-// written by the expand phase of the same workgroup), the loop state has been checked, and
-// the row's queues, visited list, popped ids and exclusions have been placed in LDS by
-// stage_row (the global reads were issued at the start of the kernel).
-// refine (fused step only): called once the visited list is current and before the candidates are
-// looked at, with the last slots of both queues; it may replace candidate distances that are only known
-// as bounds by exact ones and drop candidates that provably cannot enter a queue.
-struct NoRefine {
-    __device__ __forceinline__ void operator()(const int32_t *, int, bool, uint64_t, uint64_t, uint8_t *, uint64_t *) const {}
-};
-
-// RESIDENT (a workgroup that takes its row through several iterations, beam_window_body): the row's queues and
-// visited list stay in LDS between iterations.  The merge phase reads them where this says and writes the merged
-// queues to the *_out arrays instead of memory; nothing of the row goes to memory here.
-struct ResidentRow {
-    uint64_t *qa, *qa_out;    // search queue [0, L) as keys
-    uint64_t *va, *va_out;    // visit queue, all VL slots (the popped heads first)
-    int32_t *seen_a, *seen_b; // visited list before / after this iteration
-    int32_t *exl;
-    uint8_t *fl;
-    int *quiet;               // per-query stop: the row's count of quiet iterations
-};
-struct MergeResult {
-    int cnt;           // fill of the visited list after this iteration
-    bool queue_moved;  // RESIDENT: the search queue was written to qa_out (else it is unchanged in qa)
-};
-
-// PREFILTERED: the caller has already dropped every candidate that the updated visited list holds.
-template <int THREADS, bool FUSED, class Refine = NoRefine, bool RESIDENT = false, bool PREFILTERED = false>
-__device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned char *smem, RowState pre = RowState{0, 0},
-                                                 Refine refine = Refine(), const ResidentRow *rr = nullptr) {
-    static_assert(FUSED || !RESIDENT, "a resident row is a fused one");
+// The two-launch form's merge of one row; the candidates come from the expand kernel through memory.
+template <int THREADS>
+__device__ __forceinline__ void merge_row(const MergeArgs &a, unsigned char *smem) {
     const int Pc = a.Pc;
     uint64_t *raw = reinterpret_cast<uint64_t *>(smem);  // candidate keys as they arrive
     uint64_t *uk = raw + Pc;                             // the candidates that can matter, then sorted
     uint64_t *cc = raw;                                  // filtered for one merge (raw is no longer needed by then)
-    uint64_t *qa = RESIDENT ? rr->qa : uk + Pc;          // search queue [0, L)
-    uint64_t *va = RESIDENT ? rr->va + a.Vt : qa + a.L;  // visit queue [Vt, VL)
-    int32_t *seen_a = RESIDENT ? rr->seen_a : reinterpret_cast<int32_t *>(va + a.VL);
-    int32_t *seen_b = RESIDENT ? rr->seen_b : seen_a + a.E;
-    int32_t *exl = RESIDENT ? rr->exl : seen_b + a.E;
-    uint8_t *fl = RESIDENT ? rr->fl : reinterpret_cast<uint8_t *>(exl + a.excl_cols);  // per candidate: bit0 wanted, bit1 rest
+    uint64_t *qa = uk + Pc;                              // search queue [0, L)
+    uint64_t *va = qa + a.L;                             // visit queue [Vt, VL)
+    int32_t *seen_a = reinterpret_cast<int32_t *>(va + a.VL);
+    int32_t *seen_b = seen_a + a.E;
+    int32_t *exl = seen_b + a.E;
+    uint8_t *fl = reinterpret_cast<uint8_t *>(exl + a.excl_cols);  // per candidate: bit0 wanted, bit1 rest
     __shared__ int wave_cnt[kQueueWaves];
     __shared__ uint64_t red[2 * kQueueWaves];
-    int32_t *const newv = g_new_s;
+    __shared__ int32_t newv[kMaxVisit];  // the ids the merge adds to the visited list
+    __shared__ int n_ex_s;               // exclusion ids before the row's first empty one
     __shared__ int n_new_s;
-    __shared__ int row_changed_s;  // per-query stop: some slot of the search queue's first L changed
-    int &n_ex_s = g_n_ex_s;
 
     BeamCtrl *c = a.ctrl;
     const int t = a.iter;
@@ -512,19 +417,13 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
     const int nva = a.VL - a.Vt;
     int *first_next = &c->first[(t + 1) % 3];
 
-    const int stop = FUSED ? 0 : c->stop;
-    const int first_prev = FUSED ? 0 : c->first[(t - 1) % 3];
-    const int first = FUSED ? pre.first : c->first[t % 3];
-    int cnt = FUSED ? pre.cnt : a.seen_count[row];
+    const int stop = c->stop;
+    const int first_prev = c->first[(t - 1) % 3];
+    const int first = c->first[t % 3];
+    int cnt = a.seen_count[row];
     // the ids popped at the start of this iteration (queue.py:87-95), before the row is rewritten
     int32_t popped = VL_MAXINT;
-    if constexpr (FUSED) {
-        if (threadIdx.x < kWave && (int)threadIdx.x < a.Vt) popped = g_visit_s[threadIdx.x];
-        if (threadIdx.x == 0) {
-            n_new_s = 0;
-            row_changed_s = 0;
-        }
-    } else {
+    {
         // the visited list's fill is at most Vt ids per earlier iteration, so the row can be
         // fetched without first waiting for the exact count
         const int seen_bound = min(a.E, a.Vt * (t - 1));
@@ -539,7 +438,6 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
         if (threadIdx.x == 0) {
             n_ex_s = a.excl ? a.excl_cols : 0;
             n_new_s = 0;
-            row_changed_s = 0;
         }
         __syncthreads();
         if (a.excl) {
@@ -551,14 +449,12 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
             }
         }
     }
-    if (stop) return MergeResult{cnt, false};
-    if constexpr (!FUSED) {
-        if (!beam_row_state_ok(c, cnt, min(a.E, a.Vt * (t - 1)), threadIdx.x == 0)) return MergeResult{0, false};
-    }
-    if (!FUSED && t >= 2 && first_prev >= a.E) {
+    if (stop) return;
+    if (!beam_row_state_ok(c, cnt, min(a.E, a.Vt * (t - 1)), threadIdx.x == 0)) return;
+    if (t >= 2 && first_prev >= a.E) {
         // the visit queue is no longer fed: every candidate of this iteration is empty
         if (threadIdx.x == 0) raise_running_max(first_next, cnt, min(a.E, a.Vt * t));
-        return MergeResult{cnt, false};
+        return;
     }
     const bool seen_full = first >= a.E;
     const bool checking = (t % a.readahead) == 0;
@@ -597,24 +493,13 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
             seen_b[lower_bound(seen_a, cnt, newv[threadIdx.x]) + threadIdx.x] = newv[threadIdx.x];
         __syncthreads();
         cnt += n_new;
-        if constexpr (!RESIDENT) {
-            if (n_new) {
-                int32_t *srow = a.seen + row * a.E;
-                for (int i = threadIdx.x; i < cnt; i += blockDim.x) srow[i] = seen_b[i];
-            }
-            if (threadIdx.x == 0 && n_new) a.seen_count[row] = cnt;
+        if (n_new) {
+            int32_t *srow = a.seen + row * a.E;
+            for (int i = threadIdx.x; i < cnt; i += blockDim.x) srow[i] = seen_b[i];
         }
+        if (threadIdx.x == 0 && n_new) a.seen_count[row] = cnt;
     }
-    if constexpr (!RESIDENT) {
-        if (threadIdx.x == 0) raise_running_max(first_next, cnt, min(a.E, a.Vt * t));
-    }
-    if constexpr (FUSED) {
-        refine(seen_b, cnt, seen_full, qa[a.L - 1], nva > 0 ? va[nva - 1] : 0ull, fl, red);
-        // a thread packs the slots it (or a lane of its own wavefront, before the barrier above or in refine) wrote
-        const int32_t *li = reinterpret_cast<const int32_t *>(uk);
-        const float *ld = reinterpret_cast<const float *>(li + a.m);
-        for (int i = threadIdx.x; i < a.m; i += blockDim.x) raw[i] = vl_make_key(li[i], ld[i]);
-    }
+    if (threadIdx.x == 0) raise_running_max(first_next, cnt, min(a.E, a.Vt * t));
 
     // ---- which candidates can matter at all -------------------------------------------
     // search queue: only keys below its last slot can enter.  visit queue (VL slots, Vt of
@@ -632,7 +517,7 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
         if (id != VL_MAXINT) {
             if (k < ws) f |= 1;
             if (!seen_full && k != wv) {  // k == wv is the visit queue's own last slot again
-                bool unseen = PREFILTERED || !sorted_contains(seen_b, cnt, id);
+                bool unseen = !sorted_contains(seen_b, cnt, id);
                 if (unseen) f |= (k < wv) ? 1 : 2;
             }
         }
@@ -688,9 +573,7 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
         for (int i = threadIdx.x; i < a.L; i += blockDim.x) {
             uint64_t k = qa[i];
             int r = i + key_lower_bound(cc, n_s, k);
-            if constexpr (RESIDENT) {
-                if (r < a.L) rr->qa_out[r] = k;
-            } else if (r != i && r < a.L) {
+            if (r != i && r < a.L) {
                 qi[r] = vl_key_id(k);
                 qd[r] = vl_key_dist(k);
             }
@@ -699,37 +582,18 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
             uint64_t k = cc[j];
             int r = j + key_lower_bound(qa, a.L, k);
             if (r < a.L) {
-                if constexpr (RESIDENT) {
-                    rr->qa_out[r] = k;
-                } else {
-                    qi[r] = vl_key_id(k);
-                    qd[r] = vl_key_dist(k);
-                }
+                qi[r] = vl_key_id(k);
+                qd[r] = vl_key_dist(k);
                 diff = true;  // a new id inside the first L slots: the row changed (queue.py:57-59)
             }
         }
     }
     int *flag = &c->changed[(t / a.readahead) & 63];  // every writer stores the same 1: no atomic needed
-    if (a.row_quiet) {
-        // Per-query stop: a row is finished after `readahead` iterations in a row that left its first L
-        // slots as they were, or when the visited list has no free column (no pop yields a real id from
-        // then on); a row that is not finished at a checking iteration keeps the loop going.
-        if (diff) row_changed_s = 1;  // every writer stores the same 1
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            int quiet = row_changed_s ? 0 : (RESIDENT ? *rr->quiet : a.row_quiet[row]) + 1;
-            if (seen_full) quiet = a.readahead;
-            if constexpr (RESIDENT) *rr->quiet = quiet;
-            else a.row_quiet[row] = quiet;
-            if (checking && quiet < a.readahead &&
-                __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-                __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    } else if (checking && __ballot(diff) && lane == 0) {
+    if (checking && __ballot(diff) && lane == 0) {
         if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
             __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (seen_full) return MergeResult{cnt, n_s > 0};
+    if (seen_full) return;
     __syncthreads();  // cc is reused below
 
     // ---- visit_queue.insert(candidates, exclude=seen) : ann.py:85-88 --------------------
@@ -737,7 +601,7 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
         uint64_t k = uk[i];
         int32_t id = vl_key_id(k);
         if (i > 0 && id == vl_key_id(uk[i - 1])) return false;
-        if (!PREFILTERED && sorted_contains(seen_b, cnt, id)) return false;      // kernels.py:471-488
+        if (sorted_contains(seen_b, cnt, id)) return false;                      // kernels.py:471-488
         int p = key_lower_bound(va, nva, k);
         return !(p < nva && va[p] == k);
     };
@@ -746,469 +610,38 @@ __device__ __forceinline__ MergeResult merge_row(const MergeArgs &a, unsigned ch
         uint64_t k = va[i];
         int r = i + key_lower_bound(cc, n_v, k);
         if (r < a.VL) {
-            if constexpr (RESIDENT) {
-                rr->va_out[r] = k;
-            } else {
-                vi[r] = vl_key_id(k);
-                vd[r] = vl_key_dist(k);
-            }
+            vi[r] = vl_key_id(k);
+            vd[r] = vl_key_dist(k);
         }
     }
     for (int j = threadIdx.x; j < n_v; j += blockDim.x) {
         uint64_t k = cc[j];
         int r = j + key_lower_bound(va, nva, k);
         if (r < a.VL) {
-            if constexpr (RESIDENT) {
-                rr->va_out[r] = k;
-            } else {
-                vi[r] = vl_key_id(k);
-                vd[r] = vl_key_dist(k);
-            }
+            vi[r] = vl_key_id(k);
+            vd[r] = vl_key_dist(k);
         }
     }
     for (int r = nva + n_v + threadIdx.x; r < a.VL; r += blockDim.x) {  // the popped slots end up here, empty
-        if constexpr (RESIDENT) {
-            rr->va_out[r] = vl_make_key(VL_MAXINT, VL_MAXFLOAT);
-        } else {
-            vi[r] = VL_MAXINT;
-            vd[r] = VL_MAXFLOAT;
-        }
+        vi[r] = VL_MAXINT;
+        vd[r] = VL_MAXFLOAT;
     }
-    return MergeResult{cnt, n_s > 0};
 }
 
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void beam_merge2_kernel(MergeArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
-    merge_row<THREADS, false>(a, smem);
+    merge_row<THREADS>(a, smem);
 }
 
-// ---- one launch per iteration -------------------------------------------------
-// The expand phase (HBM bound) and the merge phase (LDS / latency bound) of one
+// ---- the fused step: one launch per iteration, or per window of iterations ------
+// The expand phase (memory bound) and the merge phase (LDS / latency bound) of one
 // row run in the same workgroup, so on every CU some workgroups stream candidate
 // rows while others merge: the merge time hides behind the memory traffic, the
 // candidate ids and distances never leave LDS, and an iteration is one launch.
-struct StepArgs {
-    MergeArgs m;
-    const float *queries;
-    const float *vectors;
-    const int32_t *beams;
-    int64_t n_vectors;
-    int dim, nchunks, width;
-    uint32_t width_magic;  // floor(2^32 / width) + 1: slot / width == umulhi(slot, width_magic) for slot * width < 2^32
-    uint64_t *memo;
-    int memo_shift;
-    int32_t *memo_rate;   // per row: share (x 256) of the candidates of iteration kMemoDecide that were cached; bit 16: the row uses the sketch
-    int memo_min_rate;    // the cache stays in use only if that share is at least this (x 256)
-    int count_evals;
-    int l2;  // 0: cosine distance, 1: squared L2
-    const uint8_t *sketch;     // 8-bit sketch of `vectors` (sketch_device.h), or null
-    const uint8_t *sketch_tails;  // the table's second part: 8 bytes per vector
-    int sketch_chunks;         // 16-byte chunks of data in a sketch row
-    const uint8_t *rounded_queries;  // the call's query rows rounded for the sketch (sketch_device.h)
-    int64_t rounded_query_bytes;
-    int window;     // beam_window_kernel: iterations m.iter ... m.iter + window - 1 in this launch
-    int lds_slots;  // beam_window_kernel: entries of the row's distance table in LDS (a power of two, or 0)
-    BeamReport *report;  // pinned host memory that hears of the progress checks, or null
-};
-
-// A probe of the distance cache is a random 8-byte read and every evaluated distance a random 8-byte
-// write - a memory sector each, and one more round trip before the candidate rows can be asked for - so
-// the cache only pays when enough probes hit; how many depends on the row size (short rows are cheap to
-// fetch again).  Each row therefore decides for itself: it uses the cache during its first kMemoDecide - 1
-// iterations, measures the share of hits in iteration kMemoDecide, and leaves the cache alone for the rest
-// of the call if that share is below the break-even share.  A hit returns the bits that would be computed
-// again, so the decision never changes a result.
-constexpr int kMemoDecide = 9;
-
-// Elements of a row that one thread brings in at the start of the fused step and keeps in registers until
-// the workgroup's other reads have been issued: search queue, visit queue, visited list.  Longer rows load
-// their remainder the slow way (read, wait, store) - none of the benchmark shapes has one.
-constexpr int kPreQ = 2, kPreV = 2, kPreS = 4;
-
-// SCPL > 0: the kernel can look at candidates through the sketch first (SCPL chunks per lane, SLPR lanes
-// per sketch row, SU loads in flight).  A row that does so gets bounds for the candidates the distance cache
-// does not know from a quarter of the bytes, then exact distances for the few whose lower bound is not above
-// every threshold that decides what the merge phase keeps; it stops doing so when most of them turn out to
-// need their exact distance (bit 16 of its word in memo_rate: set at the start of the call, cleared then).
-template <int CPL, int LPR, int U, bool GENERIC, int THREADS, int SCPL = 0, int SLPR = 64, int SU = 1>
-__device__ __forceinline__ void beam_step_body(const StepArgs &s) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const MergeArgs &a = s.m;
-    BeamCtrl *c = a.ctrl;
-    const int t = a.iter;
-    const int tid = threadIdx.x;
-    const int64_t row = blockIdx.x;
-    // ---- every read that depends on nothing else goes out first: loop state, the row's counters, the ids
-    // to visit, both queues, the visited list, the exclusions.  A round trip to memory costs more than
-    // anything this workgroup computes, so the number of dependent round trips is what it pays for: this
-    // one, then the neighbour lists of the visited ids, the cache probes, the candidate rows.
-    int32_t *vi = a.v_ids + row * a.VL;
-    float *vd = a.v_d + row * a.VL;
-    const int32_t *qi = a.q_ids + row * a.cap;
-    const float *qd = a.q_d + row * a.cap;
-    const int32_t *srow = a.seen + row * a.E;
-    const int nva = a.VL - a.Vt;
-    const int seen_bound = min(a.E, a.Vt * (t - 1));  // the fill is at most Vt ids per earlier iteration
-    const int32_t my_visit = tid < a.Vt ? vi[tid] : VL_MAXINT;
-    RowState pre;
-    pre.cnt = a.seen_count[row];
-    pre.first = c->first[t % 3];
-    const int quiet = a.row_quiet ? a.row_quiet[row] : 0;
-    const int memo_word = s.memo_rate[row];
-    const int memo_rate = memo_word & 0xffff;
-    int32_t pq_i[kPreQ], pv_i[kPreV], ps[kPreS];
-    float pq_d[kPreQ], pv_d[kPreV];
-#pragma unroll
-    for (int j = 0; j < kPreQ; ++j) {
-        const int i = tid + j * THREADS;
-        pq_i[j] = i < a.L ? qi[i] : VL_MAXINT;
-        pq_d[j] = i < a.L ? qd[i] : VL_MAXFLOAT;
-    }
-#pragma unroll
-    for (int j = 0; j < kPreV; ++j) {
-        const int i = tid + j * THREADS;
-        pv_i[j] = i < nva ? vi[a.Vt + i] : VL_MAXINT;
-        pv_d[j] = i < nva ? vd[a.Vt + i] : VL_MAXFLOAT;
-    }
-#pragma unroll
-    for (int j = 0; j < kPreS; ++j) {
-        const int i = tid + j * THREADS;
-        ps[j] = i < seen_bound ? srow[i] : VL_MAXINT;
-    }
-    int32_t my_excl = VL_MAXINT;
-    if (a.excl && tid < a.excl_cols) my_excl = a.excl[row * a.excl_cols + tid];
-
-    const int gate = beam_gate(c, t, a.readahead, a.E, blockIdx.x == 0 && tid == 0, s.report);
-    if (gate == 2) return;
-    if (!beam_row_state_ok(c, pre.cnt, seen_bound, tid == 0)) return;
-    if (gate == 1 || (a.row_quiet && quiet >= a.readahead)) {
-        // the visit queue is no longer fed (every candidate of this iteration is empty), or this row has
-        // stopped on its own: nothing changes, only the running maximum is kept current
-        if (tid == 0) raise_running_max(&c->first[(t + 1) % 3], pre.cnt, min(a.E, a.Vt * t));
-        return;
-    }
-    uint64_t *raw = reinterpret_cast<uint64_t *>(smem);
-    uint64_t *uk = raw + a.Pc;
-    uint64_t *qa = uk + a.Pc;
-    uint64_t *va = qa + a.L;
-    int32_t *seen_a = reinterpret_cast<int32_t *>(va + a.VL);
-    int32_t *exl = seen_a + 2 * a.E;
-    int32_t *li = reinterpret_cast<int32_t *>(uk);
-    float *ld = reinterpret_cast<float *>(li + a.m);
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    const float *q_row = s.queries + row * s.dim;
-    uint64_t *memo_row = s.memo ? s.memo + ((uint64_t)row << (32 - s.memo_shift)) : nullptr;
-    __shared__ int probe_hits_s, probe_asked_s;
-    uint8_t *const lane_order_s = reinterpret_cast<uint8_t *>(g_new_s);  // 64 bytes per wavefront (see g_new_s)
-    const bool resample = memo_row && t == kMemoDecide;
-    if (memo_row && memo_rate < s.memo_min_rate) memo_row = nullptr;
-    bool sketching = false;
-    // (not in the first iteration: the visit queue starts with empty slots, so everything unvisited is kept and
-    // would be fetched anyway)
-    if constexpr (SCPL > 0) sketching = (memo_word >> 16) != 0 && t > 1;
-    const bool probing = memo_row != nullptr;
-    if (tid < a.Vt) g_visit_s[tid] = my_visit;
-    if (tid == 0) {
-        g_n_ex_s = a.excl ? a.excl_cols : 0;
-        probe_hits_s = 0;
-        probe_asked_s = 0;
-    }
-    // The neighbour lists of the nodes visited in one iteration share ids; only one copy of an id is evaluated.
-    // Every candidate claims its id in a hash set in LDS (the second copy of the visited list, which the merge
-    // phase fills only later: E slots, each the slot number of the claiming candidate; used when that leaves the
-    // set at most two thirds full); a candidate that finds its id claimed becomes the empty pair before anything
-    // is asked of memory for it.  The reference evaluates every copy (kernels.py:238-255) and drops all but one
-    // when the queues are sorted (kernels.py:314-349): copies carry the same distance, so what the queues receive
-    // is the same.
-    int32_t *const dset = seen_a + a.E;
-    const uint32_t dsize = (uint32_t)a.E;
-    const bool dedup = 2 * a.E >= 3 * a.m;
-    if (dedup)
-        for (int i = tid; i < a.E; i += THREADS) dset[i] = -1;
-    __syncthreads();
-
-    // ---- expand: ann.py:69-73 (pop the visit heads, gather their neighbour lists, distances) ----
-    // candidate id of slot c0 + lane: the neighbour list of a visited node
-    auto resolve = [&](int c0) -> int32_t {
-        const int slot = c0 + lane;
-        int32_t id = VL_MAXINT;
-        if (slot < a.m) {
-            int sidx = s.width == 1 ? slot : (int)__umulhi((uint32_t)slot, s.width_magic), k = slot - sidx * s.width;
-            int32_t node = g_visit_s[sidx];
-            if (node != VL_MAXINT && (uint32_t)node < (uint64_t)s.n_vectors) id = s.beams[(int64_t)node * s.width + k];
-        }
-        return id;
-    };
-    int32_t id = resolve(wave * kWave);
-    // The row's own state, read at the top, goes to LDS now that the first neighbour lists are on their
-    // way.  (Outside the loop below on purpose: inside it, its addresses would be kept in registers across
-    // the distance code.)
-    {
-#pragma unroll
-        for (int j = 0; j < kPreQ; ++j) {
-            const int i = tid + j * THREADS;
-            if (i < a.L) qa[i] = vl_make_key(pq_i[j], pq_d[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < kPreV; ++j) {
-            const int i = tid + j * THREADS;
-            if (i < nva) va[i] = vl_make_key(pv_i[j], pv_d[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < kPreS; ++j) {
-            const int i = tid + j * THREADS;
-            if (i < seen_bound) seen_a[i] = ps[j];
-        }
-        if (a.excl && tid < a.excl_cols) {
-            exl[tid] = my_excl;
-            if (my_excl == VL_MAXINT) atomicMin(&g_n_ex_s, tid);
-        }
-        for (int i = tid + kPreQ * THREADS; i < a.L; i += THREADS) qa[i] = vl_make_key(qi[i], qd[i]);
-        for (int i = tid + kPreV * THREADS; i < nva; i += THREADS) va[i] = vl_make_key(vi[a.Vt + i], vd[a.Vt + i]);
-        for (int i = tid + kPreS * THREADS; i < seen_bound; i += THREADS) seen_a[i] = srow[i];
-        for (int i = tid + THREADS; i < a.excl_cols; i += THREADS) {
-            int32_t e = a.excl[row * a.excl_cols + i];
-            exl[i] = e;
-            if (e == VL_MAXINT) atomicMin(&g_n_ex_s, i);
-        }
-    }
-    int n_wanted = 0, n_fetched = 0, n_sketched = 0;  // counts of this wavefront
-    float *le = reinterpret_cast<float *>(raw);                     // upper bounds (raw is filled in the merge phase)
-    uint8_t *xf = reinterpret_cast<uint8_t *>(exl + a.excl_cols);   // the merge phase's per-candidate flags; 16 = exact
-    // A candidate that the visited list holds once this iteration has updated it - an id visited earlier, or one
-    // popped now that the list still has room for (utils.py:73-75) - can change neither queue: the visit queue
-    // excludes it (ann.py:85-88), and the search queue met it with this very distance when it was first a candidate
-    // (every visited id came out of the visit queue, which is fed from the search queue's heads and then with the
-    // candidates the search queue is offered in the same iteration, ann.py:75-88), so it either still sits there
-    // or lies beyond its last slot, which only ever moves down.  Such candidates become the empty pair here,
-    // before a probe or a row is spent on them, and the merge phase knows the others to be unvisited.
-    const int n_popped_kept = pre.first >= a.E ? 0 : min(min(a.E - pre.first, a.Vt), a.E - pre.cnt);
-    __syncthreads();  // the visited list is in LDS
-    // first pass over this wavefront's candidates: ids to LDS, visited ids and later copies of an id out
-    for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-        if (c0 != wave * kWave) id = resolve(c0);
-        const int slot = c0 + lane;
-        const bool has = slot < a.m;
-        bool ok = has && id != VL_MAXINT && id >= 0 && (int64_t)id < s.n_vectors;
-        if (s.count_evals || resample) n_wanted += __popcll(__ballot(ok));
-        if (ok) {
-            bool visited = sorted_contains(seen_a, pre.cnt, id);
-            for (int j = 0; j < n_popped_kept; ++j) visited |= g_visit_s[j] == id;
-            ok = !visited;
-        }
-        if (has) li[slot] = ok ? id : VL_MAXINT;  // (before the claim: a candidate that meets this one in the set reads it)
-        if (ok && dedup) {
-            uint32_t h = __umulhi((uint32_t)id * 2654435761u, dsize);
-            for (;;) {
-                const int owner = atomicCAS(&dset[h], -1, slot);
-                if (owner == -1) break;     // first of its id
-                if (li[owner] == id) {      // a copy: only the first is evaluated
-                    ok = false;
-                    break;
-                }
-                h = h + 1 == dsize ? 0 : h + 1;
-            }
-            if (!ok) li[slot] = VL_MAXINT;
-        }
-        if (has && !ok) ld[slot] = VL_MAXFLOAT;
-    }
-    if constexpr (SCPL > 0) {
-        if (sketching) {
-            SketchQuery<SCPL> sq;
-            sketch_query_load<SCPL, SLPR>(sq, s.rounded_queries + row * s.rounded_query_bytes, s.sketch_chunks);
-            for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-                const int slot = c0 + lane;
-                const bool has = slot < a.m;
-                id = has ? li[slot] : VL_MAXINT;
-                bool ok = id != VL_MAXINT;
-                if (has) xf[slot] = 0;
-                // The cache serves two kinds of repeats: a candidate evaluated exactly before comes back with its
-                // distance, one that was only bounded comes back with its bounds (dist_device.h) - either way
-                // nothing is fetched for it now.
-                if (probing && ok) {
-                    const uint64_t e = memo_load(memo_row, s.memo_shift, id);
-                    if ((int32_t)((uint32_t)e & ~kMemoBounds) == id) {
-                        if ((uint32_t)e & kMemoBounds) {
-                            ld[slot] = memo_bound_lo(e);
-                            le[slot] = memo_bound_hi(e);
-                        } else {
-                            const float d = __builtin_bit_cast(float, (uint32_t)(e >> 32));
-                            ld[slot] = d;
-                            le[slot] = d;
-                            xf[slot] = 16;  // exact already
-                        }
-                        ok = false;
-                    }
-                }
-                if (s.count_evals || resample) n_sketched += __popcll(__ballot(ok));
-                wave_sketch<SCPL, SLPR, SU>(sq, s.sketch, s.sketch_tails, s.sketch_chunks, id, ok, ld + c0, le + c0,
-                                            lane_order_s + wave * kWave, memo_row, s.memo_shift);
-            }
-            n_fetched = n_sketched;  // for the share of cache hits: what the cache did not answer
-        }
-    }
-    for (int c0 = wave * kWave; c0 < a.m && !sketching; c0 += THREADS) {
-        const int slot = c0 + lane;
-        const bool has = slot < a.m;
-        id = has ? li[slot] : VL_MAXINT;
-        bool ok = id != VL_MAXINT;
-        if (probing && ok) {
-            uint64_t e = memo_load(memo_row, s.memo_shift, id);
-            if ((int32_t)(uint32_t)e == id) {
-                ld[slot] = __builtin_bit_cast(float, (uint32_t)(e >> 32));
-                ok = false;
-            }
-        }
-        if (s.count_evals || resample) n_fetched += __popcll(__ballot(ok));
-        if constexpr (GENERIC)
-            wave_distances_generic(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0, memo_row, s.memo_shift, s.l2 != 0);
-        else
-            wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0, lane_order_s + wave * kWave,
-                                            memo_row, s.memo_shift, s.l2 != 0);
-    }
-    if (s.count_evals && lane == 0) {
-        const int stripe = (int)((blockIdx.x * (THREADS / kWave) + wave) & (kBeamStripes - 1));
-        if (n_wanted) atomicAdd(&c->wanted[stripe], (unsigned long long)n_wanted);
-        if (n_fetched && !sketching) atomicAdd(&c->evals[stripe], (unsigned long long)n_fetched);
-        if (n_sketched) atomicAdd(&c->sketched[stripe], (unsigned long long)n_sketched);
-    }
-    if (resample && lane == 0) {
-        atomicAdd(&probe_asked_s, n_wanted);
-        atomicAdd(&probe_hits_s, n_wanted - n_fetched);
-    }
-    __syncthreads();
-    if (resample && tid == 0)
-        s.memo_rate[row] = (probe_asked_s > 0 ? (probe_hits_s * 256) / probe_asked_s : 256) | (memo_word & (1 << 16));
-    // ---- merge: ann.py:75-88 ----
-    if constexpr (SCPL > 0) {
-        // A sketched row knows every candidate distance only as lo <= d <= hi (ld holds lo, le holds hi).
-        // What the merge phase keeps of the candidates: keys below the search queue's last slot (ws),
-        // unvisited keys below the visit queue's last live slot (wv), and the Vt smallest distinct
-        // unvisited keys above wv.  Take any Vt distinct unvisited candidates that are certainly above wv
-        // (lo > wv) - those with the smallest hi, the likely winners - evaluate them, and let tv be the
-        // largest of their distances: Vt candidates are then known to be at most tv, so a candidate with
-        // lo > tv is not one of the Vt smallest.  Hence a candidate whose lo is above ws, and which is
-        // visited or has lo above both wv and tv, cannot enter either queue and is dropped; all others are
-        // evaluated exactly, by the same code and in the same order as an unsketched row's, in two rounds
-        // (the second one needs tv).  Comparisons are written so that a NaN bound counts as "evaluate".
-        auto refine = [&](const int32_t *seen_b, int cnt, bool seen_full, uint64_t ws, uint64_t wv, uint8_t *flags,
-                          uint64_t *red) {
-            if (!sketching) return;  // uniform over the workgroup
-            const float ws_d = vl_key_dist(ws);
-            const float wv_d = nva > 0 ? vl_key_dist(wv) : -1.0f;
-            for (int i = tid; i < a.m; i += THREADS) {
-                const int32_t cid = li[i];
-                uint8_t f = flags[i] & 16;  // set by the expand phase for a distance that came from the cache
-                if (cid != VL_MAXINT) {
-                    const float lo = ld[i];
-                    bool need = !(lo > ws_d);
-                    if (!seen_full) {  // (every candidate left is unvisited)
-                        if (!(lo > wv_d)) need = true;
-                        else f |= 2;  // unvisited and certainly above the visit queue's last live slot
-                    }
-                    if (need) f |= 4;
-                }
-                flags[i] = f;
-            }
-            // The Vt candidates of distinct ids with the smallest upper bounds among those certainly above wv
-            // (bit 8), found one block-wide minimum at a time; fewer than Vt of them: every one may be taken.
-            // Every copy of a chosen id is marked - copies may carry different bounds (one fresh from the sketch,
-            // one decoded from the cache) and must not count twice.
-            bool all_rest = false;
-            if (!seen_full) {
-                for (int r = 0; r < a.Vt; ++r) {
-                    uint32_t mine = 0xFFFFFFFFu;
-                    for (int i = tid; i < a.m; i += THREADS) {
-                        if ((flags[i] & (2 | 8)) != 2) continue;
-                        const uint32_t k = bound_slot_key(le[i], i);
-                        if (k < mine) mine = k;
-                    }
-                    const uint32_t mn = block_min_u32(mine, reinterpret_cast<uint32_t *>(red), r);
-                    if (mn == 0xFFFFFFFFu) {
-                        all_rest = true;
-                        break;
-                    }
-                    const int32_t chosen = li[mn & (kMaxCandidates - 1)];
-                    for (int i = tid; i < a.m; i += THREADS)
-                        if ((flags[i] & 2) && li[i] == chosen) flags[i] |= 8;
-                }
-            }
-            int n_exact = 0, n_real = 0;
-            // first round: everything below a queue's last slot, and those Vt candidates
-            for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-                const int slot = c0 + lane;
-                const bool has = slot < a.m;
-                const int32_t cid = has ? li[slot] : VL_MAXINT;
-                const uint8_t f = has ? flags[slot] : 0;
-                const bool ok = ((f & (4 | 8)) || (all_rest && (f & 2))) && !(f & 16);
-                if (ok) flags[slot] = f | 16;  // its distance is exact from here on
-                n_exact += __popcll(__ballot(ok));
-                n_real += __popcll(__ballot(cid != VL_MAXINT && !(f & 16)));  // candidates known by bounds only
-                wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, cid, ok, ld + c0,
-                                                lane_order_s + wave * kWave, memo_row, s.memo_shift, false);
-            }
-            __syncthreads();
-            // tv: the largest exact distance of those Vt candidates.  Vt distinct unvisited candidates above wv
-            // are at most tv, so a candidate whose lower bound is above tv is not one of the Vt smallest.
-            float tv = -1.0f;
-            if (!seen_full && !all_rest) {
-                uint32_t mine = 0xFFFFFFFFu;  // (no distance has the key 0)
-                for (int i = tid; i < a.m; i += THREADS)
-                    if (flags[i] & 8) {
-                        const uint32_t k = ~vl_float_key(ld[i]);
-                        mine = k < mine ? k : mine;
-                    }
-                const uint32_t mn = block_min_u32(mine, reinterpret_cast<uint32_t *>(red), a.Vt);
-                tv = mn == 0xFFFFFFFFu ? -1.0f : vl_key_float(~mn);
-            }
-            // second round: the candidates above wv that may still be among the Vt smallest
-            for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-                const int slot = c0 + lane;
-                const bool has = slot < a.m;
-                const int32_t cid = has ? li[slot] : VL_MAXINT;
-                const uint8_t f = has ? flags[slot] : 0;
-                const bool ok = (f & 2) && !(f & 16) && !(ld[slot] > tv);
-                if (has && cid != VL_MAXINT && !ok && !(f & 16)) {
-                    li[slot] = VL_MAXINT;
-                    ld[slot] = VL_MAXFLOAT;
-                }
-                n_exact += __popcll(__ballot(ok));
-                wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, cid, ok, ld + c0,
-                                                lane_order_s + wave * kWave, memo_row, s.memo_shift, false);
-            }
-            if (s.count_evals && lane == 0 && n_exact)
-                atomicAdd(&c->evals[(int)((blockIdx.x * (THREADS / kWave) + wave) & (kBeamStripes - 1))],
-                          (unsigned long long)n_exact);
-            // A row that has to evaluate more than half of the candidates it knew by bounds exactly after all
-            // (they lie within the sketch's error of the queues' last slots: real neighbour lists) gives the
-            // sketch up for the rest of the call.  The first iterations fill the visit queue and keep a lot, so
-            // until iteration kMemoDecide only a row that evaluates nearly all of them (7 in 8) does.
-            if (t > 2 && !resample) {  // (the iteration that measures the cache uses the same two counters)
-                if (lane == 0) {
-                    atomicAdd(&probe_asked_s, n_real);
-                    atomicAdd(&probe_hits_s, n_exact);
-                }
-                __syncthreads();
-                const bool quit = t > kMemoDecide ? 2 * probe_hits_s > probe_asked_s : 8 * probe_hits_s > 7 * probe_asked_s;
-                if (tid == 0 && quit) {
-                    s.memo_rate[row] = memo_rate;
-                    atomicAdd(&c->sketch_rows, -1);
-                }
-            } else {
-                __syncthreads();
-            }
-        };
-        merge_row<THREADS, true, decltype(refine), false, true>(a, smem, pre, refine);
-    } else {
-        merge_row<THREADS, true, NoRefine, false, true>(a, smem, pre);
-    }
-}
-
 template <int CPL, int LPR, int U, bool GENERIC, int THREADS>
 __global__ __launch_bounds__(THREADS) void beam_step_kernel(StepArgs s) {
-    beam_step_body<CPL, LPR, U, GENERIC, THREADS>(s);
+    beam_row<CPL, LPR, U, GENERIC, THREADS>(s);
 }
 // The same kernel built to leave room for WPP wavefronts per SIMD.  Its vector registers would allow that anyway;
 // what does not is its scalar registers (more than 96 of them mean seven wavefronts instead of eight), which the
@@ -1216,457 +649,15 @@ __global__ __launch_bounds__(THREADS) void beam_step_kernel(StepArgs s) {
 template <int CPL, int LPR, int U, int THREADS, int WPP>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPP)))
 void beam_step_kernel_w(StepArgs s) {
-    beam_step_body<CPL, LPR, U, false, THREADS>(s);
+    beam_row<CPL, LPR, U, false, THREADS>(s);
 }
-
-// ---- several iterations per launch ----------------------------------------------
-// While parallel_visit_count * t <= E (the visited list's width) no row's visited list can be full at
-// iteration t, so every row appends all the ids it pops (utils.py:73-75 with room for them in every row)
-// and nothing one row does in iterations t0 ... t0 + W - 1 depends on another row of the batch; the only
-// batch-wide facts, the progress flag of the checking iteration (ann.py:90-91) and the largest fill after
-// the last of them, are written once.  One workgroup then takes its row through W = speculative_readahead
-// iterations in one launch: search queue, visit queue and visited list are read once, stay in LDS (the merge
-// phase writes the merged rows to a second set of arrays, which becomes the current one) and go back to
-// memory once.  A small direct-mapped table in LDS keeps the (id, distance) or (id, bounds) entries the
-// row met in these iterations, so a repeat inside the window costs an LDS read instead of a probe of the
-// cache in memory.  Same candidates, same order, same merge code as beam_step_body: the rows are
-// bit-identical.  The launch must start right after a progress check (t0 = k * readahead + 1, W = readahead).
-template <int CPL, int LPR, int U, int THREADS, int SCPL = 0, int SLPR = 64, int SU = 1>
-__device__ __forceinline__ void beam_window_body(const StepArgs &s) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    MergeArgs a = s.m;
-    BeamCtrl *c = a.ctrl;
-    const int t0 = a.iter, W = s.window;
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    const int64_t row = blockIdx.x;
-    int32_t *vi = a.v_ids + row * a.VL;
-    float *vd = a.v_d + row * a.VL;
-    int32_t *qi = a.q_ids + row * a.cap;
-    float *qd = a.q_d + row * a.cap;
-    int32_t *srow = a.seen + row * a.E;
-    const int nva = a.VL - a.Vt;
-    const int seen_bound = min(a.E, a.Vt * (t0 - 1));  // the fill is at most Vt ids per earlier iteration
-    // ---- every read that depends on nothing else goes out first (as in beam_step_body)
-    const int32_t my_visit = tid < a.Vt ? vi[tid] : VL_MAXINT;
-    int cnt = a.seen_count[row];
-    const int quiet0 = a.row_quiet ? a.row_quiet[row] : 0;
-    const int memo_word0 = s.memo_rate[row];
-    int32_t pq_i[kPreQ], pv_i[kPreV], ps[kPreS];
-    float pq_d[kPreQ], pv_d[kPreV];
-#pragma unroll
-    for (int j = 0; j < kPreQ; ++j) {
-        const int i = tid + j * THREADS;
-        pq_i[j] = i < a.L ? qi[i] : VL_MAXINT;
-        pq_d[j] = i < a.L ? qd[i] : VL_MAXFLOAT;
-    }
-#pragma unroll
-    for (int j = 0; j < kPreV; ++j) {
-        const int i = tid + j * THREADS;
-        pv_i[j] = i < a.VL ? vi[i] : VL_MAXINT;
-        pv_d[j] = i < a.VL ? vd[i] : VL_MAXFLOAT;
-    }
-#pragma unroll
-    for (int j = 0; j < kPreS; ++j) {
-        const int i = tid + j * THREADS;
-        ps[j] = i < seen_bound ? srow[i] : VL_MAXINT;
-    }
-    int32_t my_excl = VL_MAXINT;
-    if (a.excl && tid < a.excl_cols) my_excl = a.excl[row * a.excl_cols + tid];
-
-    // (the visited lists cannot be full in these iterations; the slots of `first` are not read here, because rows
-    // of this very launch that finish early write the one the next launch reads)
-    const int gate = beam_gate(c, t0, a.readahead, a.E, blockIdx.x == 0 && tid == 0, s.report, false);
-    if (gate == 2) return;
-    if (!beam_row_state_ok(c, cnt, seen_bound, tid == 0)) return;
-    int *first_after = &c->first[(t0 + W) % 3];  // what the launch of iteration t0 + W reads
-    const int bound_after = min(a.E, a.Vt * (t0 + W - 1));
-    if (a.row_quiet && quiet0 >= a.readahead) {
-        // this row has stopped on its own: nothing changes, only the running maximum is kept current
-        if (tid == 0) raise_running_max(first_after, cnt, bound_after);
-        return;
-    }
-    const int Pc = a.Pc;
-    uint64_t *raw = reinterpret_cast<uint64_t *>(smem);
-    uint64_t *uk = raw + Pc;
-    // two copies of each queue and of the visited list, the second right behind the first
-    uint64_t *const q0 = uk + Pc;
-    uint64_t *const v0 = q0 + 2 * a.L;
-    auto qbuf = [&](int k) -> uint64_t * { return q0 + k * a.L; };
-    auto vbuf = [&](int k) -> uint64_t * { return v0 + k * a.VL; };
-    LdsMemo lds;
-    lds.tab = s.lds_slots > 0 ? v0 + 2 * a.VL : nullptr;
-    lds.shift = 32 - (31 - __builtin_clz(s.lds_slots > 0 ? s.lds_slots : 1));
-    int32_t *const s0 = reinterpret_cast<int32_t *>(v0 + 2 * a.VL + s.lds_slots);
-    auto sbuf = [&](int k) -> int32_t * { return s0 + k * a.E; };
-    int32_t *exl = s0 + 2 * a.E;
-    const float *const q_row0 = s.queries + row * s.dim;
-    const uint8_t *const rounded_row0 = s.rounded_queries + row * s.rounded_query_bytes;
-    uint64_t *const memo_table = s.memo ? s.memo + ((uint64_t)row << (32 - s.memo_shift)) : nullptr;
-    __shared__ int probe_hits_s, probe_asked_s, quiet_s, memo_word_s;
-    uint8_t *const lane_order_s = reinterpret_cast<uint8_t *>(g_new_s);  // 64 bytes per wavefront (see g_new_s)
-    int cur_q = 0, cur_v = 0, cur_s = 0;
-    bool queue_dirty = false;
-
-    // candidate id of slot c0 + lane: the neighbour list of a visited node
-    auto resolve = [&](int c0) -> int32_t {
-        const int slot = c0 + lane;
-        int32_t id = VL_MAXINT;
-        if (slot < a.m) {
-            int sidx = s.width == 1 ? slot : (int)__umulhi((uint32_t)slot, s.width_magic), k = slot - sidx * s.width;
-            int32_t node = g_visit_s[sidx];
-            if (node != VL_MAXINT && (uint32_t)node < (uint64_t)s.n_vectors) id = s.beams[(int64_t)node * s.width + k];
-        }
-        return id;
-    };
-    if (tid < a.Vt) g_visit_s[tid] = my_visit;
-    if (tid == 0) {
-        g_n_ex_s = a.excl ? a.excl_cols : 0;
-        quiet_s = quiet0;
-        memo_word_s = memo_word0;
-        probe_hits_s = 0;
-        probe_asked_s = 0;
-    }
-    __syncthreads();
-    int32_t id = resolve(wave * kWave);
-    {
-        // the row's state, read at the top, goes to LDS while the first neighbour lists are on their way
-#pragma unroll
-        for (int j = 0; j < kPreQ; ++j) {
-            const int i = tid + j * THREADS;
-            if (i < a.L) qbuf(0)[i] = vl_make_key(pq_i[j], pq_d[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < kPreV; ++j) {
-            const int i = tid + j * THREADS;
-            if (i < a.VL) vbuf(0)[i] = vl_make_key(pv_i[j], pv_d[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < kPreS; ++j) {
-            const int i = tid + j * THREADS;
-            if (i < seen_bound) sbuf(0)[i] = ps[j];
-        }
-        if (a.excl && tid < a.excl_cols) {
-            exl[tid] = my_excl;
-            if (my_excl == VL_MAXINT) atomicMin(&g_n_ex_s, tid);
-        }
-        for (int i = tid + kPreQ * THREADS; i < a.L; i += THREADS) qbuf(0)[i] = vl_make_key(qi[i], qd[i]);
-        for (int i = tid + kPreV * THREADS; i < a.VL; i += THREADS) vbuf(0)[i] = vl_make_key(vi[i], vd[i]);
-        for (int i = tid + kPreS * THREADS; i < seen_bound; i += THREADS) sbuf(0)[i] = srow[i];
-        for (int i = tid + THREADS; i < a.excl_cols; i += THREADS) {
-            int32_t e = a.excl[row * a.excl_cols + i];
-            exl[i] = e;
-            if (e == VL_MAXINT) atomicMin(&g_n_ex_s, i);
-        }
-        for (int i = tid; i < s.lds_slots; i += THREADS) lds.tab[i] = (uint64_t)(uint32_t)VL_MAXINT;  // no probe asks for it
-        __syncthreads();  // the table is probed below
-    }
-
-    for (int w = 0; w < W; ++w) {
-        const int t = t0 + w;
-        a.iter = t;
-        // The LDS addresses of an iteration are formed again from an offset the compiler cannot see through
-        // (always 0): hoisted out of this loop, the per-thread addresses of every array below would occupy some
-        // thirty registers through all of it, and cost a wavefront per SIMD.
-        int z = 0;
-        asm volatile("" : "+s"(z));
-        unsigned char *const base = smem + z;
-        uint64_t *const raw = reinterpret_cast<uint64_t *>(base);
-        uint64_t *const uk = raw + Pc;
-        uint64_t *const q0 = uk + Pc;
-        uint64_t *const v0 = q0 + 2 * a.L;
-        auto qbuf = [&](int k) -> uint64_t * { return q0 + k * a.L; };
-        auto vbuf = [&](int k) -> uint64_t * { return v0 + k * a.VL; };
-        LdsMemo lds;
-        lds.tab = s.lds_slots > 0 ? v0 + 2 * a.VL : nullptr;
-        lds.shift = 32 - (31 - __builtin_clz(s.lds_slots > 0 ? s.lds_slots : 1));
-        int32_t *const s0 = reinterpret_cast<int32_t *>(v0 + 2 * a.VL + s.lds_slots);
-        auto sbuf = [&](int k) -> int32_t * { return s0 + k * a.E; };
-        int32_t *const exl = s0 + 2 * a.E;
-        uint8_t *const xf = reinterpret_cast<uint8_t *>(exl + a.excl_cols);  // the merge phase's per-candidate flags; 16 = exact
-        int32_t *const li = reinterpret_cast<int32_t *>(uk);                 // candidate ids, distances behind them
-        float *const ld = reinterpret_cast<float *>(li + a.m);
-        float *const le = reinterpret_cast<float *>(raw);                    // upper bounds (raw is filled in the merge phase)
-        if (w > 0) {
-            if (tid < a.Vt) g_visit_s[tid] = vl_key_id(vbuf(cur_v)[tid]);  // queue.py:87-95: the heads are popped
-            if (tid == 0) {
-                probe_hits_s = 0;
-                probe_asked_s = 0;
-            }
-            __syncthreads();
-            id = resolve(wave * kWave);
-        }
-        // The query row (and its rounded form) is read again in every iteration, as a launch per iteration
-        // does: loaded once before the loop it would hold some forty registers through all of it, merge
-        // phases included.  The empty asm hides from the compiler that the address is the same each time.
-        const float *q_row = q_row0;
-        const uint8_t *rounded_row = rounded_row0;
-        asm volatile("" : "+s"(q_row), "+s"(rounded_row));
-        const int memo_word = memo_word_s;
-        const int memo_rate = memo_word & 0xffff;
-        uint64_t *memo_row = memo_table;
-        const bool resample = memo_row && t == kMemoDecide;
-        if (memo_row && memo_rate < s.memo_min_rate) memo_row = nullptr;
-        bool sketching = false;
-        if constexpr (SCPL > 0) sketching = s.sketch != nullptr && (memo_word >> 16) != 0 && t > 1;
-        const bool probing = memo_row != nullptr;
-
-        // ---- expand: ann.py:69-73 ----
-        int n_wanted = 0, n_fetched = 0, n_sketched = 0;  // counts of this wavefront
-        // A candidate the row met before comes back from the LDS table or, failing that, from the cache in
-        // memory: with its distance, or (rows that use the sketch) with its bounds.  Returns the entry or 0.
-        auto probe = [&](int32_t cid, bool bounds_too) -> uint64_t {
-            uint64_t e = 0;
-            bool hit = false;
-            if (lds.tab) {
-                e = lds_memo_load(lds, cid);
-                hit = (int32_t)((uint32_t)e & (bounds_too ? ~kMemoBounds : ~0u)) == cid;
-            }
-            if (!hit && probing) {
-                e = memo_load(memo_row, s.memo_shift, cid);
-                hit = (int32_t)((uint32_t)e & (bounds_too ? ~kMemoBounds : ~0u)) == cid;
-                if (hit && lds.tab) lds_memo_store(lds, cid, e);
-            }
-            return hit ? e : 0ull;
-        };
-        if constexpr (SCPL > 0) {
-            if (sketching) {
-                SketchQuery<SCPL> sq;
-                sketch_query_load<SCPL, SLPR>(sq, rounded_row, s.sketch_chunks);
-                for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-                    if (c0 != wave * kWave) id = resolve(c0);
-                    const int slot = c0 + lane;
-                    const bool has = slot < a.m;
-                    bool ok = has && id != VL_MAXINT && id >= 0 && (int64_t)id < s.n_vectors;
-                    if (has) {
-                        li[slot] = ok ? id : VL_MAXINT;
-                        if (!ok) ld[slot] = VL_MAXFLOAT;
-                        xf[slot] = 0;
-                    }
-                    if (s.count_evals || resample) n_wanted += __popcll(__ballot(ok));
-                    if (ok) {
-                        const uint64_t e = probe(id, true);
-                        if (e) {  // (id 0 at distance 0 is the one entry that is all zeros: it reads as a miss and is evaluated again)
-                            if ((uint32_t)e & kMemoBounds) {
-                                ld[slot] = memo_bound_lo(e);
-                                le[slot] = memo_bound_hi(e);
-                            } else {
-                                const float d = __builtin_bit_cast(float, (uint32_t)(e >> 32));
-                                ld[slot] = d;
-                                le[slot] = d;
-                                xf[slot] = 16;  // exact already
-                            }
-                            ok = false;
-                        }
-                    }
-                    if (s.count_evals || resample) n_sketched += __popcll(__ballot(ok));
-                    wave_sketch<SCPL, SLPR, SU>(sq, s.sketch, s.sketch_tails, s.sketch_chunks, id, ok, ld + c0, le + c0,
-                                                lane_order_s + wave * kWave, memo_row, s.memo_shift, lds);
-                }
-                n_fetched = n_sketched;  // for the share of cache hits: what the cache did not answer
-            }
-        }
-        for (int c0 = wave * kWave; c0 < a.m && !sketching; c0 += THREADS) {
-            if (c0 != wave * kWave) id = resolve(c0);
-            const int slot = c0 + lane;
-            const bool has = slot < a.m;
-            bool ok = has && id != VL_MAXINT && id >= 0 && (int64_t)id < s.n_vectors;
-            if (has) {
-                li[slot] = ok ? id : VL_MAXINT;
-                if (!ok) ld[slot] = VL_MAXFLOAT;
-            }
-            if (s.count_evals || resample) n_wanted += __popcll(__ballot(ok));
-            if (ok) {
-                const uint64_t e = probe(id, false);
-                if (e) {
-                    ld[slot] = __builtin_bit_cast(float, (uint32_t)(e >> 32));
-                    ok = false;
-                }
-            }
-            if (s.count_evals || resample) n_fetched += __popcll(__ballot(ok));
-            wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0, lane_order_s + wave * kWave,
-                                            memo_row, s.memo_shift, s.l2 != 0, lds);
-        }
-        if (s.count_evals && lane == 0) {
-            const int stripe = (int)((blockIdx.x * (THREADS / kWave) + wave) & (kBeamStripes - 1));
-            if (n_wanted) atomicAdd(&c->wanted[stripe], (unsigned long long)n_wanted);
-            if (n_fetched && !sketching) atomicAdd(&c->evals[stripe], (unsigned long long)n_fetched);
-            if (n_sketched) atomicAdd(&c->sketched[stripe], (unsigned long long)n_sketched);
-        }
-        if (resample && lane == 0) {
-            atomicAdd(&probe_asked_s, n_wanted);
-            atomicAdd(&probe_hits_s, n_wanted - n_fetched);
-        }
-        __syncthreads();
-        if (resample && tid == 0) {
-            const int word = (probe_asked_s > 0 ? (probe_hits_s * 256) / probe_asked_s : 256) | (memo_word & (1 << 16));
-            s.memo_rate[row] = word;
-            memo_word_s = word;
-        }
-        // ---- merge: ann.py:75-88 ----
-        ResidentRow rr;
-        rr.qa = qbuf(cur_q); rr.qa_out = qbuf(cur_q ^ 1);
-        rr.va = vbuf(cur_v); rr.va_out = vbuf(cur_v ^ 1);
-        rr.seen_a = sbuf(cur_s); rr.seen_b = sbuf(cur_s ^ 1);
-        rr.exl = exl; rr.fl = xf; rr.quiet = &quiet_s;
-        const RowState pre{cnt, a.Vt * (t - 1)};  // every row has room for the Vt ids it pops (Vt * t <= E)
-        MergeResult mr;
-        if constexpr (SCPL > 0) {
-            // the same rule as beam_step_body's refine (see there), with the row's LDS table kept current
-            auto refine = [&](const int32_t *seen_b, int cnt_now, bool seen_full, uint64_t ws, uint64_t wv, uint8_t *flags,
-                              uint64_t *red) {
-                if (!sketching) return;  // uniform over the workgroup
-                const float ws_d = vl_key_dist(ws);
-                const float wv_d = nva > 0 ? vl_key_dist(wv) : -1.0f;
-                for (int i = tid; i < a.m; i += THREADS) {
-                    const int32_t cid = li[i];
-                    uint8_t f = flags[i] & 16;
-                    if (cid != VL_MAXINT) {
-                        const float lo = ld[i];
-                        bool need = !(lo > ws_d);
-                        if (!seen_full && !sorted_contains(seen_b, cnt_now, cid)) {
-                            if (!(lo > wv_d)) need = true;
-                            else f |= 2;
-                        }
-                        if (need) f |= 4;
-                    }
-                    flags[i] = f;
-                }
-                bool all_rest = false;
-                if (!seen_full) {
-                    for (int r = 0; r < a.Vt; ++r) {
-                        uint32_t mine = 0xFFFFFFFFu;
-                        for (int i = tid; i < a.m; i += THREADS) {
-                            if ((flags[i] & (2 | 8)) != 2) continue;
-                            const uint32_t k = bound_slot_key(le[i], i);
-                            if (k < mine) mine = k;
-                        }
-                        const uint32_t mn = block_min_u32(mine, reinterpret_cast<uint32_t *>(red), r);
-                        if (mn == 0xFFFFFFFFu) {
-                            all_rest = true;
-                            break;
-                        }
-                        const int32_t chosen = li[mn & (kMaxCandidates - 1)];
-                        for (int i = tid; i < a.m; i += THREADS)
-                            if ((flags[i] & 2) && li[i] == chosen) flags[i] |= 8;
-                    }
-                }
-                int n_exact = 0, n_real = 0;
-                for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-                    const int slot = c0 + lane;
-                    const bool has = slot < a.m;
-                    const int32_t cid = has ? li[slot] : VL_MAXINT;
-                    const uint8_t f = has ? flags[slot] : 0;
-                    const bool ok = ((f & (4 | 8)) || (all_rest && (f & 2))) && !(f & 16);
-                    if (ok) flags[slot] = f | 16;
-                    n_exact += __popcll(__ballot(ok));
-                    n_real += __popcll(__ballot(cid != VL_MAXINT && !(f & 16)));
-                    wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, cid, ok, ld + c0,
-                                                    lane_order_s + wave * kWave, memo_row, s.memo_shift, false, lds);
-                }
-                __syncthreads();
-                float tv = -1.0f;
-                if (!seen_full && !all_rest) {
-                    uint32_t mine = 0xFFFFFFFFu;  // (no distance has the key 0)
-                    for (int i = tid; i < a.m; i += THREADS)
-                        if (flags[i] & 8) {
-                            const uint32_t k = ~vl_float_key(ld[i]);
-                            mine = k < mine ? k : mine;
-                        }
-                    const uint32_t mn = block_min_u32(mine, reinterpret_cast<uint32_t *>(red), a.Vt);
-                    tv = mn == 0xFFFFFFFFu ? -1.0f : vl_key_float(~mn);
-                }
-                for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-                    const int slot = c0 + lane;
-                    const bool has = slot < a.m;
-                    const int32_t cid = has ? li[slot] : VL_MAXINT;
-                    const uint8_t f = has ? flags[slot] : 0;
-                    const bool ok = (f & 2) && !(f & 16) && !(ld[slot] > tv);
-                    if (has && cid != VL_MAXINT && !ok && !(f & 16)) {
-                        li[slot] = VL_MAXINT;
-                        ld[slot] = VL_MAXFLOAT;
-                    }
-                    n_exact += __popcll(__ballot(ok));
-                    wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, cid, ok, ld + c0,
-                                                    lane_order_s + wave * kWave, memo_row, s.memo_shift, false, lds);
-                }
-                if (s.count_evals && lane == 0 && n_exact)
-                    atomicAdd(&c->evals[(int)((blockIdx.x * (THREADS / kWave) + wave) & (kBeamStripes - 1))],
-                              (unsigned long long)n_exact);
-                if (t > 2 && !resample) {
-                    if (lane == 0) {
-                        atomicAdd(&probe_asked_s, n_real);
-                        atomicAdd(&probe_hits_s, n_exact);
-                    }
-                    __syncthreads();
-                    const bool quit = t > kMemoDecide ? 2 * probe_hits_s > probe_asked_s : 8 * probe_hits_s > 7 * probe_asked_s;
-                    if (tid == 0 && quit) {
-                        s.memo_rate[row] = memo_rate;
-                        memo_word_s = memo_rate;
-                        atomicAdd(&c->sketch_rows, -1);
-                    }
-                } else {
-                    __syncthreads();
-                }
-            };
-            mr = merge_row<THREADS, true, decltype(refine), true>(a, base, pre, refine, &rr);
-        } else {
-            mr = merge_row<THREADS, true, NoRefine, true>(a, base, pre, NoRefine(), &rr);
-        }
-        cnt = mr.cnt;
-        if (mr.queue_moved) {
-            cur_q ^= 1;
-            queue_dirty = true;
-        }
-        cur_v ^= 1;
-        cur_s ^= 1;
-        __syncthreads();  // the merged rows are read below and by the next iteration
-        if (a.row_quiet && quiet_s >= a.readahead) break;  // the row has stopped on its own (uniform)
-    }
-    // ---- the row goes back to memory once ----
-    // (addresses formed afresh: kept from the loads at the top they would sit in registers, or in scratch memory,
-    // through the whole loop)
-    asm volatile("" : "+s"(qi), "+s"(qd), "+s"(vi), "+s"(vd), "+s"(srow));
-    if (queue_dirty) {
-        const uint64_t *qf = qbuf(cur_q);
-        for (int i = tid; i < a.L; i += THREADS) {
-            const uint64_t k = qf[i];
-            qi[i] = vl_key_id(k);
-            qd[i] = vl_key_dist(k);
-        }
-    }
-    {
-        const uint64_t *vf = vbuf(cur_v);
-        for (int i = tid; i < a.VL; i += THREADS) {
-            const uint64_t k = vf[i];
-            vi[i] = vl_key_id(k);
-            vd[i] = vl_key_dist(k);
-        }
-        const int32_t *sf = sbuf(cur_s);
-        for (int i = tid; i < cnt; i += THREADS) srow[i] = sf[i];
-    }
-    if (tid == 0) {
-        a.seen_count[row] = cnt;
-        if (a.row_quiet) a.row_quiet[row] = quiet_s;
-        raise_running_max(first_after, cnt, bound_after);
-    }
+template <int CPL, int LPR, int U, bool GENERIC, int THREADS>
+__global__ __launch_bounds__(THREADS) void beam_window_kernel(StepArgs s) {
+    beam_row<CPL, LPR, U, GENERIC, THREADS, 0, 64, 1, true>(s);
 }
-
-// WPE: wavefronts per SIMD asked of the compiler.  The row's phases each wait on memory, so a launch is as fast
-// as it has wavefronts to switch to: the registers are capped at what the one-iteration kernel of the same shape
-// uses, and what the longer body holds beyond that (addresses for the write-back at the end, mostly) lives in
-// scratch memory, stored once and read back rarely.
-template <int CPL, int LPR, int U, int THREADS, int WPE>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
-void beam_window_kernel(StepArgs s) {
-    beam_window_body<CPL, LPR, U, THREADS>(s);
-}
-
-template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int WPE>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
-void beam_window_sketch_kernel(StepArgs s) {
-    beam_window_body<CPL, LPR, U, THREADS, SCPL, SLPR, SU>(s);
+template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU>
+__global__ __launch_bounds__(THREADS) void beam_window_sketch_kernel(StepArgs s) {
+    beam_row<CPL, LPR, U, false, THREADS, SCPL, SLPR, SU, true>(s);
 }
 
 // The same step for rows that may use the sketch.  WPE: wavefronts per SIMD the compiler is asked to leave room
@@ -1680,69 +671,33 @@ void beam_window_sketch_kernel(StepArgs s) {
 template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int WPE>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
 void beam_step_sketch_kernel(StepArgs s) {
-    beam_step_body<CPL, LPR, U, false, THREADS, SCPL, SLPR, SU>(s);
+    beam_row<CPL, LPR, U, false, THREADS, SCPL, SLPR, SU>(s);
 }
 
-template <int CPL, int LPR, int U, bool GENERIC, int SCPL = 0, int SLPR = 64, int SU = 1, int WPE = 4, int UX = U,
-          int WPW = WPE, int WPP = 0>
-void launch_step(const StepArgs &s, int threads, size_t smem, hipStream_t st) {
-    dim3 grid((unsigned)s.m.n_rows);
+template <class Kernel>
+void launch_rows(Kernel kernel, int threads, const StepArgs &s, size_t smem, hipStream_t st) {
+    if (vl_allow_lds(kernel, smem) != hipSuccess) return;  // seen by the launch check
+    hipLaunchKernelGGL(kernel, dim3((unsigned)s.m.n_rows), dim3((unsigned)threads), smem, st, s);
+}
+
+template <int THREADS, int CPL, int LPR, int U, bool GENERIC, int SCPL, int SLPR, int SU, int WPE, int UX, int WPP>
+void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
     if constexpr (SCPL > 0) {
-        if (!s.sketch) return launch_step<CPL, LPR, U, GENERIC, 0, 64, 1, WPE, U, WPW, WPP>(s, threads, smem, st);
-    }
-    if constexpr (!GENERIC) {
-        if (s.window > 0) {  // several iterations in this launch (smem is the window kernel's size)
-            if constexpr (SCPL > 0) {
-                if (threads == 128) {
-                    auto kernel = beam_window_sketch_kernel<CPL, LPR, UX, 128, SCPL, SLPR, SU, WPW>;
-                    if (vl_allow_lds(kernel, smem) != hipSuccess) return;  // seen by the launch check
-                    hipLaunchKernelGGL(kernel, grid, dim3(128), smem, st, s);
-                } else {
-                    auto kernel = beam_window_sketch_kernel<CPL, LPR, UX, 256, SCPL, SLPR, SU, WPW>;
-                    if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-                    hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, s);
-                }
-            } else if (threads == 128) {
-                auto kernel = beam_window_kernel<CPL, LPR, U, 128, WPW>;
-                if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-                hipLaunchKernelGGL(kernel, grid, dim3(128), smem, st, s);
-            } else {
-                auto kernel = beam_window_kernel<CPL, LPR, U, 256, WPW>;
-                if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-                hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, s);
-            }
+        if (s.sketch) {
+            if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU>, THREADS, s, smem, st);
+            else launch_rows(beam_step_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, WPE>, THREADS, s, smem, st);
             return;
         }
     }
-    if constexpr (SCPL > 0) {
-        if (threads == 128) {
-            auto kernel = beam_step_sketch_kernel<CPL, LPR, UX, 128, SCPL, SLPR, SU, WPE>;
-            if (vl_allow_lds(kernel, smem) != hipSuccess) return;  // seen by the launch check
-            hipLaunchKernelGGL(kernel, grid, dim3(128), smem, st, s);
-        } else {
-            auto kernel = beam_step_sketch_kernel<CPL, LPR, UX, 256, SCPL, SLPR, SU, WPE>;
-            if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-            hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, s);
-        }
-    } else if constexpr (WPP > 0 && !GENERIC) {
-        if (threads == 128) {
-            auto kernel = beam_step_kernel_w<CPL, LPR, U, 128, WPP>;
-            if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-            hipLaunchKernelGGL(kernel, grid, dim3(128), smem, st, s);
-        } else {
-            auto kernel = beam_step_kernel_w<CPL, LPR, U, 256, WPP>;
-            if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-            hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, s);
-        }
-    } else if (threads == 128) {
-        auto kernel = beam_step_kernel<CPL, LPR, U, GENERIC, 128>;
-        if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-        hipLaunchKernelGGL(kernel, grid, dim3(128), smem, st, s);
-    } else {
-        auto kernel = beam_step_kernel<CPL, LPR, U, GENERIC, 256>;
-        if (vl_allow_lds(kernel, smem) != hipSuccess) return;
-        hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, s);
-    }
+    if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, GENERIC, THREADS>, THREADS, s, smem, st);
+    else if constexpr (WPP > 0 && !GENERIC) launch_rows(beam_step_kernel_w<CPL, LPR, U, THREADS, WPP>, THREADS, s, smem, st);
+    else launch_rows(beam_step_kernel<CPL, LPR, U, GENERIC, THREADS>, THREADS, s, smem, st);
+}
+
+template <int CPL, int LPR, int U, bool GENERIC, int SCPL = 0, int SLPR = 64, int SU = 1, int WPE = 4, int UX = U, int WPP = 0>
+void launch_step(const StepArgs &s, int threads, size_t smem, hipStream_t st) {
+    if (threads == 128) launch_step_threads<128, CPL, LPR, U, GENERIC, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
+    else launch_step_threads<256, CPL, LPR, U, GENERIC, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
 }
 
 // VL_DIST_VARIANT (experiments only): 1 = two rows per load for rows of up to 512 bytes (32 lanes each) and
@@ -1758,8 +713,7 @@ int dist_variant() {
 // The numbers after `false` are the sketch's lane shape for rows of that size (chunks per lane, lanes per row,
 // loads in flight), the wavefronts per SIMD asked for, the whole rows in flight in the sketch kernel (it fetches
 // few of them, so fewer in flight cost nothing and leave registers for another wavefront: 0.40 -> 0.36 ms per
-// launch at 384 columns), where given, the wavefronts per SIMD asked for in the kernels that run several
-// iterations per launch, and last the wavefronts per SIMD asked for in the kernel without the sketch
+// launch at 384 columns), and last the wavefronts per SIMD asked for in the kernel without the sketch
 // (beam_step_kernel_w; 0 = the compiler's own choice, which is seven at most: the step holds 106 scalar registers).
 // Eight wavefronts per SIMD - every workgroup slot a compute unit has - is what the launches that wait on memory
 // round trips rather than on bytes want, and the shapes that reach it without spilling a vector register ask for it
@@ -1771,13 +725,13 @@ int launch_step_by_dim(const StepArgs &s, bool aligned, int threads, size_t smem
     const int nchunks = s.nchunks;
     const int variant = dist_variant();
     if (!aligned || nchunks > 512) launch_step<1, 64, 1, true>(s, threads, smem, st);
-    else if (nchunks <= 16) launch_step<1, 16, 8, false, 1, 8, 4, 5, 8, 6, 8>(s, threads, smem, st);
+    else if (nchunks <= 16) launch_step<1, 16, 8, false, 1, 8, 4, 5, 8, 8>(s, threads, smem, st);
     else if (nchunks <= 32 && variant == 1) launch_step<1, 32, 8, false>(s, threads, smem, st);
-    else if (nchunks <= 32) launch_step<2, 16, 4, false, 1, 8, 4, 5, 4, 6, 8>(s, threads, smem, st);
-    else if (nchunks <= 64) launch_step<1, 64, 8, false, 2, 8, 2, 5, 8, 6, 8>(s, threads, smem, st);
-    else if (nchunks <= 96 && variant != 1) launch_step<3, 32, 2, false, 3, 8, 1, 8, 1, 6, 8>(s, threads, smem, st);
+    else if (nchunks <= 32) launch_step<2, 16, 4, false, 1, 8, 4, 5, 4, 8>(s, threads, smem, st);
+    else if (nchunks <= 64) launch_step<1, 64, 8, false, 2, 8, 2, 5, 8, 8>(s, threads, smem, st);
+    else if (nchunks <= 96 && variant != 1) launch_step<3, 32, 2, false, 3, 8, 1, 8, 1, 8>(s, threads, smem, st);
     else if (nchunks <= 128) launch_step<2, 64, 8, false, 2, 16, 2, 6, 2>(s, threads, smem, st);
-    else if (nchunks <= 192) launch_step<3, 64, 2, false, 3, 16, 1, 8, 1, 6, 8>(s, threads, smem, st);
+    else if (nchunks <= 192) launch_step<3, 64, 2, false, 3, 16, 1, 8, 1, 8>(s, threads, smem, st);
     else if (nchunks <= 256) launch_step<4, 64, 4, false, 4, 16, 2, 5, 2>(s, threads, smem, st);
     else if (nchunks <= 320) launch_step<5, 64, 2, false, 3, 32, 2, 6, 1>(s, threads, smem, st);
     else if (nchunks <= 384) launch_step<6, 64, 2, false, 3, 32, 2, 6, 1>(s, threads, smem, st);
@@ -1946,15 +900,18 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     const size_t smem = use_sort_merge
         ? (size_t)Pmax * 8 + (size_t)a.L * 4 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4
         : (size_t)a.Pc * 16 + (size_t)(a.L + a.VL) * 8 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4 + (size_t)a.m + 16;
-    VL_REQUIRE(smem + 2048 <= kLdsPerCu, "queues of this size need %zu bytes of LDS (a compute unit has %zu)", smem,
-               kLdsPerCu);
-
+    const int hash_slots = row_hash_slots(a.E, a.m);
+    const size_t smem_step = row_layout(a.m, a.L, a.VL, hash_slots, a.excl_cols, false).bytes;
+    const size_t smem_window = row_layout(a.m, a.L, a.VL, hash_slots, a.excl_cols, true).bytes;
     // VL_BEAM_FUSED=0 runs an iteration as two launches (expand, merge) instead of the fused step
     static const bool fused_env = [] {
         const char *e = getenv("VL_BEAM_FUSED");
         return !(e && e[0] == '0');
     }();
     const bool use_fused = fused_env && !use_sort_merge && merge_threads != 64 && !(p->flags & VL_BEAM_TWO_LAUNCHES);
+    VL_REQUIRE((use_fused ? smem_step : smem) + 2048 <= kLdsPerCu, "queues of this size need %zu bytes of LDS (a compute unit has %zu)",
+               use_fused ? smem_step : smem,
+               kLdsPerCu);
     VL_REQUIRE(!per_query || use_fused, "the per-query stop is only built into the fused step");
     if (!use_fused) {
         if (use_sort_merge) VL_HIP(vl_allow_lds(beam_merge_kernel, smem));
@@ -1988,7 +945,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     step.sketch_tails = sketch ? sketch + sketch_tails_offset(p->n_vectors, p->dim) : nullptr;
     step.sketch_chunks = (int)sketch_data_chunks(p->dim);
     step.window = 0;
-    step.lds_slots = 0;
+    step.hash_slots = hash_slots;
     step.report = nullptr;
     step.memo_shift = 32;
     if (step.memo) {
@@ -2019,28 +976,15 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     }
 
     const int R = (int)p->speculative_readahead;
-    // Several iterations per launch (beam_window_body; VL_BEAM_WINDOWS in flags, or VL_BEAM_WINDOW=1 in the
-    // environment): the R iterations between two progress checks run in one launch while no visited list can fill
-    // up in them, i.e. while Vt * (last iteration) <= E; the stretch after that runs one iteration per launch.
-    // Off by default: the longer kernel body needs some fifty registers more than the one-iteration kernel, and what
-    // it saves (one read and one write of the row's queues per iteration, four launches in five) is less than what
-    // the spilled registers or the lost wavefront per SIMD cost (measured at 1M x 768: 0.61 ms per iteration either
-    // way on the first optimisation loop's state, 0.48 instead of 0.42 ms on the second's).
-    static const bool window_env = [] {
+    // Several iterations per launch (beam_row; VL_BEAM_WINDOWS in flags, or VL_BEAM_WINDOW=1 in the environment): the R
+    // iterations between two progress checks run in one launch while no visited list can fill up in them, i.e. while
+    // Vt * (last iteration) <= E; the stretch after that runs one iteration per launch.
+    static const int window_env = [] {
         const char *e = getenv("VL_BEAM_WINDOW");
-        return e && e[0] == '1';
-    }();
-    // entries of the row's distance table in LDS: room for the candidates of one iteration, 256 to 1024
-    static const int lds_slots_env = [] {
-        const char *e = getenv("VL_BEAM_LDS_SLOTS");
         return e ? atoi(e) : -1;
     }();
-    int lds_slots = a.Pc < 256 ? 256 : (a.Pc > 1024 ? 1024 : a.Pc);
-    if (lds_slots_env >= 0) lds_slots = lds_slots_env ? vl_next_pow2(lds_slots_env) : 0;
-    const size_t smem_window = (size_t)a.Pc * 16 + (size_t)(a.L + a.VL) * 16 + (size_t)lds_slots * 8 + (size_t)a.E * 8 +
-                               (size_t)a.excl_cols * 4 + (size_t)a.m + 16;
-    const bool use_window = use_fused && (window_env || (p->flags & VL_BEAM_WINDOWS)) && R >= 2 && aligned &&
-                            step.nchunks <= 512 && smem_window + 2048 <= kLdsPerCu;
+    const bool want_window = window_env >= 0 ? window_env != 0 : (p->flags & VL_BEAM_WINDOWS) != 0;
+    const bool use_window = use_fused && want_window && R >= 2 && hash_slots < 0xffff && smem_window + 2048 <= kLdsPerCu;
     auto window_fits = [&](int64_t first_iteration) { return use_window && l.Vt * (first_iteration + R - 1) <= l.E; };
     const int step_threads = merge_threads == 128 ? 128 : 256;
     if (fixed_iterations > 0) {
@@ -2051,8 +995,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
             step.m = a;
             const bool windowed = window_fits(t) && (t - 1) % R == 0 && t + R - 1 <= fixed_iterations;
             step.window = windowed ? R : 0;
-            step.lds_slots = windowed ? lds_slots : 0;
-            rc = launch_step_by_dim(step, aligned, step_threads, windowed ? smem_window : smem, st);
+            rc = launch_step_by_dim(step, aligned, step_threads, windowed ? smem_window : smem_step, st);
             if (rc < 0) return rc;
             t += windowed ? R : 1;
         }
@@ -2098,8 +1041,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
         // (the sketch kernel also for a first window: its rows leave the sketch alone in iteration 1)
         step.sketch = ((windowed || t > 0) && 2 * (int64_t)sketch_rows >= p->n_rows) ? sketch_table : nullptr;
         step.window = windowed ? R : 0;
-        step.lds_slots = windowed ? lds_slots : 0;
-        const int e = launch_step_by_dim(step, aligned, step_threads, windowed ? smem_window : smem, st);
+        const int e = launch_step_by_dim(step, aligned, step_threads, windowed ? smem_window : smem_step, st);
         t += windowed ? R : 1;
         return e;
     };

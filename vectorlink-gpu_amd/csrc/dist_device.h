@@ -57,21 +57,6 @@ __device__ __forceinline__ void memo_store_bounds(uint64_t *memo_row, int shift,
 __device__ __forceinline__ float memo_bound_lo(uint64_t e) { return (float)(uint32_t)(e >> 48) * (1.0f / 65535.0f); }
 __device__ __forceinline__ float memo_bound_hi(uint64_t e) { return (float)((uint32_t)(e >> 32) & 0xffffu) * (1.0f / 65535.0f); }
 
-// The same entries in a small direct-mapped table in LDS (a workgroup that takes a row through several
-// iterations keeps one): a repeat inside those iterations never leaves the compute unit.  An entry moves as one
-// 8-byte LDS access; shift = 32 - log2(slots); tab == nullptr: no table.
-struct LdsMemo {
-    uint64_t *tab;
-    int shift;
-};
-__device__ __forceinline__ uint32_t lds_memo_slot(int32_t id, int shift) { return ((uint32_t)id * 2654435761u) >> shift; }
-__device__ __forceinline__ uint64_t lds_memo_load(const LdsMemo &t, int32_t id) {
-    return __hip_atomic_load(t.tab + lds_memo_slot(id, t.shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void lds_memo_store(const LdsMemo &t, int32_t id, uint64_t e) {
-    __hip_atomic_store(t.tab + lds_memo_slot(id, t.shift), e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 // Folds the partial sums of a group of LPR lanes: lane l += lane l + h for h = LPR/2 ... 1, so the
 // group's first lane ends with the sum in the fixed order.  Steps of 32 and 16 lanes swap register
 // halves / rows (v_permlane32_swap, v_permlane16_swap), steps inside a row of 16 lanes are DPP row
@@ -109,7 +94,7 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
                                                const float *__restrict__ vectors, int dim,
                                                int nchunks, int32_t my_id, bool ok,
                                                float *__restrict__ out_d, uint64_t *memo_row,
-                                               int memo_shift, bool l2 = false, LdsMemo lds = LdsMemo{nullptr, 0}) {
+                                               int memo_shift, bool l2 = false) {
     constexpr int G = kWave / LPR;
     const int lane = threadIdx.x & (kWave - 1);
     const int grp = lane / LPR;
@@ -206,7 +191,6 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
                 float d = finish_distance(acc, l2);
                 out_d[mysrc[u]] = d;
                 if (memo_row) memo_store(memo_row, memo_shift, ids[u], d);
-                if (lds.tab) lds_memo_store(lds, ids[u], memo_entry(ids[u], d));
             }
         }
     }
@@ -224,7 +208,7 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
                                                    const float *__restrict__ vectors, int dim,
                                                    int nchunks, int32_t my_id, bool ok,
                                                    float *out_d, uint8_t *order, uint64_t *memo_row,
-                                                   int memo_shift, bool l2 = false, LdsMemo lds = LdsMemo{nullptr, 0}) {
+                                                   int memo_shift, bool l2 = false) {
     constexpr int G = kWave / LPR;
     uint64_t mask = __ballot(ok);
     if (!mask) return;  // uniform over the wavefront
@@ -311,7 +295,6 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
         const float d = finish_distance(out_d[lane], l2);  // the sum was parked there by the first lane of the row's group
         out_d[lane] = d;
         if (memo_row) memo_store(memo_row, memo_shift, my_id, d);
-        if (lds.tab) lds_memo_store(lds, my_id, memo_entry(my_id, d));
     }
 }
 

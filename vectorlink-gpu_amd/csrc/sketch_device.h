@@ -109,8 +109,7 @@ template <int SCPL, int SLPR, int SU>
 __device__ __forceinline__ void wave_sketch(const SketchQuery<SCPL> &sq, const uint8_t *__restrict__ table,
                                             const uint8_t *__restrict__ tails, int data_chunks, int32_t my_id, bool ok,
                                             float *out_lo, float *out_hi, uint8_t *order,
-                                            uint64_t *memo_row = nullptr, int memo_shift = 0,
-                                            LdsMemo lds = LdsMemo{nullptr, 0}) {
+                                            uint64_t *memo_row = nullptr, int memo_shift = 0) {
     constexpr int G = kWave / SLPR;
     const uint64_t mask = __ballot(ok);
     if (!mask) return;  // uniform over the wavefront
@@ -172,6 +171,5 @@ __device__ __forceinline__ void wave_sketch(const SketchQuery<SCPL> &sq, const u
         out_lo[lane] = lo;
         out_hi[lane] = hi;
         if (memo_row) memo_store_bounds(memo_row, memo_shift, my_id, lo, hi);
-        if (lds.tab) lds_memo_store(lds, my_id, memo_bounds_entry(my_id, lo, hi));
     }
 }
