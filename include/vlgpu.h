@@ -212,15 +212,17 @@ typedef struct vl_beam_params {
  * (vl_closest_vectors_with_sketch): the workspace then also holds the call's
  * query rows rounded for it (32 bytes per 16 columns and row). */
 #define VL_BEAM_USES_SKETCH 16
-/* Same loop, same result, several iterations per launch: the fused step takes
- * a row through the speculative_readahead iterations between two progress
- * checks in ONE launch, with the row's queues and visited list resident in LDS
- * and a small LDS table of the (id, distance) pairs met in them, for as long as
- * no visited list can fill up within them (parallel_visit_count * iteration <=
- * exclude_factor * visit queue length); the stretch after that runs one
- * iteration per launch.  Off by default (it measures slower on an MI355X: the
- * longer kernel runs with fewer wavefronts per SIMD). */
+/* Several iterations per launch, or one (same loop, same result): the fused
+ * step can take a row through the speculative_readahead iterations between two
+ * progress checks in ONE launch, with the row's queues and visited list
+ * resident in LDS, for as long as no visited list can fill up within them
+ * (parallel_visit_count * iteration <= exclude_factor * visit queue length); the
+ * stretch after that runs one iteration per launch.  By default it does so
+ * unless the call's sketch is small enough for the GPU's L2 caches, where more
+ * rows in flight are worth more.  VL_BEAM_WINDOWS: always, VL_BEAM_NO_WINDOWS:
+ * never. */
 #define VL_BEAM_WINDOWS 32
+#define VL_BEAM_NO_WINDOWS 64
 
 int64_t vl_beam_workspace_bytes(const vl_beam_params *p);
 

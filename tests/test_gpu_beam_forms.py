@@ -1,0 +1,58 @@
+"""The forms of the fused beam step against the oracle's loop: one iteration per launch, several per launch, and whatever
+the library picks.  A launch's LDS depends on the rows of the call and on the iteration, so the row counts go from one
+workgroup on the chip to more than it holds at once."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+
+
+def bits(t):
+    return t.cpu().numpy().view(np.uint32)
+
+
+# rows of the call, vectors, columns, degree, build queue factor, visited-list factor
+SHAPES = [
+    (1, 300, 24, 6, 2, 5),
+    (257, 700, 52, 8, 2, 5),      # one row more than compute units
+    (700, 700, 256, 16, 2, 5),    # rows of 1 KiB: the sketch
+    (900, 900, 16, 24, 3, 2),     # 288 candidates in 128 threads, a visited list that fills up
+    (2300, 2300, 12, 4, 2, 5),    # more rows than the chip holds at once
+    (40, 1200, 8, 64, 2, 5),      # 512 candidates, 256 threads
+]
+
+
+@pytest.mark.parametrize("rows,n,dim,beam,bqf,ef", SHAPES)
+def test_forms_agree_with_the_oracle(rows, n, dim, beam, bqf, ef):
+    print(f"beam forms rows={rows} n={n} dim={dim} beam={beam}", flush=True)
+    from vectorlink_gpu import Queue
+    from vectorlink_gpu.ann import BEAM_NO_WINDOWS, BEAM_WINDOWS, closest_vectors, excluding_self
+    from vectorlink_gpu.kernels import build_sketch
+
+    rng = np.random.default_rng(rows + dim)
+    v = rng.standard_normal((n, dim)).astype(np.float32)
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    c = dict(orc.DEFAULT_CONFIG)
+    c.update(beam_size=beam, beam_queue_factor=bqf, exclude_factor=ef)
+    ql = beam * bqf
+    beams = orc.generate_circulant_beams(n, orc.primes(ql))
+    d = orc.calculate_distances(v, beams)
+    want = orc.Queue(rows, ql, ql + ql * 4)
+    want.insert(beams[:rows], d[:rows])
+    t_want = orc.closest_vectors(v[:rows], want, v, beams, c, orc.excluding_self(0, rows))
+    gv, gb, gd = dev(v), dev(beams), dev(d)
+    for sketch in ([None, build_sketch(gv)] if dim >= 256 else [None]):
+        for flags in (0, BEAM_NO_WINDOWS, BEAM_WINDOWS):
+            q = Queue(rows, ql, ql + ql * 4)
+            q.insert(gb[:rows], gd[:rows])
+            t = closest_vectors(gv[:rows], q, gv, gb, c, excluding_self(0, rows), flags=flags, sketch=sketch)
+            assert t == t_want, (flags, sketch is not None)
+            assert np.array_equal(q.indices.cpu().numpy()[:, :ql], want.indices[:, :ql]), (flags, sketch is not None)
+            assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32)), flags

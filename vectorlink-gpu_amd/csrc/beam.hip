@@ -651,12 +651,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPP)))
 void beam_step_kernel_w(StepArgs s) {
     beam_row<CPL, LPR, U, false, THREADS>(s);
 }
-template <int CPL, int LPR, int U, bool GENERIC, int THREADS>
-__global__ __launch_bounds__(THREADS) void beam_window_kernel(StepArgs s) {
+template <int CPL, int LPR, int U, bool GENERIC, int THREADS, int WPP>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPP))) void beam_window_kernel(StepArgs s) {
     beam_row<CPL, LPR, U, GENERIC, THREADS, 0, 64, 1, true>(s);
 }
-template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU>
-__global__ __launch_bounds__(THREADS) void beam_window_sketch_kernel(StepArgs s) {
+template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int WPE>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void beam_window_sketch_kernel(StepArgs s) {
     beam_row<CPL, LPR, U, false, THREADS, SCPL, SLPR, SU, true>(s);
 }
 
@@ -684,12 +684,12 @@ template <int THREADS, int CPL, int LPR, int U, bool GENERIC, int SCPL, int SLPR
 void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
     if constexpr (SCPL > 0) {
         if (s.sketch) {
-            if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU>, THREADS, s, smem, st);
+            if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, (WPE < 6 ? WPE : 6)>, THREADS, s, smem, st);
             else launch_rows(beam_step_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, WPE>, THREADS, s, smem, st);
             return;
         }
     }
-    if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, GENERIC, THREADS>, THREADS, s, smem, st);
+    if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, GENERIC, THREADS, (WPP > 0 ? 6 : 1)>, THREADS, s, smem, st);
     else if constexpr (WPP > 0 && !GENERIC) launch_rows(beam_step_kernel_w<CPL, LPR, U, THREADS, WPP>, THREADS, s, smem, st);
     else launch_rows(beam_step_kernel<CPL, LPR, U, GENERIC, THREADS>, THREADS, s, smem, st);
 }
@@ -900,9 +900,9 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     const size_t smem = use_sort_merge
         ? (size_t)Pmax * 8 + (size_t)a.L * 4 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4
         : (size_t)a.Pc * 16 + (size_t)(a.L + a.VL) * 8 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4 + (size_t)a.m + 16;
-    const int hash_slots = row_hash_slots(a.E, a.m);
-    const size_t smem_step = row_layout(a.m, a.L, a.VL, hash_slots, a.excl_cols, false).bytes;
-    const size_t smem_window = row_layout(a.m, a.L, a.VL, hash_slots, a.excl_cols, true).bytes;
+    // the LDS of a row that has visited all it can
+    const size_t smem_step = row_layout(a.m, a.L, a.VL, row_hash_slots(a.E, a.m, false), a.excl_cols, false).bytes;
+    const size_t smem_window = row_layout(a.m, a.L, a.VL, row_hash_slots(a.E, a.m, true), a.excl_cols, true).bytes;
     // VL_BEAM_FUSED=0 runs an iteration as two launches (expand, merge) instead of the fused step
     static const bool fused_env = [] {
         const char *e = getenv("VL_BEAM_FUSED");
@@ -945,7 +945,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     step.sketch_tails = sketch ? sketch + sketch_tails_offset(p->n_vectors, p->dim) : nullptr;
     step.sketch_chunks = (int)sketch_data_chunks(p->dim);
     step.window = 0;
-    step.hash_slots = hash_slots;
+    step.hash_slots = 0;  // set for each launch (size_set)
     step.report = nullptr;
     step.memo_shift = 32;
     if (step.memo) {
@@ -976,17 +976,44 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     }
 
     const int R = (int)p->speculative_readahead;
-    // Several iterations per launch (beam_row; VL_BEAM_WINDOWS in flags, or VL_BEAM_WINDOW=1 in the environment): the R
-    // iterations between two progress checks run in one launch while no visited list can fill up in them, i.e. while
-    // Vt * (last iteration) <= E; the stretch after that runs one iteration per launch.
+    // Several iterations per launch (beam_row): the R iterations between two progress checks run in one launch while no
+    // visited list can fill up in them, i.e. while Vt * (last iteration) <= E; the stretch after that runs one iteration
+    // per launch.  Measured against one iteration per launch: searches of 256 queries at 4,096 x 128 1,500 -> 1,004 us,
+    // 1,000 at 100,003 x 1,536 1,803 -> 1,253, 10,000 at 1M x 128 2,690 -> 2,057, 10,000 at 1M x 768 3,145 -> 2,802 us;
+    // builds of 4,096 x 128 8.5 -> 6.9 ms, 100,000 x 128 320 -> 296 ms.
+    // With the sketch a window fits a compute unit six times, the one-iteration kernel eight times.  Rows that come from
+    // HBM do not need those (a batch of the first loop at 1M x 768: 148 -> 140 ms, 1M x 384 49.4 -> 47.2, 50,000 x 768
+    // 93.7 -> 91.2); while the table fits the chip's L2s (8 x 4 MiB) the launches wait on round trips and do (builds of
+    // 20,011 x 768: 133 ms without, 143 with windows, 30,000 x 768 254 and 262).
+    // VL_BEAM_WINDOWS / VL_BEAM_NO_WINDOWS in flags, or VL_BEAM_WINDOW=1 / 0 in the environment: windows always / never.
     static const int window_env = [] {
         const char *e = getenv("VL_BEAM_WINDOW");
         return e ? atoi(e) : -1;
     }();
-    const bool want_window = window_env >= 0 ? window_env != 0 : (p->flags & VL_BEAM_WINDOWS) != 0;
-    const bool use_window = use_fused && want_window && R >= 2 && hash_slots < 0xffff && smem_window + 2048 <= kLdsPerCu;
-    auto window_fits = [&](int64_t first_iteration) { return use_window && l.Vt * (first_iteration + R - 1) <= l.E; };
+    const bool all_windows = window_env >= 0 ? window_env != 0 : (p->flags & VL_BEAM_WINDOWS) != 0;
+    const bool no_windows = window_env >= 0 ? window_env == 0 : (p->flags & VL_BEAM_NO_WINDOWS) != 0;
+    constexpr int64_t kL2Bytes = 32 << 20;
+    const bool sketch_window = all_windows || p->n_vectors * sketch_row_bytes(p->dim) > kL2Bytes;
     const int step_threads = merge_threads == 128 ? 128 : 256;
+    const bool use_window = use_fused && !no_windows && R >= 2 && row_hash_slots_most(a.E, a.m) < 0xffff &&
+                            smem_window + 2048 <= kLdsPerCu;
+    // A launch's LDS.  The visited ids of its last iteration and the candidates share the hash set, and the emptier it is
+    // the sooner each finds its place, so it takes what LDS the workgroups that a compute unit can hold (or that there are)
+    // leave it.
+    auto size_set = [&](int64_t last_iteration, bool windowed) -> size_t {
+        const int64_t visited = l.Vt * last_iteration < l.E ? l.Vt * last_iteration : l.E;
+        const int waves = step_threads / kWave;
+        int64_t resident = (windowed ? 4 * 6 : 4 * 8) / waves;
+        const int64_t per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits;
+        if (resident > per_cu) resident = per_cu;
+        const int least = row_hash_slots(visited, a.m, windowed), most = row_hash_slots_most(visited, a.m);
+        const int64_t room = (int64_t)(kLdsPerCu / resident) - 1024 - row_layout(a.m, a.L, a.VL, 0, a.excl_cols, windowed).bytes;
+        int64_t slots = (room < 0 ? 0 : room) / 4;
+        slots = slots > most ? most : slots;
+        step.hash_slots = (int)(slots < least ? least : slots) & ~3;
+        return row_layout(a.m, a.L, a.VL, step.hash_slots, a.excl_cols, windowed).bytes;
+    };
+    auto window_fits = [&](int64_t first_iteration) { return use_window && l.Vt * (first_iteration + R - 1) <= l.E; };
     if (fixed_iterations > 0) {
         VL_REQUIRE(use_fused, "a fixed number of iterations is only built for the fused step");
         step.count_evals = 0;
@@ -995,7 +1022,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
             step.m = a;
             const bool windowed = window_fits(t) && (t - 1) % R == 0 && t + R - 1 <= fixed_iterations;
             step.window = windowed ? R : 0;
-            rc = launch_step_by_dim(step, aligned, step_threads, windowed ? smem_window : smem_step, st);
+            rc = launch_step_by_dim(step, aligned, step_threads, size_set(windowed ? t + R - 1 : t, windowed), st);
             if (rc < 0) return rc;
             t += windowed ? R : 1;
         }
@@ -1035,14 +1062,15 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     const bool ahead = use_fused && !prof && slot.get() != nullptr;
     step.report = ahead ? slot.get() : nullptr;
     auto launch_next = [&]() -> int {  // the fused launch that follows iteration t; moves t on
-        const bool windowed = window_fits(t + 1) && t % R == 0;
+        const bool want_sketch = sketch_table && 2 * (int64_t)sketch_rows >= p->n_rows;
+        const bool windowed = window_fits(t + 1) && t % R == 0 && (!want_sketch || sketch_window);
         a.iter = (int)(t + 1);
         step.m = a;
         // (the sketch kernel also for a first window: its rows leave the sketch alone in iteration 1)
-        step.sketch = ((windowed || t > 0) && 2 * (int64_t)sketch_rows >= p->n_rows) ? sketch_table : nullptr;
+        step.sketch = ((windowed || t > 0) && want_sketch) ? sketch_table : nullptr;
         step.window = windowed ? R : 0;
-        const int e = launch_step_by_dim(step, aligned, step_threads, windowed ? smem_window : smem_step, st);
         t += windowed ? R : 1;
+        const int e = launch_step_by_dim(step, aligned, step_threads, size_set(t, windowed), st);
         return e;
     };
     int64_t checked = 0;  // iterations up to the last progress check

@@ -57,21 +57,26 @@ struct StepArgs {
     int sketch_chunks;         // 16-byte chunks of data in a sketch row
     const uint8_t *rounded_queries;  // the call's query rows rounded for the sketch (sketch_device.h)
     int64_t rounded_query_bytes;
-    int hash_slots;      // slots of the LDS hash set: row_hash_slots(E, m)
+    int hash_slots;      // slots of the LDS hash set (row_hash_slots)
     int window;          // > 0: iterations m.iter ... m.iter + window - 1 in this launch
     BeamReport *report;  // pinned host memory that hears of the progress checks, or null
 };
 
-// Slots of a row's hash set: visited ids and candidates fill three quarters of it at most, a multiple of 4 (it is
-// cleared 16 bytes at a time).
-__host__ __device__ inline int row_hash_slots(int64_t E, int64_t m) { return (int)(((E + m) * 4 / 3 + 7) & ~3ll); }
+// Slots of a row's hash set, a multiple of 4 (it is cleared 16 bytes at a time).  The fewest: three quarters of them taken
+// by visited ids and candidates; outside windows also room for m keys.  The most that are any use: a quarter taken.
+__host__ __device__ inline int row_hash_slots(int64_t visited, int64_t m, bool window) {
+    int64_t slots = (visited + m) * 4 / 3 + 7;
+    if (!window && slots < 2 * m + 3) slots = 2 * m + 3;
+    return (int)(slots & ~3ll);
+}
+__host__ __device__ inline int row_hash_slots_most(int64_t visited, int64_t m) { return (int)(4 * (visited + m)); }
 
 // LDS of a row's workgroup, in bytes from the start of its dynamic LDS.
 //   keys   m keys: the survivors; before that the sketched candidates' upper bounds
 //   cand   m ids and m distances; after the survivors have been picked m keys, the new ones of the search queue
 //   qa, vq the queues as keys (all VL slots of the visit queue, the popped heads first); a window keeps two of each
 //   set    the hash set
-//   fresh  m keys, the new ones of the visit queue: over the hash set where that is done with by then and long enough
+//   fresh  m keys, the new ones of the visit queue: over the hash set, which is done with by then except in a window
 struct RowLayout {
     int cand, qa, vq, set, fresh, slot, exl, flags, bytes;
 };
@@ -84,7 +89,7 @@ __host__ __device__ inline RowLayout row_layout(int m, int L, int VL, int hash_s
     o.set = (o.vq + 8 * copies * VL + 15) & ~15;
     int end = o.set + 4 * hash_slots;
     o.fresh = o.set;
-    if (window || 2 * m > hash_slots) {
+    if (window) {
         o.fresh = (end + 7) & ~7;
         end = o.fresh + 8 * m;
     }
@@ -133,18 +138,21 @@ constexpr int kMemoDecide = 9;
 // their remainder the slow way (read, wait, store) - none of the benchmark shapes has one.
 constexpr int kPreQ = 2, kPreV = 2, kPreS = 4;
 
-// Takes id's place in an open-addressed set (-1: empty).  False: the id is there already.  The set has more slots than
-// it ever holds ids, so an empty one is met.
+// Takes id's place in an open-addressed set (-1: empty).  False: the id is there already.  The places tried are those of a
+// sequence that runs through all 32-bit values (a full-period congruence), so an empty one is met.  64 ids wait for the
+// longest of their searches, which is why the set is kept as empty as LDS allows: 256 queries at 4,096 x 128 take 1,462 us
+// with three quarters of the set taken and the next place tried after a taken one, 1,004 us with a quarter of it taken.
 __device__ __forceinline__ bool set_claim(int32_t *set, uint32_t slots, int32_t id, uint32_t *at) {
-    uint32_t h = __umulhi((uint32_t)id * 2654435761u, slots);
+    uint32_t x = (uint32_t)id * 2654435761u;
     for (;;) {
+        const uint32_t h = __umulhi(x, slots);
         const int32_t there = atomicCAS(&set[h], -1, id);
         if (there == -1) {
             *at = h;
             return true;
         }
         if (there == id) return false;
-        h = h + 1 == slots ? 0 : h + 1;
+        x = x * 1664525u + 1013904223u;
     }
 }
 
@@ -216,9 +224,9 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     const MergeArgs &a = s.m;
     BeamCtrl *c = a.ctrl;
     const int t0 = a.iter;
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
+    int tid = threadIdx.x;
+    int lane = tid & (kWave - 1);
+    int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int64_t row = blockIdx.x;
     const int nva = a.VL - a.Vt;
     // ---- every read that depends on nothing else goes out first: loop state, the row's counters, the ids
@@ -287,7 +295,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     uint64_t *qa = reinterpret_cast<uint64_t *>(smem + at.qa);
     uint64_t *vq = reinterpret_cast<uint64_t *>(smem + at.vq);
     uint64_t *qa_next = qa + a.L, *vq_next = vq + a.VL;  // WINDOW only
-    const float *const q_row = s.queries + row * s.dim;
+    const float *q_row = s.queries + row * s.dim;
     uint64_t *const memo_table = s.memo ? s.memo + ((uint64_t)row << (32 - s.memo_shift)) : nullptr;
     uint8_t *const order = order_s + wave * kWave;
 
@@ -348,6 +356,13 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
 
     for (int w = 0; w < iterations; ++w) {
         const int t = t0 + w;
+        if constexpr (WINDOW) {
+            // what follows from these is worked out in every iteration again: kept across iterations, the lane masks,
+            // addresses and query row took 30 registers more than the one-iteration kernel has
+            asm volatile("" : "+v"(tid), "+s"(q_row));
+            lane = tid & (kWave - 1);
+            wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+        }
         if (WINDOW && w > 0) {
             if (tid < a.Vt) visit_s[tid] = vl_key_id(vq[tid]);  // queue.py:87-95: the heads are popped
             if (tid == 0) {

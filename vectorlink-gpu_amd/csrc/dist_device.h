@@ -4,6 +4,13 @@
 #pragma once
 #include "vl_common.h"
 
+// The lane's number, as something the compiler cannot work out ahead of a loop: what follows from it is cheap and not
+// worth registers that stay taken around the loop.
+__device__ __forceinline__ int own_lane() {
+    int lane = threadIdx.x & (kWave - 1);
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
 
 __device__ __forceinline__ float clamp_distance(float cos_theta) {
     float r = (1.0f - cos_theta) * 0.5f;  // kernels.py:109
@@ -96,7 +103,7 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
                                                float *__restrict__ out_d, uint64_t *memo_row,
                                                int memo_shift, bool l2 = false) {
     constexpr int G = kWave / LPR;
-    const int lane = threadIdx.x & (kWave - 1);
+    const int lane = own_lane();
     const int grp = lane / LPR;
     const int lig = lane % LPR;
 
@@ -212,7 +219,7 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
     constexpr int G = kWave / LPR;
     uint64_t mask = __ballot(ok);
     if (!mask) return;  // uniform over the wavefront
-    const int lane = threadIdx.x & (kWave - 1);
+    const int lane = own_lane();
     const int grp = lane / LPR;
     const int lig = lane % LPR;
     const int n = __popcll(mask);
@@ -304,7 +311,7 @@ __device__ __forceinline__ void wave_distances_generic(const float *__restrict__
                                                        int nchunks, int32_t my_id, bool ok,
                                                        float *__restrict__ out_d, uint64_t *memo_row,
                                                        int memo_shift, bool l2 = false) {
-    const int lane = threadIdx.x & (kWave - 1);
+    const int lane = own_lane();
     uint64_t mask = __ballot(ok);
     while (mask) {
         int s = __builtin_ctzll(mask);

@@ -76,7 +76,7 @@ __host__ __device__ inline int64_t sketch_query_bytes(int64_t dim) { return sket
 template <int SCPL, int SLPR>
 __device__ __forceinline__ void sketch_query_load(SketchQuery<SCPL> &sq, const uint8_t *__restrict__ rounded_row,
                                                   int data_chunks) {
-    const int lig = (threadIdx.x & (kWave - 1)) % SLPR;
+    const int lig = own_lane() % SLPR;
     const uint4 *words = reinterpret_cast<const uint4 *>(rounded_row);
 #pragma unroll
     for (int i = 0; i < SCPL; ++i) {
@@ -113,7 +113,7 @@ __device__ __forceinline__ void wave_sketch(const SketchQuery<SCPL> &sq, const u
     constexpr int G = kWave / SLPR;
     const uint64_t mask = __ballot(ok);
     if (!mask) return;  // uniform over the wavefront
-    const int lane = threadIdx.x & (kWave - 1);
+    const int lane = own_lane();
     const int grp = lane / SLPR;
     const int lig = lane % SLPR;
     const int n = __popcll(mask);

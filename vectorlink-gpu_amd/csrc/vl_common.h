@@ -57,6 +57,7 @@ static inline unsigned vl_grid_for(int64_t n, int per_block) {
 // more dynamic LDS than the 64 KiB every kernel is allowed by default has to raise that kernel's limit first.
 constexpr size_t kLdsDefault = 64 * 1024;
 constexpr size_t kLdsPerCu = 160 * 1024;
+constexpr int kComputeUnits = 256;
 template <class Kernel>
 static inline hipError_t vl_allow_lds(Kernel kernel, size_t smem) {
     if (smem + 1024 <= kLdsDefault) return hipSuccess;  // 1 KiB of slack for the kernels' static LDS
