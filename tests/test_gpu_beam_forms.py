@@ -56,3 +56,52 @@ def test_forms_agree_with_the_oracle(rows, n, dim, beam, bqf, ef):
             assert t == t_want, (flags, sketch is not None)
             assert np.array_equal(q.indices.cpu().numpy()[:, :ql], want.indices[:, :ql]), (flags, sketch is not None)
             assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32)), flags
+
+
+# lengths around a multiple of 4 at the edges of the shapes (16, 32, 64, 96, 128, 192, 256, 320, 384, 448, 512 chunks)
+ODD_DIMS = [1, 3, 5, 50, 62, 65, 127, 130, 253, 259, 383, 386, 511, 514, 766, 1022, 1026, 1279, 1534, 1790, 2045, 2049]
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("dim", ODD_DIMS)
+def test_rows_of_odd_length(dim, metric):
+    """Distances and the loop on rows that do not start on 16-byte boundaries; the last row ends with the table."""
+    print(f"odd rows dim={dim} {metric}", flush=True)
+    from vectorlink_gpu import Queue
+    from vectorlink_gpu.ann import closest_vectors, excluding_self
+    from vectorlink_gpu.kernels import gather_distances
+
+    rng = np.random.default_rng(dim)
+    (n, beam) = (90, 6)
+    v = rng.standard_normal((n, dim)).astype(np.float32)
+    if metric == "cosine":
+        v /= np.linalg.norm(v, axis=1, keepdims=True)
+    c = dict(orc.DEFAULT_CONFIG)
+    c.update(beam_size=beam, beam_queue_factor=2, metric=metric)
+    ql = 2 * beam
+    beams = orc.generate_circulant_beams(n, orc.primes(ql))
+    ids = np.concatenate([beams, np.full((n, 1), n - 1, np.int32)], axis=1)
+    with orc.metric(metric):
+        d = orc.gather_distances(v, v, ids)
+        want = orc.Queue(n, ql, ql + ql * 4)
+        want.insert(beams, np.ascontiguousarray(d[:, :ql]))
+        t_want = orc.closest_vectors(v, want, v, beams, c, orc.excluding_self(0, n))
+    assert np.array_equal(bits(gather_distances(dev(v), dev(v), dev(ids), metric=metric)), d.view(np.uint32))
+    q = Queue(n, ql, ql + ql * 4)
+    q.insert(dev(beams), dev(d[:, :ql]))
+    assert closest_vectors(dev(v), q, dev(v), dev(beams), c, excluding_self(0, n)) == t_want
+    assert np.array_equal(q.indices.cpu().numpy()[:, :ql], want.indices[:, :ql])
+    assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32))
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_odd_rows_with_values_that_are_not_finite(value):
+    """A row of 7 elements is read as elements 0-3 and 3-6: element 3 counts once, whatever it is."""
+    from vectorlink_gpu.kernels import gather_distances
+
+    v = np.linspace(-1, 1, 63, dtype=np.float32).reshape(9, 7)
+    v[4, 3] = value
+    ids = np.tile(np.arange(9, dtype=np.int32), (9, 1))
+    want = orc.gather_distances(v, v, ids)
+    got = gather_distances(dev(v), dev(v), dev(ids)).cpu().numpy()
+    assert np.array_equal(got, want, equal_nan=True)

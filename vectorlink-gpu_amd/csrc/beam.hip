@@ -17,7 +17,7 @@
 // the host only reads the changed flag every speculative_readahead
 // iterations, the cadence at which the reference tests for progress
 // (ann.py:68,90-91).
-#include "beam_row.h"
+#include "beam_kernels.h"
 #include <stddef.h>
 #include <stdlib.h>
 #include <atomic>
@@ -634,72 +634,6 @@ __global__ __launch_bounds__(THREADS) void beam_merge2_kernel(MergeArgs a) {
     merge_row<THREADS>(a, smem);
 }
 
-// ---- the fused step: one launch per iteration, or per window of iterations ------
-// The expand phase (memory bound) and the merge phase (LDS / latency bound) of one
-// row run in the same workgroup, so on every CU some workgroups stream candidate
-// rows while others merge: the merge time hides behind the memory traffic, the
-// candidate ids and distances never leave LDS, and an iteration is one launch.
-template <int CPL, int LPR, int U, bool GENERIC, int THREADS>
-__global__ __launch_bounds__(THREADS) void beam_step_kernel(StepArgs s) {
-    beam_row<CPL, LPR, U, GENERIC, THREADS>(s);
-}
-// The same kernel built to leave room for WPP wavefronts per SIMD.  Its vector registers would allow that anyway;
-// what does not is its scalar registers (more than 96 of them mean seven wavefronts instead of eight), which the
-// compiler keeps within bounds when asked, at the price of a few moves to and from lanes of a vector register.
-template <int CPL, int LPR, int U, int THREADS, int WPP>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPP)))
-void beam_step_kernel_w(StepArgs s) {
-    beam_row<CPL, LPR, U, false, THREADS>(s);
-}
-template <int CPL, int LPR, int U, bool GENERIC, int THREADS, int WPP>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPP))) void beam_window_kernel(StepArgs s) {
-    beam_row<CPL, LPR, U, GENERIC, THREADS, 0, 64, 1, true>(s);
-}
-template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int WPE>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void beam_window_sketch_kernel(StepArgs s) {
-    beam_row<CPL, LPR, U, false, THREADS, SCPL, SLPR, SU, true>(s);
-}
-
-// The same step for rows that may use the sketch.  WPE: wavefronts per SIMD the compiler is asked to leave room
-// for.  The sketch's copy of the query row takes 16 registers per chunk and lane, and a row's phases (sketch
-// pass, two rounds of exact rows, merge) each wait on memory, so residency is worth a few spilled registers:
-// measured at 768 and 384 columns, five wavefronts per SIMD with two loads in flight beat three wavefronts
-// with four (0.84 -> 0.75 ms and 0.61 -> 0.43 ms per launch).  Residency is what a launch that is not bound by
-// memory traffic responds to (768 columns, state of the second optimisation loop, workgroups per compute unit
-// limited through LDS: 4 / 5 / 6 -> 0.53 / 0.46 / 0.42 ms per launch; 8 with one load in flight and 62 registers:
-// 0.415), which is also why the step's LDS arrays are overlaid where their lifetimes allow.
-template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int WPE>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
-void beam_step_sketch_kernel(StepArgs s) {
-    beam_row<CPL, LPR, U, false, THREADS, SCPL, SLPR, SU>(s);
-}
-
-template <class Kernel>
-void launch_rows(Kernel kernel, int threads, const StepArgs &s, size_t smem, hipStream_t st) {
-    if (vl_allow_lds(kernel, smem) != hipSuccess) return;  // seen by the launch check
-    hipLaunchKernelGGL(kernel, dim3((unsigned)s.m.n_rows), dim3((unsigned)threads), smem, st, s);
-}
-
-template <int THREADS, int CPL, int LPR, int U, bool GENERIC, int SCPL, int SLPR, int SU, int WPE, int UX, int WPP>
-void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
-    if constexpr (SCPL > 0) {
-        if (s.sketch) {
-            if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, (WPE < 6 ? WPE : 6)>, THREADS, s, smem, st);
-            else launch_rows(beam_step_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, WPE>, THREADS, s, smem, st);
-            return;
-        }
-    }
-    if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, GENERIC, THREADS, (WPP > 0 ? 6 : 1)>, THREADS, s, smem, st);
-    else if constexpr (WPP > 0 && !GENERIC) launch_rows(beam_step_kernel_w<CPL, LPR, U, THREADS, WPP>, THREADS, s, smem, st);
-    else launch_rows(beam_step_kernel<CPL, LPR, U, GENERIC, THREADS>, THREADS, s, smem, st);
-}
-
-template <int CPL, int LPR, int U, bool GENERIC, int SCPL = 0, int SLPR = 64, int SU = 1, int WPE = 4, int UX = U, int WPP = 0>
-void launch_step(const StepArgs &s, int threads, size_t smem, hipStream_t st) {
-    if (threads == 128) launch_step_threads<128, CPL, LPR, U, GENERIC, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
-    else launch_step_threads<256, CPL, LPR, U, GENERIC, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
-}
-
 // VL_DIST_VARIANT (experiments only): 1 = two rows per load for rows of up to 512 bytes (32 lanes each) and
 // one row per load for rows of up to 1536 bytes, the shapes used before lane groups of 16 / 32 took them over.
 int dist_variant() {
@@ -724,19 +658,20 @@ int dist_variant() {
 int launch_step_by_dim(const StepArgs &s, bool aligned, int threads, size_t smem, hipStream_t st) {
     const int nchunks = s.nchunks;
     const int variant = dist_variant();
-    if (!aligned || nchunks > 512) launch_step<1, 64, 1, true>(s, threads, smem, st);
-    else if (nchunks <= 16) launch_step<1, 16, 8, false, 1, 8, 4, 5, 8, 8>(s, threads, smem, st);
-    else if (nchunks <= 32 && variant == 1) launch_step<1, 32, 8, false>(s, threads, smem, st);
-    else if (nchunks <= 32) launch_step<2, 16, 4, false, 1, 8, 4, 5, 4, 8>(s, threads, smem, st);
-    else if (nchunks <= 64) launch_step<1, 64, 8, false, 2, 8, 2, 5, 8, 8>(s, threads, smem, st);
-    else if (nchunks <= 96 && variant != 1) launch_step<3, 32, 2, false, 3, 8, 1, 8, 1, 8>(s, threads, smem, st);
-    else if (nchunks <= 128) launch_step<2, 64, 8, false, 2, 16, 2, 6, 2>(s, threads, smem, st);
-    else if (nchunks <= 192) launch_step<3, 64, 2, false, 3, 16, 1, 8, 1, 8>(s, threads, smem, st);
-    else if (nchunks <= 256) launch_step<4, 64, 4, false, 4, 16, 2, 5, 2>(s, threads, smem, st);
-    else if (nchunks <= 320) launch_step<5, 64, 2, false, 3, 32, 2, 6, 1>(s, threads, smem, st);
-    else if (nchunks <= 384) launch_step<6, 64, 2, false, 3, 32, 2, 6, 1>(s, threads, smem, st);
-    else if (nchunks <= 448) launch_step<7, 64, 2, false, 4, 32, 2, 5, 1>(s, threads, smem, st);
-    else launch_step<8, 64, 2, false, 4, 32, 2, 5, 1>(s, threads, smem, st);
+    if (nchunks > 512 || (!aligned && s.dim < 4)) launch_step<1, 64, 1, kRowScalar>(s, threads, smem, st);
+    else if (!aligned) vl_launch_step_unaligned(s, threads, smem, st);
+    else if (nchunks <= 16) launch_step<1, 16, 8, kRowAligned, 1, 8, 4, 5, 8, 8>(s, threads, smem, st);
+    else if (nchunks <= 32 && variant == 1) launch_step<1, 32, 8, kRowAligned>(s, threads, smem, st);
+    else if (nchunks <= 32) launch_step<2, 16, 4, kRowAligned, 1, 8, 4, 5, 4, 8>(s, threads, smem, st);
+    else if (nchunks <= 64) launch_step<1, 64, 8, kRowAligned, 2, 8, 2, 5, 8, 8>(s, threads, smem, st);
+    else if (nchunks <= 96 && variant != 1) launch_step<3, 32, 2, kRowAligned, 3, 8, 1, 8, 1, 8>(s, threads, smem, st);
+    else if (nchunks <= 128) launch_step<2, 64, 8, kRowAligned, 2, 16, 2, 6, 2>(s, threads, smem, st);
+    else if (nchunks <= 192) launch_step<3, 64, 2, kRowAligned, 3, 16, 1, 8, 1, 8>(s, threads, smem, st);
+    else if (nchunks <= 256) launch_step<4, 64, 4, kRowAligned, 4, 16, 2, 5, 2>(s, threads, smem, st);
+    else if (nchunks <= 320) launch_step<5, 64, 2, kRowAligned, 3, 32, 2, 6, 1>(s, threads, smem, st);
+    else if (nchunks <= 384) launch_step<6, 64, 2, kRowAligned, 3, 32, 2, 6, 1>(s, threads, smem, st);
+    else if (nchunks <= 448) launch_step<7, 64, 2, kRowAligned, 4, 32, 2, 5, 1>(s, threads, smem, st);
+    else launch_step<8, 64, 2, kRowAligned, 4, 32, 2, 5, 1>(s, threads, smem, st);
     VL_LAUNCH_CHECK("beam_step_kernel");
     g_step_launches.fetch_add(1, std::memory_order_relaxed);
     return VL_OK;

@@ -1,0 +1,77 @@
+// The kernels of the fused beam step and their launches; which shape serves which rows is decided in beam.hip and
+// beam_unaligned.hip.
+#pragma once
+#include "beam_row.h"
+
+namespace {
+
+// ---- the fused step: one launch per iteration, or per window of iterations ------
+// The expand phase (memory bound) and the merge phase (LDS / latency bound) of one
+// row run in the same workgroup, so on every CU some workgroups stream candidate
+// rows while others merge: the merge time hides behind the memory traffic, the
+// candidate ids and distances never leave LDS, and an iteration is one launch.
+template <int CPL, int LPR, int U, RowForm FORM, int THREADS>
+__global__ __launch_bounds__(THREADS) void beam_step_kernel(StepArgs s) {
+    beam_row<CPL, LPR, U, FORM, THREADS>(s);
+}
+// The same kernel built to leave room for WPP wavefronts per SIMD.  Its vector registers would allow that anyway;
+// what does not is its scalar registers (more than 96 of them mean seven wavefronts instead of eight), which the
+// compiler keeps within bounds when asked, at the price of a few moves to and from lanes of a vector register.
+template <int CPL, int LPR, int U, int THREADS, int WPP>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPP)))
+void beam_step_kernel_w(StepArgs s) {
+    beam_row<CPL, LPR, U, kRowAligned, THREADS>(s);
+}
+template <int CPL, int LPR, int U, RowForm FORM, int THREADS, int WPP>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPP))) void beam_window_kernel(StepArgs s) {
+    beam_row<CPL, LPR, U, FORM, THREADS, 0, 64, 1, true>(s);
+}
+template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int WPE>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void beam_window_sketch_kernel(StepArgs s) {
+    beam_row<CPL, LPR, U, kRowAligned, THREADS, SCPL, SLPR, SU, true>(s);
+}
+
+// The same step for rows that may use the sketch.  WPE: wavefronts per SIMD the compiler is asked to leave room
+// for.  The sketch's copy of the query row takes 16 registers per chunk and lane, and a row's phases (sketch
+// pass, two rounds of exact rows, merge) each wait on memory, so residency is worth a few spilled registers:
+// measured at 768 and 384 columns, five wavefronts per SIMD with two loads in flight beat three wavefronts
+// with four (0.84 -> 0.75 ms and 0.61 -> 0.43 ms per launch).  Residency is what a launch that is not bound by
+// memory traffic responds to (768 columns, state of the second optimisation loop, workgroups per compute unit
+// limited through LDS: 4 / 5 / 6 -> 0.53 / 0.46 / 0.42 ms per launch; 8 with one load in flight and 62 registers:
+// 0.415), which is also why the step's LDS arrays are overlaid where their lifetimes allow.
+template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int WPE>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
+void beam_step_sketch_kernel(StepArgs s) {
+    beam_row<CPL, LPR, U, kRowAligned, THREADS, SCPL, SLPR, SU>(s);
+}
+
+template <class Kernel>
+void launch_rows(Kernel kernel, int threads, const StepArgs &s, size_t smem, hipStream_t st) {
+    if (vl_allow_lds(kernel, smem) != hipSuccess) return;  // seen by the launch check
+    hipLaunchKernelGGL(kernel, dim3((unsigned)s.m.n_rows), dim3((unsigned)threads), smem, st, s);
+}
+
+template <int THREADS, int CPL, int LPR, int U, RowForm FORM, int SCPL, int SLPR, int SU, int WPE, int UX, int WPP>
+void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
+    if constexpr (SCPL > 0) {
+        if (s.sketch) {
+            if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, (WPE < 6 ? WPE : 6)>, THREADS, s, smem, st);
+            else launch_rows(beam_step_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, WPE>, THREADS, s, smem, st);
+            return;
+        }
+    }
+    if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, FORM, THREADS, (WPP > 0 ? 6 : 1)>, THREADS, s, smem, st);
+    else if constexpr (WPP > 0 && FORM != kRowScalar) launch_rows(beam_step_kernel_w<CPL, LPR, U, THREADS, WPP>, THREADS, s, smem, st);
+    else launch_rows(beam_step_kernel<CPL, LPR, U, FORM, THREADS>, THREADS, s, smem, st);
+}
+
+template <int CPL, int LPR, int U, RowForm FORM, int SCPL = 0, int SLPR = 64, int SU = 1, int WPE = 4, int UX = U, int WPP = 0>
+void launch_step(const StepArgs &s, int threads, size_t smem, hipStream_t st) {
+    if (threads == 128) launch_step_threads<128, CPL, LPR, U, FORM, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
+    else launch_step_threads<256, CPL, LPR, U, FORM, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
+}
+
+}  // namespace
+
+// Rows whose addresses are not all multiples of 16 bytes, of 4 to 2,048 elements (beam_unaligned.hip).
+void vl_launch_step_unaligned(const StepArgs &s, int threads, size_t smem, hipStream_t st);

@@ -211,7 +211,7 @@ __device__ __forceinline__ void two_lower_bounds(const uint64_t *a, int na, int 
 // between two progress checks depends on another row of the batch; the only batch-wide facts, the progress flag of the
 // checking iteration (ann.py:90-91) and the largest fill after the last of them, are written once.  Such a launch starts
 // right after a progress check (m.iter = k * readahead + 1, window = readahead).
-template <int CPL, int LPR, int U, bool GENERIC, int THREADS, int SCPL = 0, int SLPR = 64, int SU = 1, bool WINDOW = false>
+template <int CPL, int LPR, int U, RowForm FORM, int THREADS, int SCPL = 0, int SLPR = 64, int SU = 1, bool WINDOW = false>
 __device__ __forceinline__ void beam_row(const StepArgs &s) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kRows16 = THREADS / 16;
@@ -477,11 +477,11 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                 }
             }
             if (s.count_evals || resample) n_fetched += __popcll(__ballot(ok));
-            if constexpr (GENERIC)
+            if constexpr (FORM == kRowScalar)
                 wave_distances_generic(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0, memo_row, s.memo_shift, s.l2 != 0);
             else
-                wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0, order, memo_row,
-                                                s.memo_shift, s.l2 != 0);
+                wave_distances_lds<CPL, LPR, U, FORM == kRowUnaligned>(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0,
+                                                                       order, memo_row, s.memo_shift, s.l2 != 0);
         }
         const int stripe = (int)((blockIdx.x * (THREADS / kWave) + wave) & (kBeamStripes - 1));
         if (s.count_evals && lane == 0) {

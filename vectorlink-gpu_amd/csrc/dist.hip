@@ -65,7 +65,7 @@ __device__ __forceinline__ bool map_block(const ExpandArgs &a, int64_t &row, int
     return row < a.n_rows;
 }
 
-template <int CPL, int LPR, int U, bool GENERIC>
+template <int CPL, int LPR, int U, RowForm FORM>
 __global__ __launch_bounds__(256) void expand_kernel(ExpandArgs a) {
     int gate = 0;
     if (a.ctrl) {
@@ -122,34 +122,35 @@ __global__ __launch_bounds__(256) void expand_kernel(ExpandArgs a) {
         if (lane == 0 && okm) atomicAdd(&a.ctrl->evals[blockIdx.x & (kBeamStripes - 1)], (unsigned long long)__popcll(okm));
     }
     const float *q_row = a.queries + row * a.dim;
-    if constexpr (GENERIC)
+    if constexpr (FORM == kRowScalar)
         wave_distances_generic(q_row, a.vectors, a.dim, a.nchunks, id, ok, out_d, memo_row, a.memo_shift, a.l2 != 0);
     else
-        wave_distances<CPL, LPR, U>(q_row, a.vectors, a.dim, a.nchunks, id, ok, out_d, memo_row, a.memo_shift, a.l2 != 0);
+        wave_distances<CPL, LPR, U, FORM == kRowUnaligned>(q_row, a.vectors, a.dim, a.nchunks, id, ok, out_d, memo_row, a.memo_shift, a.l2 != 0);
 }
 
 template <int CPL, int LPR, int U>
-void launch_fast(const ExpandArgs &a, dim3 grid, hipStream_t st) {
-    hipLaunchKernelGGL((expand_kernel<CPL, LPR, U, false>), grid, dim3(256), 0, st, a);
+void launch_fast(const ExpandArgs &a, bool aligned, dim3 grid, hipStream_t st) {
+    if (aligned) hipLaunchKernelGGL((expand_kernel<CPL, LPR, U, kRowAligned>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((expand_kernel<CPL, LPR, U, kRowUnaligned>), grid, dim3(256), 0, st, a);
 }
 
 // one launch: c.n_rows * c.parts workgroups, rounded up to whole groups of 8 rows
 void launch_expand_piece(const ExpandArgs &a, bool aligned, hipStream_t st) {
     const int nchunks = a.nchunks;
     dim3 grid((unsigned)((a.n_rows + 7) / 8 * 8 * a.parts));
-    if (!aligned || nchunks > 512) {
-        hipLaunchKernelGGL((expand_kernel<1, 64, 1, true>), grid, dim3(256), 0, st, a);
-    } else if (nchunks <= 16) launch_fast<1, 16, 8>(a, grid, st);
-    else if (nchunks <= 32) launch_fast<2, 16, 4>(a, grid, st);
-    else if (nchunks <= 64) launch_fast<1, 64, 8>(a, grid, st);
-    else if (nchunks <= 96) launch_fast<3, 32, 4>(a, grid, st);
-    else if (nchunks <= 128) launch_fast<2, 64, 8>(a, grid, st);
-    else if (nchunks <= 192) launch_fast<3, 64, 4>(a, grid, st);
-    else if (nchunks <= 256) launch_fast<4, 64, 4>(a, grid, st);
-    else if (nchunks <= 320) launch_fast<5, 64, 2>(a, grid, st);
-    else if (nchunks <= 384) launch_fast<6, 64, 2>(a, grid, st);
-    else if (nchunks <= 448) launch_fast<7, 64, 2>(a, grid, st);
-    else launch_fast<8, 64, 2>(a, grid, st);
+    if (nchunks > 512 || (!aligned && a.dim < 4)) {
+        hipLaunchKernelGGL((expand_kernel<1, 64, 1, kRowScalar>), grid, dim3(256), 0, st, a);
+    } else if (nchunks <= 16) launch_fast<1, 16, 8>(a, aligned, grid, st);
+    else if (nchunks <= 32) launch_fast<2, 16, 4>(a, aligned, grid, st);
+    else if (nchunks <= 64) launch_fast<1, 64, 8>(a, aligned, grid, st);
+    else if (nchunks <= 96) launch_fast<3, 32, 4>(a, aligned, grid, st);
+    else if (nchunks <= 128) launch_fast<2, 64, 8>(a, aligned, grid, st);
+    else if (nchunks <= 192) launch_fast<3, 64, 4>(a, aligned, grid, st);
+    else if (nchunks <= 256) launch_fast<4, 64, 4>(a, aligned, grid, st);
+    else if (nchunks <= 320) launch_fast<5, 64, 2>(a, aligned, grid, st);
+    else if (nchunks <= 384) launch_fast<6, 64, 2>(a, aligned, grid, st);
+    else if (nchunks <= 448) launch_fast<7, 64, 2>(a, aligned, grid, st);
+    else launch_fast<8, 64, 2>(a, aligned, grid, st);
 }
 
 }  // namespace

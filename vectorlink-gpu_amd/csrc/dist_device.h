@@ -12,6 +12,9 @@ __device__ __forceinline__ int own_lane() {
     return lane;
 }
 
+// How rows are read: 16 bytes at a time (at multiples of 16, or of 4), or element by element.
+enum RowForm { kRowAligned, kRowUnaligned, kRowScalar };
+
 __device__ __forceinline__ float clamp_distance(float cos_theta) {
     float r = (1.0f - cos_theta) * 0.5f;  // kernels.py:109
     if (r < 0.0f) r = 0.0f;               // kernels.py:110-113
@@ -94,9 +97,38 @@ __device__ __forceinline__ float fold_group(float acc) {
     return acc;
 }
 
+// The chunks of a row that a lane of an LPR-lane group holds: lig, lig + LPR, ... (CPL of them; the row's last chunk is
+// somebody's CPL-th, which is how the shapes are chosen).  UNALIGNED: rows of any length from 4 elements on, at any
+// address.  The loads are as wide (gfx950 takes them at any multiple of 4 bytes); the one of a short last chunk ends with
+// the row's last element, and what it holds of the chunk before becomes zero - in the query row as well, so these products
+// add nothing and the others keep their order.
+template <int CPL, int LPR, bool UNALIGNED>
+struct RowChunks {
+    typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
+    bool valid[CPL];
+    int lig, last, drop;  // UNALIGNED: first element of the last load, elements of it that belong to the chunk before
+
+    __device__ __forceinline__ RowChunks(int lig_, int dim, int nchunks) : lig(lig_) {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) valid[i] = lig + LPR * i < nchunks;
+        if constexpr (UNALIGNED) {
+            last = 4 * (lig + LPR * (CPL - 1));
+            drop = max(last + 4 - dim, 0);
+            last -= drop;
+        }
+    }
+    __device__ __forceinline__ float4 load(const float *row, int i) const {
+        if (!valid[i]) return make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (!UNALIGNED) return reinterpret_cast<const float4 *>(row)[lig + LPR * i];
+        const float4_any v = *reinterpret_cast<const float4_any *>(row + (i == CPL - 1 ? last : 4 * (lig + LPR * i)));
+        if (i < CPL - 1) return make_float4(v.x, v.y, v.z, v.w);
+        return make_float4(drop > 0 ? 0.f : v.x, drop > 1 ? 0.f : v.y, drop > 2 ? 0.f : v.z, v.w);
+    }
+};
+
 // One wavefront: lane j holds candidate id `my_id` (valid when `ok`); the
 // distance of candidate lane j to the query goes to out_d[j].
-template <int CPL, int LPR, int U>
+template <int CPL, int LPR, int U, bool UNALIGNED = false>
 __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
                                                const float *__restrict__ vectors, int dim,
                                                int nchunks, int32_t my_id, bool ok,
@@ -107,14 +139,10 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
     const int grp = lane / LPR;
     const int lig = lane % LPR;
 
+    const RowChunks<CPL, LPR, UNALIGNED> chunks(lig, dim, nchunks);
     float4 q[CPL];
-    bool cvalid[CPL];
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-        int c = lig + LPR * i;
-        cvalid[i] = c < nchunks;
-        q[i] = cvalid[i] ? reinterpret_cast<const float4 *>(q_row)[c] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    for (int i = 0; i < CPL; ++i) q[i] = chunks.load(q_row, i);
 
     uint64_t mask = __ballot(ok);
     while (mask) {
@@ -147,10 +175,10 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
                 id = __shfl(my_id, s >= 0 ? s : 0);
             }
             ids[u] = id;
-            const float4 *row = reinterpret_cast<const float4 *>(vectors + (int64_t)id * dim);
+            const float *row = vectors + (int64_t)id * dim;
 #pragma unroll
             for (int i = 0; i < CPL; ++i) {
-                if (s >= 0 && cvalid[i]) r[u][i] = row[lig + LPR * i];
+                if (s >= 0) r[u][i] = chunks.load(row, i);
                 else r[u][i] = make_float4(0.f, 0.f, 0.f, 0.f);
             }
         }
@@ -210,7 +238,7 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
 // row), and the group's first lane parks the row's sum in out_d of its candidate.  Turning a sum into a distance
 // and storing the cache entry is then each lane's own work for its own candidate, once for the wavefront instead
 // of once per load.  Same loads, same additions in the same order, same bits as wave_distances.
-template <int CPL, int LPR, int U>
+template <int CPL, int LPR, int U, bool UNALIGNED = false>
 __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_row,
                                                    const float *__restrict__ vectors, int dim,
                                                    int nchunks, int32_t my_id, bool ok,
@@ -224,14 +252,10 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
     const int lig = lane % LPR;
     const int n = __popcll(mask);
 
+    const RowChunks<CPL, LPR, UNALIGNED> chunks(lig, dim, nchunks);
     float4 q[CPL];
-    bool cvalid[CPL];
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-        int c = lig + LPR * i;
-        cvalid[i] = c < nchunks;
-        q[i] = cvalid[i] ? reinterpret_cast<const float4 *>(q_row)[c] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    for (int i = 0; i < CPL; ++i) q[i] = chunks.load(q_row, i);
     if constexpr (G > 1) {
         if (ok) order[__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] = (uint8_t)lane;
     }
@@ -250,12 +274,9 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
                     src[u] = order[min(k0 + u * G + grp, n - 1)];
                     id = __shfl(my_id, src[u]);
                 }
-                const float4 *row = reinterpret_cast<const float4 *>(vectors + (int64_t)id * dim);
+                const float *row = vectors + (int64_t)id * dim;
 #pragma unroll
-                for (int i = 0; i < CPL; ++i) {
-                    if (cvalid[i]) r[u][i] = row[lig + LPR * i];
-                    else r[u][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                }
+                for (int i = 0; i < CPL; ++i) r[u][i] = chunks.load(row, i);
             }
         }
 #pragma unroll
@@ -305,7 +326,7 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
     }
 }
 
-// Any dimension, any alignment: scalar loads, same summation order.
+// Rows of fewer than 4 elements or more than 2,048: scalar loads, one row at a time, same summation order.
 __device__ __forceinline__ void wave_distances_generic(const float *__restrict__ q_row,
                                                        const float *__restrict__ vectors, int dim,
                                                        int nchunks, int32_t my_id, bool ok,
