@@ -85,6 +85,12 @@ def test_host_side_validation(lib):
     assert lib.vl_search_from_seeds(None, 0, 8, None, 4, None, 10, 4, None, 10, None, None, None) == 0
 
 
+def test_knn_workspace_of_many_queries(lib):
+    """The buffers of the bfloat16 filter (16 KB a query and more) are for a bounded number of queries."""
+    few, many = (lib.vl_knn_workspace_bytes(n, 1_000_000, 768, 10) for n in (1 << 17, 1 << 23))
+    assert 0 < few and many - few < 1024 * ((1 << 23) - (1 << 17))  # 4 lists of 10 keys and two words a query
+
+
 def test_cpu_tensors_are_refused():
     import torch
 

@@ -112,3 +112,41 @@ def test_what_the_filter_leaves_to_the_tiles(bad):
         assert torch.equal(gi[s:s + 32], fi) and torch.equal(gd[s:s + 32], fd)
     if bad == "equal rows":
         assert np.array_equal(gi[:200].cpu().numpy(), np.tile(np.arange(10, dtype=np.int32), (200, 1)))
+
+
+@pytest.mark.parametrize("n,dim,nq,k,metric", [(9000, 32, 300, 10, "cosine"), (40_000, 64, 130, 16, "l2"), (70_000, 16, 3, 4, "l2")])
+def test_a_workspace_for_the_tiles_alone(n, dim, nq, k, metric):
+    """The tiles want at most 256 lists of 16 keys a query, two words a query and one a vector; a call that brings no more
+    than that is answered by them, with the same bits."""
+    print(f"small workspace n={n} dim={dim} nq={nq} k={k} {metric}", flush=True)
+    from vectorlink_gpu import _native as nv
+    from vectorlink_gpu.kernels import knn_exact
+
+    rng = np.random.default_rng(n)
+    v, q = dev(rows(rng, n, dim)), dev(rows(rng, nq, dim))
+    (wi, wd) = knn_exact(q, v, k, metric)
+    most = nv.lib().vl_knn_workspace_bytes(nq, n, dim, k)
+    small = nq * 256 * 16 * 8 + (2 * nq + n) * 4 + 16
+    if nq > 128:
+        small = min(small, most - 1)  # one byte less than the filter's
+    ws = torch.empty(small, dtype=torch.uint8, device=DEV)
+    ids = torch.empty((nq, k), dtype=torch.int32, device=DEV)
+    d = torch.empty((nq, k), dtype=torch.float32, device=DEV)
+    nv.check(nv.lib().vl_knn_exact_metric(nv.ptr(q), nq, nv.ptr(v), n, dim, k, nv.metric_code(metric), nv.ptr(ids),
+                                          nv.ptr(d), nv.ptr(ws), ws.numel(), nv.stream()))
+    assert torch.equal(ids, wi) and torch.equal(d, wd)
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+def test_more_queries_than_the_filter_takes_at_a_time(metric):
+    """65,536 at a time: a second piece of 200, with its own block flags."""
+    print(f"two pieces of queries {metric}", flush=True)
+    from vectorlink_gpu.kernels import knn_exact
+
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    v = torch.nn.functional.normalize(torch.randn((4096, 16), generator=gen, device=DEV), dim=1)
+    q = torch.nn.functional.normalize(torch.randn((65_736, 16), generator=gen, device=DEV), dim=1)
+    (gi, gd) = knn_exact(q, v, 4, metric)
+    for s in (0, 65_408, 65_536, 65_636):
+        (fi, fd) = knn_exact(q[s:s + 100].contiguous(), v, 4, metric)
+        assert torch.equal(gi[s:s + 100], fi) and torch.equal(gd[s:s + 100], fd)

@@ -62,20 +62,18 @@ struct EventSet {
 };
 
 // Pinned host memory for the reports of the progress checks: one page of slots for the whole process, made with the
-// first call and kept; a call borrows a slot.  With every slot lent out (64 calls at once) or no page to be had, a call
+// first call that can and kept; a call borrows a slot.  With every slot lent out (64 calls at once) or no page to be had, a call
 // waits for its stream at every check and fetches the flags instead.
 class ReportSlot {
 public:
     ReportSlot() {
         std::lock_guard<std::mutex> hold(mutex_);
-        if (!page_ && !refused_) {
+        if (!page_) {
             void *p = nullptr;
             if (hipHostMalloc(&p, kSlots * sizeof(Slot), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess)
                 page_ = static_cast<Slot *>(p);
-            else {
-                refused_ = true;
+            else
                 (void)hipGetLastError();
-            }
         }
         for (int i = 0; page_ && i < kSlots; ++i)
             if (!((lent_ >> i) & 1)) {
@@ -99,7 +97,6 @@ private:
     struct alignas(64) Slot { BeamReport report; };
     static inline std::mutex mutex_;
     static inline Slot *page_ = nullptr;
-    static inline bool refused_ = false;
     static inline uint64_t lent_ = 0;
     int index_ = -1;
 };

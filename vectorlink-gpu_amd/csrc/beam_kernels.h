@@ -61,7 +61,7 @@ void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
         }
     }
     if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, FORM, THREADS, (WPP > 0 ? 6 : 1)>, THREADS, s, smem, st);
-    else if constexpr (WPP > 0 && FORM != kRowScalar) launch_rows(beam_step_kernel_w<CPL, LPR, U, THREADS, WPP>, THREADS, s, smem, st);
+    else if constexpr (WPP > 0 && FORM == kRowAligned) launch_rows(beam_step_kernel_w<CPL, LPR, U, THREADS, WPP>, THREADS, s, smem, st);
     else launch_rows(beam_step_kernel<CPL, LPR, U, FORM, THREADS>, THREADS, s, smem, st);
 }
 

@@ -403,8 +403,14 @@ struct KnnPlan {
     int64_t bytes;
 };
 
-// l2: the plan of an L2 call; its workspace is never smaller than a cosine call's.
-int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, KnnPlan *p) {
+// Queries that go through the filter at a time (whole blocks of TQ): its buffers take 16 to 20 KB a query, and a pass
+// over that many queries takes a hundred times as long as converting the table again.
+constexpr int64_t kFilterQueries = 65536;
+static_assert(kFilterQueries % TQ == 0, "flags are kept per block of TQ queries");
+
+// l2: the plan of an L2 call; its workspace is never smaller than a cosine call's.  most: bytes of workspace there are; a
+// call with too few for the form that would take it goes to the tiles alone, with the same bits.
+int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, int64_t most, KnnPlan *p) {
     VL_REQUIRE(n_queries >= 0 && n_vectors > 0 && dim > 0, "bad sizes");
     VL_REQUIRE(k >= 1 && k <= KMAX, "k must be between 1 and %d", KMAX);
     VL_REQUIRE(dim % 4 == 0, "exact kNN tiles need a dimension that is a multiple of 4");
@@ -432,16 +438,26 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
     p->n_strips = (int)strips;
     p->strip_len = len;
     p->list_len = list_length(k);
-    p->n_cand = (int)(strips * LISTS_PER_STRIP * p->list_len);
+    auto lists = [&](int64_t n_lists) {  // bytes for that many lists of a query, bounds and squared lengths
+        p->n_cand = (int)(n_lists * p->list_len);
+        p->cand_bytes = (n_queries > 0 ? n_queries : 1) * (int64_t)p->n_cand * 8;
+        return p->cand_bytes + ((2 * n_queries + n_vectors) * 4 + 15) / 16 * 16;
+    };
     p->few = vl_knn_is_few(n_queries, n_vectors, dim);
-    if (p->few) p->n_cand = (int)(vl_knn_few_lists(n_vectors) * p->list_len);
-    p->cand_bytes = (n_queries > 0 ? n_queries : 1) * (int64_t)p->n_cand * 8;
-    p->bytes = p->cand_bytes + ((2 * n_queries + n_vectors) * 4 + 15) / 16 * 16;
-    p->filter = !p->few && vl_knn_filter_plan(n_queries, n_vectors, dim, k, l2, &p->fp);
+    if (p->few) {
+        p->bytes = lists(vl_knn_few_lists(n_vectors));
+        p->filter = false;
+        if (p->bytes <= most) return VL_OK;
+        p->few = false;
+    }
+    p->bytes = lists(strips * LISTS_PER_STRIP);
+    p->filter = vl_knn_filter_plan(n_queries < kFilterQueries ? n_queries : kFilterQueries, n_vectors, dim, k, l2, &p->fp);
     if (p->filter) {
         p->off_flags = (p->bytes + 255) / 256 * 256;
         p->off_filter = (p->off_flags + q_blocks * 4 + 255) / 256 * 256;
-        p->bytes = p->off_filter + p->fp.bytes + 256;  // (the workspace itself may be 16-byte aligned only)
+        const int64_t bytes = p->off_filter + p->fp.bytes + 256;  // (the workspace itself may be 16-byte aligned only)
+        if (bytes <= most) p->bytes = bytes;
+        else p->filter = false;
     }
     return VL_OK;
 }
@@ -450,7 +466,7 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
 
 VL_EXPORT int64_t vl_knn_workspace_bytes(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k) {
     KnnPlan p;
-    int rc = knn_plan(n_queries, n_vectors, dim, k, true, &p);  // serves both metrics
+    int rc = knn_plan(n_queries, n_vectors, dim, k, true, INT64_MAX, &p);  // serves both metrics
     return rc < 0 ? rc : p.bytes;
 }
 
@@ -467,7 +483,7 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     VL_REQUIRE(metric == VL_METRIC_COSINE || metric == VL_METRIC_L2, "unknown metric %d", (int)metric);
     KnnPlan p;
     const bool l2 = metric == VL_METRIC_L2;
-    int rc = knn_plan(n_queries, n_vectors, dim, k, l2, &p);
+    int rc = knn_plan(n_queries, n_vectors, dim, k, l2, workspace_bytes, &p);
     if (rc < 0) return rc;
     if (n_queries == 0) return VL_OK;
     VL_REQUIRE(queries && vectors && ids_out && dists_out && workspace, "null pointer");
@@ -496,9 +512,12 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     if (p.filter) {
         int32_t *flags = (int32_t *)(ws + p.off_flags);
         char *const filter_ws = (char *)(((uintptr_t)(ws + p.off_filter) + 255) / 256 * 256);
-        rc = vl_knn_filter(p.fp, queries, n_queries, vectors, n_vectors, dim, k, l2, q_norm, v_norm, flags, TQ,
-                           filter_ws, ids_out, dists_out, st);
-        if (rc < 0) return rc;
+        for (int64_t q0 = 0; q0 < n_queries; q0 += kFilterQueries) {
+            const int64_t n = n_queries - q0 < kFilterQueries ? n_queries - q0 : kFilterQueries;
+            rc = vl_knn_filter(p.fp, queries + q0 * dim, n, vectors, n_vectors, dim, k, l2, q_norm + q0, v_norm,
+                               flags + q0 / TQ, TQ, filter_ws, ids_out + q0 * k, dists_out + q0 * k, st);
+            if (rc < 0) return rc;
+        }
         wanted = flags;
     } else if (l2) {
         VL_REQUIRE((n_vectors + 3) / 4 <= kMaxBlocks * 4, "too many vectors for one call");

@@ -12,7 +12,7 @@ struct KnnFilterPlan {
     int64_t off_q16, off_v16, off_qstat, off_gmax, off_bound, off_count, off_found, off_vmax, bytes;
 };
 
-// Whether a call is taken by the filter, and its plan.
+// Whether a call is taken by the filter, and its plan, which also serves a call of fewer queries.
 bool vl_knn_filter_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, KnnFilterPlan *p);
 
 // Writes the answers of every query whose candidates fit its buffer and leaves, per block of flag_queries queries,
