@@ -181,9 +181,31 @@ __device__ __forceinline__ uint32_t rank_among(const uint32_t *red, int *rank) {
     return mine;
 }
 
+// A count that all lanes of the wavefront have read from LDS, in a scalar register if SCALAR: loops up to it have no lane masks.
+template <bool SCALAR>
+__device__ __forceinline__ int same_in_all(int x) {
+    return SCALAR ? __builtin_amdgcn_readfirstlane(x) : x;
+}
+
+// keys: n of them in LDS (n the same in all lanes); places past the last are not read.  N reads are on their way at a time:
+// one after the other, a key costs the latency of LDS.
+template <int N>
 __device__ __forceinline__ int count_below(const uint64_t *keys, int n, uint64_t k) {
-    int c = 0;
-    for (int i = 0; i < n; ++i) c += keys[i] < k;
+    int c = 0, i = 0;
+    for (; i + N <= n; i += N) {
+        uint64_t x[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) x[j] = keys[i + j];
+#pragma unroll
+        for (int j = 0; j < N; ++j) c += x[j] < k;
+    }
+    if (N > 1 && i < n) {
+        uint64_t x[N];
+#pragma unroll
+        for (int j = 0; j < N - 1; ++j) x[j] = keys[i + j < n ? i + j : n - 1];
+#pragma unroll
+        for (int j = 0; j < N - 1; ++j) c += i + j < n && x[j] < k;
+    }
     return c;
 }
 
@@ -215,6 +237,13 @@ template <int CPL, int LPR, int U, RowForm FORM, int THREADS, int SCPL = 0, int 
 __device__ __forceinline__ void beam_row(const StepArgs &s) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kRows16 = THREADS / 16;
+    // Queue keys read at a time when places are counted: eight for several iterations of rows of up to 384 elements (256
+    // queries at 4,096 x 128 1,006 -> 969 us, 10,000 at 1M x 128 2,063 -> 2,017, a build of 6,007 x 384 17.5 -> 17.0 ms).
+    // Longer rows hide the latency behind each other's loads (1,000 queries at 100,003 x 1,536 1,239 us with one, 1,267 with
+    // eight; 10,000 at 1M x 768 3,513 and 3,527), and the kernels of one iteration have no registers left for it (a build of
+    // 20,011 x 768 133.1 and 133.7 ms).
+    constexpr bool kShortRows = WINDOW && SCPL == 0 && CPL * LPR <= 96;
+    constexpr int kAtOnce = kShortRows ? 8 : 1;
     __shared__ int32_t visit_s[kMaxVisit];  // the ids popped from the visit queue in this iteration
     __shared__ uint32_t red[kRows16];
     __shared__ int n_ex_s;                  // exclusion ids before the row's first empty one
@@ -499,7 +528,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
             s.memo_rate[row] = word;
             word_s = word;
         }
-        const int n_ex = n_ex_s;
+        const int n_ex = same_in_all<kShortRows>(n_ex_s);
         const uint64_t *const va = vq + a.Vt;
         const uint64_t ws = qa[a.L - 1];                       // the search queue's last slot
         const uint64_t wv = nva > 0 ? va[nva - 1] : 0ull;       // the visit queue's last live slot
@@ -654,7 +683,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
             if (want) keys[base + __popcll(all & ((1ull << lane) - 1))] = k;
         }
         __syncthreads();
-        const int n_keys = n_keys_s;
+        const int n_keys = same_in_all<kShortRows>(n_keys_s);
 
         // ---- the survivors' places in the queues; the new ones among them ----
         const int top = 1 << (31 - __builtin_clz(max(a.L, max(nva, 1))));
@@ -694,7 +723,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
             collect(new_v, k, to_visit, &n_fresh_s);
         }
         __syncthreads();
-        const int n_search = n_search_s, n_fresh = n_fresh_s;
+        const int n_search = same_in_all<kShortRows>(n_search_s), n_fresh = same_in_all<kShortRows>(n_fresh_s);
 
         // ---- search_queue.insert (ann.py:75-80) and visit_queue.insert (ann.py:85-88) ----
         auto put_search = [&](int r, uint64_t k) {
@@ -717,26 +746,26 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         if (n_search)
             for (int i = tid; i < a.L; i += THREADS) {
                 const uint64_t k = qa[i];
-                const int r = i + count_below(to_search, n_search, k);
+                const int r = i + count_below<kAtOnce>(to_search, n_search, k);
                 if (r < a.L && (WINDOW || r != i)) put_search(r, k);
             }
         if (!seen_full)
             for (int i = tid; i < nva; i += THREADS) {
                 const uint64_t k = va[i];
-                const int r = i + count_below(to_visit, n_fresh, k);
+                const int r = i + count_below<kAtOnce>(to_visit, n_fresh, k);
                 if (r < a.VL && (WINDOW || r != a.Vt + i)) put_visit(r, k);
             }
         for (int j0 = 0; j0 < n_keys; j0 += THREADS) {
             if (j0 > 0) look_up(j0 + tid, &k0, &in_q0, &in_v0, &new_q0, &new_v0);
             if (new_q0) {
-                const int r = in_q0 + count_below(to_search, n_search, k0);
+                const int r = in_q0 + count_below<kAtOnce>(to_search, n_search, k0);
                 if (r < a.L) {
                     put_search(r, k0);
                     diff = true;  // a new id inside the first L slots: the row changed (queue.py:57-59)
                 }
             }
             if (new_v0) {
-                const int r = in_v0 + count_below(to_visit, n_fresh, k0);
+                const int r = in_v0 + count_below<kAtOnce>(to_visit, n_fresh, k0);
                 if (r < a.VL) put_visit(r, k0);
             }
         }
@@ -769,7 +798,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
             // places of those stay reachable)
             for (int i = tid; i < a.m; i += THREADS)
                 if (set_slot[i] != 0xffffu) set[set_slot[i]] = -1;
-            cnt += n_new_s;
+            cnt += same_in_all<kShortRows>(n_new_s);
             if (n_search) {
                 uint64_t *const x = qa;
                 qa = qa_next;
