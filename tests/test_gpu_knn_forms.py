@@ -150,3 +150,26 @@ def test_more_queries_than_the_filter_takes_at_a_time(metric):
     for s in (0, 65_408, 65_536, 65_636):
         (fi, fd) = knn_exact(q[s:s + 100].contiguous(), v, 4, metric)
         assert torch.equal(gi[s:s + 100], fi) and torch.equal(gd[s:s + 100], fd)
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("bad", ["nan", "inf", "long"])
+def test_no_bound_in_a_short_last_piece_of_the_table(bad, metric):
+    """2 GiB of 64 columns are 16,777,216 rows: the second piece of the table is 100 rows of a tile of 256, and one of them
+    takes that piece's error bound beyond every value.  The 156 places behind the last row must not become candidates."""
+    print(f"short last piece with {bad} {metric}", flush=True)
+    from vectorlink_gpu.kernels import knn_exact
+
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    n = (1 << 24) + 100
+    v = torch.nn.functional.normalize(torch.randn((n, 4), generator=gen, device=DEV), dim=1)
+    q = torch.nn.functional.normalize(torch.randn((150, 4), generator=gen, device=DEV), dim=1)
+    if bad == "long":
+        v[n - 7] *= 1e6
+    else:
+        v[n - 7, 2] = float(bad)
+    (gi, gd) = knn_exact(q, v, 4, metric)
+    assert int(gi.max()) < n and int(gi.min()) >= 0
+    for s in range(0, 150, 32):
+        (fi, fd) = knn_exact(q[s:s + 32].contiguous(), v, 4, metric)
+        assert torch.equal(gi[s:s + 32], fi) and torch.equal(gd[s:s + 32], fd)

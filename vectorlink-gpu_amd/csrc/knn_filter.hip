@@ -199,8 +199,15 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
         if constexpr (EMIT) {
             const int64_t q = q0 + 64 * wc + 32 * cb + l32;
             thr[cb] = __builtin_inff();
-            if (q < n_queries) thr[cb] = bound[q] - value_error(qstat[q], table, dim, l2 != 0);
-            if (thr[cb] != thr[cb] || (!l2 && thr[cb] <= -0.999f)) thr[cb] = -__builtin_inff();
+            if (q < n_queries) {
+                thr[cb] = bound[q] - value_error(qstat[q], table, dim, l2 != 0);
+                // No bound (a row that is not finite, or so long that its rounding covers every value): the query is
+                // left to the tiles.  So a threshold is above -infinity, which is what rows past the strip's end hold.
+                if (!(thr[cb] > (l2 ? -__builtin_inff() : -0.999f))) {
+                    thr[cb] = __builtin_inff();
+                    if (strip == 0 && wr == 0 && half == 0) atomicAdd(&count[q], kFound + 1);
+                }
+            }
         }
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) top[cb][rb] = -__builtin_inff();
