@@ -61,62 +61,21 @@ struct EventSet {
     }
 };
 
-// Pinned host memory for the reports of the progress checks: one page of slots for the whole process, made with the
-// first call that can and kept; a call borrows a slot.  With every slot lent out (64 calls at once) or no page to be had, a call
-// waits for its stream at every check and fetches the flags instead.
-class ReportSlot {
-public:
-    ReportSlot() {
-        std::lock_guard<std::mutex> hold(mutex_);
-        if (!page_) {
-            void *p = nullptr;
-            if (hipHostMalloc(&p, kSlots * sizeof(Slot), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess)
-                page_ = static_cast<Slot *>(p);
-            else
-                (void)hipGetLastError();
-        }
-        for (int i = 0; page_ && i < kSlots; ++i)
-            if (!((lent_ >> i) & 1)) {
-                lent_ |= 1ull << i;
-                index_ = i;
-                page_[i].report.check = 0;
-                break;
-            }
+// What beam_report.h asks of the HIP runtime, for the stream of a call.
+struct StreamOfCall {
+    hipStream_t st;
+    static void *pinned(size_t bytes) {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, bytes, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
     }
-    ~ReportSlot() {
-        if (index_ < 0) return;
-        std::lock_guard<std::mutex> hold(mutex_);
-        lent_ &= ~(1ull << index_);
+    int state() const {
+        const hipError_t e = hipStreamQuery(st);
+        return e == hipSuccess ? 0 : (e == hipErrorNotReady ? 1 : -1 - (int)e);
     }
-    ReportSlot(const ReportSlot &) = delete;
-    ReportSlot &operator=(const ReportSlot &) = delete;
-    BeamReport *get() const { return index_ < 0 ? nullptr : &page_[index_].report; }
-
-private:
-    static constexpr int kSlots = 64;
-    struct alignas(64) Slot { BeamReport report; };
-    static inline std::mutex mutex_;
-    static inline Slot *page_ = nullptr;
-    static inline uint64_t lent_ = 0;
-    int index_ = -1;
+    bool drain() const { return hipStreamSynchronize(st) == hipSuccess; }
 };
-
-// Waits until the launch behind the check after iteration t has reported.  The stream is asked now and then, so that a
-// launch that failed ends the wait.
-int wait_for_report(const BeamReport *r, int t, hipStream_t st) {
-    for (unsigned spins = 1;; ++spins) {
-        if (__atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t) return VL_OK;
-        if ((spins & 0xffff) == 0) {
-            const hipError_t e = hipStreamQuery(st);
-            if (e == hipErrorNotReady) continue;
-            VL_HIP(e);
-            if (__atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t) return VL_OK;
-            vl_set_error("the progress check after iteration %d was not reported", t);
-            return VL_ERR_HIP;
-        }
-        __builtin_ia32_pause();
-    }
-}
 
 __device__ inline bool sorted_contains(const int32_t *a, int n, int32_t v) {
     int lo = 0, hi = n;
@@ -790,6 +749,15 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     VL_REQUIRE(p->n_rows * (int64_t)l.VL < (1ll << 31), "batch too large: %lld rows with visit queues of %d slots",
                (long long)p->n_rows, (int)l.VL);
     hipStream_t st = (hipStream_t)stream;
+    if (fixed_iterations == 0) {  // refused before anything is recorded: the loop waits for what its launches find
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &capturing) != hipSuccess) (void)hipGetLastError();
+        if (capturing != hipStreamCaptureStatusNone) {
+            vl_set_error("this call waits for its stream and cannot be captured into a graph "
+                         "(vl_closest_vectors_noalloc can)");
+            return VL_ERR_HIP;
+        }
+    }
     char *ws = (char *)workspace;
     int32_t *cand_ids = (int32_t *)(ws + l.off_cand_ids);
     float *cand_d = (float *)(ws + l.off_cand_d);
@@ -990,7 +958,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     // A call that is not profiled keeps the GPU busy across its progress checks: the launch after a checking iteration
     // is enqueued before the host knows what the check found - it does nothing if the check ended the loop (beam_gate)
     // - and reports it from its first workgroup.
-    ReportSlot slot;
+    ReportSlot<StreamOfCall> slot(StreamOfCall{st});
     const bool ahead = use_fused && !prof && slot.get() != nullptr;
     step.report = ahead ? slot.get() : nullptr;
     auto launch_next = [&]() -> int {  // the fused launch that follows iteration t; moves t on
@@ -1008,6 +976,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     int64_t checked = 0;  // iterations up to the last progress check
     for (;;) {
         int launches = 0;  // of this stretch between two progress checks
+        slot.launching();
         checked += R;
         while (t < checked) {
             const int at = launches++;
@@ -1039,11 +1008,18 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
         if (ahead) {
             rc = launch_next();
             if (rc < 0) return rc;
-            rc = wait_for_report(slot.get(), (int)checked, st);
-            if (rc < 0) return rc;
+            const int waited = slot.wait((int)checked);
+            if (waited < -1) VL_HIP((hipError_t)(-1 - waited));
+            if (waited < 0) {
+                vl_set_error("the progress check after iteration %lld was not reported", (long long)checked);
+                return VL_ERR_HIP;
+            }
             found = *slot.get();
             // the launch that has nothing left to do is waited for: the caller may use the workspace on another stream
-            if (!found.changed || found.error) VL_HIP(hipStreamSynchronize(st));
+            if (!found.changed || found.error) {
+                VL_HIP(hipStreamSynchronize(st));
+                slot.drained();
+            }
         } else {
             // one copy brings the ring of progress flags and the two words behind it (they are neighbours in the
             // control block): this check's flag, the rows still using the sketch, the error flag
@@ -1056,6 +1032,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
                           "changed[64], sketch_rows, error follow each other");
             VL_HIP(hipMemcpyAsync(&seen_by_host, &ctrl->changed[0], sizeof(seen_by_host), hipMemcpyDeviceToHost, st));
             VL_HIP(hipStreamSynchronize(st));
+            slot.drained();
             found.changed = seen_by_host.changed[(checked / R) & 63];
             found.sketch_rows = seen_by_host.sketch_rows;
             found.error = seen_by_host.error;

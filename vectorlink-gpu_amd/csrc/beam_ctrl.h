@@ -16,6 +16,7 @@
 // iterations of 256 queries at 4,096 x 128 take 105 us).
 #pragma once
 #include "vl_common.h"
+#include "beam_report.h"
 
 constexpr int kBeamStripes = 1024;
 
@@ -33,10 +34,6 @@ struct BeamCtrl {
     unsigned long long sketched[kBeamStripes];  // candidate rows looked at through the 8-bit sketch only
 };
 
-struct BeamReport {
-    int changed, sketch_rows, error;  // as in BeamCtrl, after the checking iteration
-    int check;                        // written last: iterations run up to that check
-};
 __device__ inline void beam_report(const BeamCtrl *c, int t, int R, BeamReport *out) {
     out->changed = c->changed[(t / R) & 63];
     out->sketch_rows = c->sketch_rows;

@@ -1,0 +1,72 @@
+// The host's side of the beam loop's progress checks.  Nothing here needs the HIP runtime: what of it is used comes in as
+// Gpu, which has
+//   static void *pinned(size_t)  host memory that the GPU writes to, or null
+//   int state()                  of the call's stream: 0 has ended, 1 still runs, below 0 an error
+//   bool drain()                 waits for the stream; false: an error, what runs there may go on
+#pragma once
+#include <stddef.h>
+#include <stdint.h>
+#include <mutex>
+
+struct BeamReport {
+    int changed, sketch_rows, error;  // as in BeamCtrl, after the checking iteration
+    int check;                        // written last: iterations run up to that check
+};
+
+// Pinned host memory for the reports: one page of slots for the whole process, made with the first call that can and kept;
+// a call borrows a slot.  With every slot lent out (64 calls at once) or no page to be had, a call waits for its stream at
+// every check and fetches the flags instead.  A slot is given back when nothing that may write to it is left on the stream:
+// a call that ends early, with launches still on their way, waits for them here (they use its workspace as well), and one
+// whose stream cannot be waited for keeps the slot for good.
+template <class Gpu>
+class ReportSlot {
+public:
+    explicit ReportSlot(Gpu gpu) : gpu_(gpu) {
+        std::lock_guard<std::mutex> hold(mutex_);
+        if (!page_) page_ = static_cast<Slot *>(Gpu::pinned(kSlots * sizeof(Slot)));
+        for (int i = 0; page_ && i < kSlots; ++i)
+            if (!((lent_ >> i) & 1)) {
+                lent_ |= 1ull << i;
+                index_ = i;
+                page_[i].report.check = 0;
+                break;
+            }
+    }
+    ~ReportSlot() {
+        if (running_ && !gpu_.drain()) return;
+        if (index_ < 0) return;
+        std::lock_guard<std::mutex> hold(mutex_);
+        lent_ &= ~(1ull << index_);
+    }
+    ReportSlot(const ReportSlot &) = delete;
+    ReportSlot &operator=(const ReportSlot &) = delete;
+
+    BeamReport *get() const { return index_ < 0 ? nullptr : &page_[index_].report; }
+    void launching() { running_ = true; }  // before anything of the call goes to the stream
+    void drained() { running_ = false; }   // the stream has been waited for
+
+    // Waits until the launch behind the check after iteration t has reported: 0, or below 0 (-1: the stream has ended
+    // without a report, others as state()).  The stream is asked now and then, so that a launch that failed ends the wait.
+    int wait(int t) const {
+        const BeamReport *r = get();
+        for (unsigned spins = 1;; ++spins) {
+            if (__atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t) return 0;
+            if ((spins & 0xffff) == 0) {
+                const int s = gpu_.state();
+                if (s < 0) return s;
+                if (s == 0) return __atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t ? 0 : -1;
+            }
+            __builtin_ia32_pause();
+        }
+    }
+
+private:
+    static constexpr int kSlots = 64;
+    struct alignas(64) Slot { BeamReport report; };
+    static inline std::mutex mutex_;
+    static inline Slot *page_ = nullptr;
+    static inline uint64_t lent_ = 0;
+    Gpu gpu_;
+    int index_ = -1;
+    bool running_ = false;
+};
