@@ -173,3 +173,26 @@ def test_no_bound_in_a_short_last_piece_of_the_table(bad, metric):
     for s in range(0, 150, 32):
         (fi, fd) = knn_exact(q[s:s + 32].contiguous(), v, 4, metric)
         assert torch.equal(gi[s:s + 32], fi) and torch.equal(gd[s:s + 32], fd)
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("k", [1, 10, 13, 16])
+@pytest.mark.parametrize("n", [20, 1000, 9000, 70_000])
+def test_values_that_are_not_finite(n, k, metric):
+    """A distance that is not finite is nobody's neighbour: a NaN query has no neighbours under the cosine, a NaN row is
+    none; all forms agree (a few queries with one and with several tiles per wavefront; a batch of 150)."""
+    print(f"not finite n={n} k={k} {metric}", flush=True)
+    from vectorlink_gpu.kernels import knn_exact
+
+    rng = np.random.default_rng(n + k)
+    v, q = rows(rng, n, 20), rows(rng, 150, 20)
+    v[5, 3], v[6, 2], v[7, 0], v[8] = np.nan, np.inf, -np.inf, 3e38
+    q[1, 1], q[2, 4], q[3, 0], q[4] = np.nan, -np.inf, np.inf, 3e38
+    (gv, gq) = (dev(v), dev(q))
+    (mi, md) = knn_exact(gq, gv, k, metric)
+    (fi, fd) = knn_exact(gq[:30].contiguous(), gv, k, metric)
+    assert torch.equal(mi[:30], fi) and torch.equal(md[:30], fd)
+    assert not md.isnan().any()
+    assert ((md == orc.MAXFLOAT) == (mi == orc.MAXINT)).all()
+    if metric == "cosine":
+        assert (fi[1] == orc.MAXINT).all() and (fi != 5).all()

@@ -66,7 +66,7 @@ void knn_few_kernel(const float *__restrict__ queries, int n_queries, const floa
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int v = v_lane + 8 * (r >> 2) + (r & 3);
-                key[r] = v < v_limit ? vl_make_key(v, d[r]) : kPadKey;
+                key[r] = v < v_limit && d[r] < __builtin_inff() ? vl_make_key(v, d[r]) : kPadKey;  // as list_insert takes them
                 least = key[r] < least ? key[r] : least;
             }
             if (q < n_queries) {
