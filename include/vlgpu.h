@@ -400,6 +400,14 @@ int vl_knn_exact_metric(const float *queries, int64_t n_queries,
                         const float *vectors, int64_t n_vectors, int64_t dim, int64_t k,
                         int32_t metric, int32_t *ids_out, float *dists_out,
                         void *workspace, int64_t workspace_bytes, void *stream);
+/* The form that takes such a call: the kernel for a few queries, the bfloat16
+ * filter (all distances returned are float32 ones) or the float32 tiles, which
+ * need the least workspace.  Their answers have the same bits. */
+#define VL_KNN_TILES 0
+#define VL_KNN_FEW 1
+#define VL_KNN_FILTER 2
+int vl_knn_form(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
+                int64_t workspace_bytes);
 
 #ifdef __cplusplus
 }

@@ -91,6 +91,20 @@ def test_knn_workspace_of_many_queries(lib):
     assert 0 < few and many - few < 1024 * ((1 << 23) - (1 << 17))  # 4 lists of 10 keys and two words a query
 
 
+@pytest.mark.parametrize("metric", [0, 1])
+def test_knn_workspace_serves_both_metrics(lib, metric):
+    """What vl_knn_workspace_bytes asks for admits the form that a call with any amount of it would take."""
+    import random
+
+    rng = random.Random(11)
+    sizes = [(200, 3_000_000, 512, 10), (500, 3_000_000, 512, 10), (200, 9_000_000, 128, 10), (200, 9_000_000, 256, 10),
+             (200, 9_000_000, 320, 4)]
+    sizes += [(rng.randint(1, 20_000), rng.randint(100, 20_000_000), 4 * rng.randint(1, 600), rng.randint(1, 16))
+              for _ in range(300)]
+    for s in sizes:
+        assert lib.vl_knn_form(*s, metric, lib.vl_knn_workspace_bytes(*s)) == lib.vl_knn_form(*s, metric, 1 << 60), s
+
+
 def test_cpu_tensors_are_refused():
     import torch
 

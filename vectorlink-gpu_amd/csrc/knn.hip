@@ -408,8 +408,8 @@ struct KnnPlan {
 constexpr int64_t kFilterQueries = 65536;
 static_assert(kFilterQueries % TQ == 0, "flags are kept per block of TQ queries");
 
-// l2: the plan of an L2 call; its workspace is never smaller than a cosine call's.  most: bytes of workspace there are; a
-// call with too few for the form that would take it goes to the tiles alone, with the same bits.
+// most: bytes of workspace there are; a call with too few for the form that would take it goes to the tiles alone, with the
+// same bits.
 int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, int64_t most, KnnPlan *p) {
     VL_REQUIRE(n_queries >= 0 && n_vectors > 0 && dim > 0, "bad sizes");
     VL_REQUIRE(k >= 1 && k <= KMAX, "k must be between 1 and %d", KMAX);
@@ -465,9 +465,23 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
 }  // namespace
 
 VL_EXPORT int64_t vl_knn_workspace_bytes(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k) {
+    int64_t bytes = 0;
+    for (const bool l2 : {false, true}) {  // either may be the larger: pieces of the filter's table are whole tiles
+        KnnPlan p;
+        const int rc = knn_plan(n_queries, n_vectors, dim, k, l2, INT64_MAX, &p);
+        if (rc < 0) return rc;
+        bytes = p.bytes > bytes ? p.bytes : bytes;
+    }
+    return bytes;
+}
+
+VL_EXPORT int vl_knn_form(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
+                          int64_t workspace_bytes) {
+    VL_REQUIRE(metric == VL_METRIC_COSINE || metric == VL_METRIC_L2, "unknown metric %d", (int)metric);
     KnnPlan p;
-    int rc = knn_plan(n_queries, n_vectors, dim, k, true, INT64_MAX, &p);  // serves both metrics
-    return rc < 0 ? rc : p.bytes;
+    const int rc = knn_plan(n_queries, n_vectors, dim, k, metric == VL_METRIC_L2, workspace_bytes, &p);
+    if (rc < 0) return rc;
+    return p.few ? VL_KNN_FEW : (p.filter ? VL_KNN_FILTER : VL_KNN_TILES);
 }
 
 VL_EXPORT int vl_knn_exact(const float *queries, int64_t n_queries, const float *vectors,
