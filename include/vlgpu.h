@@ -408,6 +408,12 @@ int vl_knn_exact_metric(const float *queries, int64_t n_queries,
 #define VL_KNN_FILTER 2
 int vl_knn_form(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
                 int64_t workspace_bytes);
+/* Where in the workspace of a call that the filter takes an int32 holds, once
+ * the call has run, how many of its queries were left to the float32 tiles (their
+ * numbers follow it): those with more vectors within the bfloat16 rounding of
+ * their k-th best than the filter keeps, or with no bound on that rounding. */
+int64_t vl_knn_left_offset(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
+                           int64_t workspace_bytes);
 
 #ifdef __cplusplus
 }

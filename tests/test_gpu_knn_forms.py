@@ -196,3 +196,49 @@ def test_values_that_are_not_finite(n, k, metric):
     assert ((md == orc.MAXFLOAT) == (mi == orc.MAXINT)).all()
     if metric == "cosine":
         assert (fi[1] == orc.MAXINT).all() and (fi != 5).all()
+
+
+def call(q, v, k, metric="cosine"):
+    """(ids, distances, the queries left to the tiles or None if the filter does not take the call)."""
+    from vectorlink_gpu import _native as nv
+
+    (nq, dim) = q.shape
+    sizes = (nq, v.shape[0], dim, k, nv.metric_code(metric))
+    ws = torch.empty(nv.lib().vl_knn_workspace_bytes(nq, v.shape[0], dim, k), dtype=torch.uint8, device=DEV)
+    ids = torch.empty((nq, k), dtype=torch.int32, device=DEV)
+    d = torch.empty((nq, k), dtype=torch.float32, device=DEV)
+    nv.check(nv.lib().vl_knn_exact_metric(nv.ptr(q), nq, nv.ptr(v), v.shape[0], dim, k, nv.metric_code(metric), nv.ptr(ids),
+                                          nv.ptr(d), nv.ptr(ws), ws.numel(), nv.stream()))
+    if nv.lib().vl_knn_form(*sizes, ws.numel()) != 2:
+        return ids, d, None
+    at = nv.lib().vl_knn_left_offset(*sizes, ws.numel())
+    words = ws[at:at + 4 * (1 + nq)].view(torch.int32).cpu()
+    return ids, d, words[1:1 + int(words[0])].tolist()
+
+
+def agrees_with_a_few_queries(q, v, k, metric, ids, d):
+    from vectorlink_gpu.kernels import knn_exact
+
+    for s in range(0, q.shape[0], 32):
+        (fi, fd) = knn_exact(q[s:s + 32].contiguous(), v, k, metric)
+        assert torch.equal(ids[s:s + 32], fi) and torch.equal(d[s:s + 32], fd)
+
+
+@pytest.mark.parametrize("n,dim,nq,k,metric,crowded", [
+    (60_000, 64, 1000, 10, "cosine", [0, 130, 131, 511, 999]), (40_000, 128, 2500, 16, "l2", [2499]),
+    (20_000, 64, 700, 4, "cosine", list(range(100, 400))), (9000, 256, 300, 12, "cosine", list(range(300)))])
+def test_only_the_queries_that_overflow_are_left_to_the_tiles(n, dim, nq, k, metric, crowded):
+    """3,000 rows within the rounding of each other around some of the queries; the others are answered by the filter."""
+    print(f"crowded queries n={n} dim={dim} nq={nq} k={k} {metric}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    v = torch.nn.functional.normalize(torch.randn((n, dim), generator=gen, device=DEV), dim=1)
+    q = torch.nn.functional.normalize(torch.randn((nq, dim), generator=gen, device=DEV), dim=1)
+    centre = q[crowded[0]].clone()
+    q = torch.nn.functional.normalize(q - (q @ centre)[:, None] * centre, dim=1)  # the others: none of the 3,000 near them
+    at = torch.randperm(n, generator=gen, device=DEV)[:3000]
+    v[at] = torch.nn.functional.normalize(centre + 1e-4 * torch.randn((3000, dim), generator=gen, device=DEV), dim=1)
+    for c in crowded:
+        q[c] = torch.nn.functional.normalize(centre + 1e-4 * q[c], dim=0)
+    (ids, d, left) = call(q, v, k, metric)
+    assert left == crowded
+    agrees_with_a_few_queries(q, v, k, metric, ids, d)

@@ -28,6 +28,7 @@ constexpr int KMAX = 16;      // longest list kept per lane and query
 constexpr int TQ = 128;       // queries per workgroup
 constexpr int TV = 128;       // vectors per step
 constexpr int LISTS_PER_STRIP = 4;  // two half-waves x two wave rows see the same query
+constexpr int kMaxStrips = 64;      // of the vector set
 // workgroups of the tile kernel resident at once: two per compute unit (64 KB of LDS each), 256 CUs on an MI355X;
 // the count is read from the device on first use
 int64_t resident_workgroups() {
@@ -67,15 +68,40 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float *__restrict_
     if (lane == 0) out[row] = s;
 }
 
+// The work of the tiles.  left != null: only the queries of a list that the filter leaves on the device (left[0] of them,
+// numbers behind it), in as many strips as the workgroups and the lists that the launch has for all its queries allow.
+struct TileWork {
+    int64_t n_queries;
+    int64_t strip_len;
+    int n_strips, n_qblocks;
+    __device__ __forceinline__ TileWork(int64_t all, int64_t n_vectors, int64_t len, int strips, const int32_t *left)
+        : n_queries(all), strip_len(len), n_strips(strips) {
+        if (left) n_queries = left[0];
+        n_qblocks = (int)((n_queries + TQ - 1) / TQ);
+        if (left && n_qblocks > 0) {
+            const int64_t tiles = (n_vectors + TV - 1) / TV;
+            int64_t s = (all + TQ - 1) / TQ * strips / n_qblocks;
+            s = min(min(s, all * strips / n_queries), min(tiles, (int64_t)kMaxStrips));
+            const int64_t per = (tiles + s - 1) / s;
+            strip_len = per * TV;
+            n_strips = (int)((tiles + per - 1) / per);
+        }
+    }
+};
+
 // L2: distances are |q|^2 + |v|^2 - 2 q.v from the rows' squared lengths (q_norm, v_norm)
 template <int KK, bool L2>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void knn_tile_kernel(const float *__restrict__ queries, int64_t n_queries,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void knn_tile_kernel(const float *__restrict__ queries, int64_t all_queries,
                                                       const float *__restrict__ vectors, int64_t n_vectors,
-                                                      int dim, int64_t strip_len, int n_strips,
-                                                      int n_qblocks, int q_group, uint64_t *__restrict__ cand,
+                                                      int dim, int64_t all_strip_len, int all_strips,
+                                                      int q_group, uint64_t *__restrict__ cand,
                                                       const float *__restrict__ q_norm,
                                                       const float *__restrict__ v_norm, uint32_t *__restrict__ q_bound,
-                                                      const int32_t *__restrict__ wanted) {
+                                                      const int32_t *__restrict__ left) {
+    const TileWork work(all_queries, n_vectors, all_strip_len, all_strips, left);
+    const int64_t n_queries = work.n_queries, strip_len = work.strip_len;
+    const int n_strips = work.n_strips, n_qblocks = work.n_qblocks;
+    const int32_t *const list = left ? left + 1 : nullptr;
     // two buffers per operand as separate arrays: the compiler can then tell that the loads
     // landing in one buffer do not touch the one being read
     __shared__ __align__(16) float sV0[TILE];
@@ -111,7 +137,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             q_block = (n_qblocks / q_group) * q_group + (int)(w - (int64_t)strip * rest);
         }
     }
-    if (wanted && wanted[q_block] == 0) return;  // (uniform over the workgroup) answered by the filter
     const int64_t q0 = (int64_t)q_block * TQ;
     const int64_t v_begin = strip * strip_len;
     const int64_t v_end = min(n_vectors, v_begin + strip_len);
@@ -149,13 +174,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     const bool ragged = (dim % KT) != 0;
     const float *qp[4], *vp[4];
-    duty_pointers(queries, q0, n_queries - 1, dim, wave, lane, qp);
+    duty_pointers(queries, q0, n_queries - 1, dim, wave, lane, qp, list);
     float qn[2] = {0.0f, 0.0f};
     if constexpr (L2) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
-            const int64_t q = q0 + 64 * wc + 32 * cb + l32;
-            qn[cb] = q_norm[q < n_queries ? q : n_queries - 1];
+            const int64_t q = min(q0 + 64 * wc + 32 * cb + l32, n_queries - 1);
+            qn[cb] = q_norm[list ? list[q] : q];
         }
     }
 
@@ -334,13 +359,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // wavefront merges them as a tournament: a lane keeps the heads of its lists (lane, lane + 64, ...)
 // and the key behind each head; the smallest head of the wavefront is the next result and the lane
 // that held it moves on in that list.  Only the heads and the few keys behind a winner are read.
-constexpr int kSelectLists = 4;  // lists per lane: 64 strips x 4 lists at most
+constexpr int kSelectLists = kMaxStrips * LISTS_PER_STRIP / 64;  // lists per lane
 
-__global__ __launch_bounds__(256) void knn_select_kernel(const uint64_t *__restrict__ cand, int n_lists, int KK, int k,
+__global__ __launch_bounds__(256) void knn_select_kernel(const uint64_t *__restrict__ cand, int all_strips, int KK, int k,
                                                          int32_t *__restrict__ ids_out, float *__restrict__ d_out,
-                                                         int64_t n_queries, const int32_t *__restrict__ wanted) {
+                                                         int64_t all_queries, int64_t n_vectors, int64_t all_strip_len,
+                                                         const int32_t *__restrict__ left) {
+    const TileWork work(all_queries, n_vectors, all_strip_len, all_strips, left);
+    const int n_lists = work.n_strips * LISTS_PER_STRIP;
     const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (q >= n_queries || (wanted && wanted[q / TQ] == 0)) return;  // the whole wavefront leaves
+    if (q >= work.n_queries) return;  // the whole wavefront leaves
     const int lane = threadIdx.x & 63;
     const uint64_t *base = cand + q * n_lists * KK;
     uint64_t head[kSelectLists], next[kSelectLists];
@@ -382,8 +410,9 @@ __global__ __launch_bounds__(256) void knn_select_kernel(const uint64_t *__restr
     }
     if (lane < k) {
         const bool real = result != kPadKey;
-        ids_out[q * k + lane] = real ? vl_key_id(result) : VL_MAXINT;
-        d_out[q * k + lane] = real ? vl_key_dist(result) : VL_MAXFLOAT;
+        const int64_t to = left ? left[1 + q] : q;
+        ids_out[to * k + lane] = real ? vl_key_id(result) : VL_MAXINT;
+        d_out[to * k + lane] = real ? vl_key_dist(result) : VL_MAXFLOAT;
     }
 }
 
@@ -397,16 +426,16 @@ struct KnnPlan {
     bool few;     // the kernel of knn_few.hip takes the call (see vl_knn_exact_metric)
     bool filter;  // the filter of knn_filter.hip takes it, and the tiles what it leaves
     KnnFilterPlan fp;
-    int64_t off_flags, off_filter;
+    int64_t off_left, off_filter;
     int n_cand;
     int64_t cand_bytes;  // per-lane candidate lists; the queries' shared bounds and the rows' squared lengths (L2) follow
     int64_t bytes;
 };
 
-// Queries that go through the filter at a time (whole blocks of TQ): its buffers take 16 to 20 KB a query, and a pass
-// over that many queries takes a hundred times as long as converting the table again.
+// Queries that go through the filter at a time: its buffers take 16 KB a query for the candidates, 2 for the groups' maxima
+// and the query's bfloat16 row, and a pass over that many queries takes a hundred times as long as converting the table
+// again.
 constexpr int64_t kFilterQueries = 65536;
-static_assert(kFilterQueries % TQ == 0, "flags are kept per block of TQ queries");
 
 // most: bytes of workspace there are; a call with too few for the form that would take it goes to the tiles alone, with the
 // same bits.
@@ -417,13 +446,13 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
     VL_REQUIRE(n_vectors < (1ll << 30), "ids must stay below 2^30");
     int64_t q_blocks = (n_queries + TQ - 1) / TQ;
     if (q_blocks < 1) q_blocks = 1;
-    // The vector set is cut into at most 64 strips of whole tiles; q_blocks * strips workgroups
+    // The vector set is cut into at most kMaxStrips strips of whole tiles; q_blocks * strips workgroups
     // share resident_workgroups() slots (two per compute unit), so the run lasts
     // ceil(workgroups / slots) strips' worth of tiles.  Take the strip count with the shortest
     // run; a strip more costs a sixteenth of a tile (wider merge afterwards).
     const int64_t tiles = (n_vectors + TV - 1) / TV;
     int64_t strips = 1, best_cost = -1;
-    for (int64_t s = 1; s <= 64 && s <= tiles; ++s) {
+    for (int64_t s = 1; s <= kMaxStrips && s <= tiles; ++s) {
         int64_t len_t = (tiles + s - 1) / s;
         int64_t s2 = (tiles + len_t - 1) / len_t;
         if (s2 != s) continue;
@@ -453,8 +482,8 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
     p->bytes = lists(strips * LISTS_PER_STRIP);
     p->filter = vl_knn_filter_plan(n_queries < kFilterQueries ? n_queries : kFilterQueries, n_vectors, dim, k, l2, &p->fp);
     if (p->filter) {
-        p->off_flags = (p->bytes + 255) / 256 * 256;
-        p->off_filter = (p->off_flags + q_blocks * 4 + 255) / 256 * 256;
+        p->off_left = (p->bytes + 255) / 256 * 256;
+        p->off_filter = (p->off_left + (1 + n_queries) * 4 + 255) / 256 * 256;
         const int64_t bytes = p->off_filter + p->fp.bytes + 256;  // (the workspace itself may be 16-byte aligned only)
         if (bytes <= most) p->bytes = bytes;
         else p->filter = false;
@@ -482,6 +511,16 @@ VL_EXPORT int vl_knn_form(int64_t n_queries, int64_t n_vectors, int64_t dim, int
     const int rc = knn_plan(n_queries, n_vectors, dim, k, metric == VL_METRIC_L2, workspace_bytes, &p);
     if (rc < 0) return rc;
     return p.few ? VL_KNN_FEW : (p.filter ? VL_KNN_FILTER : VL_KNN_TILES);
+}
+
+VL_EXPORT int64_t vl_knn_left_offset(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
+                                     int64_t workspace_bytes) {
+    VL_REQUIRE(metric == VL_METRIC_COSINE || metric == VL_METRIC_L2, "unknown metric %d", (int)metric);
+    KnnPlan p;
+    const int rc = knn_plan(n_queries, n_vectors, dim, k, metric == VL_METRIC_L2, workspace_bytes, &p);
+    if (rc < 0) return rc;
+    VL_REQUIRE(!p.few && p.filter, "such a call does not go through the filter");
+    return p.off_left;
 }
 
 VL_EXPORT int vl_knn_exact(const float *queries, int64_t n_queries, const float *vectors,
@@ -520,19 +559,19 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     float *q_norm = reinterpret_cast<float *>(q_bound + n_queries);
     float *v_norm = q_norm + n_queries;
     // A batch goes to the kernel for a few queries (knn_few.h says where the line lies), else through the bfloat16 filter,
-    // which leaves the query blocks it cannot answer to the float32 tiles below; a table below 4,096 rows to the tiles.
-    const int32_t *wanted = nullptr;
+    // which leaves the queries it cannot answer to the float32 tiles below; a table below 4,096 rows goes to the tiles.
+    const int32_t *left = nullptr;
     char *const ws = (char *)workspace;
     if (p.filter) {
-        int32_t *flags = (int32_t *)(ws + p.off_flags);
+        int32_t *const list = (int32_t *)(ws + p.off_left);
         char *const filter_ws = (char *)(((uintptr_t)(ws + p.off_filter) + 255) / 256 * 256);
         for (int64_t q0 = 0; q0 < n_queries; q0 += kFilterQueries) {
             const int64_t n = n_queries - q0 < kFilterQueries ? n_queries - q0 : kFilterQueries;
-            rc = vl_knn_filter(p.fp, queries + q0 * dim, n, vectors, n_vectors, dim, k, l2, q_norm + q0, v_norm,
-                               flags + q0 / TQ, TQ, filter_ws, ids_out + q0 * k, dists_out + q0 * k, st);
+            rc = vl_knn_filter(p.fp, queries + q0 * dim, n, vectors, n_vectors, dim, k, l2, q_norm + q0, v_norm, q0, list,
+                               q_bound, filter_ws, ids_out + q0 * k, dists_out + q0 * k, st);
             if (rc < 0) return rc;
         }
-        wanted = flags;
+        left = list;
     } else if (l2) {
         VL_REQUIRE((n_vectors + 3) / 4 <= kMaxBlocks * 4, "too many vectors for one call");
         hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, queries,
@@ -544,18 +583,20 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     if (p.few)
         return vl_knn_few(queries, n_queries, vectors, n_vectors, dim, k, p.list_len, l2, q_norm, v_norm, cand, ids_out,
                           dists_out, st);
-    hipLaunchKernelGGL(knn_bound_init_kernel, dim3(vl_grid_for(n_queries, 256)), dim3(256), 0, st, q_bound, n_queries);
-    VL_LAUNCH_CHECK("knn_bound_init_kernel");
+    if (!left) {
+        hipLaunchKernelGGL(knn_bound_init_kernel, dim3(vl_grid_for(n_queries, 256)), dim3(256), 0, st, q_bound, n_queries);
+        VL_LAUNCH_CHECK("knn_bound_init_kernel");
+    }
 #define VL_KNN_LAUNCH(KK)                                                                                     \
     do {                                                                                                      \
         if (l2)                                                                                               \
             hipLaunchKernelGGL((knn_tile_kernel<KK, true>), dim3((unsigned)blocks), dim3(256), 0, st, queries, \
-                               n_queries, vectors, n_vectors, (int)dim, p.strip_len, p.n_strips, (int)q_blocks, \
-                               (int)q_group, cand, q_norm, v_norm, q_bound, wanted);                          \
+                               n_queries, vectors, n_vectors, (int)dim, p.strip_len, p.n_strips, (int)q_group,  \
+                               cand, q_norm, v_norm, q_bound, left);                          \
         else                                                                                                  \
             hipLaunchKernelGGL((knn_tile_kernel<KK, false>), dim3((unsigned)blocks), dim3(256), 0, st, queries, \
-                               n_queries, vectors, n_vectors, (int)dim, p.strip_len, p.n_strips, (int)q_blocks, \
-                               (int)q_group, cand, nullptr, nullptr, q_bound, wanted);                        \
+                               n_queries, vectors, n_vectors, (int)dim, p.strip_len, p.n_strips, (int)q_group,  \
+                               cand, nullptr, nullptr, q_bound, left);                        \
     } while (0)
     switch (p.list_len) {
         case 1: VL_KNN_LAUNCH(1); break;
@@ -567,10 +608,8 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     }
 #undef VL_KNN_LAUNCH
     VL_LAUNCH_CHECK("knn_tile_kernel");
-    const int n_lists = p.n_strips * LISTS_PER_STRIP;
-    VL_REQUIRE(n_lists <= 64 * kSelectLists, "too many candidate lists per query");
-    hipLaunchKernelGGL(knn_select_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, cand, n_lists,
-                       p.list_len, (int)k, ids_out, dists_out, n_queries, wanted);
+    hipLaunchKernelGGL(knn_select_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, cand, p.n_strips,
+                       p.list_len, (int)k, ids_out, dists_out, n_queries, n_vectors, p.strip_len, left);
     VL_LAUNCH_CHECK("knn_select_kernel");
     return VL_OK;
 }

@@ -39,15 +39,17 @@ __device__ __forceinline__ int swz(int r) { return (r >> 1) & (CH - 1); }
 // registers in between).  A wavefront instruction fills 1 KB = 8 tile rows and lane i writes
 // slot i of those rows, so it fetches the chunk that belongs there.  Each lane has four such
 // (row, chunk) duties per operand; their source addresses at k = 0 are kept as pointers.
-// Rows past `last` repeat row `last` (their results are discarded later).
+// Rows past `last` repeat row `last` (their results are discarded later).  list: the rows' numbers, or null.
 __device__ __forceinline__ void duty_pointers(const float *__restrict__ src, int64_t first, int64_t last, int dim,
-                                              int wave, int lane, const float *(&p)[4]) {
+                                              int wave, int lane, const float *(&p)[4],
+                                              const int32_t *__restrict__ list = nullptr) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int r = 8 * (4 * wave + i) + (lane >> 3);
         const int c = (lane & (CH - 1)) ^ swz(r);
         int64_t row = first + r;
         row = row < last ? row : last;
+        if (list) row = list[row];
         p[i] = src + row * dim + 4 * c;
     }
 }

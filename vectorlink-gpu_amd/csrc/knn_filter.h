@@ -15,9 +15,10 @@ struct KnnFilterPlan {
 // Whether a call is taken by the filter, and its plan, which also serves a call of fewer queries.
 bool vl_knn_filter_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, KnnFilterPlan *p);
 
-// Writes the answers of every query whose candidates fit its buffer and leaves, per block of flag_queries queries,
-// flags[block] = 1 where some query's did not (its answer is not written then, nor are others of the block to be kept).
-// ws: p.bytes bytes, 256-byte aligned.  q_norm / v_norm: squared lengths (written here when l2, else not used).
+// Writes the answers of every query whose candidates fit its buffer; appends the others to left: left[0] is how many there
+// are, their numbers (q_first + place in this call) follow in order.  tile_bound[i] is set for the i-th of them.  A call
+// with q_first == 0 starts the list.  ws: p.bytes bytes, 256-byte aligned.  q_norm / v_norm: squared lengths (written here
+// when l2, else not used).
 int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_queries, const float *vectors, int64_t n_vectors,
-                  int64_t dim, int64_t k, bool l2, float *q_norm, float *v_norm, int32_t *flags, int flag_queries, char *ws,
-                  int32_t *ids_out, float *dists_out, hipStream_t st);
+                  int64_t dim, int64_t k, bool l2, float *q_norm, float *v_norm, int64_t q_first, int32_t *left,
+                  uint32_t *tile_bound, char *ws, int32_t *ids_out, float *dists_out, hipStream_t st);

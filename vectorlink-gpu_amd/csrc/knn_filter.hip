@@ -16,7 +16,7 @@
 //   finish    their float32 dot products - one fused multiply-add after the other in the order in which the float32 tiles'
 //             matrix instructions take the elements, which gives the tiles' bits - and the k best of them
 // A query with more candidates than its buffer holds (thousands of rows within the rounding of each other) is left to the
-// float32 tiles.  For squared L2 the values are <q, v> - |v|^2 / 2: three more columns hold -|v|^2 / 2 as a sum of three
+// float32 tiles, which take all such queries of a call together.  For squared L2 the values are <q, v> - |v|^2 / 2: three more columns hold -|v|^2 / 2 as a sum of three
 // bfloat16 numbers (24 bits), and ones on the query side.
 //
 // The pass: 256 vectors x 256 queries per workgroup of eight wavefronts (128 x 64 each, 128 accumulator registers), 64
@@ -430,10 +430,41 @@ __global__ __launch_bounds__(256) void bound_kernel(const float *__restrict__ gm
     }
 }
 
-__global__ void filter_clear_kernel(uint32_t *__restrict__ vmax, int64_t n, int32_t *__restrict__ flags, int64_t n_flags) {
+__global__ void filter_clear_kernel(uint32_t *__restrict__ vmax, int64_t n, int32_t *__restrict__ left) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) vmax[i] = 0;
-    if (i < n_flags) flags[i] = 0;
+    if (i == 0 && left) left[0] = 0;
+}
+
+// Appends the queries with more candidates than a buffer holds to the list that the tiles take, in order, and gives their
+// places the bound they start from.  One workgroup: it is the only one to touch the list.  (A place for each from an atomic
+// counter took 8 ns a query where all were left.)
+constexpr int kLeftThreads = 1024;
+__global__ __launch_bounds__(kLeftThreads) void left_kernel(const int32_t *__restrict__ count, int n, int q_first,
+                                                            int32_t *__restrict__ left, uint32_t *__restrict__ tile_bound) {
+    constexpr int kWaves = kLeftThreads / kWave;
+    __shared__ int part[2][kWaves];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    int have = left[0];
+    for (int base = 0, round = 0; base < n; base += kLeftThreads, round ^= 1) {
+        const int q = base + tid;
+        const bool mine = q < n && count[q] > kFound;
+        const uint64_t all = __ballot(mine);
+        if (lane == 0) part[round][wave] = __popcll(all);
+        __syncthreads();
+        int at = have + __popcll(all & ((1ull << lane) - 1));
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const int theirs = part[round][w];
+            have += theirs;
+            if (w < wave) at += theirs;
+        }
+        if (mine) {
+            left[1 + at] = q_first + q;
+            tile_bound[at] = 0x7F800000u;
+        }
+    }
+    if (tid == 0) left[0] = have;
 }
 
 // The dot product of a lane's row with the query: the products of knn_tile_kernel one fused multiply-add after the other,
@@ -494,7 +525,6 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(const float *__r
                                                                 const uint32_t *__restrict__ vmax, int slabs,
                                                                 const float *__restrict__ q_norm,
                                                                 const float *__restrict__ v_norm, int64_t q_first,
-                                                                int flag_queries, int32_t *__restrict__ flags,
                                                                 int32_t *__restrict__ ids_out, float *__restrict__ d_out) {
     __shared__ uint64_t keys[kFound];
     __shared__ uint32_t values[kFound];
@@ -504,10 +534,7 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(const float *__r
     const int64_t q = q_first + blockIdx.x;
     const int tid = threadIdx.x;
     const int n = count[q];
-    if (n > kFound) {  // uniform; every writer of a flag stores the same 1
-        if (tid == 0) flags[q / flag_queries] = 1;
-        return;
-    }
+    if (n > kFound) return;  // uniform; left to the tiles
     if (tid == 0) {
         kth_s = 0;
         n_s = 0;
@@ -630,8 +657,8 @@ bool vl_knn_filter_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64
 }
 
 int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_queries, const float *vectors, int64_t n_vectors,
-                  int64_t dim, int64_t k, bool l2, float *q_norm, float *v_norm, int32_t *flags, int flag_queries, char *ws,
-                  int32_t *ids_out, float *dists_out, hipStream_t st) {
+                  int64_t dim, int64_t k, bool l2, float *q_norm, float *v_norm, int64_t q_first, int32_t *left,
+                  uint32_t *tile_bound, char *ws, int32_t *ids_out, float *dists_out, hipStream_t st) {
     __bf16 *q16 = (__bf16 *)(ws + p.off_q16), *v16 = (__bf16 *)(ws + p.off_v16);
     RowStat *qstat = (RowStat *)(ws + p.off_qstat);
     float *gmax = (float *)(ws + p.off_gmax), *bound = (float *)(ws + p.off_bound);
@@ -640,17 +667,15 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     uint32_t *vmax = (uint32_t *)(ws + p.off_vmax);
     const int kp = (int)p.kp, kp2 = kp / 2;
     const int64_t slabs = (n_vectors + p.slab_rows - 1) / p.slab_rows;
-    const int64_t n_flags = (n_queries + flag_queries - 1) / flag_queries;
     const int64_t n_words = (slabs + 1) * kStripes * kStripeWords;
-    const int64_t n_clear = n_words > n_flags ? n_words : n_flags;
     const size_t smem = 4 * TR * KT * sizeof(float);
     auto allow = [&]() -> hipError_t {
         const hipError_t e = vl_allow_lds(pass_kernel<false>, smem);
         return e == hipSuccess ? vl_allow_lds(pass_kernel<true>, smem) : e;
     };
     VL_HIP(allow());
-    hipLaunchKernelGGL(filter_clear_kernel, dim3((unsigned)((n_clear + 255) / 256)), dim3(256), 0, st, vmax,
-                       n_words, flags, n_flags);
+    hipLaunchKernelGGL(filter_clear_kernel, dim3((unsigned)((n_words + 255) / 256)), dim3(256), 0, st, vmax,
+                       n_words, q_first == 0 ? left : nullptr);
     auto prepare = [&](const float *rows, int64_t n, int64_t step, int extra, __bf16 *out, float *norm2, RowStat *stat, uint32_t *top) {
         const int64_t blocks = (n + 3) / 4 < 2048 ? (n + 3) / 4 : 2048;
         hipLaunchKernelGGL(prepare_kernel, dim3((unsigned)blocks), dim3(256), 0, st, rows, n, (int)dim, kp, step, l2 ? extra : 0, out, norm2,
@@ -690,11 +715,13 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
         const dim3 grid((unsigned)(n_queries - q0 < kMaxBlocks ? n_queries - q0 : kMaxBlocks));
         if (l2)
             hipLaunchKernelGGL(finish_kernel<true>, grid, dim3(kFinishThreads), 0, st, queries, vectors, (int)dim, (int)k,
-                               count, found, qstat, vmax, (int)slabs, q_norm, v_norm, q0, flag_queries, flags, ids_out, dists_out);
+                               count, found, qstat, vmax, (int)slabs, q_norm, v_norm, q0, ids_out, dists_out);
         else
             hipLaunchKernelGGL(finish_kernel<false>, grid, dim3(kFinishThreads), 0, st, queries, vectors, (int)dim, (int)k,
-                               count, found, qstat, vmax, (int)slabs, q_norm, v_norm, q0, flag_queries, flags, ids_out, dists_out);
+                               count, found, qstat, vmax, (int)slabs, q_norm, v_norm, q0, ids_out, dists_out);
     }
     VL_LAUNCH_CHECK("knn finish_kernel");
+    hipLaunchKernelGGL(left_kernel, dim3(1), dim3(kLeftThreads), 0, st, count, (int)n_queries, (int)q_first, left, tile_bound);
+    VL_LAUNCH_CHECK("knn left_kernel");
     return VL_OK;
 }
