@@ -242,3 +242,24 @@ def test_only_the_queries_that_overflow_are_left_to_the_tiles(n, dim, nq, k, met
     (ids, d, left) = call(q, v, k, metric)
     assert left == crowded
     agrees_with_a_few_queries(q, v, k, metric, ids, d)
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("order", ["random", "by cluster", "in turn"])
+@pytest.mark.parametrize("n,dim,members,nq,k", [(60_000, 128, 200, 600, 10), (9000, 64, 90, 300, 16), (131_075, 256, 500, 400, 1)])
+def test_the_order_of_the_rows_does_not_matter(n, dim, members, nq, k, order, metric):
+    """Clusters whose rows follow each other, or come one from each in turn: the sample that bounds are taken from meets all
+    of them, and no query has more candidates than its buffer holds."""
+    print(f"order {order} n={n} dim={dim} members={members} nq={nq} k={k} {metric}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(n + k)
+    count = n // members
+    at = torch.arange(n, device=DEV)
+    group = {"random": at[torch.randperm(n, generator=gen, device=DEV)] % count, "by cluster": at * count // n,
+             "in turn": at % count}[order]
+    centres = torch.randn((count, dim), generator=gen, device=DEV)
+    v = centres[group] + 0.15 * torch.randn((n, dim), generator=gen, device=DEV)
+    q = centres[torch.randint(0, count, (nq,), generator=gen, device=DEV)] + 0.15 * torch.randn((nq, dim), generator=gen, device=DEV)
+    (v, q) = (torch.nn.functional.normalize(x, dim=1) for x in (v, q))
+    (ids, d, left) = call(q, v, k, metric)
+    assert left == []
+    agrees_with_a_few_queries(q, v, k, metric, ids, d)

@@ -5,7 +5,7 @@
 struct KnnFilterPlan {
     int64_t kp;             // columns of a bfloat16 row: dim (and three more for L2) padded to a multiple of 64
     int64_t sample_rows;    // rows of the sample that bounds are taken from (whole tiles)
-    int64_t sample_step;    // its tiles are every sample_step-th of the table
+    int64_t sample_stride;  // between the places of two rows of the sample that follow each other in the table
     int sample_strips;
     int groups;             // maxima per query that the sample pass leaves
     int64_t slab_rows;      // rows of the table converted at a time

@@ -50,18 +50,35 @@ struct RowStat {
 
 __device__ __forceinline__ float up(float x) { return x * 1.00001f; }  // norms are sums of dim rounded terms: never below
 
-// Row j of the output is row (j / TR) * TR * step + j % TR of the input, rounded to bfloat16 and padded with zeros to kp
-// columns.  extra: 0, 1 = a query row for L2 (three ones behind the columns), 2 = a vector for L2 (-|v|^2 / 2 there).  One wavefront per row.  vmax: the largest resid and norm as float bits (all values are >= 0; what is not
+// The sample takes one row of each of n_sample equal stretches of the table, at a place of its own in each, and deals
+// neighbours to groups far apart: a table whose rows come in the order of their clusters, or in turn from each, is sampled
+// like one in random order.  (Whole tiles at equal distances met 1 in 16 of the clusters of a table in their order, and the
+// bounds from those that were met let thousands of candidates through.)
+struct SampleRows {
+    int64_t n_sample, n_table;
+    int64_t stride;  // has no common divisor with n_sample
+    __device__ __forceinline__ int64_t source(int64_t i) const {
+        const int64_t first = i * n_table / n_sample, room = (i + 1) * n_table / n_sample - first;
+        uint32_t h = (uint32_t)i * 2654435761u;  // (the finaliser of MurmurHash3)
+        h = (h ^ (h >> 16)) * 0x85ebca6bu;
+        h = (h ^ (h >> 13)) * 0xc2b2ae35u;
+        return first + (int64_t)__umulhi(h ^ (h >> 16), (uint32_t)room);
+    }
+    __device__ __forceinline__ int64_t place(int64_t i) const { return i * stride % n_sample; }
+};
+
+// Rows of the input (all n, or a sample of n) rounded to bfloat16 and padded with zeros to kp columns.  extra: 0, 1 = a query row for L2 (three ones behind the columns), 2 = a vector for L2 (-|v|^2 / 2 there).  One wavefront per row.  vmax: the largest resid and norm as float bits (all values are >= 0; what is not
 // finite counts as infinity), over kStripes stripes that table_stat puts together - with one pair of words for all, the
 // 32,768 atomic operations of a large table queued up for 280 us.
+template <bool SAMPLE>
 __global__ __launch_bounds__(256) void prepare_kernel(const float *__restrict__ rows, int64_t n, int dim, int kp,
-                                                      int64_t step, int extra, __bf16 *__restrict__ out,
+                                                      SampleRows sample, int extra, __bf16 *__restrict__ out,
                                                       float *__restrict__ norm2,
                                                       RowStat *__restrict__ stat, uint32_t *__restrict__ vmax) {
     const int lane = threadIdx.x & (kWave - 1);
     float top_resid = 0.0f, top_norm = 0.0f;
-    for (int64_t j = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave; j < n; j += (int64_t)gridDim.x * 4) {
-        const int64_t row = step == 1 ? j : (j / TR) * TR * step + j % TR;
+    for (int64_t i = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave; i < n; i += (int64_t)gridDim.x * 4) {
+        const int64_t row = SAMPLE ? sample.source(i) : i, j = SAMPLE ? sample.place(i) : i;
         const float4 *src = reinterpret_cast<const float4 *>(rows + row * dim);
         bf16x4 *dst = reinterpret_cast<bf16x4 *>(out + j * kp);
         float s = 0.0f, e2 = 0.0f;
@@ -94,9 +111,9 @@ __global__ __launch_bounds__(256) void prepare_kernel(const float *__restrict__ 
             if (extra == 2) {
                 float left = -0.5f * s;
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    h[i] = (__bf16)left;
-                    left -= (float)h[i];
+                for (int c = 0; c < 3; ++c) {
+                    h[c] = (__bf16)left;
+                    left -= (float)h[c];
                 }
             }
             dst[dim / 4] = h;
@@ -616,20 +633,22 @@ int64_t strips_for(int64_t q_blocks, int64_t tiles, int64_t most) {
 }
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
+inline int64_t gcd(int64_t a, int64_t b) { return b ? gcd(b, a % b) : a; }
 
 }  // namespace
 
 bool vl_knn_filter_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, KnnFilterPlan *p) {
     if (n_vectors < 4096 || dim > 8192) return false;
     p->kp = (dim + (l2 ? 3 : 0) + 63) / 64 * 64;
-    const int64_t tiles = n_vectors / TR;  // whole ones: the sample repeats no row
+    const int64_t tiles = n_vectors / TR;
     // The sample: a sixteenth of the table (an eighth for long lists, whose expected number of candidates, k times the
     // share's inverse and half as much again for E, would come near kFound) and 32 tiles at least: a candidate costs as much
     // as some hundred products of 64 columns (32,768 entry points x 64 columns: 16 tiles 298 us, 32 tiles 242 us).
     int64_t sample = tiles / (k > 10 ? 8 : 16);
     if (sample < 32) sample = tiles / 2 < 32 ? (tiles + 1) / 2 : 32;
-    p->sample_step = tiles / sample;
     p->sample_rows = sample * TR;
+    p->sample_stride = p->sample_rows * 618 / 1000 | 1;
+    while (gcd(p->sample_stride, p->sample_rows) != 1) p->sample_stride += 2;
     const int64_t q_blocks = (n_queries + TR - 1) / TR;
     int64_t strips = strips_for(q_blocks, sample, kMaxGroups / kGroupsPerStrip);
     // enough groups that the k-th largest maximum is close to the k-th best of the sample
@@ -676,9 +695,10 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     VL_HIP(allow());
     hipLaunchKernelGGL(filter_clear_kernel, dim3((unsigned)((n_words + 255) / 256)), dim3(256), 0, st, vmax,
                        n_words, q_first == 0 ? left : nullptr);
-    auto prepare = [&](const float *rows, int64_t n, int64_t step, int extra, __bf16 *out, float *norm2, RowStat *stat, uint32_t *top) {
+    const SampleRows sample{p.sample_rows, n_vectors, p.sample_stride};
+    auto prepare = [&](auto kernel, const float *rows, int64_t n, int extra, __bf16 *out, float *norm2, RowStat *stat, uint32_t *top) {
         const int64_t blocks = (n + 3) / 4 < 2048 ? (n + 3) / 4 : 2048;
-        hipLaunchKernelGGL(prepare_kernel, dim3((unsigned)blocks), dim3(256), 0, st, rows, n, (int)dim, kp, step, l2 ? extra : 0, out, norm2,
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, rows, n, (int)dim, kp, sample, l2 ? extra : 0, out, norm2,
                            stat, top);
     };
     const int64_t q_blocks = (n_queries + TR - 1) / TR;
@@ -696,8 +716,8 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
         if (emit) go(pass_kernel<true>);
         else go(pass_kernel<false>);
     };
-    prepare(queries, n_queries, 1, 1, q16, l2 ? q_norm : nullptr, qstat, nullptr);
-    prepare(vectors, p.sample_rows, p.sample_step, 2, v16, nullptr, nullptr, vmax);
+    prepare(prepare_kernel<false>, queries, n_queries, 1, q16, l2 ? q_norm : nullptr, qstat, nullptr);
+    prepare(prepare_kernel<true>, vectors, p.sample_rows, 2, v16, nullptr, nullptr, vmax);
     VL_LAUNCH_CHECK("knn prepare_kernel");
     pass(false, p.sample_rows, p.sample_strips, vmax, 0);
     VL_LAUNCH_CHECK("knn pass_kernel (sample)");
@@ -707,7 +727,7 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     for (int64_t s = 0; s < slabs; ++s) {
         const int64_t r0 = s * p.slab_rows;
         const int64_t rows = n_vectors - r0 < p.slab_rows ? n_vectors - r0 : p.slab_rows;
-        prepare(vectors + r0 * dim, rows, 1, 2, v16, l2 ? v_norm + r0 : nullptr, nullptr, vmax + (s + 1) * kStripes * kStripeWords);
+        prepare(prepare_kernel<false>, vectors + r0 * dim, rows, 2, v16, l2 ? v_norm + r0 : nullptr, nullptr, vmax + (s + 1) * kStripes * kStripeWords);
         pass(true, rows, strips_for(q_blocks, (rows + TR - 1) / TR, 1024), vmax + (s + 1) * kStripes * kStripeWords, r0);
         VL_LAUNCH_CHECK("knn pass_kernel (filter)");
     }
