@@ -263,3 +263,27 @@ def test_the_order_of_the_rows_does_not_matter(n, dim, members, nq, k, order, me
     (ids, d, left) = call(q, v, k, metric)
     assert left == []
     agrees_with_a_few_queries(q, v, k, metric, ids, d)
+
+
+# candidates of a query around the wavefronts' shares of 8, 16, 32 and 64 rows, one round of a workgroup and several;
+# rows that end within a line of 32 columns, with and without a chunk on its own
+@pytest.mark.parametrize("nq", [200, 600])
+@pytest.mark.parametrize("members,dim,k,metric", [
+    (3, 20, 16, "cosine"), (9, 64, 1, "cosine"), (17, 36, 10, "l2"), (33, 132, 4, "cosine"), (64, 256, 16, "cosine"),
+    (65, 28, 12, "l2"), (129, 60, 10, "cosine"), (300, 300, 16, "cosine"), (1025, 768, 10, "cosine"), (1900, 4, 8, "l2")])
+def test_candidates_of_every_number(members, dim, k, metric, nq):
+    """Rows close to each other in groups: a query has its whole group to evaluate."""
+    print(f"candidates members={members} dim={dim} nq={nq} k={k} {metric}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(members)
+    n = 12_007
+    count = n // members
+    group = torch.arange(n, device=DEV) % count
+    centres = torch.randn((count, dim), generator=gen, device=DEV)
+    v = centres[group] + 1e-3 * torch.randn((n, dim), generator=gen, device=DEV)
+    q = centres[torch.randint(0, count, (nq,), generator=gen, device=DEV)] + 1e-3 * torch.randn((nq, dim), generator=gen, device=DEV)
+    if metric == "cosine":
+        (v, q) = (torch.nn.functional.normalize(x, dim=1) for x in (v, q))
+    v[n // 2] = v[n // 3]  # a tie that the ids decide
+    (ids, d, left) = call(q, v, k, metric)
+    assert left == [] or dim == 4  # (groups of 4 columns lie on top of each other)
+    agrees_with_a_few_queries(q, v, k, metric, ids, d)

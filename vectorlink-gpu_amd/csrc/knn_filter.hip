@@ -484,12 +484,39 @@ __global__ __launch_bounds__(kLeftThreads) void left_kernel(const int32_t *__res
     if (tid == 0) left[0] = have;
 }
 
-// The dot product of a lane's row with the query: the products of knn_tile_kernel one fused multiply-add after the other,
-// as its matrix instructions form them (element x of the two chunks of a pair, then y, z, w).  The query row is the same
-// for all lanes.  kLines cache lines of 128 bytes are on their way at a time: the lanes' rows are scattered, so a line is
-// a round trip to memory, and one after the other they took 370 us for 1,000 queries at 1,536 columns.
-constexpr int kLines = 4;
-__device__ __forceinline__ float dot_in_tile_order(const float *__restrict__ row, const float *__restrict__ q, int dim) {
+// The dot products of up to 8 NG rows with the query, one row per lane: the products of knn_tile_kernel one fused
+// multiply-add after the other, as its matrix instructions form them (element x of the two chunks of a pair, then y, z, w).
+// The query row is the same for all lanes.  Rows come in lines of 32 columns, eight lanes to a line, and change hands in LDS
+// (8 KB a wavefront, a chunk's place as in the tiles' operands): read by its own lane, a row costs a cycle of the address
+// unit per 16 bytes (10,000 queries with some 950 rows each to evaluate at 32,768 x 768: 6.7 ms a call, 4.5 this way, which
+// is 7.5 TB/s of rows).  Eight loads per lane are on their way whatever the number of rows, 8 / NG lines of each.
+template <int NG>
+__device__ __forceinline__ float dots_in_tile_order(const float *__restrict__ vectors, const int32_t *ids, int n,
+                                                    const float *__restrict__ q, int dim, float4 *buf) {
+    constexpr int D = 8 / NG;
+    const int lane = threadIdx.x & (kWave - 1), c = lane & 7;
+    const float *src[NG];
+    int to[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int r = 8 * g + (lane >> 3);
+        src[g] = vectors + (int64_t)ids[min(r, n - 1)] * dim + 4 * c;
+        to[g] = r * CH + (c ^ swz(r));
+    }
+    const int own = lane & (8 * NG - 1);
+    const float4 *const mine = buf + own * CH;
+    const int lines = (dim + 31) / 32;
+    float4 x[8];
+    auto load = [&](int l0) {
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+#pragma unroll
+            for (int g = 0; g < NG; ++g)
+                if (8 * g < n && 32 * (l0 + d) + 4 * c < dim) x[d * NG + g] = *reinterpret_cast<const float4 *>(src[g] + 32 * (l0 + d));
+    };
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    load(0);
     float s = 0.0f;
     auto pair = [&](const float4 &a, const float4 &b, const float *p) {
         s = fmaf(a.x, p[0], s); s = fmaf(b.x, p[4], s);
@@ -497,66 +524,94 @@ __device__ __forceinline__ float dot_in_tile_order(const float *__restrict__ row
         s = fmaf(a.z, p[2], s); s = fmaf(b.z, p[6], s);
         s = fmaf(a.w, p[3], s); s = fmaf(b.w, p[7], s);
     };
-    const float4 *r4 = reinterpret_cast<const float4 *>(row);
-    const int lines = dim / 32;
-    float4 x[kLines][8];
-    auto load = [&](float4 (&to)[8], int l) {
-        if (l < lines)
+    for (int l0 = 0; l0 < lines; l0 += D) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) to[i] = r4[8 * l + i];
-    };
+        for (int d = 0; d < D; ++d)
 #pragma unroll
-    for (int j = 0; j < kLines; ++j) load(x[j], j);
-    for (int l = 0; l < lines; l += kLines)
+            for (int g = 0; g < NG; ++g) buf[d * 8 * NG * CH + to[g]] = x[d * NG + g];
+        __builtin_amdgcn_wave_barrier();
+        if (l0 + D < lines) load(l0 + D);
 #pragma unroll
-        for (int j = 0; j < kLines; ++j)
-            if (l + j < lines) {  // uniform
+        for (int d = 0; d < D; ++d) {
+            const int left = dim - 32 * (l0 + d);  // columns
+            const float *const p = q + 32 * (l0 + d);
+            const float4 *const line = mine + d * 8 * NG * CH;
+            if (left >= 32) {
+                float4 a[8];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) pair(x[j][2 * i], x[j][2 * i + 1], q + 32 * (l + j) + 8 * i);
-                load(x[j], l + j + kLines);
+                for (int i = 0; i < 8; ++i) a[i] = line[i ^ swz(own)];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) pair(a[2 * i], a[2 * i + 1], p + 8 * i);
+            } else {
+                for (int i = 0; 8 * i < left; ++i) {
+                    const float4 a = line[(2 * i) ^ swz(own)];
+                    if (8 * i + 4 == left) {  // a last chunk on its own
+                        s = fmaf(a.x, p[8 * i], s); s = fmaf(a.y, p[8 * i + 1], s); s = fmaf(a.z, p[8 * i + 2], s); s = fmaf(a.w, p[8 * i + 3], s);
+                    } else {
+                        pair(a, line[(2 * i + 1) ^ swz(own)], p + 8 * i);
+                    }
+                }
             }
-    int c = lines * 8;
-    for (; c + 2 <= dim / 4; c += 2) pair(r4[c], r4[c + 1], q + 4 * c);
-    if (c < dim / 4) {  // a last chunk on its own
-        const float4 a = r4[c];
-        const float *p = q + 4 * c;
-        s = fmaf(a.x, p[0], s);
-        s = fmaf(a.y, p[1], s);
-        s = fmaf(a.z, p[2], s);
-        s = fmaf(a.w, p[3], s);
+        }
+        __builtin_amdgcn_wave_barrier();
     }
     return s;
 }
 
+// The k-th smallest of n values in LDS, 1 <= k <= n <= kFound, bit by bit; each wavefront finds it for itself.
+template <int PER>
+__device__ __forceinline__ uint32_t kth_of(const uint32_t *values, int n, int k) {
+    const int lane = threadIdx.x & (kWave - 1);
+    uint32_t v[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) v[j] = kWave * j + lane < n ? values[kWave * j + lane] : 0xFFFFFFFFu;
+    uint32_t at = 0;
+    for (uint32_t bit = 1u << 31; bit; bit >>= 1) {
+        const uint32_t mid = at | bit;
+        int below = 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) below += __popcll(__builtin_amdgcn_ballot_w64(v[j] < mid));
+        if (below < k) at = mid;
+    }
+    return at;
+}
+__device__ __forceinline__ uint32_t kth_smallest(const uint32_t *values, int n, int k) {
+    if (n <= kWave) return kth_of<1>(values, n, k);
+    if (n <= 4 * kWave) return kth_of<4>(values, n, k);
+    if (n <= 16 * kWave) return kth_of<16>(values, n, k);
+    return kth_of<kFound / kWave>(values, n, k);
+}
+
 // One workgroup per query.  The sample's bound let through several times k candidates; the k-th best value among all of
 // them bounds the k-th best float32 value far better, so most are dropped before their rows are fetched (at 1,000 queries
-// x 32,768 x 1,536, k = 16: 350 candidates, 390 us when all were evaluated).  What is left is evaluated, and every
-// candidate's rank among them is counted.
-constexpr int kFinishThreads = 128;
-template <bool L2>
-__global__ __launch_bounds__(kFinishThreads) void finish_kernel(const float *__restrict__ queries,
-                                                                const float *__restrict__ vectors, int dim, int k,
-                                                                const int32_t *__restrict__ count,
-                                                                const uint64_t *__restrict__ found,
-                                                                const RowStat *__restrict__ qstat,
-                                                                const uint32_t *__restrict__ vmax, int slabs,
-                                                                const float *__restrict__ q_norm,
-                                                                const float *__restrict__ v_norm, int64_t q_first,
-                                                                int32_t *__restrict__ ids_out, float *__restrict__ d_out) {
-    __shared__ uint64_t keys[kFound];
-    __shared__ uint32_t values[kFound];
+// x 32,768 x 1,536, k = 16: 350 candidates, 390 us when all were evaluated).  What is left is evaluated, and those not
+// above the k-th best distance are ranked.
+template <bool L2, int THREADS>
+__global__ __launch_bounds__(THREADS) void finish_kernel(const float *__restrict__ queries,
+                                                         const float *__restrict__ vectors, int dim, int k,
+                                                         const int32_t *__restrict__ count,
+                                                         const uint64_t *__restrict__ found,
+                                                         const RowStat *__restrict__ qstat,
+                                                         const uint32_t *__restrict__ vmax, int slabs,
+                                                         const float *__restrict__ q_norm,
+                                                         const float *__restrict__ v_norm, int64_t q_first,
+                                                         int32_t *__restrict__ ids_out, float *__restrict__ d_out) {
+    constexpr int kWaves = THREADS / kWave;
+    __shared__ float4 buf[kWaves][kWave * CH];
+    __shared__ uint32_t values[kFound];  // of the pass, smallest is best; then the distances, as keys
     __shared__ int32_t ids[kFound];
-    __shared__ uint32_t kth_s;
-    __shared__ int n_s;
+    __shared__ int n_s, n_keys_s;
+    uint64_t *const keys = reinterpret_cast<uint64_t *>(&buf[0][0]);
+    static_assert(sizeof(buf) >= kFound * sizeof(uint64_t), "room for all keys");
     const int64_t q = q_first + blockIdx.x;
     const int tid = threadIdx.x;
     const int n = count[q];
     if (n > kFound) return;  // uniform; left to the tiles
     if (tid == 0) {
-        kth_s = 0;
         n_s = 0;
+        n_keys_s = 0;
     }
-    for (int i = tid; i < n; i += kFinishThreads) values[i] = vl_float_key(__builtin_bit_cast(float, (uint32_t)(found[q * kFound + i] >> 32)));  // larger is better
+    for (int i = tid; i < n; i += THREADS) values[i] = ~vl_float_key(__builtin_bit_cast(float, (uint32_t)(found[q * kFound + i] >> 32)));
     RowStat table = {0.0f, 0.0f};
     for (int s = 1; s <= slabs; ++s) {
         const RowStat one = table_stat(vmax + (int64_t)s * kStripes * kStripeWords);
@@ -564,45 +619,62 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(const float *__r
         table.norm = fmaxf(table.norm, one.norm);
     }
     __syncthreads();
-    if (n > k)
-        for (int i = tid; i < n; i += kFinishThreads) {
-            const uint32_t mine = values[i];
-            int rank = 0;
-            for (int j = 0; j < n; ++j) rank += values[j] > mine || (values[j] == mine && j < i);
-            if (rank == k - 1) kth_s = mine;
-        }
-    __syncthreads();
-    const float error = value_error(qstat[q], table, dim, L2);
-    float least = vl_key_float(kth_s) - error;
-    if (!L2) least = fminf(least, 1.0f - 1e-6f);  // values of 1 and more are one distance, 0
-    least -= error;
-    if (n <= k || (!L2 && least <= -0.999f)) least = -__builtin_inff();
-    for (int i = tid; i < n; i += kFinishThreads)
-        if (!(vl_key_float(values[i]) < least)) ids[atomicAdd(&n_s, 1)] = (int32_t)(uint32_t)found[q * kFound + i];
+    float least = -__builtin_inff();
+    if (n > k) {
+        const float error = value_error(qstat[q], table, dim, L2);
+        least = vl_key_float(~kth_smallest(values, n, k)) - error;
+        if (!L2) least = fminf(least, 1.0f - 1e-6f);  // values of 1 and more are one distance, 0
+        least -= error;
+        if (!L2 && least <= -0.999f) least = -__builtin_inff();
+    }
+    for (int i = tid; i < n; i += THREADS)
+        if (!(vl_key_float(~values[i]) < least)) ids[atomicAdd(&n_s, 1)] = (int32_t)(uint32_t)found[q * kFound + i];
     __syncthreads();
     const int left = n_s;
-    const float *q_row = queries + q * dim;
-    for (int i = tid; i < left; i += kFinishThreads) {
-        const int32_t id = ids[i];
-        const float s = dot_in_tile_order(vectors + (int64_t)id * dim, q_row, dim);
-        keys[i] = vl_make_key(id, tile_distance<L2>(s, L2 ? q_norm[q] : 0.0f, L2 ? v_norm[id] : 0.0f));
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    for (int base = 0; base < left; base += THREADS) {
+        // the same number of rows for each wavefront
+        const int rows = min(left - base, THREADS), per = (rows + kWaves - 1) / kWaves;
+        const int first = base + wave * per, mine = min(per, base + rows - first);
+        if (mine <= 0) continue;
+        float s;
+        auto dots = [&](auto groups) {
+            return dots_in_tile_order<decltype(groups)::value>(vectors, ids + first, mine, queries + q * dim, dim, buf[wave]);
+        };
+        if (mine <= 8) s = dots(std::integral_constant<int, 1>{});
+        else if (mine <= 16) s = dots(std::integral_constant<int, 2>{});
+        else if (mine <= 32) s = dots(std::integral_constant<int, 4>{});
+        else s = dots(std::integral_constant<int, 8>{});
+        const int i = first + (tid & (kWave - 1));
+        if (i < first + mine) {
+            const int32_t id = ids[i];
+            values[i] = (uint32_t)(vl_make_key(id, tile_distance<L2>(s, L2 ? q_norm[q] : 0.0f, L2 ? v_norm[id] : 0.0f)) >> 32);
+        }
     }
     __syncthreads();
-    for (int i = tid; i < left || i < k; i += kFinishThreads) {
-        if (i >= left) {  // fewer vectors than asked for
+    const uint32_t last = left > k ? kth_smallest(values, left, k) : 0xFFFFFFFFu;
+    for (int i = tid; i < left; i += THREADS)
+        if (values[i] <= last) keys[atomicAdd(&n_keys_s, 1)] = ((uint64_t)values[i] << 32) | (uint32_t)ids[i];
+    __syncthreads();
+    const int n_keys = n_keys_s;
+    for (int i = tid; i < n_keys || i < k; i += THREADS) {
+        if (i >= n_keys) {  // fewer vectors than asked for
             ids_out[q * k + i] = VL_MAXINT;
             d_out[q * k + i] = VL_MAXFLOAT;
             continue;
         }
         const uint64_t key = keys[i];
         int rank = 0;
-        for (int j = 0; j < left; ++j) rank += keys[j] < key;  // keys are unique
+        for (int j = 0; j < n_keys; ++j) rank += keys[j] < key;  // keys are unique
         if (rank < k) {
             ids_out[q * k + rank] = vl_key_id(key);
             d_out[q * k + rank] = vl_key_dist(key);
         }
     }
 }
+
+// Batches of so few queries leave compute units idle: 512 threads per query instead of 128.
+constexpr int64_t kFinishWide = 512;
 
 int64_t compute_units() {
     static const int64_t n = [] {
@@ -733,12 +805,12 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     }
     for (int64_t q0 = 0; q0 < n_queries; q0 += kMaxBlocks) {
         const dim3 grid((unsigned)(n_queries - q0 < kMaxBlocks ? n_queries - q0 : kMaxBlocks));
-        if (l2)
-            hipLaunchKernelGGL(finish_kernel<true>, grid, dim3(kFinishThreads), 0, st, queries, vectors, (int)dim, (int)k,
-                               count, found, qstat, vmax, (int)slabs, q_norm, v_norm, q0, ids_out, dists_out);
-        else
-            hipLaunchKernelGGL(finish_kernel<false>, grid, dim3(kFinishThreads), 0, st, queries, vectors, (int)dim, (int)k,
-                               count, found, qstat, vmax, (int)slabs, q_norm, v_norm, q0, ids_out, dists_out);
+        auto go = [&](auto kernel, int threads) {
+            hipLaunchKernelGGL(kernel, grid, dim3((unsigned)threads), 0, st, queries, vectors, (int)dim, (int)k, count, found,
+                               qstat, vmax, (int)slabs, q_norm, v_norm, q0, ids_out, dists_out);
+        };
+        if (n_queries <= kFinishWide) l2 ? go(finish_kernel<true, 512>, 512) : go(finish_kernel<false, 512>, 512);
+        else l2 ? go(finish_kernel<true, 128>, 128) : go(finish_kernel<false, 128>, 128);
     }
     VL_LAUNCH_CHECK("knn finish_kernel");
     hipLaunchKernelGGL(left_kernel, dim3(1), dim3(kLeftThreads), 0, st, count, (int)n_queries, (int)q_first, left, tile_bound);
