@@ -275,7 +275,7 @@ def test_candidates_of_every_number(members, dim, k, metric, nq):
     """Rows close to each other in groups: a query has its whole group to evaluate."""
     print(f"candidates members={members} dim={dim} nq={nq} k={k} {metric}", flush=True)
     gen = torch.Generator(device=DEV).manual_seed(members)
-    n = 12_007
+    n = 12_007 if members < 1000 else 80_003  # (in a short table the tiles take queries with so many)
     count = n // members
     group = torch.arange(n, device=DEV) % count
     centres = torch.randn((count, dim), generator=gen, device=DEV)
@@ -287,3 +287,21 @@ def test_candidates_of_every_number(members, dim, k, metric, nq):
     (ids, d, left) = call(q, v, k, metric)
     assert left == [] or dim == 4  # (groups of 4 columns lie on top of each other)
     agrees_with_a_few_queries(q, v, k, metric, ids, d)
+
+
+@pytest.mark.parametrize("n,dim,members,nq,k", [(16_384, 1536, 977, 1000, 10), (100_000, 64, 20_000, 300, 1), (9000, 128, 3000, 513, 16)])
+def test_queries_that_the_tiles_answer_sooner_are_left_to_them(n, dim, members, nq, k):
+    """The sample shows that a query has more candidates than are worth evaluating one by one; half the queries have few."""
+    print(f"expected candidates n={n} dim={dim} members={members} nq={nq} k={k}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    v = torch.nn.functional.normalize(torch.randn((n, dim), generator=gen, device=DEV), dim=1)
+    q = torch.nn.functional.normalize(torch.randn((nq, dim), generator=gen, device=DEV), dim=1)
+    crowd = torch.nn.functional.normalize(torch.randn((1, dim), generator=gen, device=DEV), dim=1)
+    q -= (q @ crowd.T) * crowd
+    at = torch.randperm(n, generator=gen, device=DEV)[:members]
+    v[at] = crowd + 1e-3 * v[at]
+    q[::2] = crowd + 1e-3 * q[::2]
+    (v, q) = (torch.nn.functional.normalize(x, dim=1) for x in (v, q))
+    (ids, d, left) = call(q, v, k)
+    assert left == list(range(0, nq, 2))
+    agrees_with_a_few_queries(q, v, k, "cosine", ids, d)

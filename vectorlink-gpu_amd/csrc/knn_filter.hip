@@ -15,8 +15,9 @@
 //   filter    the pass over all: ids of the values that are not out, per query
 //   finish    their float32 dot products - one fused multiply-add after the other in the order in which the float32 tiles'
 //             matrix instructions take the elements, which gives the tiles' bits - and the k best of them
-// A query with more candidates than its buffer holds (thousands of rows within the rounding of each other) is left to the
-// float32 tiles, which take all such queries of a call together.  For squared L2 the values are <q, v> - |v|^2 / 2: three more columns hold -|v|^2 / 2 as a sum of three
+// A query with more candidates than its buffer holds (thousands of rows within the rounding of each other), or than the
+// tiles are worth, is left to the float32 tiles, which take all such queries of a call together; most are known from the
+// sample and are not looked for in the pass.  For squared L2 the values are <q, v> - |v|^2 / 2: three more columns hold -|v|^2 / 2 as a sum of three
 // bfloat16 numbers (24 bits), and ones on the query side.
 //
 // The pass: 256 vectors x 256 queries per workgroup of eight wavefronts (128 x 64 each, 128 accumulator registers), 64
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *__restrict__ v16, int64_t n_vectors,
                  int kp2, int64_t strip_len, int n_strips, int n_qblocks, int q_group, float *__restrict__ gmax,
                  const float *__restrict__ bound, const RowStat *__restrict__ qstat, const uint32_t *__restrict__ vmax,
-                 int dim, int l2, int64_t id0, int32_t *__restrict__ count,
+                 const uint32_t *__restrict__ sample_vmax, int dim, int l2, int64_t id0, int32_t *__restrict__ count,
                  uint64_t *__restrict__ found) {
     extern __shared__ __align__(16) float smem[];
     constexpr int T = TR * KT;  // floats of a staged operand
@@ -209,18 +210,23 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
     const int64_t v_end = min(n_vectors, v_begin + strip_len);
 
     float thr[CB], top[CB][RB];
-    RowStat table = {0.0f, 0.0f};
-    if constexpr (EMIT) table = table_stat(vmax);
+    RowStat table = {0.0f, 0.0f}, sampled = {0.0f, 0.0f};
+    if constexpr (EMIT) {
+        table = table_stat(vmax);
+        sampled = table_stat(sample_vmax);
+    }
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
         if constexpr (EMIT) {
             const int64_t q = q0 + 64 * wc + 32 * cb + l32;
             thr[cb] = __builtin_inff();
             if (q < n_queries) {
-                thr[cb] = bound[q] - value_error(qstat[q], table, dim, l2 != 0);
-                // No bound (a row that is not finite, or so long that its rounding covers every value): the query is
-                // left to the tiles.  So a threshold is above -infinity, which is what rows past the strip's end hold.
-                if (!(thr[cb] > (l2 ? -__builtin_inff() : -0.999f))) {
+                const float error = value_error(qstat[q], table, dim, l2 != 0);
+                thr[cb] = bound[q] - error;
+                // No bound (a row that is not finite), or one that lets everything through because a row is far longer than
+                // those of the sample: the query is left to the tiles.  So a threshold is above -infinity, which is what
+                // rows past the strip's end hold.
+                if (!(thr[cb] > (l2 ? -__builtin_inff() : -0.999f)) || error > 16.0f * value_error(qstat[q], sampled, dim, l2 != 0)) {
                     thr[cb] = __builtin_inff();
                     if (strip == 0 && wr == 0 && half == 0) atomicAdd(&count[q], kFound + 1);
                 }
@@ -229,6 +235,8 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) top[cb][rb] = -__builtin_inff();
     }
+    if constexpr (EMIT)
+        if (!__syncthreads_or(thr[0] < __builtin_inff() || thr[1] < __builtin_inff())) return;  // none of these queries is looked for
     int a_off[RB], b_off[CB];
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
@@ -404,11 +412,12 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
     }
 }
 
-// bound[q]: what the k-th best float32 value of query q is not below, from the k-th largest of its groups' maxima.
+// bound[q]: what the k-th best float32 value of query q is not below, from the k-th largest of its groups' maxima.  A query
+// that too many vectors (most of them) are expected to pass is left to the tiles before the pass: its bound is infinite.
 __global__ __launch_bounds__(256) void bound_kernel(const float *__restrict__ gmax, int groups, int k, int64_t n_queries,
                                                     const RowStat *__restrict__ qstat, const uint32_t *__restrict__ vmax,
-                                                    int dim, int l2, float *__restrict__ bound,
-                                                    int32_t *__restrict__ count) {
+                                                    int dim, int l2, float rows_per_sample_row, int most,
+                                                    float *__restrict__ bound, int32_t *__restrict__ count) {
     const int64_t q = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
     if (q >= n_queries) return;
     const int lane = threadIdx.x & (kWave - 1);
@@ -439,11 +448,23 @@ __global__ __launch_bounds__(256) void bound_kernel(const float *__restrict__ gm
         }
     }
     const RowStat table = table_stat(vmax);
+    const float error = value_error(qstat[q], table, dim, l2 != 0);
+    float t = vl_key_float(~kth) - error;
+    if (!l2) t = fminf(t, 1.0f - 1e-6f);  // values of 1 and more are one distance, 0
+    // How many vectors will not be out: their rows of the sample lie in any group with the same chance, so a share of
+    // exp(-m / groups) of the groups holds none of m such rows.
+    const float limit = t - error;
+    int without = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int g = lane + kWave * j;
+        without += __popcll(__ballot(g < groups && gmax[q * groups + min(g, groups - 1)] < limit));
+    }
+    const float vectors = -(float)groups * logf((float)without / (float)groups) * rows_per_sample_row;  // infinite if none is without
     if (lane == 0) {
-        float t = vl_key_float(~kth) - value_error(qstat[q], table, dim, l2 != 0);
-        if (!l2) t = fminf(t, 1.0f - 1e-6f);  // values of 1 and more are one distance, 0
-        bound[q] = t == t ? t : -__builtin_inff();
-        count[q] = 0;
+        const bool fits = vectors <= (float)most;  // (no bound: no group is without)
+        bound[q] = fits ? t : __builtin_inff();
+        count[q] = fits ? 0 : kFound + 1;
     }
 }
 
@@ -733,6 +754,12 @@ bool vl_knn_filter_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64
     p->slab_rows = (2ll << 30) / (p->kp * 2) / TR * TR;
     if (p->slab_rows < p->sample_rows) p->slab_rows = p->sample_rows;
     if (p->slab_rows > n_vectors) p->slab_rows = n_vectors;
+    // A query with more candidates than this is left to the tiles.  On full batches the tiles take 0.0163 ps per product and
+    // 0.14 ps per place of their lists for a vector, a candidate 40 ps and 0.4 ps a column, and the pass, which such a query
+    // saves as well, 0.002 ps per product.  A guess somewhat above what the buffer holds is still tried: the sample is off
+    // by a tenth (4,000 queries with 2,000 candidates each at 500,000 x 384: 4.5 ms, with the tiles 12.8).
+    const double even = (double)n_vectors * (0.014 * (double)dim + 0.14 * (double)k) / (40.0 + 0.4 * (double)dim);
+    p->most = (int)(even < kFound * 1.25 ? even : kFound * 1.25);
     int64_t o = 0;
     p->off_q16 = o; o = align256(o + n_queries * p->kp * 2);
     p->off_v16 = o; o = align256(o + p->slab_rows * p->kp * 2);
@@ -783,7 +810,7 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), smem, st, (const float *)q16, n_queries,
                                (const float *)v16, rows, kp2, len, (int)strips, (int)q_blocks, (int)q_group, gmax, bound,
-                               qstat, top, (int)dim, l2 ? 1 : 0, id0, count, found);
+                               qstat, top, vmax, (int)dim, l2 ? 1 : 0, id0, count, found);
         };
         if (emit) go(pass_kernel<true>);
         else go(pass_kernel<false>);
@@ -794,7 +821,7 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     pass(false, p.sample_rows, p.sample_strips, vmax, 0);
     VL_LAUNCH_CHECK("knn pass_kernel (sample)");
     hipLaunchKernelGGL(bound_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, gmax, p.groups, (int)k,
-                       n_queries, qstat, vmax, (int)dim, l2 ? 1 : 0, bound, count);
+                       n_queries, qstat, vmax, (int)dim, l2 ? 1 : 0, (float)n_vectors / (float)p.sample_rows, p.most, bound, count);
     VL_LAUNCH_CHECK("knn bound_kernel");
     for (int64_t s = 0; s < slabs; ++s) {
         const int64_t r0 = s * p.slab_rows;
