@@ -15,7 +15,7 @@ After the build:
   * roofline pass: the first K batches of the state every optimisation loop
     started from are run again with the hooks ON (HIP events around the
     launches on the launch stream, fetched rows counted on the device); the
-    per-loop averages are combined with the timed build's launch counts;
+    per-loop averages are combined with the timed build's launches;
   * measured ceilings of the box: a 1 GiB device copy, and the library's own
     gathered-distance kernel over a 4.3 GiB and a 120 MiB table with ids in
     memory order and with uniformly random ids;
@@ -47,6 +47,7 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0   # MI355X published HBM3E bandwidth
 MFMA_FP32_PEAK = 157.3  # MI355X published dense fp32 matrix TFLOP/s
+MFMA_BF16_PEAK = 2500.0  # and bf16, which forms all pairs of an exact-kNN call that goes through the filter
 
 PROFILE_DIR = os.path.join(ROOT, "profiles")
 LINE_LIMIT = 3072       # the one JSON line on stdout stays below this many bytes
@@ -83,6 +84,34 @@ def traffic_from_profiles(workload):
     return out, os.path.relpath(path, ROOT)
 
 
+def profiled_algorithmic_bytes(workload):
+    """Algorithmic bytes per launch of the committed profile's own run, per optimisation-loop state ([] without one)."""
+    path = os.path.join(PROFILE_DIR, f"beam_step_kernel_{workload}_by_phase.txt")
+    if not os.path.exists(path):
+        return []
+    with open(path) as f:
+        found = re.findall(r"^  state of loop (\d+): .* algorithmic bytes per launch ([0-9.]+) GB", f.read(), re.M)
+    return [float(b) * 1e9 for (_, b) in sorted(found, key=lambda x: int(x[0]))]
+
+
+def launches_for(iterations, replay):
+    """Launches that so many iterations of the timed build take, at the iterations per launch of its replay."""
+    return int(round(iterations / max(replay["iterations_per_launch"], 1.0)))
+
+
+def same_launches(per_loop, profiled):
+    """Whether launches of this run move what those of the profiled run did: counters per launch say nothing about
+    launches of another number of iterations."""
+    return len(profiled) >= len(per_loop) and all(
+        0.8 < r["algorithmic_bytes_per_launch"] / b < 1.25 for r, b in zip(per_loop, profiled))
+
+
+def knn_peak(nv, queries, n, dim, k):
+    """Peak of the unit that forms all pairs of such an exact-kNN call."""
+    form = nv.check(nv.lib().vl_knn_form(queries, n, dim, k, 0, (1 << 63) - 1))
+    return MFMA_BF16_PEAK if form == nv.KNN_FORMS["filter"] else MFMA_FP32_PEAK
+
+
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
@@ -108,7 +137,8 @@ def step_roofline(prof, dim, batch_rows):
     gbs = algo / secs / 1e9 if secs > 0 else 0.0
     ref_equiv = (prof["wanted"] * per_eval + q_loads) / secs / 1e9 if secs > 0 else 0.0
     wanted = max(prof["wanted"], 1.0)
-    return dict(launches=int(prof["expand_launches"]), avg_launch_ms=prof["expand_ms"] / launches,
+    return dict(launches=int(prof["expand_launches"]), iterations_per_launch=prof["iterations"] / launches,
+                avg_launch_ms=prof["expand_ms"] / launches,
                 algorithmic_bytes_per_launch=algo / launches, achieved_gbs=gbs, frac=gbs / HBM_PEAK_GBS,
                 reference_equivalent_gbs=ref_equiv,
                 candidate_rows_fetched=prof["evals"] / wanted,
@@ -437,7 +467,7 @@ def main():
     torch.cuda.synchronize()
 
     if args.knn_only:
-        out = {"metric": "dense distance tiles (fp32 MFMA), TFLOP/s", "unit": "TFLOP/s", "n_gpus": 1,
+        out = {"metric": "exact kNN (all pairs), TFLOP/s", "unit": "TFLOP/s", "n_gpus": 1,
                "higher_is_better": True, "dtype": "f32", "data": "synthetic",
                "config": {"workload": args.workload, "n": n, "dim": dim, "queries": int(qdev.shape[0])}}
         from vectorlink_gpu.ann import entry_point_ids
@@ -452,10 +482,11 @@ def main():
             torch.cuda.synchronize()
             dt = (time.time() - t0) / reps
             flops = 2.0 * qdev.shape[0] * table.shape[0] * dim
+            peak = knn_peak(nv, qdev.shape[0], table.shape[0], dim, k)
             out[name] = dict(bound="mfma", vectors=int(table.shape[0]), k=k, seconds=dt, tflops=flops / dt / 1e12,
-                             peak_tflops=MFMA_FP32_PEAK, frac=flops / dt / 1e12 / MFMA_FP32_PEAK, calls=reps + 1)
+                             peak_tflops=peak, frac=flops / dt / 1e12 / peak, calls=reps + 1)
         out["value"] = out["exact_knn"]["tflops"]
-        out["roofline"] = dict(bound="mfma", achieved=out["exact_knn"]["tflops"], peak=MFMA_FP32_PEAK, unit="TFLOP/s",
+        out["roofline"] = dict(bound="mfma", achieved=out["exact_knn"]["tflops"], peak=out["exact_knn"]["peak_tflops"], unit="TFLOP/s",
                                frac=out["exact_knn"]["frac"], traffic=None)
         print(json.dumps(out))
         return
@@ -521,7 +552,9 @@ def main():
         torch.cuda.synchronize()
         r = step_roofline(profile_read(nv, reset=True, enable=0), dim, batch_rows)
         phases.mark(f"roofline pass, state of loop {li}")
-        r.update(loop=li, replayed_batches=replay, build_launches_of_this_loop=int(build.stats[li]["iterations"]),
+        iterations = int(build.stats[li]["iterations"])
+        r.update(loop=li, replayed_batches=replay, build_iterations_of_this_loop=iterations,
+                 build_launches_of_this_loop=launches_for(iterations, r),
                  build_seconds_of_this_loop=build.stats[li]["seconds"])
         per_loop.append(r)
         del rb
@@ -532,7 +565,8 @@ def main():
     achieved = w_bytes / (w_time / 1e3) / 1e9 if w_time > 0 else 0.0
     (per_loop_traffic, traffic_file) = traffic_from_profiles(args.workload)
     traffic = traffic_detail = None
-    if per_loop_traffic and len(per_loop_traffic) >= len(per_loop) and args.n is None:
+    if (per_loop_traffic and len(per_loop_traffic) >= len(per_loop) and args.n is None
+            and same_launches(per_loop, profiled_algorithmic_bytes(args.workload))):
         traffic = sum(wt * tb for wt, tb in zip(weights, per_loop_traffic)) / w_launch
         for tb, r in zip(per_loop_traffic, per_loop):
             r["traffic_bytes_per_launch"] = tb
@@ -546,7 +580,8 @@ def main():
             bytes_per_launch_by_loop=per_loop_traffic[:len(per_loop)])
     roofline = dict(
         bound="hbm",
-        kernel="beam_step_kernel (one beam-search iteration: gathered cosine distances + queue merge per row)",
+        kernel="beam_window / beam_step kernels (the iterations between two progress checks, or one: gathered cosine "
+               "distances + queue merge per row)",
         achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s", frac=achieved / HBM_PEAK_GBS,
         frac_scope="algorithmic bytes over the published HBM peak; the bytes are served by the path beyond L2 "
                    "(memory-side cache + HBM), see gather_gbs_measured for what that path delivers on this box",
@@ -564,7 +599,8 @@ def main():
                             batches_in_flight=args.concurrent_batches),
         method=f"hooks are off in the timed build; the first {replay} batches of the tables each optimisation loop "
                "started from were run again with HIP events around the launches (on the launch stream) and the fetched "
-               "rows counted on the device; per-loop averages below, combined here with the timed build's launch counts",
+               "rows counted on the device; per-loop averages below, combined here with the timed build's launches (its "
+               "iterations over those that a launch of the replay took)",
         per_loop=per_loop)
     log(f"[bench] roofline: {achieved:.0f} GB/s = {achieved / HBM_PEAK_GBS:.3f} of peak; per loop: "
         + ", ".join(f"{r['avg_launch_ms']:.3f} ms {r['frac']:.3f}" for r in per_loop))
@@ -598,8 +634,9 @@ def main():
         torch.cuda.synchronize()
         t_knn = time.time() - t0
         flops = 2.0 * qdev.shape[0] * n * dim
-        result["exact_knn"] = dict(seconds=t_knn, tflops=flops / t_knn / 1e12, peak_tflops=MFMA_FP32_PEAK,
-                                   frac=flops / t_knn / 1e12 / MFMA_FP32_PEAK, bound="mfma")
+        peak = knn_peak(nv, qdev.shape[0], n, dim, 10)
+        result["exact_knn"] = dict(seconds=t_knn, tflops=flops / t_knn / 1e12, peak_tflops=peak,
+                                   frac=flops / t_knn / 1e12 / peak, bound="mfma")
         log(f"[bench] exact kNN: {t_knn:.3f} s = {result['exact_knn']['tflops']:.1f} TFLOP/s")
 
         def one_search(qs, seeding, mode, runs=args.search_runs):
@@ -669,7 +706,8 @@ def main():
         result["search"]["roofline"] = dict(
             iterations=dict(bound="hbm", queue=qs, **sr),
             seeding_tiles=dict(bound="mfma", seconds=t_seed, tflops=seed_flops / t_seed / 1e12,
-                               frac=seed_flops / t_seed / 1e12 / MFMA_FP32_PEAK,
+                               frac=seed_flops / t_seed / 1e12 / knn_peak(nv, qdev.shape[0], entry_vectors.shape[0],
+                                                                          entry_vectors.shape[1], k_seed),
                                entry_points=int(entry_vectors.shape[0])))
         # the same graph searched with other settings of the additions (entry points of the dense seeding, queue
         # length, how often progress is checked, which stop): the fastest of them that still reaches recall@10 >= 0.95

@@ -86,3 +86,35 @@ def test_traffic_is_read_from_the_committed_profile():
     assert source == os.path.join("profiles", "beam_step_kernel_mix-1m-768_by_phase.txt")
     assert len(per_loop) == 3 and all(1e8 < b < 1e11 for b in per_loop)
     assert bench.traffic_from_profiles("no-such-workload") == (None, None)
+
+
+def test_launches_of_several_iterations_are_not_counted_as_iterations():
+    """A replay of 500 iterations in 100 launches: a build of 5,000 iterations took 1,000 of them, not 5,000, and
+    counters of launches of one iteration each say nothing about these."""
+    sys.path.insert(0, ROOT)
+    import bench
+
+    prof = dict(expand_ms=200.0, merge_ms=0.0, expand_launches=100, merge_launches=100, evals=10**7, sketched=0,
+                wanted=10**7, rows=10**4, iterations=500)
+    r = bench.step_roofline(prof, 768, 10_000)
+    assert r["launches"] == 100 and r["iterations_per_launch"] == 5.0
+    assert bench.launches_for(5000, r) == 1000
+    one = bench.step_roofline(dict(prof, expand_launches=500), 768, 10_000)
+    assert bench.launches_for(5000, one) == 5000
+    assert one["algorithmic_bytes_per_launch"] * 5 == r["algorithmic_bytes_per_launch"]
+    assert bench.same_launches([r], [1.1 * r["algorithmic_bytes_per_launch"]])
+    assert not bench.same_launches([r], [one["algorithmic_bytes_per_launch"]])
+    assert not bench.same_launches([r], [])
+    assert len(bench.profiled_algorithmic_bytes("mix-1m-768")) == 3
+    assert bench.profiled_algorithmic_bytes("no-such-workload") == []
+
+
+def test_exact_knn_is_compared_with_the_unit_that_forms_all_pairs():
+    sys.path.insert(0, ROOT)
+    sys.path.insert(0, os.path.join(ROOT, "vectorlink-gpu_amd"))
+    import bench
+    from vectorlink_gpu import _native as nv
+
+    assert bench.knn_peak(nv, 10_000, 1_000_000, 768, 10) == bench.MFMA_BF16_PEAK   # the filter
+    assert bench.knn_peak(nv, 10_000, 2_000, 768, 10) == bench.MFMA_FP32_PEAK       # tiles
+    assert bench.knn_peak(nv, 1, 1_000_000, 768, 10) == bench.MFMA_FP32_PEAK        # a few queries

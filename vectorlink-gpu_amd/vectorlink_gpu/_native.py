@@ -24,6 +24,7 @@ class BeamParams(C.Structure):
 
 
 METRICS = {"cosine": 0, "l2": 1}  # include/vlgpu.h: VL_METRIC_COSINE, VL_METRIC_L2
+KNN_FORMS = {"tiles": 0, "few": 1, "filter": 2}  # VL_KNN_TILES, VL_KNN_FEW, VL_KNN_FILTER
 
 
 def metric_code(name: str) -> int:
