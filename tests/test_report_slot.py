@@ -79,3 +79,11 @@ def output(tmp_path_factory):
 
 def test_slots_and_waits(output):
     assert output.returncode == 0, output.stdout
+
+
+def test_a_long_wait_leaves_the_core_to_others(output):
+    """The stand-in GPU reports after 200 ms: a wait that only looks takes 200 ms of a core.  One that sleeps takes the 1 ms
+    until it does, and a look of some us every 20 us and more (the rest: starting the program, allocating)."""
+    assert output.returncode == 0, output.stdout
+    cpu_ms = int(output.stdout.split("cpu_ms")[1].split()[0])
+    assert cpu_ms < 60, cpu_ms

@@ -6,7 +6,9 @@
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
+#include <chrono>
 #include <mutex>
+#include <thread>
 
 struct BeamReport {
     int changed, sketch_rows, error;  // as in BeamCtrl, after the checking iteration
@@ -47,21 +49,35 @@ public:
 
     // Waits until the launch behind the check after iteration t has reported: 0, or below 0 (-1: the stream has ended
     // without a report, others as state()).  The stream is asked now and then, so that a launch that failed ends the wait.
+    // A wait of a short call is some 60 us and looks all the time; from kLook on it lets other threads have the core
+    // between two looks, and from kYield on - the launches of a large batch take 2 to 15 ms, and the next one is on the
+    // stream already - it sleeps.
     int wait(int t) const {
+        using Clock = std::chrono::steady_clock;
         const BeamReport *r = get();
-        for (unsigned spins = 1;; ++spins) {
-            if (__atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t) return 0;
-            if ((spins & 0xffff) == 0) {
+        const auto start = Clock::now();
+        auto asked = start;
+        for (;;) {
+            for (int i = 0; i < 64; ++i) {
+                if (__atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t) return 0;
+                __builtin_ia32_pause();
+            }
+            const auto now = Clock::now();
+            if (now - start < kLook) continue;
+            if (now - asked > kAsk) {
+                asked = now;
                 const int s = gpu_.state();
                 if (s < 0) return s;
                 if (s == 0) return __atomic_load_n(&r->check, __ATOMIC_ACQUIRE) == t ? 0 : -1;
             }
-            __builtin_ia32_pause();
+            if (now - start < kYield) std::this_thread::yield();
+            else std::this_thread::sleep_for(kSleep);
         }
     }
 
 private:
     static constexpr int kSlots = 64;
+    static constexpr std::chrono::microseconds kLook{200}, kYield{1000}, kSleep{20}, kAsk{2000};
     struct alignas(64) Slot { BeamReport report; };
     static inline std::mutex mutex_;
     static inline Slot *page_ = nullptr;
