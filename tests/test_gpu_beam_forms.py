@@ -105,3 +105,27 @@ def test_odd_rows_with_values_that_are_not_finite(value):
     want = orc.gather_distances(v, v, ids)
     got = gather_distances(dev(v), dev(v), dev(ids)).cpu().numpy()
     assert np.array_equal(got, want, equal_nan=True)
+
+
+@pytest.mark.parametrize("n,dim,windows", [(45_000, 768, True), (45_000, 772, False), (20_000, 768, False)])
+def test_which_calls_with_a_sketch_take_several_iterations_per_launch(n, dim, windows):
+    """More than 32 MiB of sketch and at most 768 columns: the launches of a call tell."""
+    print(f"sketch windows n={n} dim={dim}", flush=True)
+    from vectorlink_gpu import Queue, _native
+    from vectorlink_gpu.ann import closest_vectors, excluding_self
+    from vectorlink_gpu.kernels import build_sketch, calculate_distances
+    from vectorlink_gpu.utils import generate_circulant_beams, primes
+
+    gen = torch.Generator(device="cuda").manual_seed(n + dim)
+    v = torch.nn.functional.normalize(torch.randn((n, dim), generator=gen, device="cuda"), dim=1)
+    (rows, ql) = (64, 32)
+    beams = generate_circulant_beams(n, primes(ql, "cuda"))
+    q = Queue(rows, ql, ql + ql * 4, device="cuda")
+    q.insert(beams[:rows], calculate_distances(v, beams)[:rows])
+    c = dict(orc.DEFAULT_CONFIG)
+    c.update(beam_size=16, beam_queue_factor=2)
+    before = _native.lib().vl_beam_launches()
+    t = closest_vectors(v[:rows], q, v, beams, c, excluding_self(0, rows, ql, "cuda"), sketch=build_sketch(v))
+    launches = _native.lib().vl_beam_launches() - before
+    assert t >= 10  # (one launch more than needed is on its way when the loop ends, of five iterations or of one)
+    assert (launches < t) == windows, (launches, t)

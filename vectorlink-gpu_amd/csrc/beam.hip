@@ -41,9 +41,10 @@ struct BeamProfile {
     double expand_ms = 0, merge_ms = 0;
     int64_t expand_launches = 0, merge_launches = 0, evals = 0, rows = 0, iterations = 0, wanted = 0, sketched = 0;
 };
-// The only mutable state of the library besides the thread-local error text.  A call
-// sums into a BeamProfile of its own and adds it here once, under the mutex, when it
-// returns, so calls on different host threads do not tear each other's sums.
+// A call sums into a BeamProfile of its own and adds it here once, under the mutex, when
+// it returns, so calls on different host threads do not tear each other's sums.  (The
+// library's other mutable state: the launch counter below, the page of report slots in
+// beam_report.h, the thread-local error text.)
 BeamProfile g_prof;
 std::mutex g_prof_mutex;
 std::atomic<int64_t> g_step_launches{0};  // vl_beam_launches
@@ -884,7 +885,13 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     // With the sketch a window fits a compute unit six times, the one-iteration kernel eight times.  Rows that come from
     // HBM do not need those (a batch of the first loop at 1M x 768: 148 -> 140 ms, 1M x 384 49.4 -> 47.2, 50,000 x 768
     // 93.7 -> 91.2); while the table fits the chip's L2s (8 x 4 MiB) the launches wait on round trips and do (builds of
-    // 20,011 x 768: 133 ms without, 143 with windows, 30,000 x 768 254 and 262).
+    // 20,011 x 768: 133 ms without, 143 with windows, 30,000 x 768 254 and 262).  From 769 columns on the sketch window
+    // spills vector registers, and what it saves in launches goes there: a batch of the first loop at 600,000 x 2,048 534.8
+    // ms without and 541.9 with windows, 100,000 x 2,048 356 and 362, 600,000 x 1,536 373.1 and 373.5, 600,000 x 1,024 228.9
+    // and 228.8, builds of 24,000 x 1,536 199.9 and 205.0, 50,000 x 1,024 510 and 514 (600,000 x 512: 121.0 and 114.9).
+    // Without a sketch windows are faster for every length of a row (10,000 queries at 150,000 rows of 512 columns 7.34 ->
+    // 6.68 ms, 1,024 9.26 -> 7.79, 1,536 9.91 -> 9.15, 2,048 12.17 -> 11.74; 1,000 queries 1.46 -> 0.95, 1.67 -> 1.12,
+    // 1.82 -> 1.27, 2.00 -> 1.83).
     // VL_BEAM_WINDOWS / VL_BEAM_NO_WINDOWS in flags, or VL_BEAM_WINDOW=1 / 0 in the environment: windows always / never.
     static const int window_env = [] {
         const char *e = getenv("VL_BEAM_WINDOW");
@@ -893,7 +900,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     const bool all_windows = window_env >= 0 ? window_env != 0 : (p->flags & VL_BEAM_WINDOWS) != 0;
     const bool no_windows = window_env >= 0 ? window_env == 0 : (p->flags & VL_BEAM_NO_WINDOWS) != 0;
     constexpr int64_t kL2Bytes = 32 << 20;
-    const bool sketch_window = all_windows || p->n_vectors * sketch_row_bytes(p->dim) > kL2Bytes;
+    const bool sketch_window = all_windows || (p->dim <= 768 && p->n_vectors * sketch_row_bytes(p->dim) > kL2Bytes);
     const int step_threads = merge_threads == 128 ? 128 : 256;
     const bool use_window = use_fused && !no_windows && R >= 2 && row_hash_slots_most(a.E, a.m) < 0xffff &&
                             smem_window + 2048 <= kLdsPerCu;
