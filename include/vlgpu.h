@@ -379,7 +379,7 @@ int64_t vl_optimize_graph_workspace_bytes(int64_t n, int64_t width, int64_t degr
 int vl_optimize_graph(const int32_t *beams, int64_t n, int64_t width, int64_t degree,
                       int32_t *out, void *workspace, int64_t workspace_bytes, void *stream);
 
-/* ---- exact k nearest neighbours on dense fp32 MFMA tiles -------------- */
+/* ---- exact k nearest neighbours on the matrix cores -------------------- */
 /* No counterpart in the reference (its recall is self-recall@1 only,
  * ann.py:235-259); used for ground truth recall@k.  ids_out/dists_out are
  * [n_queries, k], ordered by (distance, id).  k <= 16, dim % 4 == 0,

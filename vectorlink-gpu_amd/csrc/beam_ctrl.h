@@ -6,7 +6,8 @@
 //                 modulo 3 (iteration t reads t-1 and t, raises t+1, and rows of
 //                 one launch may be in different phases); it is the first column
 //                 that is empty in every row (utils.py:63-66) because rows are
-//                 kept sorted
+//                 packed at the front (the fused step appends, the merge kernels
+//                 keep them sorted as well)
 //   changed[64] - ring of "some row changed" flags, one per checking iteration
 //   sketch_rows - how many rows currently use the 8-bit sketch (they opt in once and may opt out once)
 //   error       - a row found its own state impossible (see beam_row_state_ok)

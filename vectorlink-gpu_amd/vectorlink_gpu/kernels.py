@@ -160,9 +160,11 @@ def queue_sort_(ids: Tensor, distances: Tensor):
 
 
 def knn_exact(queries: Tensor, vectors: Tensor, k: int, metric: str = "cosine") -> Tuple[Tensor, Tensor]:
-    """Exact k nearest neighbours under `metric` on dense fp32 MFMA tiles
-    (no counterpart in the reference; ground truth for recall@k).  Returns
-    (ids [Q, k] int32, distances [Q, k] float32) ordered by (distance, id)."""
+    """Exact k nearest neighbours under `metric` on the matrix cores (no
+    counterpart in the reference; ground truth for recall@k).  Returns
+    (ids [Q, k] int32, distances [Q, k] float32) ordered by (distance, id).
+    Every distance is a float32 one; larger calls find the vectors that can be
+    among the k best with bfloat16 products and proven bounds first."""
     _check_f32(queries, "queries")
     _check_f32(vectors, "vectors")
     nv.require_gpu(queries, vectors)
