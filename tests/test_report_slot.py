@@ -82,7 +82,7 @@ def test_slots_and_waits(output):
 
 
 def test_a_long_wait_leaves_the_core_to_others(output):
-    """The stand-in GPU reports after 200 ms: a wait that only looks takes 200 ms of a core.  One that sleeps takes the 1 ms
+    """The stand-in GPU reports after 200 ms: a wait that only looks takes 200 ms of a core.  One that sleeps takes the 2 ms
     until it does, and a look of some us every 20 us and more (the rest: starting the program, allocating)."""
     assert output.returncode == 0, output.stdout
     cpu_ms = int(output.stdout.split("cpu_ms")[1].split()[0])

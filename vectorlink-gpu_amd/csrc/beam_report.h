@@ -50,8 +50,8 @@ public:
     // Waits until the launch behind the check after iteration t has reported: 0, or below 0 (-1: the stream has ended
     // without a report, others as state()).  The stream is asked now and then, so that a launch that failed ends the wait.
     // A wait of a short call is some 60 us and looks all the time; from kLook on it lets other threads have the core
-    // between two looks, and from kYield on - the launches of a large batch take 2 to 15 ms, and the next one is on the
-    // stream already - it sleeps.
+    // between two looks, and from kYield on it sleeps between them (a build's waits are 2 to 15 ms, and the next launch is
+    // on the stream already).
     int wait(int t) const {
         using Clock = std::chrono::steady_clock;
         const BeamReport *r = get();
@@ -77,7 +77,7 @@ public:
 
 private:
     static constexpr int kSlots = 64;
-    static constexpr std::chrono::microseconds kLook{200}, kYield{1000}, kSleep{20}, kAsk{2000};
+    static constexpr std::chrono::microseconds kLook{200}, kYield{2000}, kSleep{20}, kAsk{2000};
     struct alignas(64) Slot { BeamReport report; };
     static inline std::mutex mutex_;
     static inline Slot *page_ = nullptr;
