@@ -408,6 +408,12 @@ int vl_knn_exact_metric(const float *queries, int64_t n_queries,
 #define VL_KNN_FILTER 2
 int vl_knn_form(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
                 int64_t workspace_bytes);
+/* Added to the metric of this, vl_knn_left_offset and vl_knn_exact_metric: the
+ * filter takes the call whatever the sizes (from 4,096 vectors on, in a workspace
+ * of vl_knn_metric_workspace_bytes), for tests and measurements. */
+#define VL_KNN_ANY_SIZE 256
+/* The workspace of a call with that metric. */
+int64_t vl_knn_metric_workspace_bytes(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric);
 /* Where in the workspace of a call that the filter takes an int32 holds, once
  * the call has run, how many of its queries were left to the float32 tiles (their
  * numbers follow it): those with more vectors within the bfloat16 rounding of

@@ -105,6 +105,25 @@ def test_knn_workspace_serves_both_metrics(lib, metric):
         assert lib.vl_knn_form(*s, metric, lib.vl_knn_workspace_bytes(*s)) == lib.vl_knn_form(*s, metric, 1 << 60), s
 
 
+def test_the_filter_is_left_out_where_the_tiles_are_sooner(lib):
+    """Short calls stay with the float32 tiles; long ones go through the filter, and so does any if asked for."""
+    few, tiles, filt = 1, 0, 2
+    form = lambda *s: lib.vl_knn_form(*s, 0, 1 << 60)
+    assert form(300, 4096, 64, 10) == tiles and form(10_000, 4096, 64, 10) == tiles
+    assert form(1500, 6000, 768, 10) == tiles and form(300, 32_768, 64, 1) == tiles and form(129, 12_000, 20, 16) == tiles
+    assert form(10_000, 32_768, 64, 4) == filt and form(1000, 32_768, 1536, 16) == filt
+    assert form(10_000, 1_000_000, 768, 10) == filt and form(300, 150_000, 64, 10) == filt and form(10_000, 6000, 768, 10) == filt
+    assert form(32, 32_768, 64, 1) == few
+    for s in [(300, 4096, 64, 10), (32, 32_768, 64, 1), (1, 4096, 4, 1)]:
+        for metric in (0, 1):
+            need = lib.vl_knn_metric_workspace_bytes(*s, metric + 256)
+            assert lib.vl_knn_form(*s, metric + 256, need) == filt and lib.vl_knn_form(*s, metric + 256, need - 1) != filt
+    assert lib.vl_knn_form(300, 4000, 64, 10, 256, 1 << 60) == tiles
+    for metric in (2, 255, 258, -1, 512):
+        assert lib.vl_knn_form(300, 4096, 64, 10, metric, 1 << 60) < 0
+        assert lib.vl_knn_metric_workspace_bytes(300, 4096, 64, 10, metric) < 0
+
+
 def test_cpu_tensors_are_refused():
     import torch
 

@@ -199,15 +199,16 @@ def test_values_that_are_not_finite(n, k, metric):
 
 
 def call(q, v, k, metric="cosine"):
-    """(ids, distances, the queries left to the tiles or None if the filter does not take the call)."""
+    """(ids, distances, the queries left to the tiles or None if the filter does not take the call), whatever the sizes."""
     from vectorlink_gpu import _native as nv
 
     (nq, dim) = q.shape
-    sizes = (nq, v.shape[0], dim, k, nv.metric_code(metric))
-    ws = torch.empty(nv.lib().vl_knn_workspace_bytes(nq, v.shape[0], dim, k), dtype=torch.uint8, device=DEV)
+    code = nv.metric_code(metric) + nv.KNN_ANY_SIZE
+    sizes = (nq, v.shape[0], dim, k, code)
+    ws = torch.empty(nv.lib().vl_knn_metric_workspace_bytes(*sizes), dtype=torch.uint8, device=DEV)
     ids = torch.empty((nq, k), dtype=torch.int32, device=DEV)
     d = torch.empty((nq, k), dtype=torch.float32, device=DEV)
-    nv.check(nv.lib().vl_knn_exact_metric(nv.ptr(q), nq, nv.ptr(v), v.shape[0], dim, k, nv.metric_code(metric), nv.ptr(ids),
+    nv.check(nv.lib().vl_knn_exact_metric(nv.ptr(q), nq, nv.ptr(v), v.shape[0], dim, k, code, nv.ptr(ids),
                                           nv.ptr(d), nv.ptr(ws), ws.numel(), nv.stream()))
     if nv.lib().vl_knn_form(*sizes, ws.numel()) != 2:
         return ids, d, None
@@ -305,3 +306,39 @@ def test_queries_that_the_tiles_answer_sooner_are_left_to_them(n, dim, members, 
     (ids, d, left) = call(q, v, k)
     assert left == list(range(0, nq, 2))
     agrees_with_a_few_queries(q, v, k, "cosine", ids, d)
+
+
+@pytest.mark.parametrize("n,dim,nq,k,metric", [
+    (4096, 64, 129, 10, "cosine"), (4097, 4, 256, 16, "cosine"), (5000, 60, 257, 4, "l2"), (6000, 64, 300, 1, "l2"),
+    (4096, 1536, 1, 1, "cosine"), (8191, 132, 33, 12, "l2"), (33_000, 196, 513, 12, "l2"), (40_000, 192, 700, 16, "cosine")])
+def test_the_filter_against_float64(n, dim, nq, k, metric):
+    """Calls of every size through the filter: no query is left to the tiles, and the answers are those of the other forms
+    and, to the rounding of float32 sums (as in test_a_few_queries), those of 64 bits."""
+    print(f"filter against float64 n={n} dim={dim} nq={nq} k={k} {metric}", flush=True)
+    rng = np.random.default_rng(n + dim)
+    (v, q) = (rows(rng, n, dim), rows(rng, nq, dim))
+    q[nq // 2] = v[n - 1]
+    (ids, d, left) = call(dev(q), dev(v), k, metric)
+    assert left == []
+    agrees_with_a_few_queries(dev(q), dev(v), k, metric, ids, d)
+    s = q.astype(np.float64) @ v.astype(np.float64).T
+    true = np.clip((1 - s) / 2, 0, 1) if metric == "cosine" else np.maximum(
+        (q.astype(np.float64) ** 2).sum(1)[:, None] + (v.astype(np.float64) ** 2).sum(1)[None] - 2 * s, 0)
+    want = np.sort(true, axis=1)[:, :k]
+    assert np.allclose(d.cpu().numpy(), want, rtol=1e-5, atol=1e-6)
+    assert np.allclose(np.take_along_axis(true, ids.cpu().numpy().astype(np.int64), 1), want, rtol=1e-5, atol=2e-6)
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_the_filter_of_a_short_table_with_values_that_are_not_finite(value, metric):
+    print(f"filter of a short table with {value} {metric}", flush=True)
+    rng = np.random.default_rng(3)
+    (v, q) = (rows(rng, 5000, 20), rows(rng, 200, 20))
+    q[3, 7] = value
+    for bad in (False, True):
+        if bad:
+            v[4999, 2] = value
+        (ids, d, left) = call(dev(q), dev(v), 10, metric)
+        assert left == (list(range(200)) if bad else [3])
+        agrees_with_a_few_queries(dev(q), dev(v), 10, metric, ids, d)

@@ -3,8 +3,8 @@
 // vectorlink_gpu/ann.py:235-259); this is the ground truth for recall@k and the
 // only contraction-shaped step of the path.
 //
-// Small batches go to knn_few.hip and most others through knn_filter.hip; this file holds the float32 tiles, which take
-// tables of fewer than 4,096 rows and what the filter cannot decide.  All three give the same bits.
+// Small batches go to knn_few.hip and long calls through knn_filter.hip; this file holds the float32 tiles, which take
+// short calls, tables of fewer than 4,096 rows and what the filter cannot decide.  All three give the same bits.
 //
 // One workgroup (4 wavefronts, 2 x 2) owns 128 queries and a strip of the
 // vector set; operand tiles go from global memory straight into LDS
@@ -437,9 +437,33 @@ struct KnnPlan {
 // again.
 constexpr int64_t kFilterQueries = 65536;
 
+// Microseconds that the tiles take for a call: rounds of two workgroups per compute unit (a last round of at most half of
+// them has the compute units to itself), strips of len tiles, stages of 32 columns.  Fitted to 7,840 calls of 4,096 to
+// 500,000 vectors of 16 to 1,536 columns, 129 to 40,000 queries and k up to 16: nine in ten are within 12 %.
+double tiles_us(int64_t workgroups, int64_t len, int64_t dim, int list_len, int64_t n_queries) {
+    const int64_t slots = resident_workgroups(), full = workgroups / slots, rest = workgroups % slots;
+    const double rounds = (double)full + (rest == 0 ? 0.0 : (2 * rest <= slots ? 0.55 : 1.0));
+    return 23.0 + rounds * (double)len * (4.0 * (double)((dim + KT - 1) / KT) + 1.4 + 0.71 * list_len) +
+           1.9 * list_len * (double)(full + (rest != 0)) + 0.0022 * (double)n_queries;
+}
+
+// The filter takes a call that would keep the tiles busy for longer than this.  It has eleven launches, works some 10 ns for a
+// query whatever the table, its sample is at least 8,192 rows - half a short table, 1/16 of a long one - and queries that it
+// leaves to the tiles cost both.  Us with the tiles / the filter, rows in no clusters, in clusters of 244 and of 977:
+//   4,096 x 64, 300 queries, k = 10        54 / 68     57 / 106    54 / 89     tiles
+//   6,000 x 768, 1,500, k = 10             251 / 134   259 / 314   249 / 307   tiles
+//   12,000 x 64, 10,000, k = 10            351 / 205   354 / 345   351 / 520   filter
+//   32,768 x 64, 300, k = 10               100 / 82    104 / 107   100 / 139   tiles
+//   12,000 x 768, 1,500, k = 10            364 / 158   371 / 257   362 / 423   filter
+//   32,768 x 768, 10,000, k = 10           4,288 / 949 4,356 / 1,834  4,284 / 4,718  filter
+//   150,000 x 64, 300, k = 10              276 / 140   276 / 175   276 / 230   filter
+// Of 7,840 calls of such sizes the filter answers 4,166, in a geometric mean of 0.71 of the tiles' time over all of them (0.77 with the
+// filter for every call); 500 take more than 1.1 times as long, nearly all of them with clusters of a thirtieth of the table and more.
+double filter_from_us(int64_t n_queries, int64_t n_vectors) { return 80.0 + 2e6 / (double)n_vectors + 0.015 * (double)n_queries; }
+
 // most: bytes of workspace there are; a call with too few for the form that would take it goes to the tiles alone, with the
-// same bits.
-int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, int64_t most, KnnPlan *p) {
+// same bits.  any_size: the filter also where the tiles are expected to be faster.
+int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool l2, bool any_size, int64_t most, KnnPlan *p) {
     VL_REQUIRE(n_queries >= 0 && n_vectors > 0 && dim > 0, "bad sizes");
     VL_REQUIRE(k >= 1 && k <= KMAX, "k must be between 1 and %d", KMAX);
     VL_REQUIRE(dim % 4 == 0, "exact kNN tiles need a dimension that is a multiple of 4");
@@ -472,7 +496,7 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
         p->cand_bytes = (n_queries > 0 ? n_queries : 1) * (int64_t)p->n_cand * 8;
         return p->cand_bytes + ((2 * n_queries + n_vectors) * 4 + 15) / 16 * 16;
     };
-    p->few = vl_knn_is_few(n_queries, n_vectors, dim);
+    p->few = !any_size && vl_knn_is_few(n_queries, n_vectors, dim);
     if (p->few) {
         p->bytes = lists(vl_knn_few_lists(n_vectors));
         p->filter = false;
@@ -480,7 +504,8 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
         p->few = false;
     }
     p->bytes = lists(strips * LISTS_PER_STRIP);
-    p->filter = vl_knn_filter_plan(n_queries < kFilterQueries ? n_queries : kFilterQueries, n_vectors, dim, k, l2, &p->fp);
+    p->filter = (any_size || tiles_us(q_blocks * strips, len / TV, dim, p->list_len, n_queries) >= filter_from_us(n_queries, n_vectors)) &&
+                vl_knn_filter_plan(n_queries < kFilterQueries ? n_queries : kFilterQueries, n_vectors, dim, k, l2, &p->fp);
     if (p->filter) {
         p->off_left = (p->bytes + 255) / 256 * 256;
         p->off_filter = (p->off_left + (1 + n_queries) * 4 + 255) / 256 * 256;
@@ -493,31 +518,44 @@ int knn_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, bool 
 
 }  // namespace
 
+// A metric, possibly with VL_KNN_ANY_SIZE added.
+#define VL_KNN_METRIC(metric, l2, any_size)                                                              \
+    const bool any_size = ((metric) & VL_KNN_ANY_SIZE) != 0, l2 = ((metric) & ~VL_KNN_ANY_SIZE) == VL_METRIC_L2; \
+    VL_REQUIRE(l2 || ((metric) & ~VL_KNN_ANY_SIZE) == VL_METRIC_COSINE, "unknown metric %d", (int)(metric))
+
+// Enough for the filter where it could take the call, whether or not it does.
 VL_EXPORT int64_t vl_knn_workspace_bytes(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k) {
     int64_t bytes = 0;
-    for (const bool l2 : {false, true}) {  // either may be the larger: pieces of the filter's table are whole tiles
-        KnnPlan p;
-        const int rc = knn_plan(n_queries, n_vectors, dim, k, l2, INT64_MAX, &p);
+    const int any_size = vl_knn_is_few(n_queries, n_vectors, dim) ? 0 : VL_KNN_ANY_SIZE;
+    for (const int32_t metric : {VL_METRIC_COSINE, VL_METRIC_L2}) {  // either may be the larger: pieces of the filter's table are whole tiles
+        const int64_t rc = vl_knn_metric_workspace_bytes(n_queries, n_vectors, dim, k, metric + any_size);
         if (rc < 0) return rc;
-        bytes = p.bytes > bytes ? p.bytes : bytes;
+        bytes = rc > bytes ? rc : bytes;
     }
     return bytes;
 }
 
+VL_EXPORT int64_t vl_knn_metric_workspace_bytes(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric) {
+    VL_KNN_METRIC(metric, l2, any_size);
+    KnnPlan p;
+    const int rc = knn_plan(n_queries, n_vectors, dim, k, l2, any_size, INT64_MAX, &p);
+    return rc < 0 ? rc : p.bytes;
+}
+
 VL_EXPORT int vl_knn_form(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
                           int64_t workspace_bytes) {
-    VL_REQUIRE(metric == VL_METRIC_COSINE || metric == VL_METRIC_L2, "unknown metric %d", (int)metric);
+    VL_KNN_METRIC(metric, l2, any_size);
     KnnPlan p;
-    const int rc = knn_plan(n_queries, n_vectors, dim, k, metric == VL_METRIC_L2, workspace_bytes, &p);
+    const int rc = knn_plan(n_queries, n_vectors, dim, k, l2, any_size, workspace_bytes, &p);
     if (rc < 0) return rc;
     return p.few ? VL_KNN_FEW : (p.filter ? VL_KNN_FILTER : VL_KNN_TILES);
 }
 
 VL_EXPORT int64_t vl_knn_left_offset(int64_t n_queries, int64_t n_vectors, int64_t dim, int64_t k, int32_t metric,
                                      int64_t workspace_bytes) {
-    VL_REQUIRE(metric == VL_METRIC_COSINE || metric == VL_METRIC_L2, "unknown metric %d", (int)metric);
+    VL_KNN_METRIC(metric, l2, any_size);
     KnnPlan p;
-    const int rc = knn_plan(n_queries, n_vectors, dim, k, metric == VL_METRIC_L2, workspace_bytes, &p);
+    const int rc = knn_plan(n_queries, n_vectors, dim, k, l2, any_size, workspace_bytes, &p);
     if (rc < 0) return rc;
     VL_REQUIRE(!p.few && p.filter, "such a call does not go through the filter");
     return p.off_left;
@@ -533,10 +571,9 @@ VL_EXPORT int vl_knn_exact(const float *queries, int64_t n_queries, const float 
 VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const float *vectors,
                                   int64_t n_vectors, int64_t dim, int64_t k, int32_t metric, int32_t *ids_out,
                                   float *dists_out, void *workspace, int64_t workspace_bytes, void *stream) {
-    VL_REQUIRE(metric == VL_METRIC_COSINE || metric == VL_METRIC_L2, "unknown metric %d", (int)metric);
+    VL_KNN_METRIC(metric, l2, any_size);
     KnnPlan p;
-    const bool l2 = metric == VL_METRIC_L2;
-    int rc = knn_plan(n_queries, n_vectors, dim, k, l2, workspace_bytes, &p);
+    int rc = knn_plan(n_queries, n_vectors, dim, k, l2, any_size, workspace_bytes, &p);
     if (rc < 0) return rc;
     if (n_queries == 0) return VL_OK;
     VL_REQUIRE(queries && vectors && ids_out && dists_out && workspace, "null pointer");
@@ -559,7 +596,7 @@ VL_EXPORT int vl_knn_exact_metric(const float *queries, int64_t n_queries, const
     float *q_norm = reinterpret_cast<float *>(q_bound + n_queries);
     float *v_norm = q_norm + n_queries;
     // A batch goes to the kernel for a few queries (knn_few.h says where the line lies), else through the bfloat16 filter,
-    // which leaves the queries it cannot answer to the float32 tiles below; a table below 4,096 rows goes to the tiles.
+    // which leaves the queries it cannot answer to the float32 tiles below; short calls go to the tiles (filter_from_us).
     const int32_t *left = nullptr;
     char *const ws = (char *)workspace;
     if (p.filter) {

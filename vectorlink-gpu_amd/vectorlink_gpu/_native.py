@@ -25,6 +25,7 @@ class BeamParams(C.Structure):
 
 METRICS = {"cosine": 0, "l2": 1}  # include/vlgpu.h: VL_METRIC_COSINE, VL_METRIC_L2
 KNN_FORMS = {"tiles": 0, "few": 1, "filter": 2}  # VL_KNN_TILES, VL_KNN_FEW, VL_KNN_FILTER
+KNN_ANY_SIZE = 256  # VL_KNN_ANY_SIZE
 
 
 def metric_code(name: str) -> int:
@@ -66,6 +67,7 @@ _SIGNATURES = {
     "vl_optimize_graph_workspace_bytes": (C.c_int64, [_i64, _i64, _i64]),
     "vl_optimize_graph": (C.c_int, [_ptr, _i64, _i64, _i64, _ptr, _ptr, _i64, _ptr]),
     "vl_knn_workspace_bytes": (C.c_int64, [_i64, _i64, _i64, _i64]),
+    "vl_knn_metric_workspace_bytes": (C.c_int64, [_i64, _i64, _i64, _i64, C.c_int32]),
     "vl_knn_form": (C.c_int, [_i64, _i64, _i64, _i64, C.c_int32, _i64]),
     "vl_knn_left_offset": (C.c_int64, [_i64, _i64, _i64, _i64, C.c_int32, _i64]),
     "vl_knn_exact": (C.c_int, [_ptr, _i64, _ptr, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr]),
