@@ -342,3 +342,23 @@ def test_the_filter_of_a_short_table_with_values_that_are_not_finite(value, metr
         (ids, d, left) = call(dev(q), dev(v), 10, metric)
         assert left == (list(range(200)) if bad else [3])
         agrees_with_a_few_queries(dev(q), dev(v), 10, metric, ids, d)
+
+
+@pytest.mark.parametrize("nq,share,want", [(300, 3, "none"), (300, 1.5, "all"), (512, 1.9, "all"), (513, 1.9, "crowd"), (1000, 1.5, "crowd"), (1000, 3, "none")])
+def test_what_a_batch_leaves_to_the_tiles_before_the_pass(nq, share, want):
+    """Queries with 1,100 candidates, somewhat more than cost what the tiles do for one (858): a small batch is left as a
+    whole or not at all, a large one leaves them if they are many."""
+    print(f"left before the pass nq={nq} share={share}", flush=True)
+    (n, dim) = (32_768, 256)
+    gen = torch.Generator(device=DEV).manual_seed(nq)
+    v = torch.nn.functional.normalize(torch.randn((n, dim), generator=gen, device=DEV), dim=1)
+    q = torch.nn.functional.normalize(torch.randn((nq, dim), generator=gen, device=DEV), dim=1)
+    crowd = torch.nn.functional.normalize(torch.randn((1, dim), generator=gen, device=DEV), dim=1)
+    q -= (q @ crowd.T) * crowd
+    v[torch.randperm(n, generator=gen, device=DEV)[:1100]] = crowd + 1e-3 * torch.randn((1100, dim), generator=gen, device=DEV)
+    at = torch.randperm(nq, generator=gen, device=DEV)[:int(nq / share)].sort().values
+    q[at] = crowd + 1e-3 * q[at]
+    (v, q) = (torch.nn.functional.normalize(x, dim=1) for x in (v, q))
+    (ids, d, left) = call(q, v, 1)
+    assert left == {"none": [], "all": list(range(nq)), "crowd": at.tolist()}[want]
+    agrees_with_a_few_queries(q, v, 1, "cosine", ids, d)

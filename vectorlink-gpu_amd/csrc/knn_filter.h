@@ -8,7 +8,7 @@ struct KnnFilterPlan {
     int64_t sample_stride;  // between the places of two rows of the sample that follow each other in the table
     int sample_strips;
     int groups;             // maxima per query that the sample pass leaves
-    int most;               // candidates of a query that are worth evaluating
+    int most;               // candidates of a query that cost what the tiles do for it
     int64_t slab_rows;      // rows of the table converted at a time
     int64_t off_q16, off_v16, off_qstat, off_gmax, off_bound, off_count, off_found, off_vmax, bytes;
 };

@@ -16,9 +16,9 @@
 //   finish    their float32 dot products - one fused multiply-add after the other in the order in which the float32 tiles'
 //             matrix instructions take the elements, which gives the tiles' bits - and the k best of them
 // A query with more candidates than its buffer holds (thousands of rows within the rounding of each other), or than the
-// tiles are worth, is left to the float32 tiles, which take all such queries of a call together; most are known from the
-// sample and are not looked for in the pass.  For squared L2 the values are <q, v> - |v|^2 / 2: three more columns hold -|v|^2 / 2 as a sum of three
-// bfloat16 numbers (24 bits), and ones on the query side.
+// tiles are worth (expected_limit), is left to the float32 tiles, which take all such queries of a call together; most are
+// known from the sample and are not looked for in the pass.  For squared L2 the values are <q, v> - |v|^2 / 2: three more
+// columns hold -|v|^2 / 2 as a sum of three bfloat16 numbers (24 bits), and ones on the query side.
 //
 // The pass: 256 vectors x 256 queries per workgroup of eight wavefronts (128 x 64 each, 128 accumulator registers), 64
 // columns per stage through two LDS buffers per operand (128 KB), v_mfma_f32_32x32x16_bf16.  A wavefront reads 6 KB of
@@ -43,10 +43,19 @@ constexpr int RB = 4, CB = 2;     // 32-row and 32-column blocks of a wavefront
 constexpr int kGroupsPerStrip = 2 * 2 * RB;  // maxima that a strip's workgroup leaves per query
 constexpr int kFound = 2048;      // candidates per query
 constexpr int kMaxGroups = 512;
-constexpr int kStripes = 64, kStripeWords = 32;  // partial maxima of a piece of the table, a cache line each
+constexpr int kStripes = 64, kStripeWords = 32;  // partial maxima of a piece of the table, a cache line each (in the sample's: a third word, bound_kernel)
+constexpr float kMostExpected = 1.25f * kFound;  // expected candidates with which a query is still looked for: the sample is off by a tenth
+// Batches of so few queries leave compute units idle: 512 threads per query evaluate its candidates instead of 128.
+constexpr int64_t kFinishWide = 512;
 
 struct RowStat {
     float resid, norm;  // not below ||x - x^||_2 and ||x||_2
+};
+// What the sample tells of a query.
+struct alignas(16) Sampled {
+    float value;       // the k-th best float32 value is not below this
+    float expected;    // how many vectors the pass will not rule out
+    float error;       // value_error with the sample's rows
 };
 
 __device__ __forceinline__ float up(float x) { return x * 1.00001f; }  // norms are sums of dim rounded terms: never below
@@ -158,6 +167,23 @@ __device__ __forceinline__ float value_error(RowStat q, RowStat v, int dim, bool
     return up(q.resid * v_norm + (q.norm + q.resid) * v_resid) + (float)dim * 2.4e-7f * sums + ties;
 }
 
+// The expected number of candidates up to which the pass looks for a query's.  `most` candidates cost what the tiles do for
+// one query of a full batch, `above` of the n queries expect more.  The tiles take as long for one query as for a few hundred, so a small
+// batch is left to them as a whole, if most of its queries expect too many, or not at all; in a large one the queries
+// far above, or if they are many all that are above, are left.  (32,768 x 768 in clusters of 977, k = 1, us with the tiles / the
+// filter that left every query above / this: 300 queries 235 / 484 / 306, 1,000 456 / 610 / 492, 4,000 1,672 / 1,952 / 1,730.)
+__device__ __forceinline__ float expected_limit(const uint32_t *__restrict__ sample_vmax, int64_t n, float most) {
+    int above = (int)sample_vmax[(threadIdx.x & (kWave - 1)) * kStripeWords + 2];
+    above += __builtin_amdgcn_update_dpp(0, above, 0x128, 0xf, 0xf, false);  // row_ror:8
+    above += __builtin_amdgcn_update_dpp(0, above, 0x124, 0xf, 0xf, false);  // row_ror:4
+    above += __builtin_amdgcn_update_dpp(0, above, 0x122, 0xf, 0xf, false);  // row_ror:2
+    above += __builtin_amdgcn_update_dpp(0, above, 0x121, 0xf, 0xf, false);  // row_ror:1
+    above = __builtin_amdgcn_readlane(above, 0) + __builtin_amdgcn_readlane(above, 16) + __builtin_amdgcn_readlane(above, 32) +
+            __builtin_amdgcn_readlane(above, 48);
+    if (n <= kFinishWide) return 2 * above > n ? -1.0f : kMostExpected;
+    return 2 * above >= n ? most : fminf(2.0f * most, kMostExpected);
+}
+
 // Staging of 256-row operands by eight wavefronts: wavefront w brings rows 32 w ... 32 w + 31, eight per instruction.
 __device__ __forceinline__ void stage256(const float *const (&p)[4], int kt, float *tile, int wave) {
 #pragma unroll
@@ -171,9 +197,9 @@ template <bool EMIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *__restrict__ v16, int64_t n_vectors,
                  int kp2, int64_t strip_len, int n_strips, int n_qblocks, int q_group, float *__restrict__ gmax,
-                 const float *__restrict__ bound, const RowStat *__restrict__ qstat, const uint32_t *__restrict__ vmax,
-                 const uint32_t *__restrict__ sample_vmax, int dim, int l2, int64_t id0, int32_t *__restrict__ count,
-                 uint64_t *__restrict__ found) {
+                 const Sampled *__restrict__ bound, const RowStat *__restrict__ qstat, const uint32_t *__restrict__ vmax,
+                 const uint32_t *__restrict__ sample_vmax, float most, int dim, int l2,
+                 int64_t id0, int32_t *__restrict__ count, uint64_t *__restrict__ found) {
     extern __shared__ __align__(16) float smem[];
     constexpr int T = TR * KT;  // floats of a staged operand
     float *const sV0 = smem, *const sV1 = smem + T, *const sQ0 = smem + 2 * T, *const sQ1 = smem + 3 * T;
@@ -210,10 +236,19 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
     const int64_t v_end = min(n_vectors, v_begin + strip_len);
 
     float thr[CB], top[CB][RB];
-    RowStat table = {0.0f, 0.0f}, sampled = {0.0f, 0.0f};
+    RowStat table = {0.0f, 0.0f}, q_stat[CB];
+    float limit = 0.0f;
+    Sampled sampled[CB];
     if constexpr (EMIT) {
+        // (read without conditions, so that one round trip to memory brings all of it)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            const int64_t q = min(q0 + 64 * wc + 32 * cb + l32, n_queries - 1);
+            sampled[cb] = bound[q];
+            q_stat[cb] = qstat[q];
+        }
         table = table_stat(vmax);
-        sampled = table_stat(sample_vmax);
+        limit = expected_limit(sample_vmax, n_queries, most);
     }
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
@@ -221,12 +256,12 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
             const int64_t q = q0 + 64 * wc + 32 * cb + l32;
             thr[cb] = __builtin_inff();
             if (q < n_queries) {
-                const float error = value_error(qstat[q], table, dim, l2 != 0);
-                thr[cb] = bound[q] - error;
-                // No bound (a row that is not finite), or one that lets everything through because a row is far longer than
-                // those of the sample: the query is left to the tiles.  So a threshold is above -infinity, which is what
-                // rows past the strip's end hold.
-                if (!(thr[cb] > (l2 ? -__builtin_inff() : -0.999f)) || error > 16.0f * value_error(qstat[q], sampled, dim, l2 != 0)) {
+                const float error = value_error(q_stat[cb], table, dim, l2 != 0);
+                thr[cb] = sampled[cb].value - error;
+                // Too many expected, no bound (a row that is not finite), or one that lets everything through because a row is
+                // far longer than those of the sample: the query is left to the tiles.  So a threshold is above -infinity,
+                // which is what rows past the strip's end hold.
+                if (!(sampled[cb].expected <= limit) || !(thr[cb] > (l2 ? -__builtin_inff() : -0.999f)) || error > 16.0f * sampled[cb].error) {
                     thr[cb] = __builtin_inff();
                     if (strip == 0 && wr == 0 && half == 0) atomicAdd(&count[q], kFound + 1);
                 }
@@ -235,8 +270,17 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) top[cb][rb] = -__builtin_inff();
     }
-    if constexpr (EMIT)
-        if (!__syncthreads_or(thr[0] < __builtin_inff() || thr[1] < __builtin_inff())) return;  // none of these queries is looked for
+    if constexpr (EMIT) {
+        // a workgroup none of whose queries is looked for ends here (the words are in a buffer that the first stage leaves alone)
+        int *const looked_for = reinterpret_cast<int *>(sQ1);
+        const bool mine = __builtin_amdgcn_ballot_w64(thr[0] < __builtin_inff() || thr[1] < __builtin_inff()) != 0;
+        if (lane == 0) looked_for[wave] = mine;
+        __syncthreads();
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < kThreads / kWave; ++w) any |= looked_for[w];
+        if (!any) return;
+    }
     int a_off[RB], b_off[CB];
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
@@ -412,22 +456,23 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
     }
 }
 
-// bound[q]: what the k-th best float32 value of query q is not below, from the k-th largest of its groups' maxima.  A query
-// that too many vectors (most of them) are expected to pass is left to the tiles before the pass: its bound is infinite.
+// What the sample tells of a query, from the k-th largest of its groups' maxima.  The queries that expect more than `most`
+// vectors are counted in vmax.
 __global__ __launch_bounds__(256) void bound_kernel(const float *__restrict__ gmax, int groups, int k, int64_t n_queries,
-                                                    const RowStat *__restrict__ qstat, const uint32_t *__restrict__ vmax,
-                                                    int dim, int l2, float rows_per_sample_row, int most,
-                                                    float *__restrict__ bound, int32_t *__restrict__ count) {
+                                                    const RowStat *__restrict__ qstat, uint32_t *__restrict__ vmax,
+                                                    int dim, int l2, float rows_per_sample_row, float most,
+                                                    Sampled *__restrict__ bound, int32_t *__restrict__ count) {
     const int64_t q = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
     if (q >= n_queries) return;
     const int lane = threadIdx.x & (kWave - 1);
     constexpr int PER = kMaxGroups / kWave;
+    float top[PER];
     uint32_t key[PER];  // largest value first
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const int g = lane + kWave * j;
-        const float x = g < groups ? gmax[q * groups + g] : -__builtin_inff();
-        key[j] = ~vl_float_key(x == x ? x : -__builtin_inff());  // a NaN bounds nothing
+        top[j] = g < groups ? gmax[q * groups + g] : -__builtin_inff();
+        key[j] = ~vl_float_key(top[j] == top[j] ? top[j] : -__builtin_inff());  // a NaN bounds nothing
     }
     uint32_t kth = 0xFFFFFFFFu;
     for (int i = 0; i < k; ++i) {
@@ -458,13 +503,13 @@ __global__ __launch_bounds__(256) void bound_kernel(const float *__restrict__ gm
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const int g = lane + kWave * j;
-        without += __popcll(__ballot(g < groups && gmax[q * groups + min(g, groups - 1)] < limit));
+        without += __popcll(__ballot(g < groups && top[j] < limit));
     }
     const float vectors = -(float)groups * logf((float)without / (float)groups) * rows_per_sample_row;  // infinite if none is without
     if (lane == 0) {
-        const bool fits = vectors <= (float)most;  // (no bound: no group is without)
-        bound[q] = fits ? t : __builtin_inff();
-        count[q] = fits ? 0 : kFound + 1;
+        bound[q] = Sampled{t, vectors, error};  // (no bound: no group is without)
+        count[q] = 0;
+        if (!(vectors <= most)) atomicAdd(vmax + (blockIdx.x & (kStripes - 1)) * kStripeWords + 2, 1u);
     }
 }
 
@@ -549,7 +594,8 @@ __device__ __forceinline__ float dots_in_tile_order(const float *__restrict__ ve
 #pragma unroll
         for (int d = 0; d < D; ++d)
 #pragma unroll
-            for (int g = 0; g < NG; ++g) buf[d * 8 * NG * CH + to[g]] = x[d * NG + g];
+            for (int g = 0; g < NG; ++g)
+                if (d == 0 || l0 + d < lines) buf[d * 8 * NG * CH + to[g]] = x[d * NG + g];
         __builtin_amdgcn_wave_barrier();
         if (l0 + D < lines) load(l0 + D);
 #pragma unroll
@@ -579,6 +625,20 @@ __device__ __forceinline__ float dots_in_tile_order(const float *__restrict__ ve
     return s;
 }
 
+// The k-th smallest of up to 64 values in LDS, a lane each: four values are looked at together (those past the last are not
+// counted).  Bit by bit, as below, is 32 steps that wait for each other.
+__device__ __forceinline__ uint32_t kth_of_a_few(const uint4 *values, int n, int k) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t mine = reinterpret_cast<const uint32_t *>(values)[min(lane, n - 1)];
+    int below = 0, same = 0;
+    for (int j = 0; 4 * j < n; ++j) {
+        const uint4 x = values[j];
+        below += (x.x < mine) + (4 * j + 1 < n && x.y < mine) + (4 * j + 2 < n && x.z < mine) + (4 * j + 3 < n && x.w < mine);
+        same += (x.x == mine) + (4 * j + 1 < n && x.y == mine) + (4 * j + 2 < n && x.z == mine) + (4 * j + 3 < n && x.w == mine);
+    }
+    return (uint32_t)__builtin_amdgcn_readlane((int)mine, __builtin_ctzll(__builtin_amdgcn_ballot_w64(below < k && k <= below + same)));
+}
+
 // The k-th smallest of n values in LDS, 1 <= k <= n <= kFound, bit by bit; each wavefront finds it for itself.
 template <int PER>
 __device__ __forceinline__ uint32_t kth_of(const uint32_t *values, int n, int k) {
@@ -597,7 +657,7 @@ __device__ __forceinline__ uint32_t kth_of(const uint32_t *values, int n, int k)
     return at;
 }
 __device__ __forceinline__ uint32_t kth_smallest(const uint32_t *values, int n, int k) {
-    if (n <= kWave) return kth_of<1>(values, n, k);
+    if (n <= kWave) return kth_of_a_few(reinterpret_cast<const uint4 *>(values), n, k);
     if (n <= 4 * kWave) return kth_of<4>(values, n, k);
     if (n <= 16 * kWave) return kth_of<16>(values, n, k);
     return kth_of<kFound / kWave>(values, n, k);
@@ -607,6 +667,9 @@ __device__ __forceinline__ uint32_t kth_smallest(const uint32_t *values, int n, 
 // them bounds the k-th best float32 value far better, so most are dropped before their rows are fetched (at 1,000 queries
 // x 32,768 x 1,536, k = 16: 350 candidates, 390 us when all were evaluated).  What is left is evaluated, and those not
 // above the k-th best distance are ranked.
+// A few candidates with rows of up to so many columns are all evaluated at once: the bound on them would wait for LDS longer
+// than their rows take (10,000 queries with 20 candidates of 64 columns each: 57.8 us with it, 44.5 without).
+constexpr int kShortRow = 128;
 template <bool L2, int THREADS>
 __global__ __launch_bounds__(THREADS) void finish_kernel(const float *__restrict__ queries,
                                                          const float *__restrict__ vectors, int dim, int k,
@@ -619,7 +682,7 @@ __global__ __launch_bounds__(THREADS) void finish_kernel(const float *__restrict
                                                          int32_t *__restrict__ ids_out, float *__restrict__ d_out) {
     constexpr int kWaves = THREADS / kWave;
     __shared__ float4 buf[kWaves][kWave * CH];
-    __shared__ uint32_t values[kFound];  // of the pass, smallest is best; then the distances, as keys
+    __shared__ __align__(16) uint32_t values[kFound];  // of the pass, smallest is best; then the distances, as keys
     __shared__ int32_t ids[kFound];
     __shared__ int n_s, n_keys_s;
     uint64_t *const keys = reinterpret_cast<uint64_t *>(&buf[0][0]);
@@ -632,26 +695,34 @@ __global__ __launch_bounds__(THREADS) void finish_kernel(const float *__restrict
         n_s = 0;
         n_keys_s = 0;
     }
-    for (int i = tid; i < n; i += THREADS) values[i] = ~vl_float_key(__builtin_bit_cast(float, (uint32_t)(found[q * kFound + i] >> 32)));
-    RowStat table = {0.0f, 0.0f};
-    for (int s = 1; s <= slabs; ++s) {
-        const RowStat one = table_stat(vmax + (int64_t)s * kStripes * kStripeWords);
-        table.resid = fmaxf(table.resid, one.resid);
-        table.norm = fmaxf(table.norm, one.norm);
+    const uint64_t own = tid < n ? found[q * kFound + tid] : 0;
+    int left = n;
+    if (n <= kWave && dim <= kShortRow) {
+        if (tid < n) ids[tid] = (int32_t)(uint32_t)own;
+        __syncthreads();
+    } else {
+        if (tid < n) values[tid] = ~vl_float_key(__builtin_bit_cast(float, (uint32_t)(own >> 32)));
+        for (int i = tid + THREADS; i < n; i += THREADS) values[i] = ~vl_float_key(__builtin_bit_cast(float, (uint32_t)(found[q * kFound + i] >> 32)));
+        RowStat table = {0.0f, 0.0f};
+        for (int s = 1; s <= slabs; ++s) {
+            const RowStat one = table_stat(vmax + (int64_t)s * kStripes * kStripeWords);
+            table.resid = fmaxf(table.resid, one.resid);
+            table.norm = fmaxf(table.norm, one.norm);
+        }
+        __syncthreads();
+        float least = -__builtin_inff();
+        if (n > k) {
+            const float error = value_error(qstat[q], table, dim, L2);
+            least = vl_key_float(~kth_smallest(values, n, k)) - error;
+            if (!L2) least = fminf(least, 1.0f - 1e-6f);  // values of 1 and more are one distance, 0
+            least -= error;
+            if (!L2 && least <= -0.999f) least = -__builtin_inff();
+        }
+        for (int i = tid; i < n; i += THREADS)
+            if (!(vl_key_float(~values[i]) < least)) ids[atomicAdd(&n_s, 1)] = (int32_t)(uint32_t)(i == tid ? own : found[q * kFound + i]);
+        __syncthreads();
+        left = __builtin_amdgcn_readfirstlane(n_s);
     }
-    __syncthreads();
-    float least = -__builtin_inff();
-    if (n > k) {
-        const float error = value_error(qstat[q], table, dim, L2);
-        least = vl_key_float(~kth_smallest(values, n, k)) - error;
-        if (!L2) least = fminf(least, 1.0f - 1e-6f);  // values of 1 and more are one distance, 0
-        least -= error;
-        if (!L2 && least <= -0.999f) least = -__builtin_inff();
-    }
-    for (int i = tid; i < n; i += THREADS)
-        if (!(vl_key_float(~values[i]) < least)) ids[atomicAdd(&n_s, 1)] = (int32_t)(uint32_t)found[q * kFound + i];
-    __syncthreads();
-    const int left = n_s;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     for (int base = 0; base < left; base += THREADS) {
         // the same number of rows for each wavefront
@@ -673,11 +744,17 @@ __global__ __launch_bounds__(THREADS) void finish_kernel(const float *__restrict
         }
     }
     __syncthreads();
-    const uint32_t last = left > k ? kth_smallest(values, left, k) : 0xFFFFFFFFu;
-    for (int i = tid; i < left; i += THREADS)
-        if (values[i] <= last) keys[atomicAdd(&n_keys_s, 1)] = ((uint64_t)values[i] << 32) | (uint32_t)ids[i];
-    __syncthreads();
-    const int n_keys = n_keys_s;
+    int n_keys = left;
+    if (left <= kWave) {  // a few are ranked as they are
+        if (tid < left) keys[tid] = ((uint64_t)values[tid] << 32) | (uint32_t)ids[tid];
+        __syncthreads();
+    } else {
+        const uint32_t last = kth_smallest(values, left, k);
+        for (int i = tid; i < left; i += THREADS)
+            if (values[i] <= last) keys[atomicAdd(&n_keys_s, 1)] = ((uint64_t)values[i] << 32) | (uint32_t)ids[i];
+        __syncthreads();
+        n_keys = __builtin_amdgcn_readfirstlane(n_keys_s);
+    }
     for (int i = tid; i < n_keys || i < k; i += THREADS) {
         if (i >= n_keys) {  // fewer vectors than asked for
             ids_out[q * k + i] = VL_MAXINT;
@@ -693,9 +770,6 @@ __global__ __launch_bounds__(THREADS) void finish_kernel(const float *__restrict
         }
     }
 }
-
-// Batches of so few queries leave compute units idle: 512 threads per query instead of 128.
-constexpr int64_t kFinishWide = 512;
 
 int64_t compute_units() {
     static const int64_t n = [] {
@@ -754,18 +828,18 @@ bool vl_knn_filter_plan(int64_t n_queries, int64_t n_vectors, int64_t dim, int64
     p->slab_rows = (2ll << 30) / (p->kp * 2) / TR * TR;
     if (p->slab_rows < p->sample_rows) p->slab_rows = p->sample_rows;
     if (p->slab_rows > n_vectors) p->slab_rows = n_vectors;
-    // A query with more candidates than this is left to the tiles.  On full batches the tiles take 0.0163 ps per product and
-    // 0.14 ps per place of their lists for a vector, a candidate 40 ps and 0.4 ps a column, and the pass, which such a query
-    // saves as well, 0.002 ps per product.  A guess somewhat above what the buffer holds is still tried: the sample is off
-    // by a tenth (4,000 queries with 2,000 candidates each at 500,000 x 384: 4.5 ms, with the tiles 12.8).
+    // On full batches the tiles take 0.0163 ps per product and 0.14 ps per place of their lists for a vector, a candidate
+    // 40 ps and 0.4 ps a column, and the pass, which a query left to the tiles saves as well, 0.002 ps per product.  A guess
+    // somewhat above what the buffer holds is still tried (4,000 queries with 2,000 candidates each at 500,000 x 384: 4.5 ms,
+    // with the tiles 12.8).
     const double even = (double)n_vectors * (0.014 * (double)dim + 0.14 * (double)k) / (40.0 + 0.4 * (double)dim);
-    p->most = (int)(even < kFound * 1.25 ? even : kFound * 1.25);
+    p->most = (int)(even < kMostExpected ? even : kMostExpected);
     int64_t o = 0;
     p->off_q16 = o; o = align256(o + n_queries * p->kp * 2);
     p->off_v16 = o; o = align256(o + p->slab_rows * p->kp * 2);
     p->off_qstat = o; o = align256(o + n_queries * (int64_t)sizeof(RowStat));
     p->off_gmax = o; o = align256(o + n_queries * p->groups * 4);
-    p->off_bound = o; o = align256(o + n_queries * 4);
+    p->off_bound = o; o = align256(o + n_queries * (int64_t)sizeof(Sampled));
     p->off_count = o; o = align256(o + n_queries * 4);
     p->off_found = o; o = align256(o + n_queries * kFound * 8);
     const int64_t slabs = (n_vectors + p->slab_rows - 1) / p->slab_rows;
@@ -779,7 +853,8 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
                   uint32_t *tile_bound, char *ws, int32_t *ids_out, float *dists_out, hipStream_t st) {
     __bf16 *q16 = (__bf16 *)(ws + p.off_q16), *v16 = (__bf16 *)(ws + p.off_v16);
     RowStat *qstat = (RowStat *)(ws + p.off_qstat);
-    float *gmax = (float *)(ws + p.off_gmax), *bound = (float *)(ws + p.off_bound);
+    float *gmax = (float *)(ws + p.off_gmax);
+    Sampled *bound = (Sampled *)(ws + p.off_bound);
     int32_t *count = (int32_t *)(ws + p.off_count);
     uint64_t *found = (uint64_t *)(ws + p.off_found);
     uint32_t *vmax = (uint32_t *)(ws + p.off_vmax);
@@ -810,7 +885,7 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), smem, st, (const float *)q16, n_queries,
                                (const float *)v16, rows, kp2, len, (int)strips, (int)q_blocks, (int)q_group, gmax, bound,
-                               qstat, top, vmax, (int)dim, l2 ? 1 : 0, id0, count, found);
+                               qstat, top, vmax, (float)p.most, (int)dim, l2 ? 1 : 0, id0, count, found);
         };
         if (emit) go(pass_kernel<true>);
         else go(pass_kernel<false>);
@@ -821,7 +896,8 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     pass(false, p.sample_rows, p.sample_strips, vmax, 0);
     VL_LAUNCH_CHECK("knn pass_kernel (sample)");
     hipLaunchKernelGGL(bound_kernel, dim3((unsigned)((n_queries + 3) / 4)), dim3(256), 0, st, gmax, p.groups, (int)k,
-                       n_queries, qstat, vmax, (int)dim, l2 ? 1 : 0, (float)n_vectors / (float)p.sample_rows, p.most, bound, count);
+                       n_queries, qstat, vmax, (int)dim, l2 ? 1 : 0, (float)n_vectors / (float)p.sample_rows, (float)p.most, bound,
+                       count);
     VL_LAUNCH_CHECK("knn bound_kernel");
     for (int64_t s = 0; s < slabs; ++s) {
         const int64_t r0 = s * p.slab_rows;
