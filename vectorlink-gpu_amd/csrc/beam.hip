@@ -880,7 +880,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     // Several iterations per launch (beam_row): the R iterations between two progress checks run in one launch while no
     // visited list can fill up in them, i.e. while Vt * (last iteration) <= E; the stretch after that runs one iteration
     // per launch.  Measured against one iteration per launch: searches of 256 queries at 4,096 x 128 1,500 -> 1,004 us,
-    // 1,000 at 100,003 x 1,536 1,803 -> 1,253, 10,000 at 1M x 128 2,690 -> 2,057, 10,000 at 1M x 768 3,145 -> 2,802 us;
+    // 1,000 at 100,003 x 1,536 1,803 -> 1,253, 10,000 at 1M x 128 2,690 -> 2,057, 10,000 at 1M x 768 3,790 -> 3,310 to 3,640 us;
     // builds of 4,096 x 128 8.5 -> 6.9 ms, 100,000 x 128 320 -> 296 ms.
     // With the sketch a window fits a compute unit six times, the one-iteration kernel eight times.  Rows that come from
     // HBM do not need those (a batch of the first loop at 1M x 768: 148 -> 140 ms, 1M x 384 49.4 -> 47.2, 50,000 x 768

@@ -23,7 +23,7 @@
 // The pass: 256 vectors x 256 queries per workgroup of eight wavefronts (128 x 64 each, 128 accumulator registers), 64
 // columns per stage through two LDS buffers per operand (128 KB), v_mfma_f32_32x32x16_bf16.  A wavefront reads 6 KB of
 // LDS per 8 products of 32 cycles; with 64 x 64 per wavefront LDS (128 bytes per cycle) would be the bound.
-// Measured, 10,000 queries, k = 10 (k = 4 and 16 below): 1,000,000 x 768 17.3 ms of which the pass 15.0 = 1,026 TFLOP/s
+// Measured, 10,000 queries, k = 10 (k = 4 and 16 below): 1,000,000 x 768 17.5 ms of which the pass 15.0 = 1,026 TFLOP/s
 // (a library product of 16,384^3 reaches 1,345 on the same card), 124.5 ms with the float32 tiles; 32,768 x 64 0.30 ms (0.61),
 // 32,768 x 128 0.44 ms (1.34), 1,000 queries at 32,768 x 1,536 0.33 ms (0.90).  What is left of the short ones is storing the
 // candidates.
