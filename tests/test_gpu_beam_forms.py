@@ -58,6 +58,37 @@ def test_forms_agree_with_the_oracle(rows, n, dim, beam, bqf, ef):
             assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32)), flags
 
 
+@pytest.mark.parametrize("width", [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 97])
+@pytest.mark.parametrize("dim", [40, 128, 130, 300])
+def test_candidate_counts_around_the_sets_of_64(width, dim):
+    """Four neighbour lists of `width` ids: the last set of 64 candidates of a wavefront, and its last pair of sets, full,
+    short by one and begun.  Lists share ids and have empty places, so what is left to fetch lies unevenly among the sets."""
+    print(f"beam candidates width={width} dim={dim}", flush=True)
+    from vectorlink_gpu import Queue
+    from vectorlink_gpu.ann import BEAM_NO_CACHE, BEAM_NO_WINDOWS, closest_vectors
+
+    rng = np.random.default_rng(width * 1000 + dim)
+    (n, rows, length) = (500, 70, 24)
+    v = rng.standard_normal((n, dim)).astype(np.float32)
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    table = rng.integers(0, n, (n, width)).astype(np.int32)
+    table[rng.random((n, width)) < 0.1] = orc.MAXINT
+    table[::7, : width // 2] = table[0, : width // 2]
+    c = dict(orc.DEFAULT_CONFIG)
+    c.update(beam_size=12)
+    seeds = np.stack([rng.choice(n, length, replace=False) for _ in range(rows)]).astype(np.int32)
+    d = orc.gather_distances(v[:rows], v, seeds)
+    want = orc.Queue(rows, length, length + 4 * max(width, 6))
+    want.insert(seeds, d)
+    t_want = orc.closest_vectors(v[:rows], want, v, table, c, None)
+    for flags in (0, BEAM_NO_WINDOWS, BEAM_NO_CACHE):
+        q = Queue(rows, length, length + 4 * max(width, 6))
+        q.insert(dev(seeds), dev(d))
+        assert closest_vectors(dev(v[:rows]), q, dev(v), dev(table), c, flags=flags) == t_want, flags
+        assert np.array_equal(q.indices.cpu().numpy()[:, :length], want.indices[:, :length]), flags
+        assert np.array_equal(bits(q.distances)[:, :length], want.distances[:, :length].view(np.uint32)), flags
+
+
 # lengths around a multiple of 4 at the edges of the shapes (16, 32, 64, 96, 128, 192, 256, 320, 384, 448, 512 chunks)
 ODD_DIMS = [1, 3, 5, 50, 62, 65, 127, 130, 253, 259, 383, 386, 511, 514, 766, 1022, 1026, 1279, 1534, 1790, 2045, 2049]
 

@@ -21,6 +21,9 @@ FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
     "-ffp-contract=off",  # every fused multiply-add in the kernels is written explicitly
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # where a loop ends inside a branch that ends with a barrier, merging the two ends has put reloads of spilled
+    # registers into code that runs with no lane active (clang 20 of ROCm 7)
+    "-mllvm", "-amdgpu-remove-redundant-endcf=0",
     "-Wall", "-Wno-unused-function",
 ]
 

@@ -138,6 +138,9 @@ constexpr int kMemoDecide = 9;
 // their remainder the slow way (read, wait, store) - none of the benchmark shapes has one.
 constexpr int kPreQ = 2, kPreV = 2, kPreS = 4;
 
+// Sets of 64 candidates of a wavefront whose neighbour ids, claims and cache probes are on their way at a time.
+constexpr int kAhead = 2;
+
 // Takes id's place in an open-addressed set (-1: empty).  False: the id is there already.  The places tried are those of a
 // sequence that runs through all 32-bit values (a full-period congruence), so an empty one is met.  64 ids wait for the
 // longest of their searches, which is why the set is kept as empty as LDS allows: 256 queries at 4,096 x 128 take 1,462 us
@@ -213,9 +216,11 @@ __device__ __forceinline__ int count_below(const uint64_t *keys, int n, uint64_t
 __device__ __forceinline__ void two_lower_bounds(const uint64_t *a, int na, int *in_a, const uint64_t *b, int nb, int *in_b,
                                                  int top, uint64_t k) {
     int x = 0, y = 0;
-    for (int step = top; step > 0; step >>= 1) {  // top: the largest power of two not above either length
-        if (x + step <= na && a[x + step - 1] < k) x += step;
-        if (y + step <= nb && b[y + step - 1] < k) y += step;
+    for (int step = top; step > 0; step >>= 1) {  // top: the largest power of two not above the longer one's length
+        const int i = x + step, j = y + step;  // (selects, no branches: those cost more than the reads past the end they save)
+        const uint64_t in_a = a[min(i, na) - 1], in_b = b[min(j, nb) - 1];
+        x = ((i <= na) & (in_a < k)) ? i : x;
+        y = ((j <= nb) & (in_b < k)) ? j : y;
     }
     *in_a = x;
     *in_b = y;
@@ -244,10 +249,9 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     // 20,011 x 768 133.1 and 133.7 ms).
     constexpr bool kShortRows = WINDOW && SCPL == 0 && CPL * LPR <= 96;
     constexpr int kAtOnce = kShortRows ? 8 : 1;
-    __shared__ int32_t visit_s[kMaxVisit];  // the ids popped from the visit queue in this iteration
     __shared__ uint32_t red[kRows16];
     __shared__ int n_ex_s;                  // exclusion ids before the row's first empty one
-    __shared__ int n_keys_s, n_search_s, n_fresh_s, changed_s, n_new_s, probe_hits_s, probe_asked_s, quiet_s, word_s;
+    __shared__ int n_keys_s, n_search_s, n_fresh_s, n_miss_s, changed_s, n_new_s, probe_hits_s, probe_asked_s, quiet_s, word_s;
     __shared__ __align__(8) uint8_t order_s[THREADS];  // lists of candidate lanes (wave_sketch, wave_distances_lds), 64 bytes per wavefront
 
     const MergeArgs &a = s.m;
@@ -312,6 +316,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     const uint32_t slots = (uint32_t)s.hash_slots;
     const RowLayout at = row_layout(a.m, a.L, a.VL, s.hash_slots, a.excl_cols, WINDOW);
     uint64_t *const keys = reinterpret_cast<uint64_t *>(smem);
+    uint16_t *const missed = reinterpret_cast<uint16_t *>(smem);  // candidate slots to fetch (before there are keys)
     float *const le = reinterpret_cast<float *>(smem);  // upper bounds of sketched candidates (keys are picked later)
     int32_t *const li = reinterpret_cast<int32_t *>(smem + at.cand);
     float *const ld = reinterpret_cast<float *>(li + a.m);
@@ -329,27 +334,27 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     uint8_t *const order = order_s + wave * kWave;
 
     for (int i = tid; i < (int)(slots >> 2); i += THREADS) reinterpret_cast<int4 *>(set)[i] = make_int4(-1, -1, -1, -1);
-    if (tid < a.Vt) visit_s[tid] = my_visit;
+    if (tid < a.Vt) vq[tid] = vl_make_key(my_visit, VL_MAXFLOAT);  // the ids popped in the first iteration
     if (tid == 0) {
         n_ex_s = a.excl ? a.excl_cols : 0;
         quiet_s = quiet0;
-        probe_hits_s = 0;
-        probe_asked_s = 0;
     }
     __syncthreads();
 
-    // candidate id of slot c0 + lane: the neighbour list of a visited node (ann.py:69-73)
-    auto resolve = [&](int c0) -> int32_t {
-        const int slot = c0 + lane;
+    // candidate id of a slot: the neighbour list of a visited node (ann.py:69-73)
+    auto resolve = [&](int slot) -> int32_t {
         int32_t id = VL_MAXINT;
         if (slot < a.m) {
             int sidx = s.width == 1 ? slot : (int)__umulhi((uint32_t)slot, s.width_magic), k = slot - sidx * s.width;
-            int32_t node = visit_s[sidx];
+            const int32_t node = vl_key_id(vq[sidx]);  // queue.py:87-95: the heads are popped
             if (node != VL_MAXINT && (uint32_t)node < (uint64_t)s.n_vectors) id = s.beams[(int64_t)node * s.width + k];
         }
         return id;
     };
-    int32_t id = resolve(wave * kWave);
+    // (those of a wavefront's first kAhead sets of candidates are asked for ahead of everything else)
+    int32_t near[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) near[j] = wave * kWave + j * THREADS < a.m ? resolve(tid + j * THREADS) : VL_MAXINT;
     // The row's own state, read at the top, goes to LDS now that the first neighbour lists are on their
     // way.  (Outside the loops below on purpose: inside, its addresses would be kept in registers across
     // the distance code.)
@@ -393,13 +398,8 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
             wave = __builtin_amdgcn_readfirstlane(tid / kWave);
         }
         if (WINDOW && w > 0) {
-            if (tid < a.Vt) visit_s[tid] = vl_key_id(vq[tid]);  // queue.py:87-95: the heads are popped
-            if (tid == 0) {
-                probe_hits_s = 0;
-                probe_asked_s = 0;
-            }
-            __syncthreads();
-            id = resolve(wave * kWave);
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) near[j] = wave * kWave + j * THREADS < a.m ? resolve(tid + j * THREADS) : VL_MAXINT;
             memo_word = word_s;
         }
         const int first = WINDOW ? a.Vt * (t - 1) : first0;
@@ -412,12 +412,12 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         // would be fetched anyway)
         bool sketching = false;
         if constexpr (SCPL > 0) sketching = s.sketch != nullptr && (memo_word >> 16) != 0 && t > 1;
-        __syncthreads();  // the queues and the visited ids are in LDS
+        if (w == 0) __syncthreads();  // the queues and the visited ids are in LDS
 
         // ---- add_new_to_seen_ (utils.py:61-82): the popped ids that still have room become visited ----
         if (tid < kWave) {
             const int n_add = seen_full ? 0 : min(min(a.E - first, a.Vt), a.E - cnt);  // utils.py:73-75 (cnt <= first)
-            const int32_t x = tid < n_add ? visit_s[tid] : VL_MAXINT;
+            const int32_t x = tid < n_add ? vl_key_id(vq[tid]) : VL_MAXINT;
             uint32_t h;
             const bool fresh = x != VL_MAXINT && set_claim(set, slots, x, &h);
             const uint64_t all = __ballot(fresh);
@@ -430,7 +430,10 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                 n_keys_s = 0;
                 n_search_s = 0;
                 n_fresh_s = 0;
+                n_miss_s = 0;
                 changed_s = 0;
+                probe_hits_s = 0;
+                probe_asked_s = 0;
                 word_s = memo_word;
             }
         }
@@ -446,17 +449,43 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         // lies beyond its last slot, which only ever moves down.  And later copies of an id: the neighbour lists of the
         // nodes visited in one iteration share ids; the reference evaluates every copy (kernels.py:238-255) and drops
         // all but one when the queues are sorted (kernels.py:314-349); copies carry the same distance.
-        for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
-            if (c0 != wave * kWave) id = resolve(c0);
-            const int slot = c0 + lane;
-            bool ok = slot < a.m && id != VL_MAXINT && id >= 0 && (int64_t)id < s.n_vectors;
-            if (s.count_evals || resample) n_wanted += __popcll(__ballot(ok));
-            uint32_t h = 0xffff;
-            if (ok) ok = set_claim(set, slots, id, &h);
-            if (slot < a.m) {
-                li[slot] = ok ? id : VL_MAXINT;
-                if (!ok) ld[slot] = VL_MAXFLOAT;
-                if constexpr (WINDOW) set_slot[slot] = (uint16_t)(ok ? h : 0xffffu);
+        // A row without the sketch asks its cache for the others right away and lists the candidates to fetch.
+        for (int c0 = wave * kWave; c0 < a.m; c0 += kAhead * THREADS) {
+            int32_t id[kAhead];
+            bool ok[kAhead];
+            uint64_t entry[kAhead];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                const int slot = c0 + j * THREADS + lane;
+                ok[j] = false;
+                if (c0 + j * THREADS >= a.m) continue;  // uniform
+                id[j] = c0 == wave * kWave ? near[j] : resolve(slot);
+                ok[j] = slot < a.m && id[j] != VL_MAXINT && id[j] >= 0 && (int64_t)id[j] < s.n_vectors;
+                if (s.count_evals || resample) n_wanted += __popcll(__ballot(ok[j]));
+                uint32_t h = 0xffff;
+                if (ok[j]) ok[j] = set_claim(set, slots, id[j], &h);
+                if (slot < a.m) {
+                    li[slot] = ok[j] ? id[j] : VL_MAXINT;
+                    if (!ok[j]) ld[slot] = VL_MAXFLOAT;
+                    if constexpr (WINDOW) set_slot[slot] = (uint16_t)(ok[j] ? h : 0xffffu);
+                }
+                if (!sketching && memo_row && ok[j]) entry[j] = memo_load(memo_row, s.memo_shift, id[j]);
+            }
+            if (sketching) continue;
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                const int slot = c0 + j * THREADS + lane;
+                if (memo_row && ok[j] && (int32_t)(uint32_t)entry[j] == id[j]) {
+                    ld[slot] = __builtin_bit_cast(float, (uint32_t)(entry[j] >> 32));
+                    ok[j] = false;
+                }
+                const uint64_t all = __ballot(ok[j]);
+                if (all == 0) continue;
+                if (s.count_evals || resample) n_fetched += __popcll(all);
+                int base = 0;
+                if (lane == 0) base = atomicAdd(&n_miss_s, __popcll(all));
+                base = __builtin_amdgcn_readfirstlane(base);
+                if (ok[j]) missed[base + __popcll(all & ((1ull << lane) - 1))] = (uint16_t)slot;
             }
         }
         if constexpr (SCPL > 0) {
@@ -466,7 +495,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                 for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
                     const int slot = c0 + lane;
                     const bool has = slot < a.m;
-                    id = has ? li[slot] : VL_MAXINT;
+                    const int32_t id = has ? li[slot] : VL_MAXINT;
                     bool ok = id != VL_MAXINT;
                     if (has) flags[slot] = 0;
                     // The cache serves two kinds of repeats: a candidate evaluated exactly before comes back with its
@@ -494,23 +523,21 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                 n_fetched = n_sketched;  // for the share of cache hits: what the cache did not answer
             }
         }
-        for (int c0 = wave * kWave; c0 < a.m && !sketching; c0 += THREADS) {
-            const int slot = c0 + lane;
-            id = slot < a.m ? li[slot] : VL_MAXINT;
-            bool ok = id != VL_MAXINT;
-            if (memo_row && ok) {
-                const uint64_t e = memo_load(memo_row, s.memo_shift, id);
-                if ((int32_t)(uint32_t)e == id) {
-                    ld[slot] = __builtin_bit_cast(float, (uint32_t)(e >> 32));
-                    ok = false;
+        if (!sketching) {
+            __syncthreads();
+            // (a scalar count: where one in a vector register decided about barriers the compiler has reloaded registers
+            // with no lane active)
+            const int n_miss = __builtin_amdgcn_readfirstlane(n_miss_s);
+            if constexpr (FORM == kRowScalar) {
+                for (int i = wave; i < n_miss; i += THREADS / kWave) {
+                    const int slot = __builtin_amdgcn_readfirstlane(missed[i]);
+                    wave_distances_generic(q_row, s.vectors, s.dim, s.nchunks, li[slot], lane == 0, ld + slot, memo_row,
+                                           s.memo_shift, s.l2 != 0);
                 }
+            } else {
+                listed_distances<CPL, LPR, U, THREADS / kWave, FORM == kRowUnaligned>(
+                    q_row, s.vectors, s.dim, s.nchunks, li, missed, n_miss, wave, ld, memo_row, s.memo_shift, s.l2 != 0);
             }
-            if (s.count_evals || resample) n_fetched += __popcll(__ballot(ok));
-            if constexpr (FORM == kRowScalar)
-                wave_distances_generic(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0, memo_row, s.memo_shift, s.l2 != 0);
-            else
-                wave_distances_lds<CPL, LPR, U, FORM == kRowUnaligned>(q_row, s.vectors, s.dim, s.nchunks, id, ok, ld + c0,
-                                                                       order, memo_row, s.memo_shift, s.l2 != 0);
         }
         const int stripe = (int)((blockIdx.x * (THREADS / kWave) + wave) & (kBeamStripes - 1));
         if (s.count_evals && lane == 0) {
@@ -589,7 +616,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                     n_exact += __popcll(__ballot(ok));
                     n_real += __popcll(__ballot(cid != VL_MAXINT && !(f & 16)));  // candidates known by bounds only
                     wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, cid, ok, ld + c0, order, memo_row,
-                                                    s.memo_shift, false);
+                                                    s.memo_shift);
                 }
                 // tv: the largest exact distance of those Vt candidates.  Vt unvisited candidates above wv
                 // are at most tv, so a candidate whose lower bound is above tv is not one of the Vt smallest.
@@ -622,7 +649,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                     }
                     n_exact += __popcll(__ballot(ok));
                     wave_distances_lds<CPL, LPR, U>(q_row, s.vectors, s.dim, s.nchunks, cid, ok, ld + c0, order, memo_row,
-                                                    s.memo_shift, false);
+                                                    s.memo_shift);
                 }
                 if (s.count_evals && lane == 0 && n_exact) atomicAdd(&c->evals[stripe], (unsigned long long)n_exact);
                 // A row that has to evaluate more than half of the candidates it knew by bounds exactly after all
@@ -686,7 +713,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         const int n_keys = same_in_all<kShortRows>(n_keys_s);
 
         // ---- the survivors' places in the queues; the new ones among them ----
-        const int top = 1 << (31 - __builtin_clz(max(a.L, max(nva, 1))));
+        const int top = 1 << (31 - __builtin_clz(max(a.L, nva)));
         auto look_up = [&](int j, uint64_t *k, int *in_q, int *in_v, bool *new_q, bool *new_v) {
             *k = j < n_keys ? keys[j] : kPadKey;
             two_lower_bounds(qa, a.L, in_q, va, nva, in_v, top, *k);
@@ -704,10 +731,10 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
             base = __builtin_amdgcn_readfirstlane(base);
             if (mine) to[base + __popcll(all & ((1ull << lane) - 1))] = k;
         };
-        uint64_t k0;
-        int in_q0, in_v0;
-        bool new_q0, new_v0;
-        for (int j0 = 0; j0 < n_keys; j0 += THREADS) {
+        uint64_t k0 = kPadKey;
+        int in_q0 = 0, in_v0 = 0;
+        bool new_q0 = false, new_v0 = false;
+        for (int j0 = 0; j0 + wave * kWave < n_keys; j0 += THREADS) {
             uint64_t k;
             int in_q, in_v;
             bool new_q, new_v;

@@ -126,6 +126,46 @@ struct RowChunks {
     }
 };
 
+// A row's sum over the lanes of its group (in the group's first lane).  Chunk c of a row belongs to partial sum c mod 64.  A
+// lane of an LPR-lane group holds the chunks lig + LPR * i, i.e. the partial sums lig, lig + LPR, ... (V = 64 / LPR of them,
+// the (V + j)-th chunk continuing the j-th sum), and folds them at lane distances 32 and 16 itself before the group's
+// cross-lane folds: the same additions in the same order as 64 lanes with one partial sum each (sums no chunk reaches are +0).
+template <int CPL, int LPR>
+__device__ __forceinline__ float row_sum(const float4 *r, const float4 *q, bool l2) {
+    constexpr int V = kWave / LPR;
+    float part[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) part[j] = 0.0f;
+    if (l2) {  // uniform over the launch
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            const float dx = r[i].x - q[i].x, dy = r[i].y - q[i].y;
+            const float dz = r[i].z - q[i].z, dw = r[i].w - q[i].w;
+            float a = part[i % V];
+            a = __builtin_fmaf(dx, dx, a);
+            a = __builtin_fmaf(dy, dy, a);
+            a = __builtin_fmaf(dz, dz, a);
+            a = __builtin_fmaf(dw, dw, a);
+            part[i % V] = a;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            float a = part[i % V];
+            a = __builtin_fmaf(r[i].x, q[i].x, a);
+            a = __builtin_fmaf(r[i].y, q[i].y, a);
+            a = __builtin_fmaf(r[i].z, q[i].z, a);
+            a = __builtin_fmaf(r[i].w, q[i].w, a);
+            part[i % V] = a;
+        }
+    }
+#pragma unroll
+    for (int h = V / 2; h >= 1; h >>= 1)
+#pragma unroll
+        for (int j = 0; j < h; ++j) part[j] = part[j] + part[j + h];
+    return fold_group<LPR>(part[0]);
+}
+
 // One wavefront: lane j holds candidate id `my_id` (valid when `ok`); the
 // distance of candidate lane j to the query goes to out_d[j].
 template <int CPL, int LPR, int U, bool UNALIGNED = false>
@@ -184,44 +224,7 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            // Chunk c of a row belongs to partial sum c mod 64.  A lane of an LPR-lane group holds the
-            // chunks lig + LPR * i, i.e. the partial sums lig, lig + LPR, ... (V = 64 / LPR of them, the
-            // (V + j)-th chunk continuing the j-th sum), and folds them at lane distances 32 and 16 itself
-            // before the group's cross-lane folds: the same additions in the same order as 64 lanes with one
-            // partial sum each (sums no chunk reaches are +0).
-            constexpr int V = kWave / LPR;
-            float part[V];
-#pragma unroll
-            for (int j = 0; j < V; ++j) part[j] = 0.0f;
-            if (l2) {  // uniform over the launch
-#pragma unroll
-                for (int i = 0; i < CPL; ++i) {
-                    const float dx = r[u][i].x - q[i].x, dy = r[u][i].y - q[i].y;
-                    const float dz = r[u][i].z - q[i].z, dw = r[u][i].w - q[i].w;
-                    float a = part[i % V];
-                    a = __builtin_fmaf(dx, dx, a);
-                    a = __builtin_fmaf(dy, dy, a);
-                    a = __builtin_fmaf(dz, dz, a);
-                    a = __builtin_fmaf(dw, dw, a);
-                    part[i % V] = a;
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < CPL; ++i) {
-                    float a = part[i % V];
-                    a = __builtin_fmaf(r[u][i].x, q[i].x, a);
-                    a = __builtin_fmaf(r[u][i].y, q[i].y, a);
-                    a = __builtin_fmaf(r[u][i].z, q[i].z, a);
-                    a = __builtin_fmaf(r[u][i].w, q[i].w, a);
-                    part[i % V] = a;
-                }
-            }
-#pragma unroll
-            for (int h = V / 2; h >= 1; h >>= 1)
-#pragma unroll
-                for (int j = 0; j < h; ++j) part[j] = part[j] + part[j + h];
-            float acc = part[0];
-            acc = fold_group<LPR>(acc);
+            const float acc = row_sum<CPL, LPR>(r[u], q, l2);
             if (lig == 0 && mysrc[u] >= 0) {
                 float d = finish_distance(acc, l2);
                 out_d[mysrc[u]] = d;
@@ -231,19 +234,19 @@ __device__ __forceinline__ void wave_distances(const float *__restrict__ q_row,
     }
 }
 
-// The same distances for a caller whose out_d is in LDS (the fused beam-search step), with the per-row work cut to
-// the sums: the k-th candidate's lane comes from `order` (64 bytes of LDS that belong to this wavefront, filled
-// here by rank; with one row per load instruction the lanes are simply taken off the mask), a group slot past the last
+// The same cosine distances of aligned rows for a caller whose out_d is in LDS (what the sketch leaves of a wavefront's
+// candidates), with the per-row work cut to the sums: the k-th candidate's lane comes from `order` (64 bytes of LDS that
+// belong to this wavefront, filled here by rank; with one row per load instruction the lanes are simply taken off the mask), a group slot past the last
 // candidate takes the last one again (same addresses, same sum: nothing in the loop depends on a lane having a
 // row), and the group's first lane parks the row's sum in out_d of its candidate.  Turning a sum into a distance
 // and storing the cache entry is then each lane's own work for its own candidate, once for the wavefront instead
 // of once per load.  Same loads, same additions in the same order, same bits as wave_distances.
-template <int CPL, int LPR, int U, bool UNALIGNED = false>
+template <int CPL, int LPR, int U>
 __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_row,
                                                    const float *__restrict__ vectors, int dim,
                                                    int nchunks, int32_t my_id, bool ok,
                                                    float *out_d, uint8_t *order, uint64_t *memo_row,
-                                                   int memo_shift, bool l2 = false) {
+                                                   int memo_shift) {
     constexpr int G = kWave / LPR;
     uint64_t mask = __ballot(ok);
     if (!mask) return;  // uniform over the wavefront
@@ -252,7 +255,7 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
     const int lig = lane % LPR;
     const int n = __popcll(mask);
 
-    const RowChunks<CPL, LPR, UNALIGNED> chunks(lig, dim, nchunks);
+    const RowChunks<CPL, LPR, false> chunks(lig, dim, nchunks);
     float4 q[CPL];
 #pragma unroll
     for (int i = 0; i < CPL; ++i) q[i] = chunks.load(q_row, i);
@@ -282,47 +285,66 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (k0 + u * G < n) {
-                // the partial sums of wave_distances, folded in the same order
-                constexpr int V = kWave / LPR;
-                float part[V];
-#pragma unroll
-                for (int j = 0; j < V; ++j) part[j] = 0.0f;
-                if (l2) {  // uniform over the launch
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i) {
-                        const float dx = r[u][i].x - q[i].x, dy = r[u][i].y - q[i].y;
-                        const float dz = r[u][i].z - q[i].z, dw = r[u][i].w - q[i].w;
-                        float a = part[i % V];
-                        a = __builtin_fmaf(dx, dx, a);
-                        a = __builtin_fmaf(dy, dy, a);
-                        a = __builtin_fmaf(dz, dz, a);
-                        a = __builtin_fmaf(dw, dw, a);
-                        part[i % V] = a;
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i) {
-                        float a = part[i % V];
-                        a = __builtin_fmaf(r[u][i].x, q[i].x, a);
-                        a = __builtin_fmaf(r[u][i].y, q[i].y, a);
-                        a = __builtin_fmaf(r[u][i].z, q[i].z, a);
-                        a = __builtin_fmaf(r[u][i].w, q[i].w, a);
-                        part[i % V] = a;
-                    }
-                }
-#pragma unroll
-                for (int h = V / 2; h >= 1; h >>= 1)
-#pragma unroll
-                    for (int j = 0; j < h; ++j) part[j] = part[j] + part[j + h];
-                const float acc = fold_group<LPR>(part[0]);
+                const float acc = row_sum<CPL, LPR>(r[u], q, false);
                 if (lig == 0) out_d[src[u]] = acc;
             }
         }
     }
     if (ok) {
-        const float d = finish_distance(out_d[lane], l2);  // the sum was parked there by the first lane of the row's group
+        const float d = finish_distance(out_d[lane], false);  // the sum was parked there by the first lane of the row's group
         out_d[lane] = d;
         if (memo_row) memo_store(memo_row, memo_shift, my_id, d);
+    }
+}
+
+// The distances of the candidates slots[0 .. n) of a workgroup (n the same in all lanes, in a scalar register): ids[slot]
+// goes in, dists[slot] comes out, all of it in LDS.  The rows are dealt to the workgroup's WAVES wavefronts a load
+// instruction at a time, so they end together however the candidates to fetch lie among the neighbour lists (a row of
+// 10,000 queries at 1M x 768 waited 5,700 of an iteration's 32,100 cycles for its busiest wavefront, one query at 100,000 x
+// 768 10,900 of 40,400).  LDS is asked for the ids of all U loads before the first row is asked of memory: looked up load
+// by load they are two trips to LDS each in front of it (256 queries at 4,096 x 128: 8,500 cycles an iteration, 5,000 so).
+// Same sums as wave_distances.
+template <int CPL, int LPR, int U, int WAVES, bool UNALIGNED>
+__device__ __forceinline__ void listed_distances(const float *__restrict__ q_row, const float *__restrict__ vectors, int dim,
+                                                 int nchunks, const int32_t *ids, const uint16_t *slots, int n, int wave,
+                                                 float *dists, uint64_t *memo_row, int memo_shift, bool l2) {
+    constexpr int G = kWave / LPR;
+    if (wave * G >= n) return;
+    const int lane = own_lane();
+    const int grp = lane / LPR;
+    const int lig = lane % LPR;
+    const RowChunks<CPL, LPR, UNALIGNED> chunks(lig, dim, nchunks);
+    float4 q[CPL];
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) q[i] = chunks.load(q_row, i);
+    for (int i0 = wave * G; i0 < n; i0 += WAVES * G * U) {
+        float4 r[U][CPL];
+        int slot[U];
+        int32_t id[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) slot[u] = slots[min(i0 + u * WAVES * G + grp, n - 1)];  // past the last: the last again
+#pragma unroll
+        for (int u = 0; u < U; ++u) id[u] = ids[slot[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i0 + u * WAVES * G < n) {  // a load instruction with no candidate at all is not issued
+                if constexpr (G == 1) id[u] = __builtin_amdgcn_readfirstlane(id[u]);
+                const float *row = vectors + (int64_t)id[u] * dim;
+#pragma unroll
+                for (int i = 0; i < CPL; ++i) r[u][i] = chunks.load(row, i);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i0 + u * WAVES * G < n) {
+                const float acc = row_sum<CPL, LPR>(r[u], q, l2);
+                if (lig == 0) {
+                    const float d = finish_distance(acc, l2);
+                    dists[slot[u]] = d;
+                    if (memo_row) memo_store(memo_row, memo_shift, id[u], d);
+                }
+            }
+        }
     }
 }
 
