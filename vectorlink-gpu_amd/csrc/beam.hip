@@ -788,15 +788,21 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
         return e && e[0] == 's';
     }();
     const bool use_sort_merge = sort_merge_env || (p->flags & VL_BEAM_SORT_MERGE);
-    // threads per row of the merge step: small rows are latency bound and do better with
-    // more rows in flight per CU (measured: 128 wins at m=256, E=480 and at m=128, E=960; 256 wins at
-    // m=512, E=960)
+    // Threads per row.  Rows that fill the chip want as many of them in flight as it holds: 128 threads, unless a row has more
+    // candidates in an iteration than those look at in two goes.  A few rows want the wavefronts: idle ones share in the
+    // fetch.  With 128 and 256 threads (us): 37 / 256 / 512 / 1,000 / 2,000 queries at 20,011 x 50 (m = 96) 1,085 and 961,
+    // 1,131 and 995, 1,205 and 1,065, 1,274 and 1,158, 1,430 and 2,061; 256 / 512 / 1,000 / 3,000 at 4,096 x 128 (m = 128) 1,003
+    // and 891, 1,390 and 1,216, 1,473 and 1,383, 2,176 and 2,984, at 100,000 x 128 in clusters of 977 684 and 698, 871 and 886,
+    // 1,073 and 1,129, 1,893 and 2,781; 1,000 / 3,000 / 10,000 at 50,000 x 384 (m = 192) 918 and 864, 1,502 and 1,815, 4,244 and
+    // 5,152, at 100,000 x 768 (m = 256) 618 and 566, 1,136 and 1,171, 3,163 and 3,264; a build of 100,000 x 128 (m = 256) 278 and
+    // 319 ms, of 2,000 x 128 2.58 and 2.50, of 8,000 x 200 with m = 256 / 288 / 384 / 512 17.7 and 19.2, 18.8 and 20.3, 27.3 and
+    // 23.9, 29.6 and 22.2, with the sketch (8,000 x 384) 20.7 and 23.2, 20.3 and 22.9, 39.0 and 37.3, 48.5 and 39.3.
     static const int merge_threads_env = [] {
         const char *e = getenv("VL_BEAM_MERGE_THREADS");
         return e ? atoi(e) : 0;
     }();
     const int merge_threads = merge_threads_env ? merge_threads_env
-                              : ((l.m <= 128 || (l.m + l.E + l.VL + p->queue_length) <= 1024) ? 128 : 256);
+                              : ((l.m > 320 || p->n_rows <= (l.m <= 128 ? 2 : 4) * kComputeUnits) ? 256 : 128);
     const int Pmax = a.Ps > a.Pv ? a.Ps : a.Pv;
     const size_t smem = use_sort_merge
         ? (size_t)Pmax * 8 + (size_t)a.L * 4 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4
@@ -834,7 +840,16 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
             const char *e = getenv("VL_BEAM_MEMO_MIN_RATE");
             return e ? atoi(e) : -1;
         }();
-        int64_t r = (205ll * 256) / (4 * p->dim);
+        const int64_t row_bytes = 4 * p->dim;
+        int64_t r = (205ll * 256) / row_bytes;
+        // What is measured in one early iteration says little where rows ask for so many candidates until their visited lists
+        // are full that they meet most vectors several times: the share grows then, and the cache stays in use.  Measured
+        // without a share to reach, against the share above (asked: candidates a row asks for, over the vectors there are):
+        // builds of 6,000 x 25 (asked 4.3) 0.84, 10,000 x 50 (2.6) 0.94, 9,000 x 128 (3.4) 0.86, 4,096 x 128 (7.5) 0.76, 3,000 x 64
+        // (20) 0.92; 10,000 queries at 4,096 x 64 (3.8) 0.93, 8,000 x 128 (1.9) 1.03, 20,000 x 128 (0.8) 1.21, 20,000 x 50 (0.4)
+        // 1.08, 20,000 x 300 (1.7) 0.65.
+        const int64_t asked = l.E * p->width;
+        if (row_bytes <= 512 ? 2 * asked >= 5 * p->n_vectors : row_bytes * asked >= 1280 * p->n_vectors) r = 0;
         step.memo_min_rate = rate_env >= 0 ? rate_env : (int)(r > 255 ? 255 : r);
     }
     // The sketch serves the cosine distance of 16-byte aligned rows in the fused step; other calls ignore it.

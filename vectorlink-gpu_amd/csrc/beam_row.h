@@ -138,9 +138,6 @@ constexpr int kMemoDecide = 9;
 // their remainder the slow way (read, wait, store) - none of the benchmark shapes has one.
 constexpr int kPreQ = 2, kPreV = 2, kPreS = 4;
 
-// Sets of 64 candidates of a wavefront whose neighbour ids, claims and cache probes are on their way at a time.
-constexpr int kAhead = 2;
-
 // Takes id's place in an open-addressed set (-1: empty).  False: the id is there already.  The places tried are those of a
 // sequence that runs through all 32-bit values (a full-period congruence), so an empty one is met.  64 ids wait for the
 // longest of their searches, which is why the set is kept as empty as LDS allows: 256 queries at 4,096 x 128 take 1,462 us
@@ -249,6 +246,9 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     // 20,011 x 768 133.1 and 133.7 ms).
     constexpr bool kShortRows = WINDOW && SCPL == 0 && CPL * LPR <= 96;
     constexpr int kAtOnce = kShortRows ? 8 : 1;
+    // Sets of 64 candidates of a wavefront whose neighbour ids and cache probes are on their way at a time.  (The kernels with
+    // the sketch, which wait on bytes, spill registers with two: a batch of the first loop at 1M x 768 141.0 and 143.1 ms.)
+    constexpr int kAhead = SCPL > 0 ? 1 : 2;
     __shared__ uint32_t red[kRows16];
     __shared__ int n_ex_s;                  // exclusion ids before the row's first empty one
     __shared__ int n_keys_s, n_search_s, n_fresh_s, n_miss_s, changed_s, n_new_s, probe_hits_s, probe_asked_s, quiet_s, word_s;
