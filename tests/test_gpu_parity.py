@@ -246,6 +246,38 @@ def test_queue_insert_pop_sequence(length, m, cap, e):
             assert np.array_equal(host(gq.indices), oq.indices)
 
 
+@pytest.mark.parametrize("length,m,cap", [(1, 1, 2), (3, 2, 9), (10, 4, 266), (64, 63, 127), (64, 64, 200), (20, 65, 300),
+                                          (128, 128, 640), (300, 257, 1000)])
+def test_first_insert_into_empty_rows(length, m, cap):
+    """Rows that hold nothing yet are sorted without their empty pairs; rows with one real slot anywhere, or with a candidate
+    beyond the empty distance (it sorts behind the empty pairs, which then separate copies of its id), are not."""
+    say(f"first insert length={length} m={m} cap={cap}")
+    from vectorlink_gpu import Queue
+
+    rng = np.random.default_rng(length + m + cap)
+    rows = 40
+    table = rng.random(50).astype(np.float32)
+    table[::9] = F  # real ids at the empty distance
+    ids = rng.integers(0, 50, (rows, m)).astype(np.int32)
+    d = table[ids].copy()
+    s = rng.random((rows, m)) < 0.1
+    ids[s], d[s] = M, F
+    ids[3, 0], d[3, 0] = ids[3, -1], np.inf   # copies of an id on both sides of the empty pairs
+    ids[4, -1], d[4, -1] = 7, np.float32(3.41e37)
+    ids[5], d[5] = M, F
+    ex = np.full((rows, 3), M, np.int32)
+    ex[::2, :2] = np.sort(rng.integers(0, 50, (rows, 2)), axis=1)[::2]
+    oq, gq = orc.Queue(rows, length, cap), Queue(rows, length, cap)
+    for (row, at) in ((7, 0), (8, length - 1), (9, cap - 1)):  # not empty
+        oq.indices[row, at], oq.distances[row, at] = 99, 0.5
+        gq.indices[row, at], gq.distances[row, at] = 99, 0.5
+    wm = oq.insert(ids, d, exclude=ex, output_update=True)
+    gm = gq.insert(dev(ids), dev(d), exclude=dev(ex), output_update=True)
+    assert np.array_equal(host(gq.indices), oq.indices)
+    assert np.array_equal(bits(host(gq.distances)), bits(oq.distances))
+    assert np.array_equal(host(gm), wm)
+
+
 def test_seen_add_sequence():
     from vectorlink_gpu.utils import add_new_to_seen_
 

@@ -97,9 +97,11 @@ struct PlaceScratch {
 // before/changed (optional): before[0:len) are the ids the row started with;
 // changed_bytes[i] = (new id at i != before[i]) for i < len and *any_changed
 // is or-ed with 1 when some slot differs.
+// more_empty: that many slots of the row are the empty pair and not among the keys.  They sort behind every
+// slot at VL_MAXFLOAT and ahead of those beyond it.
 __device__ inline void block_place3(const uint64_t *keys, int n, int n_out, int32_t *out_ids,
                                     float *out_d, PlaceScratch *ps, const int32_t *before,
-                                    int len, uint8_t *changed_bytes, int *any_changed) {
+                                    int len, uint8_t *changed_bytes, int *any_changed, int more_empty = 0) {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const uint32_t fkey = vl_float_key(VL_MAXFLOAT);
@@ -134,11 +136,21 @@ __device__ inline void block_place3(const uint64_t *keys, int n, int n_out, int3
     for (int c = 0; c < 3; ++c)
         if (cnt[c]) atomicAdd(&ps->total[c], cnt[c]);
     __syncthreads();
-    int run[3] = {0, ps->total[0], ps->total[0] + ps->total[1]};
+    const int empty_from = ps->total[0] + ps->total[1];
+    int run[3] = {0, ps->total[0], empty_from + more_empty};
     __syncthreads();
 
     // pass 2: stable destinations, tile by tile
     bool diff = false;
+    for (int i = empty_from + threadIdx.x; i < empty_from + more_empty && i < n_out; i += blockDim.x) {
+        out_ids[i] = VL_MAXINT;
+        out_d[i] = VL_MAXFLOAT;
+        if (before && i < len) {
+            bool ch = before[i] != VL_MAXINT;
+            diff |= ch;
+            if (changed_bytes) changed_bytes[i] = ch ? 1 : 0;
+        }
+    }
     for (int base = 0; base < n; base += blockDim.x) {
         int i = base + threadIdx.x;
         int32_t id = VL_MAXINT;
