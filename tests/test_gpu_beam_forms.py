@@ -160,3 +160,33 @@ def test_which_calls_with_a_sketch_take_several_iterations_per_launch(n, dim, wi
     launches = _native.lib().vl_beam_launches() - before
     assert t >= 10  # (one launch more than needed is on its way when the loop ends, of five iterations or of one)
     assert (launches < t) == windows, (launches, t)
+
+
+# the cache's size: a slot for every vector and a quarter (819 vectors fit 1,024 slots, 820 do not), 1,024 slots for 3,000
+# vectors of up to 128 columns, which collide; 128 threads a row and 256 on either side of one round of rows (queue 128, LDS
+# for eleven rows of 128 threads per compute unit)
+@pytest.mark.parametrize("rows,n,dim,beam,ef", [(60, 819, 40, 16, 5), (60, 820, 40, 16, 5), (60, 3000, 128, 4, 2),
+                                                (60, 3000, 132, 4, 2), (2816, 2817, 8, 64, 1), (2817, 2817, 8, 64, 1)])
+def test_cache_sizes_and_threads_per_row(rows, n, dim, beam, ef):
+    print(f"beam cache and threads rows={rows} n={n} dim={dim} beam={beam}", flush=True)
+    from vectorlink_gpu import Queue
+    from vectorlink_gpu.ann import BEAM_NO_CACHE, BEAM_NO_WINDOWS, closest_vectors
+
+    rng = np.random.default_rng(n + dim)
+    v = rng.standard_normal((n, dim)).astype(np.float32)
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    c = dict(orc.DEFAULT_CONFIG)
+    c.update(beam_size=beam, exclude_factor=ef)
+    (length, cap) = (2 * beam, 2 * beam + 4 * beam)
+    beams = orc.generate_circulant_beams(n, orc.primes(beam))
+    seeds = np.ascontiguousarray(orc.generate_circulant_beams(n, orc.primes(length))[:rows])
+    d = orc.gather_distances(v[:rows], v, seeds)
+    want = orc.Queue(rows, length, cap + length)
+    want.insert(seeds, d)
+    t_want = orc.closest_vectors(v[:rows], want, v, beams, c, None)
+    for flags in (0, BEAM_NO_WINDOWS, BEAM_NO_CACHE):
+        q = Queue(rows, length, cap + length)
+        q.insert(dev(seeds), dev(d))
+        assert closest_vectors(dev(v[:rows]), q, dev(v), dev(beams), c, flags=flags) == t_want, flags
+        assert np.array_equal(q.indices.cpu().numpy()[:, :length], want.indices[:, :length]), flags
+        assert np.array_equal(bits(q.distances)[:, :length], want.distances[:, :length].view(np.uint32)), flags

@@ -642,6 +642,16 @@ struct BeamLayout {
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
 
+// Whether rows ask for so many candidates until their visited lists are full (asked) that they meet most vectors several
+// times.  What is measured in one early iteration says little then: the share of repeats grows, and the cache stays in use.
+// Measured without a share to reach, against the share:
+// builds of 6,000 x 25 (asked 4.3 times the vectors) 0.84, 10,000 x 50 (2.6) 0.94, 9,000 x 128 (3.4) 0.86, 4,096 x 128 (7.5)
+// 0.76, 3,000 x 64 (20) 0.92; 10,000 queries at 4,096 x 64 (3.8) 0.93, 8,000 x 128 (1.9) 1.03, 20,000 x 128 (0.8) 1.21,
+// 20,000 x 50 (0.4) 1.08, 20,000 x 300 (1.7) 0.65.
+inline bool meets_again(int64_t dim, int64_t n_vectors, int64_t asked) {
+    return dim <= 128 ? 2 * asked >= 5 * n_vectors : 4 * dim * asked >= 1280 * n_vectors;
+}
+
 // lean: the layout of the entry point that allocates nothing - the fused step keeps its candidates in LDS
 // and runs without the distance cache, so neither gets room.
 int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
@@ -690,6 +700,20 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
     // iterations, fills little of a large table and would pay for clearing it on every call
     int64_t want = 128 * l->m < 512 * p->queue_length ? 128 * l->m : 512 * p->queue_length;
     int slots = vl_next_pow2(want > 65536 ? 65536 : want);
+    // ... and no more than the vectors need (a quarter of them over, for the sake of collisions): a build of 6,007 x 384
+    // 15.3 ms with 64Ki slots, 13.9 with 8Ki, 19.1 with 4Ki; of 4,096 x 128 5.10 with 32Ki, 4.86 with 8Ki, 5.12 with 4Ki; of
+    // 20,011 x 768 130.1 with 64Ki, 128.2 with 32Ki, 160.8 with 16Ki
+    const int64_t most = p->n_vectors + p->n_vectors / 4;
+    if (slots > most) slots = vl_next_pow2(most);
+    // ... and of rows of up to 512 bytes that meet few vectors again 16 per candidate: such a row is fetched again for little
+    // more than a probe, and clearing and spreading the table costs more.  Us with 128 slots per candidate (a whole table) and
+    // with 16: 10,000 queries at 1M x 128 1,991 and 1,711, at 100,000 x 128 5,389 and 5,151, at 60,000 x 50 5,969 and 5,693,
+    // builds of 100,000 x 128 275 and 269 ms, a batch of a first loop at 300,000 x 96 15.2 and 14.9.  Not with longer rows: a batch of
+    // 100,000 x 200 (no clusters, m = 512) 124.4 ms with 64Ki, 127.3 with 32Ki, 131.6 with 8Ki.
+    if (p->dim <= 128 && !meets_again(p->dim, p->n_vectors, l->E * p->width)) {
+        const int enough = vl_next_pow2(16 * l->m);
+        if (slots > enough) slots = enough;
+    }
     if (slots < 1024) slots = 1024;
     if (slots > 65536) slots = 65536;
     while (slots > 1024 && p->n_rows * (int64_t)slots * 8 > (8ll << 30)) slots >>= 1;
@@ -842,14 +866,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
         }();
         const int64_t row_bytes = 4 * p->dim;
         int64_t r = (205ll * 256) / row_bytes;
-        // What is measured in one early iteration says little where rows ask for so many candidates until their visited lists
-        // are full that they meet most vectors several times: the share grows then, and the cache stays in use.  Measured
-        // without a share to reach, against the share above (asked: candidates a row asks for, over the vectors there are):
-        // builds of 6,000 x 25 (asked 4.3) 0.84, 10,000 x 50 (2.6) 0.94, 9,000 x 128 (3.4) 0.86, 4,096 x 128 (7.5) 0.76, 3,000 x 64
-        // (20) 0.92; 10,000 queries at 4,096 x 64 (3.8) 0.93, 8,000 x 128 (1.9) 1.03, 20,000 x 128 (0.8) 1.21, 20,000 x 50 (0.4)
-        // 1.08, 20,000 x 300 (1.7) 0.65.
-        const int64_t asked = l.E * p->width;
-        if (row_bytes <= 512 ? 2 * asked >= 5 * p->n_vectors : row_bytes * asked >= 1280 * p->n_vectors) r = 0;
+        if (meets_again(p->dim, p->n_vectors, l.E * p->width)) r = 0;
         step.memo_min_rate = rate_env >= 0 ? rate_env : (int)(r > 255 ? 255 : r);
     }
     // The sketch serves the cosine distance of 16-byte aligned rows in the fused step; other calls ignore it.

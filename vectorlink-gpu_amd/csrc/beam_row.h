@@ -408,6 +408,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         const int memo_rate = memo_word & 0xffff;
         const bool resample = memo_table && t == kMemoDecide;
         uint64_t *const memo_row = memo_table && memo_rate >= s.memo_min_rate ? memo_table : nullptr;
+        const bool probing = memo_row && t > 1;  // nothing is cached before the first iteration, whose candidates are distinct
         // (not in the first iteration: the visit queue starts with empty slots, so everything unvisited is kept and
         // would be fetched anyway)
         bool sketching = false;
@@ -469,13 +470,13 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                     if (!ok[j]) ld[slot] = VL_MAXFLOAT;
                     if constexpr (WINDOW) set_slot[slot] = (uint16_t)(ok[j] ? h : 0xffffu);
                 }
-                if (!sketching && memo_row && ok[j]) entry[j] = memo_load(memo_row, s.memo_shift, id[j]);
+                if (!sketching && probing && ok[j]) entry[j] = memo_load(memo_row, s.memo_shift, id[j]);
             }
             if (sketching) continue;
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) {
                 const int slot = c0 + j * THREADS + lane;
-                if (memo_row && ok[j] && (int32_t)(uint32_t)entry[j] == id[j]) {
+                if (probing && ok[j] && (int32_t)(uint32_t)entry[j] == id[j]) {
                     ld[slot] = __builtin_bit_cast(float, (uint32_t)(entry[j] >> 32));
                     ok[j] = false;
                 }
