@@ -821,12 +821,22 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
     // 5,152, at 100,000 x 768 (m = 256) 618 and 566, 1,136 and 1,171, 3,163 and 3,264; a build of 100,000 x 128 (m = 256) 278 and
     // 319 ms, of 2,000 x 128 2.58 and 2.50, of 8,000 x 200 with m = 256 / 288 / 384 / 512 17.7 and 19.2, 18.8 and 20.3, 27.3 and
     // 23.9, 29.6 and 22.2, with the sketch (8,000 x 384) 20.7 and 23.2, 20.3 and 22.9, 39.0 and 37.3, 48.5 and 39.3.
+    // A chip full of rows with 256 threads is six to a compute unit, with 128 twelve, where their LDS leaves room for so many
+    // (taken with half of a visited list).  Where it does not, rows just beyond one round of those that fit wait for a
+    // second round of few; two rounds of six hold them better.  Queue 128, m = 256 (nine fit), 128 and 256 threads (us):
+    // 2,300 / 2,600 / 3,000 / 3,500 / 4,500 queries at 200,000 x 768 in clusters of 977 4,764 and 5,364, 6,422 and 5,781, 7,432
+    // and 6,253, 7,927 and 7,592, 9,266 and 8,983, at 100,000 x 384 3,701 and 4,275, 5,127 and 4,541, 5,719 and 4,980, 6,174 and
+    // 5,984, 7,108 and 7,199.
+    const int64_t rows_per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits;
+    const int row_bytes_128 = row_layout((int)l.m, (int)p->queue_length, (int)l.VL, row_hash_slots(l.E / 2, l.m, true), (int)p->excl_cols, true).bytes;
+    const int64_t fit_128 = (int64_t)kLdsPerCu / (row_bytes_128 + 640);
+    const bool two_rounds = fit_128 < 12 && rows_per_cu > fit_128 && rows_per_cu <= 14;
     static const int merge_threads_env = [] {
         const char *e = getenv("VL_BEAM_MERGE_THREADS");
         return e ? atoi(e) : 0;
     }();
     const int merge_threads = merge_threads_env ? merge_threads_env
-                              : ((l.m > 320 || p->n_rows <= (l.m <= 128 ? 2 : 4) * kComputeUnits) ? 256 : 128);
+                              : ((l.m > 320 || p->n_rows <= (l.m <= 128 ? 2 : 4) * kComputeUnits || two_rounds) ? 256 : 128);
     const int Pmax = a.Ps > a.Pv ? a.Ps : a.Pv;
     const size_t smem = use_sort_merge
         ? (size_t)Pmax * 8 + (size_t)a.L * 4 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4
