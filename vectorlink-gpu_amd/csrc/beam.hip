@@ -648,7 +648,12 @@ inline int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
 // builds of 6,000 x 25 (asked 4.3 times the vectors) 0.84, 10,000 x 50 (2.6) 0.94, 9,000 x 128 (3.4) 0.86, 4,096 x 128 (7.5)
 // 0.76, 3,000 x 64 (20) 0.92; 10,000 queries at 4,096 x 64 (3.8) 0.93, 8,000 x 128 (1.9) 1.03, 20,000 x 128 (0.8) 1.21,
 // 20,000 x 50 (0.4) 1.08, 20,000 x 300 (1.7) 0.65.
-inline bool meets_again(int64_t dim, int64_t n_vectors, int64_t asked) {
+// With the sketch a new candidate costs a quarter of a row, which up to 256 columns is little more than a probe.  Batches of
+// 5,000 rows (degree 64, ms): 256 columns, 20,000 vectors (asked 6.1) 26.7 without a share to reach and 28.0 with the share,
+// 40,000 (3.1) 30.4 and 30.1, 77,000 (1.6) 36.6 and 33.7, 150,000 (0.8) 36.5 and 31.7; 300 columns, 30,000 28.9 and 32.1, 77,000 40.6 and
+// 41.8, 384 columns 29.3 and 31.6, 41.0 and 42.0, 512 columns, 77,000 44.1 and 46 to 52, 768 columns 61.7 and 65.0.
+inline bool meets_again(int64_t dim, int64_t n_vectors, int64_t asked, bool sketch) {
+    if (sketch && dim <= 256) return asked >= 4 * n_vectors;
     return dim <= 128 ? 2 * asked >= 5 * n_vectors : 4 * dim * asked >= 1280 * n_vectors;
 }
 
@@ -710,7 +715,7 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
     // with 16: 10,000 queries at 1M x 128 1,991 and 1,711, at 100,000 x 128 5,389 and 5,151, at 60,000 x 50 5,969 and 5,693,
     // builds of 100,000 x 128 275 and 269 ms, a batch of a first loop at 300,000 x 96 15.2 and 14.9.  Not with longer rows: a batch of
     // 100,000 x 200 (no clusters, m = 512) 124.4 ms with 64Ki, 127.3 with 32Ki, 131.6 with 8Ki.
-    if (p->dim <= 128 && !meets_again(p->dim, p->n_vectors, l->E * p->width)) {
+    if (p->dim <= 128 && !meets_again(p->dim, p->n_vectors, l->E * p->width, (p->flags & VL_BEAM_USES_SKETCH) != 0)) {
         const int enough = vl_next_pow2(16 * l->m);
         if (slots > enough) slots = enough;
     }
@@ -876,7 +881,7 @@ int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *que
         }();
         const int64_t row_bytes = 4 * p->dim;
         int64_t r = (205ll * 256) / row_bytes;
-        if (meets_again(p->dim, p->n_vectors, l.E * p->width)) r = 0;
+        if (meets_again(p->dim, p->n_vectors, l.E * p->width, sketch && !step.l2)) r = 0;
         step.memo_min_rate = rate_env >= 0 ? rate_env : (int)(r > 255 ? 255 : r);
     }
     // The sketch serves the cosine distance of 16-byte aligned rows in the fused step; other calls ignore it.
