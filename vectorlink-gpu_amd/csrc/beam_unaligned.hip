@@ -7,7 +7,9 @@ void vl_launch_step_unaligned(const StepArgs &s, int threads, size_t smem, hipSt
     const int nchunks = s.nchunks;
     if (nchunks <= 16) launch_step<1, 16, 8, kRowUnaligned>(s, threads, smem, st);
     else if (nchunks <= 32) launch_step<2, 16, 4, kRowUnaligned>(s, threads, smem, st);
-    else if (nchunks <= 64) launch_step<1, 64, 8, kRowUnaligned>(s, threads, smem, st);
+    // (four rows in flight: eight take registers that leave five wavefronts per SIMD instead of seven; builds of 34,111 x 130 150.2 ->
+    // 133.1 ms, 20,696 x 130 109.2 -> 97.7, 30,000 x 250 163.1 -> 154.7, searches the same)
+    else if (nchunks <= 64) launch_step<1, 64, 4, kRowUnaligned>(s, threads, smem, st);
     else if (nchunks <= 96) launch_step<3, 32, 2, kRowUnaligned>(s, threads, smem, st);
     else if (nchunks <= 128) launch_step<2, 64, 4, kRowUnaligned>(s, threads, smem, st);
     else if (nchunks <= 192) launch_step<3, 64, 2, kRowUnaligned>(s, threads, smem, st);
