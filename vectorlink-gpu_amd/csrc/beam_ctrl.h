@@ -46,12 +46,12 @@ __device__ inline void beam_report(const BeamCtrl *c, int t, int R, BeamReport *
 // count beyond that was not written by this loop (its workspace is shared with another call): the row
 // must not run - its copy loops would run to that count - and the loop ends with an error.
 __device__ inline bool beam_row_state_ok(BeamCtrl *c, int cnt, int bound, bool writer) {
-    if (cnt >= 0 && cnt <= bound) return true;
-    if (writer) {
+    const bool ok = cnt >= 0 && cnt <= bound;
+    if (!ok && writer) {
         c->error = 1;
         c->stop = 1;
     }
-    return false;
+    return __builtin_amdgcn_readfirstlane(ok) != 0;  // (in a scalar register, like what beam_gate returns)
 }
 
 // State of iteration t as seen by a kernel launched for it:
@@ -65,6 +65,10 @@ __device__ inline bool beam_row_state_ok(BeamCtrl *c, int cnt, int bound, bool w
 // visited list full): state 1 is not looked for - rows of such a launch that finish early raise the slot of
 // `first` that the launch after it reads, which for some lengths is the slot of iteration t - 1 modulo 3.
 // report (may be null): where the launch after a checking iteration tells the host what that check found.
+// The result is the same in all lanes of a workgroup, but by way of the writer's own branches the compiler takes it for
+// one that lanes may disagree about, and with it everything that a kernel does after `if (gate) return`: barriers
+// and loop ends inside a branch with a lane mask of its own, where it has reloaded spilled registers with no lane active.
+// Hence the scalar register.
 __device__ inline int beam_gate(BeamCtrl *c, int t, int R, int E, bool writer, BeamReport *report = nullptr,
                                 bool look_at_fill = true) {
     int stop = c->stop;
@@ -74,13 +78,10 @@ __device__ inline int beam_gate(BeamCtrl *c, int t, int R, int E, bool writer, B
         stop = 1;
         if (writer) c->ended_after = t - 1;  // the loop ran t - 1 iterations
     }
-    if (stop) {
-        if (writer) c->stop = 1;
-        return 2;
-    }
+    if (writer && stop) c->stop = 1;
     // the slot of the check after next: this iteration itself may be a checking one (R == 1)
     // and rows of one launch set their flag while others are still here
-    if (writer && ((t - 1) % R) == 0) c->changed[((t - 1) / R + 2) & 63] = 0;
-    if (look_at_fill && t >= 2 && c->first[(t - 1) % 3] >= E) return 1;
-    return 0;
+    if (writer && !stop && ((t - 1) % R) == 0) c->changed[((t - 1) / R + 2) & 63] = 0;
+    const bool full = look_at_fill && t >= 2 && c->first[(t - 1) % 3] >= E;
+    return __builtin_amdgcn_readfirstlane(stop ? 2 : full ? 1 : 0);
 }

@@ -526,8 +526,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         }
         if (!sketching) {
             __syncthreads();
-            // (a scalar count: where one in a vector register decided about barriers the compiler has reloaded registers
-            // with no lane active)
+            // (a scalar count: the loops up to it have no lane masks)
             const int n_miss = __builtin_amdgcn_readfirstlane(n_miss_s);
             if constexpr (FORM == kRowScalar) {
                 for (int i = wave; i < n_miss; i += THREADS / kWave) {
@@ -605,6 +604,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                     if (wave == 0 && ((chosen >> lane) & 1) && !all_rest) flags[x & (kMaxCandidates - 1)] |= 8;
                 }
                 __syncthreads();
+                all_rest = __builtin_amdgcn_readfirstlane(all_rest) != 0;  // (a barrier below depends on it)
                 int n_exact = 0, n_real = 0;
                 // first round: everything below a queue's last slot, and those Vt candidates
                 for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
