@@ -249,6 +249,10 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     // Sets of 64 candidates of a wavefront whose neighbour ids and cache probes are on their way at a time.  (The kernels with
     // the sketch, which wait on bytes, spill registers with two: a batch of the first loop at 1M x 768 141.0 and 143.1 ms.)
     constexpr int kAhead = SCPL > 0 ? 1 : 2;
+    // Where the ids to visit are read from: the heads of the visit queue, and in the kernels with the sketch a copy of their
+    // own, which those need to be as fast (a batch of the first loop at 1M x 768 141.3 ms without it, 139.9 with it).
+    constexpr bool kOwnHeads = SCPL > 0;
+    __shared__ int32_t visit_s[kOwnHeads ? kMaxVisit : 1];
     __shared__ uint32_t red[kRows16];
     __shared__ int n_ex_s;                  // exclusion ids before the row's first empty one
     __shared__ int n_keys_s, n_search_s, n_fresh_s, n_miss_s, changed_s, n_new_s, probe_hits_s, probe_asked_s, quiet_s, word_s;
@@ -334,19 +338,26 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     uint8_t *const order = order_s + wave * kWave;
 
     for (int i = tid; i < (int)(slots >> 2); i += THREADS) reinterpret_cast<int4 *>(set)[i] = make_int4(-1, -1, -1, -1);
-    if (tid < a.Vt) vq[tid] = vl_make_key(my_visit, VL_MAXFLOAT);  // the ids popped in the first iteration
+    if (tid < a.Vt) {  // the ids popped in the first iteration
+        if constexpr (kOwnHeads) visit_s[tid] = my_visit;
+        else vq[tid] = vl_make_key(my_visit, VL_MAXFLOAT);
+    }
     if (tid == 0) {
         n_ex_s = a.excl ? a.excl_cols : 0;
         quiet_s = quiet0;
     }
     __syncthreads();
 
+    auto popped = [&](int i) -> int32_t {  // queue.py:87-95: the heads are popped
+        if constexpr (kOwnHeads) return visit_s[i];
+        else return vl_key_id(vq[i]);
+    };
     // candidate id of a slot: the neighbour list of a visited node (ann.py:69-73)
     auto resolve = [&](int slot) -> int32_t {
         int32_t id = VL_MAXINT;
         if (slot < a.m) {
             int sidx = s.width == 1 ? slot : (int)__umulhi((uint32_t)slot, s.width_magic), k = slot - sidx * s.width;
-            const int32_t node = vl_key_id(vq[sidx]);  // queue.py:87-95: the heads are popped
+            const int32_t node = popped(sidx);
             if (node != VL_MAXINT && (uint32_t)node < (uint64_t)s.n_vectors) id = s.beams[(int64_t)node * s.width + k];
         }
         return id;
@@ -398,6 +409,10 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
             wave = __builtin_amdgcn_readfirstlane(tid / kWave);
         }
         if (WINDOW && w > 0) {
+            if constexpr (kOwnHeads) {
+                if (tid < a.Vt) visit_s[tid] = vl_key_id(vq[tid]);
+                __syncthreads();
+            }
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) near[j] = wave * kWave + j * THREADS < a.m ? resolve(tid + j * THREADS) : VL_MAXINT;
             memo_word = word_s;
@@ -418,7 +433,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         // ---- add_new_to_seen_ (utils.py:61-82): the popped ids that still have room become visited ----
         if (tid < kWave) {
             const int n_add = seen_full ? 0 : min(min(a.E - first, a.Vt), a.E - cnt);  // utils.py:73-75 (cnt <= first)
-            const int32_t x = tid < n_add ? vl_key_id(vq[tid]) : VL_MAXINT;
+            const int32_t x = tid < n_add ? popped(tid) : VL_MAXINT;
             uint32_t h;
             const bool fresh = x != VL_MAXINT && set_claim(set, slots, x, &h);
             const uint64_t all = __ballot(fresh);
