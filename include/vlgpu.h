@@ -224,6 +224,14 @@ typedef struct vl_beam_params {
 #define VL_BEAM_WINDOWS 32
 #define VL_BEAM_NO_WINDOWS 64
 
+/* Bytes of workspace that serve a call with these parameters.  All but the last
+ * part, the distance cache, follows from n_rows, width, beam_size, the queue and
+ * visit parameters and flags (with VL_BEAM_USES_SKETCH also dim).  The cache takes
+ * 1,024 to 65,536 slots of 8 bytes per row, and how many are of use depends on
+ * n_vectors and dim as well, not always upwards: a larger table may need a
+ * smaller cache.  A workspace that was sized with another n_vectors or dim is
+ * accepted, and the cache then has the slots that fit; refused is one that could
+ * not hold 1,024 per row.  The result does not depend on it. */
 int64_t vl_beam_workspace_bytes(const vl_beam_params *p);
 
 /* Runs the whole loop of closest_vectors on the search queue in place and

@@ -190,3 +190,51 @@ def test_cache_sizes_and_threads_per_row(rows, n, dim, beam, ef):
         assert closest_vectors(dev(v[:rows]), q, dev(v), dev(beams), c, flags=flags) == t_want, flags
         assert np.array_equal(q.indices.cpu().numpy()[:, :length], want.indices[:, :length]), flags
         assert np.array_equal(bits(q.distances)[:, :length], want.distances[:, :length].view(np.uint32)), flags
+
+
+# sized for a table of fewer vectors, of more vectors (whose rows of up to 128 columns meet few vectors again and take a small
+# cache), of longer rows; and by what a table of one vector needs
+@pytest.mark.parametrize("dim,sized", [(768, dict(n_vectors=3000)), (768, dict(n_vectors=1)), (64, dict(n_vectors=1_000_000)),
+                                       (64, dict(dim=100, n_vectors=400_000)), (132, dict(dim=64, n_vectors=1_000_000))])
+def test_a_workspace_sized_for_another_table_serves(dim, sized):
+    print(f"workspace of another table dim={dim} {sized}", flush=True)
+    import ctypes as C
+
+    from vectorlink_gpu import Queue, _native as nv
+    from vectorlink_gpu.ann import _beam_params
+
+    rng = np.random.default_rng(dim)
+    (n, rows, beam) = (4000, 30, 32)
+    v = rng.standard_normal((n, dim)).astype(np.float32)
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    c = dict(orc.DEFAULT_CONFIG)
+    c.update(beam_size=beam)
+    (length, cap) = (2 * beam, 6 * beam)
+    gv, gb = dev(v), dev(orc.generate_circulant_beams(n, orc.primes(beam)))
+    seeds = orc.generate_circulant_beams(n, orc.primes(length))[:rows]
+    d = dev(orc.gather_distances(v[:rows], v, seeds))
+
+    def run(give):
+        """Result of a call with `give` of the bytes that its own parameters ask for, and what lies behind them."""
+        q = Queue(rows, length, cap + length)
+        q.insert(dev(seeds), d)
+        p = _beam_params(rows, dim, n, beam, q, c, 0, 0)
+        need = nv.lib().vl_beam_workspace_bytes(C.byref(p))
+        have = give(p) or need
+        ws = torch.full((max(have, need) + 256,), 0xA5, dtype=torch.uint8, device="cuda:0")
+        rc = nv.lib().vl_closest_vectors(C.byref(p), nv.ptr(gv), nv.ptr(gv), nv.ptr(gb), nv.ptr(q.indices),
+                                         nv.ptr(q.distances), None, nv.ptr(ws), have, nv.stream())
+        assert bool((ws[have:] == 0xA5).all())
+        return have, need, (rc, q.indices.cpu().numpy()[:, :length], bits(q.distances)[:, :length])
+
+    def other(p, **kw):
+        o = type(p)(**{f: getattr(p, f) for f, _ in p._fields_})
+        for k, x in kw.items():
+            setattr(o, k, x)
+        return nv.lib().vl_beam_workspace_bytes(C.byref(o))
+
+    want = run(lambda p: None)[2]
+    have, need, got = run(lambda p: other(p, **sized))
+    assert have < need and got[0] == want[0] > 0
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2])
+    assert run(lambda p: other(p, n_vectors=1) - 1)[2][0] == -3

@@ -642,6 +642,8 @@ struct BeamLayout {
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
 
+constexpr int kLeastCacheSlots = 1024;  // per row, where there is a cache
+
 // Whether rows ask for so many candidates until their visited lists are full (asked) that they meet most vectors several
 // times.  What is measured in one early iteration says little then: the share of repeats grows, and the cache stays in use.
 // Measured without a share to reach, against the share:
@@ -719,9 +721,9 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
         const int enough = vl_next_pow2(16 * l->m);
         if (slots > enough) slots = enough;
     }
-    if (slots < 1024) slots = 1024;
+    if (slots < kLeastCacheSlots) slots = kLeastCacheSlots;
     if (slots > 65536) slots = 65536;
-    while (slots > 1024 && p->n_rows * (int64_t)slots * 8 > (8ll << 30)) slots >>= 1;
+    while (slots > kLeastCacheSlots && p->n_rows * (int64_t)slots * 8 > (8ll << 30)) slots >>= 1;
     if (memo_env >= 0) slots = memo_env;
     if (lean || (p->flags & VL_BEAM_NO_CACHE)) slots = 0;
     l->memo_slots = slots;
@@ -763,13 +765,19 @@ __global__ void beam_status_kernel(const BeamCtrl *c, int iterations, int R, int
 // > 0: enqueue exactly that many iterations and return 0 without ever waiting for the device - once a
 // check finds the batch quiet the remaining launches do nothing (beam_gate) - then one small kernel writes
 // status_out[0] = 1 if the loop ended within them (else 0) and status_out[1] = the iteration count.
-int64_t beam_loop(const vl_beam_params *p, const BeamLayout &l, const float *queries, const float *vectors,
+int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, const float *vectors,
                   const int32_t *beams, int32_t *q_ids, float *q_dists, const int32_t *exclude, void *workspace,
                   int64_t workspace_bytes, int64_t fixed_iterations, int32_t *status_out, void *stream,
                   const uint8_t *sketch = nullptr) {
     int rc;
     VL_REQUIRE(queries && vectors && beams && q_ids && q_dists && workspace, "null pointer");
     VL_REQUIRE(((uintptr_t)workspace & 255) == 0, "workspace must be 256-byte aligned");
+    // A workspace sized for the same rows of a table with more or fewer vectors or columns serves: the cache, which lies at
+    // the end, takes the slots that fit.  Refused is what is too small for a table of any size.
+    while (l.total > workspace_bytes && l.memo_slots > kLeastCacheSlots) {
+        l.memo_slots >>= 1;
+        l.total = align256(l.off_memo + p->n_rows * (int64_t)l.memo_slots * 8);
+    }
     if (workspace_bytes < l.total) {
         vl_set_error("workspace of %lld bytes is smaller than the %lld needed", (long long)workspace_bytes,
                      (long long)l.total);
