@@ -105,6 +105,24 @@ def test_knn_workspace_serves_both_metrics(lib, metric):
         assert lib.vl_knn_form(*s, metric, lib.vl_knn_workspace_bytes(*s)) == lib.vl_knn_form(*s, metric, 1 << 60), s
 
 
+def test_calls_that_cannot_use_the_sketch_are_sized_as_without_it(lib):
+    """The distance cache of rows that meet most vectors again is larger, and with the sketch they have to ask for more of
+    them.  A call whose metric, row length or form rules the sketch out is judged as one without it: the sketch's own part of
+    the workspace is all that the flag adds, for tables of every size."""
+    from vectorlink_gpu import _native as nv
+
+    def size(n, flags, **kw):
+        p = dict(n_rows=100, dim=64, n_vectors=n, width=64, queue_capacity=64 + 256, queue_length=64, beam_size=64,
+                 parallel_visit_count=4, visit_queue_factor=3, exclude_factor=5, speculative_readahead=5, excl_cols=0,
+                 flags=flags, metric=0)
+        p.update(kw)
+        return lib.vl_beam_workspace_bytes(C.byref(nv.BeamParams(**p)))
+
+    for kw, flags in ((dict(metric=1), 0), (dict(dim=50), 0), (dict(), 1), (dict(), 2)):
+        adds = {size(n, 16 | flags, **kw) - size(n, flags, **kw) for n in (500, 5000, 15_000, 18_000, 24_000, 60_000, 1_000_000)}
+        assert len(adds) == 1 and adds.pop() > 0, (kw, flags)
+
+
 def test_the_filter_is_left_out_where_the_tiles_are_sooner(lib):
     """Short calls stay with the float32 tiles; long ones go through the filter, and so does any if asked for."""
     few, tiles, filt = 1, 0, 2

@@ -638,6 +638,8 @@ struct BeamLayout {
     int64_t m, VL, Vt, E, head;
     int64_t off_cand_ids, off_cand_d, off_v_ids, off_v_d, off_seen, off_seen_count, off_row_quiet, off_memo_rate, off_ctrl, off_rounded, off_memo, total;
     int memo_slots;
+    bool may_sketch;     // the call may bring a sketch and use it (as far as its parameters tell: not the rows' addresses)
+    bool rows_meet_again;  // what meets_again says
 };
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
@@ -677,6 +679,9 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
     l->m = l->Vt * p->width;
     l->E = p->exclude_factor * l->VL;                                                  // ann.py:55
     l->head = p->queue_length < l->VL ? p->queue_length : l->VL;                       // queue.py:31
+    l->may_sketch = (p->flags & VL_BEAM_USES_SKETCH) && !(p->flags & (VL_BEAM_TWO_LAUNCHES | VL_BEAM_SORT_MERGE)) &&
+                    p->metric == VL_METRIC_COSINE && p->dim % 4 == 0 && p->dim <= 2048 && l->m <= kMaxCandidates;
+    l->rows_meet_again = meets_again(p->dim, p->n_vectors, l->E * p->width, l->may_sketch);
     VL_REQUIRE(l->Vt <= kMaxVisit, "parallel_visit_count above %d is not supported", kMaxVisit);
     VL_REQUIRE(p->queue_length + l->m <= p->queue_capacity,
                "search queue capacity %lld cannot take %lld candidates after its %lld slots",
@@ -717,7 +722,7 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
     // with 16: 10,000 queries at 1M x 128 1,991 and 1,711, at 100,000 x 128 5,389 and 5,151, at 60,000 x 50 5,969 and 5,693,
     // builds of 100,000 x 128 275 and 269 ms, a batch of a first loop at 300,000 x 96 15.2 and 14.9.  Not with longer rows: a batch of
     // 100,000 x 200 (no clusters, m = 512) 124.4 ms with 64Ki, 127.3 with 32Ki, 131.6 with 8Ki.
-    if (p->dim <= 128 && !meets_again(p->dim, p->n_vectors, l->E * p->width, (p->flags & VL_BEAM_USES_SKETCH) != 0)) {
+    if (p->dim <= 128 && !l->rows_meet_again) {
         const int enough = vl_next_pow2(16 * l->m);
         if (slots > enough) slots = enough;
     }
@@ -889,7 +894,7 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         }();
         const int64_t row_bytes = 4 * p->dim;
         int64_t r = (205ll * 256) / row_bytes;
-        if (meets_again(p->dim, p->n_vectors, l.E * p->width, sketch && !step.l2)) r = 0;
+        if (l.rows_meet_again) r = 0;
         step.memo_min_rate = rate_env >= 0 ? rate_env : (int)(r > 255 ? 255 : r);
     }
     // The sketch serves the cosine distance of 16-byte aligned rows in the fused step; other calls ignore it.

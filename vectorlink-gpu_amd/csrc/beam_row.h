@@ -130,7 +130,8 @@ __device__ __forceinline__ uint32_t bound_slot_key(float hi, int slot) {
 // fetch again).  Each row therefore decides for itself: it uses the cache during its first kMemoDecide - 1
 // iterations, measures the share of hits in iteration kMemoDecide, and leaves the cache alone for the rest
 // of the call if that share is below the break-even share.  A hit returns the bits that would be computed
-// again, so the decision never changes a result.
+// again, so the decision never changes a result.  (Where rows ask for so many candidates that they meet most vectors
+// again, meets_again in beam.hip, the break-even share is 0: the cache stays in use.)
 constexpr int kMemoDecide = 9;
 
 // Elements of a row that one thread brings in at the start of the fused step and keeps in registers until
