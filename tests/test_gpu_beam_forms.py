@@ -125,6 +125,33 @@ def test_rows_of_odd_length(dim, metric):
     assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32))
 
 
+@pytest.mark.parametrize("rows", [2560, 2561, 3072, 3073])
+@pytest.mark.parametrize("dim", [390, 902])
+def test_rows_of_odd_length_in_one_round(rows, dim):
+    """From 385 columns on, ten, eleven, twelve and thirteen rows per compute unit have different numbers of rows in flight."""
+    print(f"odd rows dim={dim} rows={rows}", flush=True)
+    from vectorlink_gpu import Queue
+    from vectorlink_gpu.ann import BEAM_NO_WINDOWS, closest_vectors, excluding_self
+
+    rng = np.random.default_rng(rows + dim)
+    (beam, ql) = (3, 6)
+    v = rng.standard_normal((rows, dim)).astype(np.float32)
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    c = dict(orc.DEFAULT_CONFIG)
+    c.update(beam_size=beam, beam_queue_factor=2, exclude_factor=3)
+    beams = orc.generate_circulant_beams(rows, orc.primes(ql))
+    d = orc.calculate_distances(v, beams)
+    want = orc.Queue(rows, ql, ql + ql * 4)
+    want.insert(beams, d)
+    t_want = orc.closest_vectors(v, want, v, beams, c, orc.excluding_self(0, rows))
+    for flags in (0, BEAM_NO_WINDOWS):
+        q = Queue(rows, ql, ql + ql * 4)
+        q.insert(dev(beams), dev(d))
+        assert closest_vectors(dev(v), q, dev(v), dev(beams), c, excluding_self(0, rows), flags=flags) == t_want
+        assert np.array_equal(q.indices.cpu().numpy()[:, :ql], want.indices[:, :ql])
+        assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32))
+
+
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
 def test_odd_rows_with_values_that_are_not_finite(value):
     """A row of 7 elements is read as elements 0-3 and 3-6: element 3 counts once, whatever it is."""

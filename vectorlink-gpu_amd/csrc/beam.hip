@@ -611,7 +611,9 @@ int dist_variant() {
 // (measured: searches of 1M x 768 1.59 -> 1.69 M queries/s, the 1M x 128 build 4.4 -> 4.1 s; at 384 columns with
 // two instead of four whole rows in flight, third-loop launches 0.252 -> 0.217 ms, and the sketch kernel with one
 // load in flight 0.317 -> 0.295 ms on the first loop's).  A sketch row has a quarter of the chunks, so a quarter of
-// the lanes (or of the chunks per lane) covers it.
+// the lanes (or of the chunks per lane) covers it.  Two shapes end with the wavefronts asked for in the kernel of several
+// iterations, which are one more than the compiler leaves room for (3 to 5 spilled registers): 2,400 / 10,000 queries at
+// 60,000 x 1,280 1,762 -> 1,708 and 6,509 -> 6,359 us, 2,800 / 10,000 at 60,000 x 1,792 2,430 -> 2,324 and 8,228 -> 7,834.
 int launch_step_by_dim(const StepArgs &s, bool aligned, int threads, size_t smem, hipStream_t st) {
     const int nchunks = s.nchunks;
     const int variant = dist_variant();
@@ -625,9 +627,9 @@ int launch_step_by_dim(const StepArgs &s, bool aligned, int threads, size_t smem
     else if (nchunks <= 128) launch_step<2, 64, 8, kRowAligned, 2, 16, 2, 6, 2>(s, threads, smem, st);
     else if (nchunks <= 192) launch_step<3, 64, 2, kRowAligned, 3, 16, 1, 8, 1, 8>(s, threads, smem, st);
     else if (nchunks <= 256) launch_step<4, 64, 4, kRowAligned, 4, 16, 2, 5, 2>(s, threads, smem, st);
-    else if (nchunks <= 320) launch_step<5, 64, 2, kRowAligned, 3, 32, 2, 6, 1>(s, threads, smem, st);
+    else if (nchunks <= 320) launch_step<5, 64, 2, kRowAligned, 3, 32, 2, 6, 1, 0, 5>(s, threads, smem, st);
     else if (nchunks <= 384) launch_step<6, 64, 2, kRowAligned, 3, 32, 2, 6, 1>(s, threads, smem, st);
-    else if (nchunks <= 448) launch_step<7, 64, 2, kRowAligned, 4, 32, 2, 5, 1>(s, threads, smem, st);
+    else if (nchunks <= 448) launch_step<7, 64, 2, kRowAligned, 4, 32, 2, 5, 1, 0, 4>(s, threads, smem, st);
     else launch_step<8, 64, 2, kRowAligned, 4, 32, 2, 5, 1>(s, threads, smem, st);
     VL_LAUNCH_CHECK("beam_step_kernel");
     g_step_launches.fetch_add(1, std::memory_order_relaxed);

@@ -51,7 +51,7 @@ void launch_rows(Kernel kernel, int threads, const StepArgs &s, size_t smem, hip
     hipLaunchKernelGGL(kernel, dim3((unsigned)s.m.n_rows), dim3((unsigned)threads), smem, st, s);
 }
 
-template <int THREADS, int CPL, int LPR, int U, RowForm FORM, int SCPL, int SLPR, int SU, int WPE, int UX, int WPP>
+template <int THREADS, int CPL, int LPR, int U, RowForm FORM, int SCPL, int SLPR, int SU, int WPE, int UX, int WPP, int WPW>
 void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
     if constexpr (SCPL > 0) {
         if (s.sketch) {
@@ -60,15 +60,15 @@ void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
             return;
         }
     }
-    if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, FORM, THREADS, (WPP > 0 ? 6 : 1)>, THREADS, s, smem, st);
+    if (s.window > 0) launch_rows(beam_window_kernel<CPL, LPR, U, FORM, THREADS, WPW>, THREADS, s, smem, st);
     else if constexpr (WPP > 0 && FORM == kRowAligned) launch_rows(beam_step_kernel_w<CPL, LPR, U, THREADS, WPP>, THREADS, s, smem, st);
     else launch_rows(beam_step_kernel<CPL, LPR, U, FORM, THREADS>, THREADS, s, smem, st);
 }
 
-template <int CPL, int LPR, int U, RowForm FORM, int SCPL = 0, int SLPR = 64, int SU = 1, int WPE = 4, int UX = U, int WPP = 0>
+template <int CPL, int LPR, int U, RowForm FORM, int SCPL = 0, int SLPR = 64, int SU = 1, int WPE = 4, int UX = U, int WPP = 0, int WPW = (WPP > 0 ? 6 : 1)>
 void launch_step(const StepArgs &s, int threads, size_t smem, hipStream_t st) {
-    if (threads == 128) launch_step_threads<128, CPL, LPR, U, FORM, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
-    else launch_step_threads<256, CPL, LPR, U, FORM, SCPL, SLPR, SU, WPE, UX, WPP>(s, smem, st);
+    if (threads == 128) launch_step_threads<128, CPL, LPR, U, FORM, SCPL, SLPR, SU, WPE, UX, WPP, WPW>(s, smem, st);
+    else launch_step_threads<256, CPL, LPR, U, FORM, SCPL, SLPR, SU, WPE, UX, WPP, WPW>(s, smem, st);
 }
 
 }  // namespace
