@@ -968,15 +968,20 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
                             smem_window + 2048 <= kLdsPerCu;
     // A launch's LDS.  The visited ids of its last iteration and the candidates share the hash set, and the emptier it is
     // the sooner each finds its place, so it takes what LDS the workgroups that a compute unit can hold (or that there are)
-    // leave it.
+    // leave it.  Where a batch is one round of such workgroups, their share is counted in the pieces that LDS is handed out in:
+    // else ten, eleven or twelve that were to share a compute unit take a piece more each than there is, and the last rows
+    // run in a round of their own.  2,400 rows (ten per compute unit), share in bytes and in pieces: queries at 100,000 x 384
+    // 2,282 and 1,946 us, at 60,000 x 200 1,632 and 1,462, batches of a first loop at 60,000 x 768 (degree 32) 13.4 and 11.4 ms,
+    // at 60,000 x 130 14.2 and 9.0; 2,800 (eleven) at 60,000 x 384 (degree 24) 8.0 and 7.3 ms, 60,000 x 256 searched 3,112 and
+    // 3,155 us.  A batch of more rounds does better with the larger set (10,000 rows at 60,000 x 768 44.5 and 45.0 ms).
     auto size_set = [&](int64_t last_iteration, bool windowed) -> size_t {
         const int64_t visited = l.Vt * last_iteration < l.E ? l.Vt * last_iteration : l.E;
         const int waves = step_threads / kWave;
-        int64_t resident = (windowed ? 4 * 6 : 4 * 8) / waves;
-        const int64_t per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits;
-        if (resident > per_cu) resident = per_cu;
+        const int64_t per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits, most_resident = (windowed ? 4 * 6 : 4 * 8) / waves;
+        const int64_t share = per_cu <= most_resident ? (int64_t)(kLdsPerCu / kLdsGranule / per_cu * kLdsGranule)
+                                                     : (int64_t)kLdsPerCu / most_resident;
         const int least = row_hash_slots(visited, a.m, windowed), most = row_hash_slots_most(visited, a.m);
-        const int64_t room = (int64_t)(kLdsPerCu / resident) - 1024 - row_layout(a.m, a.L, a.VL, 0, a.excl_cols, windowed).bytes;
+        const int64_t room = share - 1024 - row_layout(a.m, a.L, a.VL, 0, a.excl_cols, windowed).bytes;
         int64_t slots = (room < 0 ? 0 : room) / 4;
         slots = slots > most ? most : slots;
         step.hash_slots = (int)(slots < least ? least : slots) & ~3;

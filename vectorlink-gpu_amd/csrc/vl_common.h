@@ -57,6 +57,7 @@ static inline unsigned vl_grid_for(int64_t n, int per_block) {
 // more dynamic LDS than the 64 KiB every kernel is allowed by default has to raise that kernel's limit first.
 constexpr size_t kLdsDefault = 64 * 1024;
 constexpr size_t kLdsPerCu = 160 * 1024;
+constexpr size_t kLdsGranule = 1280;  // a workgroup's LDS is handed out in pieces of this size
 constexpr int kComputeUnits = 256;
 template <class Kernel>
 static inline hipError_t vl_allow_lds(Kernel kernel, size_t smem) {
