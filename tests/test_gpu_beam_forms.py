@@ -128,7 +128,7 @@ def test_rows_of_odd_length(dim, metric):
 @pytest.mark.parametrize("rows", [2560, 2561, 3072, 3073])
 @pytest.mark.parametrize("dim", [390, 902])
 def test_rows_of_odd_length_in_one_round(rows, dim):
-    """From 385 columns on, ten, eleven, twelve and thirteen rows per compute unit have different numbers of rows in flight."""
+    """From 385 columns on, ten, eleven, twelve and thirteen rows per compute unit take different forms of the fetch."""
     print(f"odd rows dim={dim} rows={rows}", flush=True)
     from vectorlink_gpu import Queue
     from vectorlink_gpu.ann import BEAM_NO_WINDOWS, closest_vectors, excluding_self

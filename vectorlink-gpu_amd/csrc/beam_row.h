@@ -551,7 +551,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                                            s.memo_shift, s.l2 != 0);
                 }
             } else {
-                listed_distances<CPL, LPR, U, THREADS / kWave, FORM == kRowUnaligned>(
+                listed_distances<CPL, LPR, U, THREADS / kWave, FORM != kRowAligned, FORM == kRowUnalignedSums>(
                     q_row, s.vectors, s.dim, s.nchunks, li, missed, n_miss, wave, ld, memo_row, s.memo_shift, s.l2 != 0);
             }
         }

@@ -12,8 +12,9 @@ __device__ __forceinline__ int own_lane() {
     return lane;
 }
 
-// How rows are read: 16 bytes at a time (at multiples of 16, or of 4), or element by element.
-enum RowForm { kRowAligned, kRowUnaligned, kRowScalar };
+// How rows are read: 16 bytes at a time (at multiples of 16, or of 4), or element by element.  kRowUnalignedSums: as
+// kRowUnaligned, and the fused step turns the sums of a wavefront's rows into distances together (listed_distances).
+enum RowForm { kRowAligned, kRowUnaligned, kRowScalar, kRowUnalignedSums };
 
 __device__ __forceinline__ float clamp_distance(float cos_theta) {
     float r = (1.0f - cos_theta) * 0.5f;  // kernels.py:109
@@ -303,8 +304,16 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
 // 10,000 queries at 1M x 768 waited 5,700 of an iteration's 32,100 cycles for its busiest wavefront, one query at 100,000 x
 // 768 10,900 of 40,400).  LDS is asked for the ids of all U loads before the first row is asked of memory: looked up load
 // by load they are two trips to LDS each in front of it (256 queries at 4,096 x 128: 8,500 cycles an iteration, 5,000 so).
+// SUMS: a row's sum is parked in dists, and once a wavefront's rows are through each lane turns one of them into the distance
+// and stores its cache entry.  Otherwise the first lane of a row's lanes does so right away, between the loads - which then
+// wait for these stores as well, as both are counted together, and hold the registers of the ids meanwhile.
+// Which is the sooner depends on how much is fetched: rows that are not aligned and meet few vectors again, away and
+// together (us): 1,500 / 10,000 queries at 20,011 x 50 1,404 -> 1,368 and 4,841 -> 4,662, at 20,000 x 130 3,104 -> 2,823 and
+// 11,750 -> 10,750, 1,500 at 30,000 x 390 6,480 -> 5,814, 300 at 30,000 x 902 4,240 -> 3,276, batches of a first loop at
+// 60,000 x 130 32,813 -> 29,617; aligned rows, which mostly do meet them again, 10,000 at 100,000 x 128 5,125 -> 5,233, at
+// 60,000 x 256 10,909 -> 11,102, at 1M x 768 3,217 and 3,210.
 // Same sums as wave_distances.
-template <int CPL, int LPR, int U, int WAVES, bool UNALIGNED>
+template <int CPL, int LPR, int U, int WAVES, bool UNALIGNED, bool SUMS>
 __device__ __forceinline__ void listed_distances(const float *__restrict__ q_row, const float *__restrict__ vectors, int dim,
                                                  int nchunks, const int32_t *ids, const uint16_t *slots, int n, int wave,
                                                  float *dists, uint64_t *memo_row, int memo_shift, bool l2) {
@@ -339,11 +348,25 @@ __device__ __forceinline__ void listed_distances(const float *__restrict__ q_row
             if (i0 + u * WAVES * G < n) {
                 const float acc = row_sum<CPL, LPR>(r[u], q, l2);
                 if (lig == 0) {
-                    const float d = finish_distance(acc, l2);
-                    dists[slot[u]] = d;
-                    if (memo_row) memo_store(memo_row, memo_shift, id[u], d);
+                    if constexpr (SUMS) {
+                        dists[slot[u]] = acc;
+                    } else {
+                        const float d = finish_distance(acc, l2);
+                        dists[slot[u]] = d;
+                        if (memo_row) memo_store(memo_row, memo_shift, id[u], d);
+                    }
                 }
             }
+        }
+    }
+    if constexpr (SUMS) {
+        for (int j = lane;; j += kWave) {  // the wavefront's j-th row
+            const int i = (j / G) * (WAVES * G) + wave * G + j % G;
+            if (i >= n) break;
+            const int at = slots[i];
+            const float d = finish_distance(dists[at], l2);
+            dists[at] = d;
+            if (memo_row) memo_store(memo_row, memo_shift, ids[at], d);
         }
     }
 }
