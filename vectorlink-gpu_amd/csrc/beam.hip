@@ -832,31 +832,51 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         return e && e[0] == 's';
     }();
     const bool use_sort_merge = sort_merge_env || (p->flags & VL_BEAM_SORT_MERGE);
-    // Threads per row.  Rows that fill the chip want as many of them in flight as it holds: 128 threads, unless a row has more
-    // candidates in an iteration than those look at in two goes.  A few rows want the wavefronts: idle ones share in the
-    // fetch.  With 128 and 256 threads (us): 37 / 256 / 512 / 1,000 / 2,000 queries at 20,011 x 50 (m = 96) 1,085 and 961,
-    // 1,131 and 995, 1,205 and 1,065, 1,274 and 1,158, 1,430 and 2,061; 256 / 512 / 1,000 / 3,000 at 4,096 x 128 (m = 128) 1,003
-    // and 891, 1,390 and 1,216, 1,473 and 1,383, 2,176 and 2,984, at 100,000 x 128 in clusters of 977 684 and 698, 871 and 886,
-    // 1,073 and 1,129, 1,893 and 2,781; 1,000 / 3,000 / 10,000 at 50,000 x 384 (m = 192) 918 and 864, 1,502 and 1,815, 4,244 and
-    // 5,152, at 100,000 x 768 (m = 256) 618 and 566, 1,136 and 1,171, 3,163 and 3,264; a build of 100,000 x 128 (m = 256) 278 and
-    // 319 ms, of 2,000 x 128 2.58 and 2.50, of 8,000 x 200 with m = 256 / 288 / 384 / 512 17.7 and 19.2, 18.8 and 20.3, 27.3 and
-    // 23.9, 29.6 and 22.2, with the sketch (8,000 x 384) 20.7 and 23.2, 20.3 and 22.9, 39.0 and 37.3, 48.5 and 39.3.
-    // A chip full of rows with 256 threads is six to a compute unit, with 128 twelve, where their LDS leaves room for so many
-    // (taken with half of a visited list).  Where it does not, rows just beyond one round of those that fit wait for a
-    // second round of few; two rounds of six hold them better.  Queue 128, m = 256 (nine fit), 128 and 256 threads (us):
-    // 2,300 / 2,600 / 3,000 / 3,500 / 4,500 queries at 200,000 x 768 in clusters of 977 4,764 and 5,364, 6,422 and 5,781, 7,432
-    // and 6,253, 7,927 and 7,592, 9,266 and 8,983, at 100,000 x 384 3,701 and 4,275, 5,127 and 4,541, 5,719 and 4,980, 6,174 and
-    // 5,984, 7,108 and 7,199.
+    const bool aligned = (p->dim % 4 == 0) && (((uintptr_t)queries | (uintptr_t)vectors) % 16 == 0);
+    // VL_BEAM_WINDOWS / VL_BEAM_NO_WINDOWS in flags, or VL_BEAM_WINDOW=1 / 0 in the environment: windows always / never.
+    static const int window_env = [] {
+        const char *e = getenv("VL_BEAM_WINDOW");
+        return e ? atoi(e) : -1;
+    }();
+    const bool all_windows = window_env >= 0 ? window_env != 0 : (p->flags & VL_BEAM_WINDOWS) != 0;
+    const bool no_windows = window_env >= 0 ? window_env == 0 : (p->flags & VL_BEAM_NO_WINDOWS) != 0;
+    // Threads per row.  A few rows want the wavefronts: idle ones share in the fetch.  Rows that fill the chip want as many of
+    // them in flight as it holds: 128 threads, unless a row has more than 320 candidates in an iteration (ms of a build of
+    // 8,000 x 200 with m = 256 / 288 / 384 / 512, 128 and 256 threads: 17.7 and 19.2, 18.8 and 20.3, 27.3 and 23.9, 29.6 and
+    // 22.2, with the sketch (8,000 x 384) 20.7 and 23.2, 20.3 and 22.9, 39.0 and 37.3, 48.5 and 39.3).
+    // Few are the rows that a compute unit holds at once with 256 threads: six, and four of the shapes whose registers leave four
+    // wavefronts per SIMD (aligned rows of 385 to 512 columns without the sketch, rows of more than 768).  Time with 128
+    // threads over time with 256 at 4 / 5 / 6 / 7 rows per compute unit: queries at 20,011 x 50 (m = 96) 1.08 / 1.05 / 1.04 /
+    // 0.73, 8,000 x 130 (96) 1.29 / 1.27 / 1.25 / 0.84, 12,000 x 384 (128) 1.08 / 1.05 / 1.01 / 0.85, 50,000 x 384 (192) 1.05 /
+    // 1.04 / 1.02 / 0.82, 100,000 x 768 (256) 1.10 / 1.09 / 1.06 / 0.94, 60,000 x 200 (256) 1.12 / 1.08 / 1.08 / 0.89, 100,000 x
+    // 512 (256) 1.13 / 0.87 / 0.84 / 0.84, 100,000 x 1,536 (256) 1.06 / 0.88 / 0.88 / 0.86, rows of a first loop at 60,000 x 50
+    // (288) 1.39 / 1.35 / 1.32 / 0.85, at 60,000 x 768 with the sketch (256) 1.21 / 1.11 / 1.04 / 0.87.
+    // Aligned rows of up to 128 columns with up to 128 candidates gain less by a share in the fetch, and fewer of them are few:
+    // at 1 / 2 / 3 / 4 per compute unit 4,096 x 128 1.04 / 1.04 / 1.02 / 1.00, 100,000 x 128 in clusters of 977 1.00 / 0.99 / 0.98 /
+    // 0.96, 11,717 x 96 0.98 / 0.98 / 0.98 / 0.94.
+    // With the sketch and more than 768 columns (one iteration per launch) 256 threads are the sooner at 5 / 7 / 9 / 12 / 39 rows per
+    // compute unit too: a first loop's rows at 60,000 x 1,024 (m = 256) 1.02 / 1.03 / 1.06 / 1.08 / 1.06, (m = 288) 1.01 at 5,
+    // 1.05 at 9, 1.06 at 39, at 60,000 x 1,536 (256) 1.05 at 9, 1.06 at 39.
     const int64_t rows_per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits;
+    const bool holds_six = p->dim <= 768 && !(aligned && !sketch && p->dim > 384 && p->dim <= 512);
+    const int64_t few = l.m <= 128 && aligned && p->dim <= 128 ? 2 : holds_six ? 6 : 4;
+    // A chip full of rows with 128 threads is twelve to a compute unit, where their LDS leaves room for so many (taken with half
+    // of a visited list).  Where it does not, rows beyond those that fit take two rounds, and as long as 256 threads take two
+    // as well, those are as soon or sooner for searches that go on for long.  Only with several iterations per launch and without the
+    // sketch, where this was measured.  Queue 128, m = 256 (nine fit), 128 over 256 threads at 9 / 10 / 11 / 12 / 13 / 14 rows per
+    // compute unit: 200,000 x 768 in clusters of 977 0.90 / 1.06 / 1.11 / 1.16 / 1.03 / 1.03, 100,000 x 768 in clusters of 244
+    // (which end after fewer iterations) 0.87 / 0.90 / 0.96 / 1.05 / 0.96 / 0.96; queue 32 (ten fit) 100,000 x 384 0.89 / 0.91 / 0.91 /
+    // 1.01 / 1.00 / 0.99; four of 256 threads: 100,000 x 1,536 0.94 / 0.96 / 0.94 / 0.94 / 0.89 / 0.90.
     const int row_bytes_128 = row_layout((int)l.m, (int)p->queue_length, (int)l.VL, row_hash_slots(l.E / 2, l.m, true), (int)p->excl_cols, true).bytes;
     const int64_t fit_128 = (int64_t)kLdsPerCu / (row_bytes_128 + 640);
-    const bool two_rounds = fit_128 < 12 && rows_per_cu > fit_128 && rows_per_cu <= 14;
+    const bool two_rounds = holds_six && !sketch && !no_windows && p->speculative_readahead >= 2 && fit_128 < 12 &&
+                            rows_per_cu > fit_128 && rows_per_cu <= 12;
     static const int merge_threads_env = [] {
         const char *e = getenv("VL_BEAM_MERGE_THREADS");
         return e ? atoi(e) : 0;
     }();
     const int merge_threads = merge_threads_env ? merge_threads_env
-                              : ((l.m > 320 || p->n_rows <= (l.m <= 128 ? 2 : 4) * kComputeUnits || two_rounds) ? 256 : 128);
+                              : ((l.m > 320 || rows_per_cu <= few || two_rounds || (sketch && p->dim > 768)) ? 256 : 128);
     const int Pmax = a.Ps > a.Pv ? a.Ps : a.Pv;
     const size_t smem = use_sort_merge
         ? (size_t)Pmax * 8 + (size_t)a.L * 4 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4
@@ -880,7 +900,6 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         else if (merge_threads == 128) VL_HIP(vl_allow_lds(beam_merge2_kernel<128>, smem));
         else VL_HIP(vl_allow_lds(beam_merge2_kernel<256>, smem));
     }
-    const bool aligned = (p->dim % 4 == 0) && (((uintptr_t)queries | (uintptr_t)vectors) % 16 == 0);
     StepArgs step;
     step.queries = queries; step.vectors = vectors; step.beams = beams; step.n_vectors = p->n_vectors;
     step.dim = (int)p->dim; step.nchunks = (int)((p->dim + 3) / 4); step.width = (int)p->width;
@@ -954,13 +973,6 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     // Without a sketch windows are faster for every length of a row (10,000 queries at 150,000 rows of 512 columns 7.34 ->
     // 6.68 ms, 1,024 9.26 -> 7.79, 1,536 9.91 -> 9.15, 2,048 12.17 -> 11.74; 1,000 queries 1.46 -> 0.95, 1.67 -> 1.12,
     // 1.82 -> 1.27, 2.00 -> 1.83).
-    // VL_BEAM_WINDOWS / VL_BEAM_NO_WINDOWS in flags, or VL_BEAM_WINDOW=1 / 0 in the environment: windows always / never.
-    static const int window_env = [] {
-        const char *e = getenv("VL_BEAM_WINDOW");
-        return e ? atoi(e) : -1;
-    }();
-    const bool all_windows = window_env >= 0 ? window_env != 0 : (p->flags & VL_BEAM_WINDOWS) != 0;
-    const bool no_windows = window_env >= 0 ? window_env == 0 : (p->flags & VL_BEAM_NO_WINDOWS) != 0;
     constexpr int64_t kL2Bytes = 32 << 20;
     const bool sketch_window = all_windows || (p->dim <= 768 && p->n_vectors * sketch_row_bytes(p->dim) > kL2Bytes);
     const int step_threads = merge_threads == 128 ? 128 : 256;
