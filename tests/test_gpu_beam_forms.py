@@ -1,6 +1,9 @@
 """The forms of the fused beam step against the oracle's loop: one iteration per launch, several per launch, and whatever
 the library picks.  A launch's LDS depends on the rows of the call and on the iteration, so the row counts go from one
-workgroup on the chip to more than it holds at once."""
+workgroup on the chip to more than it holds at once.  A row has 256 threads up to two rows per compute unit (512), where it
+is aligned with at most 128 columns and 128 candidates, up to six (1,536) otherwise (four, 1,024, from 769 columns on), and with
+more than 320 candidates in an iteration; beyond that it has 128, and then a wavefront looks at its candidates in
+every second set of 64 instead of every fourth."""
 import numpy as np
 import pytest
 import torch
@@ -23,9 +26,18 @@ SHAPES = [
     (1, 300, 24, 6, 2, 5),
     (257, 700, 52, 8, 2, 5),      # one row more than compute units
     (700, 700, 256, 16, 2, 5),    # rows of 1 KiB: the sketch
-    (900, 900, 16, 24, 3, 2),     # 288 candidates in 128 threads, a visited list that fills up
+    (900, 900, 16, 24, 3, 2),     # 288 candidates in 256 threads, a visited list that fills up
+    (1600, 1600, 16, 24, 3, 2),   # the same in 128 threads
+    (1600, 1600, 12, 65, 1, 2),   # 260 and 320 candidates in 128 threads: a second and third pass over two sets of 64, begun and full
+    (1600, 1600, 12, 40, 2, 2),
+    (1600, 1600, 10, 65, 1, 2),   # the same, rows that are not aligned
+    (1600, 1600, 10, 40, 2, 2),
     (2300, 2300, 12, 4, 2, 5),    # more rows than the chip holds at once
     (40, 1200, 8, 64, 2, 5),      # 512 candidates, 256 threads
+    (40, 1200, 8, 129, 1, 2),     # 516, 580 and 640 in 256 threads: a second pass, with one set of it and with both
+    (40, 1200, 9, 145, 1, 2),
+    (40, 1200, 8, 80, 2, 2),
+    (40, 1200, 9, 80, 2, 2),
 ]
 
 
@@ -58,17 +70,20 @@ def test_forms_agree_with_the_oracle(rows, n, dim, beam, bqf, ef):
             assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32)), flags
 
 
-@pytest.mark.parametrize("width", [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 97])
-@pytest.mark.parametrize("dim", [40, 128, 130, 300])
-def test_candidate_counts_around_the_sets_of_64(width, dim):
+@pytest.mark.parametrize("rows,width,dim",
+                         [(70, w, d) for d in (40, 128, 130, 300) for w in (1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 97)] +
+                         [(70, w, d) for d in (40, 130) for w in (127, 129, 145, 160, 161)] +
+                         [(1600, w, d) for d in (40, 130) for w in (15, 16, 17, 32, 33, 64, 65, 79, 80)])
+def test_candidate_counts_around_the_sets_of_64(rows, width, dim):
     """Four neighbour lists of `width` ids: the last set of 64 candidates of a wavefront, and its last pair of sets, full,
-    short by one and begun.  Lists share ids and have empty places, so what is left to fetch lies unevenly among the sets."""
-    print(f"beam candidates width={width} dim={dim}", flush=True)
+    short by one and begun; 70 rows have 256 threads, 1,600 have 128.  Lists share ids and have empty places, so what is left to
+    fetch lies unevenly among the sets."""
+    print(f"beam candidates rows={rows} width={width} dim={dim}", flush=True)
     from vectorlink_gpu import Queue
     from vectorlink_gpu.ann import BEAM_NO_CACHE, BEAM_NO_WINDOWS, closest_vectors
 
     rng = np.random.default_rng(width * 1000 + dim)
-    (n, rows, length) = (500, 70, 24)
+    (n, length) = (max(500, rows), 24)
     v = rng.standard_normal((n, dim)).astype(np.float32)
     v /= np.linalg.norm(v, axis=1, keepdims=True)
     table = rng.integers(0, n, (n, width)).astype(np.int32)
@@ -93,17 +108,19 @@ def test_candidate_counts_around_the_sets_of_64(width, dim):
 ODD_DIMS = [1, 3, 5, 50, 62, 65, 127, 130, 253, 259, 383, 386, 511, 514, 766, 1022, 1026, 1279, 1534, 1790, 2045, 2049]
 
 
-@pytest.mark.parametrize("metric", ["cosine", "l2"])
-@pytest.mark.parametrize("dim", ODD_DIMS)
-def test_rows_of_odd_length(dim, metric):
-    """Distances and the loop on rows that do not start on 16-byte boundaries; the last row ends with the table."""
-    print(f"odd rows dim={dim} {metric}", flush=True)
+@pytest.mark.parametrize("n,dim,metric", [(90, d, m) for d in ODD_DIMS for m in ("cosine", "l2")] +
+                         [(1600, d, "cosine" if i % 2 else "l2") for i, d in
+                          enumerate([3, 50, 62, 65, 127, 130, 253, 383, 511, 766, 1022, 1279, 1534, 1790, 2045, 2049])])
+def test_rows_of_odd_length(n, dim, metric):
+    """Distances and the loop on rows that do not start on 16-byte boundaries; the last row ends with the table.  90 rows have
+    256 threads, 1,600 have 128."""
+    print(f"odd rows n={n} dim={dim} {metric}", flush=True)
     from vectorlink_gpu import Queue
     from vectorlink_gpu.ann import closest_vectors, excluding_self
     from vectorlink_gpu.kernels import gather_distances
 
     rng = np.random.default_rng(dim)
-    (n, beam) = (90, 6)
+    beam = 6
     v = rng.standard_normal((n, dim)).astype(np.float32)
     if metric == "cosine":
         v /= np.linalg.norm(v, axis=1, keepdims=True)
@@ -125,8 +142,8 @@ def test_rows_of_odd_length(dim, metric):
     assert np.array_equal(bits(q.distances)[:, :ql], want.distances[:, :ql].view(np.uint32))
 
 
-@pytest.mark.parametrize("rows", [2560, 2561, 3072, 3073])
-@pytest.mark.parametrize("dim", [390, 902])
+@pytest.mark.parametrize("rows,dim", [(r, d) for r in (2560, 2561, 3072, 3073) for d in (390, 902)] +
+                         [(3073, d) for d in (602, 1182, 1410, 1702, 2045)])
 def test_rows_of_odd_length_in_one_round(rows, dim):
     """From 385 columns on, ten, eleven, twelve and thirteen rows per compute unit take different forms of the fetch."""
     print(f"odd rows dim={dim} rows={rows}", flush=True)
