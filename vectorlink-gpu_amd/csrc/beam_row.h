@@ -136,7 +136,8 @@ constexpr int kMemoDecide = 9;
 
 // Elements of a row that one thread brings in at the start of the fused step and keeps in registers until
 // the workgroup's other reads have been issued: search queue, visit queue, visited list.  Longer rows load
-// their remainder the slow way (read, wait, store) - none of the benchmark shapes has one.
+// their remainder the slow way (read, wait, store): a visited list of more than 512 ids in 128 threads has one, which rows of
+// a degree of 35 and more reach late in a call (960 ids at degree 64), and a queue of more than 256 slots.
 constexpr int kPreQ = 2, kPreV = 2, kPreS = 4;
 
 // Takes id's place in an open-addressed set (-1: empty).  False: the id is there already.  The places tried are those of a
