@@ -1,9 +1,9 @@
 """The forms of the fused beam step against the oracle's loop: one iteration per launch, several per launch, and whatever
 the library picks.  A launch's LDS depends on the rows of the call and on the iteration, so the row counts go from one
 workgroup on the chip to more than it holds at once.  A row has 256 threads up to two rows per compute unit (512), where it
-is aligned with at most 128 columns and 128 candidates, up to six (1,536) otherwise (four, 1,024, from 769 columns on), and with
-more than 320 candidates in an iteration; beyond that it has 128, and then a wavefront looks at its candidates in
-every second set of 64 instead of every fourth."""
+is aligned with at most 128 candidates, up to six (1,536) otherwise (four, 1,024, from 769 columns on), and with more than
+320 candidates in an iteration; beyond that it has 128, and then a wavefront looks at its candidates in every second set of
+64 instead of every fourth."""
 import numpy as np
 import pytest
 import torch

@@ -847,19 +847,20 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     // Few are the rows that a compute unit holds at once with 256 threads: six, and four of the shapes whose registers leave four
     // wavefronts per SIMD (aligned rows of 385 to 512 columns without the sketch, rows of more than 768).  Time with 128
     // threads over time with 256 at 4 / 5 / 6 / 7 rows per compute unit: queries at 20,011 x 50 (m = 96) 1.08 / 1.05 / 1.04 /
-    // 0.73, 8,000 x 130 (96) 1.29 / 1.27 / 1.25 / 0.84, 12,000 x 384 (128) 1.08 / 1.05 / 1.01 / 0.85, 50,000 x 384 (192) 1.05 /
-    // 1.04 / 1.02 / 0.82, 100,000 x 768 (256) 1.10 / 1.09 / 1.06 / 0.94, 60,000 x 200 (256) 1.12 / 1.08 / 1.08 / 0.89, 100,000 x
+    // 0.73, 8,000 x 130 (96) 1.29 / 1.27 / 1.25 / 0.84, 50,000 x 384 (192) 1.05 / 1.04 / 1.02 / 0.82,
+    // 100,000 x 768 (256) 1.10 / 1.09 / 1.06 / 0.94, 60,000 x 200 (256) 1.12 / 1.08 / 1.08 / 0.89, 100,000 x
     // 512 (256) 1.13 / 0.87 / 0.84 / 0.84, 100,000 x 1,536 (256) 1.06 / 0.88 / 0.88 / 0.86, rows of a first loop at 60,000 x 50
     // (288) 1.39 / 1.35 / 1.32 / 0.85, at 60,000 x 768 with the sketch (256) 1.21 / 1.11 / 1.04 / 0.87.
-    // Aligned rows of up to 128 columns with up to 128 candidates gain less by a share in the fetch, and fewer of them are few:
-    // at 1 / 2 / 3 / 4 per compute unit 4,096 x 128 1.04 / 1.04 / 1.02 / 1.00, 100,000 x 128 in clusters of 977 1.00 / 0.99 / 0.98 /
-    // 0.96, 11,717 x 96 0.98 / 0.98 / 0.98 / 0.94.
+    // Aligned rows with up to 128 candidates, which dense seeds start near their neighbours, fetch less, and fewer of them are few: at
+    // 1 / 2 / 3 / 4 per compute unit 4,096 x 128 1.04 / 1.04 / 1.02 / 1.00, 100,000 x 128 in clusters of 977 1.00 / 0.99 / 0.98 / 0.96,
+    // 11,717 x 96 0.98 / 0.98 / 0.98 / 0.94; at 4 / 5 / 6 60,000 x 200 in clusters of 244 0.96 / 0.94 / 0.93, x 384 0.96 / 0.95 / 0.94, x
+    // 768 0.97 / 0.96 / 0.96.  (Without clusters more would do: 20,000 x 200 1.20 / 1.17 / 1.14, x 384 1.08 / 1.00 / 0.95, x 768 1.01 / 0.97 / 0.97.)
     // With the sketch and more than 768 columns (one iteration per launch) 256 threads are the sooner at 5 / 7 / 9 / 12 / 39 rows per
     // compute unit too: a first loop's rows at 60,000 x 1,024 (m = 256) 1.02 / 1.03 / 1.06 / 1.08 / 1.06, (m = 288) 1.01 at 5,
     // 1.05 at 9, 1.06 at 39, at 60,000 x 1,536 (256) 1.05 at 9, 1.06 at 39.
     const int64_t rows_per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits;
     const bool holds_six = p->dim <= 768 && !(aligned && !sketch && p->dim > 384 && p->dim <= 512);
-    const int64_t few = l.m <= 128 && aligned && p->dim <= 128 ? 2 : holds_six ? 6 : 4;
+    const int64_t few = l.m <= 128 && aligned ? 2 : holds_six ? 6 : 4;
     // A chip full of rows with 128 threads is twelve to a compute unit, where their LDS leaves room for so many (taken with half
     // of a visited list).  Where it does not, rows beyond those that fit take two rounds, and as long as 256 threads take two
     // as well, those are as soon or sooner for searches that go on for long.  Only with several iterations per launch and without the
