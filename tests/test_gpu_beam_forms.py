@@ -207,10 +207,12 @@ def test_which_calls_with_a_sketch_take_several_iterations_per_launch(n, dim, wi
 
 
 # the cache's size: a slot for every vector and a quarter (819 vectors fit 1,024 slots, 820 do not), 1,024 slots for 3,000
-# vectors of up to 128 columns, which collide; 128 threads a row and 256 on either side of one round of rows (queue 128, LDS
-# for eleven rows of 128 threads per compute unit)
+# vectors of up to 128 columns, which collide; 128 threads a row up to iteration 25 and 256 from there on (eleven rows per
+# compute unit, of which LDS holds eleven, then ten), 256 throughout (twelve), 128 up to iteration 5 (fourteen, and LDS for ten,
+# then nine)
 @pytest.mark.parametrize("rows,n,dim,beam,ef", [(60, 819, 40, 16, 5), (60, 820, 40, 16, 5), (60, 3000, 128, 4, 2),
-                                                (60, 3000, 132, 4, 2), (2816, 2817, 8, 64, 1), (2817, 2817, 8, 64, 1)])
+                                                (60, 3000, 132, 4, 2), (2816, 2817, 8, 64, 1), (2817, 2817, 8, 64, 1),
+                                                (3400, 3401, 8, 72, 1)])
 def test_cache_sizes_and_threads_per_row(rows, n, dim, beam, ef):
     print(f"beam cache and threads rows={rows} n={n} dim={dim} beam={beam}", flush=True)
     from vectorlink_gpu import Queue

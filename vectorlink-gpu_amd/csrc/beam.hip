@@ -847,10 +847,10 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     // Few are the rows that a compute unit holds at once with 256 threads: six, and four of the shapes whose registers leave four
     // wavefronts per SIMD (aligned rows of 385 to 512 columns without the sketch, rows of more than 768).  Time with 128
     // threads over time with 256 at 4 / 5 / 6 / 7 rows per compute unit: queries at 20,011 x 50 (m = 96) 1.08 / 1.05 / 1.04 /
-    // 0.73, 8,000 x 130 (96) 1.29 / 1.27 / 1.25 / 0.84, 50,000 x 384 (192) 1.05 / 1.04 / 1.02 / 0.82,
-    // 100,000 x 768 (256) 1.10 / 1.09 / 1.06 / 0.94, 60,000 x 200 (256) 1.12 / 1.08 / 1.08 / 0.89, 100,000 x
-    // 512 (256) 1.13 / 0.87 / 0.84 / 0.84, 100,000 x 1,536 (256) 1.06 / 0.88 / 0.88 / 0.86, rows of a first loop at 60,000 x 50
-    // (288) 1.39 / 1.35 / 1.32 / 0.85, at 60,000 x 768 with the sketch (256) 1.21 / 1.11 / 1.04 / 0.87.
+    // 0.73, 8,000 x 130 (96) 1.29 / 1.27 / 1.25 / 0.84, 50,000 x 384 (192) 1.05 / 1.04 / 1.02 / 0.82, 100,000 x 768 (256) 1.10 / 1.09 /
+    // 1.06 / 0.94, 60,000 x 200 (256) 1.12 / 1.08 / 1.08 / 0.89, 100,000 x 512 (256) 1.13 / 0.87 / 0.84 / 0.84, 100,000 x 1,536 (256)
+    // 1.06 / 0.88 / 0.88 / 0.86, rows of a first loop at 60,000 x 50 (288) 1.39 / 1.35 / 1.32 / 0.85, at 60,000 x 768 with the sketch
+    // (256) 1.21 / 1.11 / 1.04 / 0.87.
     // Aligned rows with up to 128 candidates, which dense seeds start near their neighbours, fetch less, and fewer of them are few: at
     // 1 / 2 / 3 / 4 per compute unit 4,096 x 128 1.04 / 1.04 / 1.02 / 1.00, 100,000 x 128 in clusters of 977 1.00 / 0.99 / 0.98 / 0.96,
     // 11,717 x 96 0.98 / 0.98 / 0.98 / 0.94; at 4 / 5 / 6 60,000 x 200 in clusters of 244 0.96 / 0.94 / 0.93, x 384 0.96 / 0.95 / 0.94, x
@@ -861,23 +861,12 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     const int64_t rows_per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits;
     const bool holds_six = p->dim <= 768 && !(aligned && !sketch && p->dim > 384 && p->dim <= 512);
     const int64_t few = l.m <= 128 && aligned ? 2 : holds_six ? 6 : 4;
-    // A chip full of rows with 128 threads is twelve to a compute unit, where their LDS leaves room for so many (taken with half
-    // of a visited list).  Where it does not, rows beyond those that fit take two rounds, and as long as 256 threads take two
-    // as well, those are as soon or sooner for searches that go on for long.  Only with several iterations per launch and without the
-    // sketch, where this was measured.  Queue 128, m = 256 (nine fit), 128 over 256 threads at 9 / 10 / 11 / 12 / 13 / 14 rows per
-    // compute unit: 200,000 x 768 in clusters of 977 0.90 / 1.06 / 1.11 / 1.16 / 1.03 / 1.03, 100,000 x 768 in clusters of 244
-    // (which end after fewer iterations) 0.87 / 0.90 / 0.96 / 1.05 / 0.96 / 0.96; queue 32 (ten fit) 100,000 x 384 0.89 / 0.91 / 0.91 /
-    // 1.01 / 1.00 / 0.99; four of 256 threads: 100,000 x 1,536 0.94 / 0.96 / 0.94 / 0.94 / 0.89 / 0.90.
-    const int row_bytes_128 = row_layout((int)l.m, (int)p->queue_length, (int)l.VL, row_hash_slots(l.E / 2, l.m, true), (int)p->excl_cols, true).bytes;
-    const int64_t fit_128 = (int64_t)kLdsPerCu / (row_bytes_128 + 640);
-    const bool two_rounds = holds_six && !sketch && !no_windows && p->speculative_readahead >= 2 && fit_128 < 12 &&
-                            rows_per_cu > fit_128 && rows_per_cu <= 12;
     static const int merge_threads_env = [] {
         const char *e = getenv("VL_BEAM_MERGE_THREADS");
         return e ? atoi(e) : 0;
     }();
     const int merge_threads = merge_threads_env ? merge_threads_env
-                              : ((l.m > 320 || rows_per_cu <= few || two_rounds || (sketch && p->dim > 768)) ? 256 : 128);
+                              : ((l.m > 320 || rows_per_cu <= few || (sketch && p->dim > 768)) ? 256 : 128);
     const int Pmax = a.Ps > a.Pv ? a.Ps : a.Pv;
     const size_t smem = use_sort_merge
         ? (size_t)Pmax * 8 + (size_t)a.L * 4 + (size_t)a.E * 8 + (size_t)a.excl_cols * 4
@@ -976,9 +965,27 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     // 1.82 -> 1.27, 2.00 -> 1.83).
     constexpr int64_t kL2Bytes = 32 << 20;
     const bool sketch_window = all_windows || (p->dim <= 768 && p->n_vectors * sketch_row_bytes(p->dim) > kL2Bytes);
-    const int step_threads = merge_threads == 128 ? 128 : 256;
     const bool use_window = use_fused && !no_windows && R >= 2 && row_hash_slots_most(a.E, a.m) < 0xffff &&
                             smem_window + 2048 <= kLdsPerCu;
+    // Threads of a launch.  With 128 a compute unit holds twelve rows (sixteen of one iteration), where their LDS leaves room
+    // for so many, and that shrinks as the visited lists grow: at queue 128, m = 256 and E = 960 eleven rows fit at first and
+    // eight in the end, sixteen wavefronts, where six rows of 256 threads are 24.  So a call whose rows do not all fit goes
+    // on with 256 threads once no more than three quarters do, or once they do not if both take two rounds (and a compute
+    // unit holds six of 256).  Early launches, and with them searches that end early, keep the rows.
+    // 128 threads throughout / 256 / this (ms), degree 64: 2,800 queries at 20,000 x 256 14.0 / 11.3 / 11.3, x 768 29.0 / 26.1 /
+    // 26.3; 4,096 at x 128 10.7 / 9.7 / 10.0, x 384 21.5 / 20.7 / 20.8, x 512 29.3 / 26.5 / 27.9, x 902 44.0 / 45.8 / 44.9, x 1,282
+    // 67.8 / 59.6 / 64.6; 10,000 at x 64 15.9 / 15.4 / 15.4, x 130 38.5 / 34.5 / 35.5; at 60,000 x 128 in clusters of 244, which end early,
+    // 3.46 / 4.08 / 3.46, x 768 5.47 / 6.02 / 5.48, in clusters of 977 19.48 / 19.88 / 19.48.  (At five sixths, ten rows, the
+    // clusters pay for it: 3.80, 5.83, 19.91.)  Not with the sketch, where it made no difference (2,800 rows of a first loop at
+    // 60,000 x 768 12.97 and 13.02).
+    auto threads_of = [&](int64_t last_iteration, bool windowed) -> int {
+        if (merge_threads != 128) return 256;
+        if (merge_threads_env || step.sketch) return 128;
+        const int64_t visited = l.Vt * last_iteration < l.E ? l.Vt * last_iteration : l.E;
+        const size_t bytes = row_layout(a.m, a.L, a.VL, row_hash_slots(visited, a.m, windowed), a.excl_cols, windowed).bytes + 128;
+        const int64_t fit = (int64_t)(kLdsPerCu / ((bytes + kLdsGranule - 1) / kLdsGranule * kLdsGranule)), most = windowed ? 12 : 16;
+        return rows_per_cu > fit && (4 * fit <= 3 * most || (holds_six && rows_per_cu <= 12)) ? 256 : 128;
+    };
     // A launch's LDS.  The visited ids of its last iteration and the candidates share the hash set, and the emptier it is
     // the sooner each finds its place, so it takes what LDS the workgroups that a compute unit can hold (or that there are)
     // leave it.  Where a batch is one round of such workgroups, their share is counted in the pieces that LDS is handed out in:
@@ -987,12 +994,12 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     // 2,282 and 1,946 us, at 60,000 x 200 1,632 and 1,462, batches of a first loop at 60,000 x 768 (degree 32) 13.4 and 11.4 ms,
     // at 60,000 x 130 14.2 and 9.0; 2,800 (eleven) at 60,000 x 384 (degree 24) 8.0 and 7.3 ms, 60,000 x 256 searched 3,112 and
     // 3,155 us.  A batch of more rounds does better with the larger set (10,000 rows at 60,000 x 768 44.5 and 45.0 ms).
-    auto size_set = [&](int64_t last_iteration, bool windowed) -> size_t {
+    auto size_set = [&](int64_t last_iteration, bool windowed, int threads) -> size_t {
         const int64_t visited = l.Vt * last_iteration < l.E ? l.Vt * last_iteration : l.E;
-        const int waves = step_threads / kWave;
-        const int64_t per_cu = (p->n_rows + kComputeUnits - 1) / kComputeUnits, most_resident = (windowed ? 4 * 6 : 4 * 8) / waves;
-        const int64_t share = per_cu <= most_resident ? (int64_t)(kLdsPerCu / kLdsGranule / per_cu * kLdsGranule)
-                                                     : (int64_t)kLdsPerCu / most_resident;
+        const int waves = threads / kWave;
+        const int64_t most_resident = (windowed ? 4 * 6 : 4 * 8) / waves;
+        const int64_t share = rows_per_cu <= most_resident ? (int64_t)(kLdsPerCu / kLdsGranule / rows_per_cu * kLdsGranule)
+                                                          : (int64_t)kLdsPerCu / most_resident;
         const int least = row_hash_slots(visited, a.m, windowed), most = row_hash_slots_most(visited, a.m);
         const int64_t room = share - 1024 - row_layout(a.m, a.L, a.VL, 0, a.excl_cols, windowed).bytes;
         int64_t slots = (room < 0 ? 0 : room) / 4;
@@ -1009,7 +1016,9 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
             step.m = a;
             const bool windowed = window_fits(t) && (t - 1) % R == 0 && t + R - 1 <= fixed_iterations;
             step.window = windowed ? R : 0;
-            rc = launch_step_by_dim(step, aligned, step_threads, size_set(windowed ? t + R - 1 : t, windowed), st);
+            const int64_t last = windowed ? t + R - 1 : t;
+            const int threads = threads_of(last, windowed);
+            rc = launch_step_by_dim(step, aligned, threads, size_set(last, windowed, threads), st);
             if (rc < 0) return rc;
             t += windowed ? R : 1;
         }
@@ -1057,8 +1066,8 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         step.sketch = ((windowed || t > 0) && want_sketch) ? sketch_table : nullptr;
         step.window = windowed ? R : 0;
         t += windowed ? R : 1;
-        const int e = launch_step_by_dim(step, aligned, step_threads, size_set(t, windowed), st);
-        return e;
+        const int threads = threads_of(t, windowed);
+        return launch_step_by_dim(step, aligned, threads, size_set(t, windowed, threads), st);
     };
     int64_t checked = 0;  // iterations up to the last progress check
     for (;;) {
