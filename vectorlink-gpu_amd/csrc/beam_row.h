@@ -248,6 +248,11 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     // 20,011 x 768 133.1 and 133.7 ms).
     constexpr bool kShortRows = WINDOW && SCPL == 0 && CPL * LPR <= 96;
     constexpr int kAtOnce = kShortRows ? 8 : 1;
+    // Whether a wavefront's sums become distances together (listed_distances).  Of aligned rows those of 129 to 256 columns: 64
+    // lanes bring one row a load, and eight loads wait for eight stores.  Away and together: batches of a first loop at 100,000 x
+    // 200 65.4 -> 63.9 ms (degree 64) and 16.2 -> 15.4 (32), builds of 8,000 x 200 16.2 -> 15.2, 300 / 1,000 / 10,000 queries at
+    // 20,000 x 200 2,950 -> 2,694, 3,194 -> 2,738 (degree 32) and 33,314 -> 32,890 us; clusters of 977 at 60,000 x 256 6,393 -> 6,508.
+    constexpr bool kSums = FORM == kRowUnalignedSums || (FORM == kRowAligned && SCPL == 0 && CPL == 1 && LPR == 64);
     // Sets of 64 candidates of a wavefront whose neighbour ids and cache probes are on their way at a time.  (The kernels with
     // the sketch, which wait on bytes, spill registers with two: a batch of the first loop at 1M x 768 141.0 and 143.1 ms.)
     constexpr int kAhead = SCPL > 0 ? 1 : 2;
@@ -552,7 +557,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                                            s.memo_shift, s.l2 != 0);
                 }
             } else {
-                listed_distances<CPL, LPR, U, THREADS / kWave, FORM != kRowAligned, FORM == kRowUnalignedSums>(
+                listed_distances<CPL, LPR, U, THREADS / kWave, FORM != kRowAligned, kSums>(
                     q_row, s.vectors, s.dim, s.nchunks, li, missed, n_miss, wave, ld, memo_row, s.memo_shift, s.l2 != 0);
             }
         }

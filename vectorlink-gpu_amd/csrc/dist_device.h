@@ -311,7 +311,7 @@ __device__ __forceinline__ void wave_distances_lds(const float *__restrict__ q_r
 // together (us): 1,500 / 10,000 queries at 20,011 x 50 1,404 -> 1,368 and 4,841 -> 4,662, at 20,000 x 130 3,104 -> 2,823 and
 // 11,750 -> 10,750, 1,500 at 30,000 x 390 6,480 -> 5,814, 300 at 30,000 x 902 4,240 -> 3,276, batches of a first loop at
 // 60,000 x 130 32,813 -> 29,617; aligned rows, which mostly do meet them again, 10,000 at 100,000 x 128 5,125 -> 5,233, at
-// 60,000 x 256 10,909 -> 11,102, at 1M x 768 3,217 and 3,210.
+// 60,000 x 256 10,909 -> 11,102, at 1M x 768 3,217 and 3,210.  (Those of 129 to 256 columns park them all the same: kSums in beam_row.h.)
 // Same sums as wave_distances.
 template <int CPL, int LPR, int U, int WAVES, bool UNALIGNED, bool SUMS>
 __device__ __forceinline__ void listed_distances(const float *__restrict__ q_row, const float *__restrict__ vectors, int dim,
