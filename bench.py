@@ -220,7 +220,7 @@ def recall_at(found, truth):
 
 
 def cpu_leg(torch, dev, base_c3, cfg_c3, cpu_rows, gpu_c3_batch):
-    """The CPU oracle as the reported CPU baseline (test infrastructure, timed here as the checker's own speed)."""
+    """The CPU oracle as the reported CPU baseline (test infrastructure, timed here as the oracle's own speed)."""
     from oracle import oracle as orc
     from vectorlink_gpu import ANN, synthetic
 
