@@ -223,6 +223,14 @@ typedef struct vl_beam_params {
  * never. */
 #define VL_BEAM_WINDOWS 32
 #define VL_BEAM_NO_WINDOWS 64
+/* The caller expects many iterations (same loop, same result): a search that
+ * starts anywhere, or a batch of a build.  Such a call is the more likely to be
+ * given the distances of all its queries and vectors ahead of the loop, which
+ * iterations then look up.  VL_BEAM_TABLE: always, where the kernels are built
+ * for the call's sizes, VL_BEAM_NO_TABLE: never. */
+#define VL_BEAM_MANY_ITERATIONS 128
+#define VL_BEAM_TABLE 256
+#define VL_BEAM_NO_TABLE 512
 
 /* Bytes of workspace that serve a call with these parameters.  All but the last
  * part, the distance cache, follows from n_rows, width, beam_size, the queue and
@@ -231,7 +239,10 @@ typedef struct vl_beam_params {
  * n_vectors and dim as well, not always upwards: a larger table may need a
  * smaller cache.  A workspace that was sized with another n_vectors or dim is
  * accepted, and the cache then has the slots that fit; refused is one that could
- * not hold 1,024 per row.  The result does not depend on it. */
+ * not hold 1,024 per row.  Calls that are worth it (VL_BEAM_MANY_ITERATIONS) also
+ * ask for the distances of all their queries and vectors, 4 bytes each and 16 GiB
+ * at most, and copies of both, in the place of the cache; with less than that they
+ * run without.  The result does not depend on it. */
 int64_t vl_beam_workspace_bytes(const vl_beam_params *p);
 
 /* Runs the whole loop of closest_vectors on the search queue in place and

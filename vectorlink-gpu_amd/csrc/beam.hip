@@ -18,6 +18,8 @@
 // iterations, the cadence at which the reference tests for progress
 // (ann.py:68,90-91).
 #include "beam_kernels.h"
+#include "beam_table.h"
+#include "pair_table.h"
 #include <stddef.h>
 #include <stdlib.h>
 #include <atomic>
@@ -117,6 +119,8 @@ __global__ __launch_bounds__(kQueueThreads) void beam_init_kernel(BeamCtrl *ctrl
         ctrl->first[0] = ctrl->first[1] = ctrl->first[2] = 0;
         ctrl->sketch_rows = sketch_rows;
         ctrl->error = 0;
+        ctrl->refused_at = 0;
+        ctrl->unordered = 0;
     }
     if (t < 64) ctrl->changed[t] = 0;
     if (t < kBeamStripes) {
@@ -642,6 +646,9 @@ struct BeamLayout {
     int memo_slots;
     bool may_sketch;     // the call may bring a sketch and use it (as far as its parameters tell: not the rows' addresses)
     bool rows_meet_again;  // what meets_again says
+    // the table of all distances (beam_table.hip) and the copies it is made from, over the cache
+    int use_table;  // TableUse
+    int64_t table_columns, off_packed_queries, off_packed_vectors, off_table, table_end;
 };
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
@@ -661,6 +668,61 @@ constexpr int kLeastCacheSlots = 1024;  // per row, where there is a cache
 inline bool meets_again(int64_t dim, int64_t n_vectors, int64_t asked, bool sketch) {
     if (sketch && dim <= 256) return asked >= 4 * n_vectors;
     return dim <= 128 ? 2 * asked >= 5 * n_vectors : 4 * dim * asked >= 1280 * n_vectors;
+}
+
+// Whether a call is worth the distances of all its queries and vectors ahead of the loop (beam_table.hip), if it runs so many
+// iterations.  Per pair and column they take some 0.02 ps as products (10,000 queries of 20,011 x 768 3.0 ms, 100,000 x 128 3.0),
+// 0.05 ps as squared differences, in whole tiles of queries, and the copies that they are made from 2 ps an element; 50 us
+// are for the launches and for the first iterations, which fill the queues.  An iteration then takes some 11 ps for each candidate of a row (6.8 to 15 measured), 4.5 us at
+// least.  Without them it takes 7.5 us at least, and where the vectors are beyond the chip's L2s 30 ps and 0.08 for each column
+// (batches of 10,000 rows of a first loop at 200,000 x 50 40, x 128 50, x 384 66, x 768 111, 100,003 x 256 55, x 1,536 210), 30
+// otherwise (20,011 x 768 48).
+bool table_pays(const vl_beam_params *p, const BeamLayout &l, double iterations) {
+    const double rows = (double)p->n_rows, candidates = rows * (double)l.m, elements = (double)p->n_vectors * (double)p->dim;
+    const double in_tiles = (double)(pair_tiles(p->n_rows) * kPairTile) * elements;
+    const double made = 50.0 + 0.02 * (double)p->dim + 2e-6 * elements + in_tiles * (p->metric == VL_METRIC_L2 ? 5e-8 : 2e-8);  // us
+    const double with = candidates * 11e-6, without = candidates * (elements > (8 << 20) ? 30e-6 + 0.08e-6 * (double)p->dim : 30e-6);
+    return made + iterations * (with > 4.5 ? with : 4.5) < 0.9 * iterations * (without > 7.5 ? without : 7.5);
+}
+// kTableAsk: if the graph is the one that builds start from.
+//   A batch of a build that says so (VL_BEAM_MANY_ITERATIONS) takes four fifths of the iterations that fill its visited lists and
+// more, a search 85 to 95 (37 to 300 queries), few queries 30; what a call that does not say takes is not known, and ten is
+// what the shortest do.  Batches of a build that come without a word
+// exclude their own ids; those of a first loop run as long as any, those of the later loops find most distances in the cache
+// (10,000 rows of 20,011 x 768 4.0 ms without and 5.6 with the table, of 100,000 x 128 6.0 and 8.5), so the graph itself is
+// looked at.  First loops without and with the table, ms: 10,000 rows of 20,011 x 768 60.2 and 12.6, 50,000 x 768 88.2 and 17.6,
+// 200,000 x 768 138.9 and 39.2, 100,003 x 1,536 263 and 40, 100,000 x 128 15.7 and 6.1, 200,000 x 50 10.8 and 6.1, 60,000 x 200 (L2)
+// 72.9 and 12.5, 1,000 rows of 200,000 x 768 15.8 and 7.0, of 50,000 x 100 1.75 and 1.03.
+enum TableUse { kTableNo, kTableYes, kTableAsk };
+constexpr int64_t kTableMostBytes = 16ll << 30;
+TableUse table_use(const vl_beam_params *p, const BeamLayout &l) {
+    if (p->flags & (VL_BEAM_NO_TABLE | VL_BEAM_TWO_LAUNCHES | VL_BEAM_SORT_MERGE | VL_BEAM_NO_WINDOWS | VL_BEAM_WINDOWS)) return kTableNo;
+    if (l.Vt > kTableMaxVisit || l.VL <= l.Vt || l.VL > kTableMaxQueue || p->queue_length > kTableMaxQueue ||
+        l.m > kTableMaxCandidates || p->excl_cols > kTableMaxExcluded || l.Vt * p->speculative_readahead > l.E || p->dim > 2048)
+        return kTableNo;
+    if (p->n_vectors < kPairTile || p->n_rows * pair_columns(p->n_vectors) * 4 > kTableMostBytes) return kTableNo;
+    if (p->flags & VL_BEAM_TABLE) return kTableYes;
+    if ((p->flags & VL_BEAM_NO_CACHE) && !(p->flags & VL_BEAM_MANY_ITERATIONS)) return kTableNo;  // (asked for a small workspace)
+    if (table_pays(p, l, 10)) return kTableYes;
+    const double all = 0.8 * (double)l.E / (double)l.Vt, search = p->n_rows >= 32 ? 30 : 20;
+    if (!table_pays(p, l, p->excl_cols > 0 || all < search ? all : search)) return kTableNo;
+    if (p->flags & VL_BEAM_MANY_ITERATIONS) return kTableYes;
+    return p->excl_cols > 0 && p->n_rows >= kComputeUnits ? kTableAsk : kTableNo;  // (asking waits for the stream: not for a few rows)
+}
+
+// *circulant = 1 if the neighbours of node i + 1 are those of node i plus one, in a sample of the nodes.
+constexpr int kCirculantNodes = 64;
+__global__ __launch_bounds__(256) void circulant_graph_kernel(const int32_t *__restrict__ beams, int64_t n, int64_t width, int *circulant) {
+    __shared__ int other;
+    if (threadIdx.x == 0) other = 0;
+    __syncthreads();
+    for (int64_t i = threadIdx.x; i < kCirculantNodes * width; i += 256) {
+        const int64_t node = i / width * (n - 1) / kCirculantNodes, k = i % width;
+        const int32_t here = beams[node * width + k], next = beams[(node + 1) * width + k];
+        if (here < 0 || here >= n || next != (here + 1 == n ? 0 : here + 1)) other = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) *circulant = !other;
 }
 
 // lean: the layout of the entry point that allocates nothing - the fused step keeps its candidates in LDS
@@ -736,6 +798,15 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
     l->memo_slots = slots;
     l->off_memo = o; o = align256(o + p->n_rows * (int64_t)slots * 8);
     l->total = o;
+    l->use_table = lean ? kTableNo : table_use(p, *l);
+    l->table_columns = l->off_packed_queries = l->off_packed_vectors = l->off_table = l->table_end = 0;
+    if (l->use_table != kTableNo) {
+        l->table_columns = pair_columns(p->n_vectors);
+        l->off_packed_queries = l->off_memo;
+        l->off_packed_vectors = l->off_packed_queries + pair_packed_bytes(p->n_rows, p->dim);
+        l->off_table = l->off_packed_vectors + pair_packed_bytes(l->table_columns, p->dim);
+        l->table_end = l->off_table + p->n_rows * l->table_columns * 4;
+    }
     return VL_OK;
 }
 
@@ -744,7 +815,7 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
 VL_EXPORT int64_t vl_beam_workspace_bytes(const vl_beam_params *p) {
     BeamLayout l;
     int rc = beam_layout(p, &l);
-    return rc < 0 ? rc : l.total;
+    return rc < 0 ? rc : l.total > l.table_end ? l.total : l.table_end;
 }
 
 namespace {
@@ -928,10 +999,26 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     }
     // with a sketch every row starts out using it (and the cache, when there is one)
     const bool sketch_from_start = step.sketch != nullptr;
-    if (step.sketch) {
-        rc = vl_launch_sketch_queries(queries, p->n_rows, p->dim, (uint8_t *)(ws + l.off_rounded), st);
-        if (rc < 0) return rc;
+    // (neither with the table of all distances)
+    bool table = use_fused && !no_windows && l.use_table != kTableNo && l.table_end <= workspace_bytes;
+    bool prof;
+    {
+        std::lock_guard<std::mutex> hold(g_prof_mutex);
+        prof = g_prof.enabled != 0 && fixed_iterations == 0;
     }
+    // what is counted are the rows that are fetched: a profiled call has the table only where it is asked for
+    if (prof && !(p->flags & (VL_BEAM_MANY_ITERATIONS | VL_BEAM_TABLE))) table = false;
+    auto make_ready = [&]() -> int {
+        if (sketch_from_start) {
+            rc = vl_launch_sketch_queries(queries, p->n_rows, p->dim, (uint8_t *)(ws + l.off_rounded), st);
+            if (rc < 0) return rc;
+        }
+        if (l.memo_slots > 0) {
+            hipLaunchKernelGGL(beam_memo_clear_kernel, dim3(4096), dim3(256), 0, st, memo, p->n_rows * (int64_t)l.memo_slots);
+            VL_LAUNCH_CHECK("beam_memo_clear_kernel");
+        }
+        return VL_OK;
+    };
     {
         int64_t n = p->n_rows * l.VL;
         if (n < kBeamStripes) n = kBeamStripes;
@@ -942,9 +1029,17 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
                            sketch_from_start ? (256 | (1 << 16)) : 256, sketch_from_start ? (int)p->n_rows : 0);
         VL_LAUNCH_CHECK("beam_init_kernel");
     }
-    if (l.memo_slots > 0) {
-        hipLaunchKernelGGL(beam_memo_clear_kernel, dim3(4096), dim3(256), 0, st, memo, p->n_rows * (int64_t)l.memo_slots);
-        VL_LAUNCH_CHECK("beam_memo_clear_kernel");
+    if (table && l.use_table == kTableAsk) {
+        hipLaunchKernelGGL(circulant_graph_kernel, dim3(1), dim3(256), 0, st, beams, p->n_vectors, p->width, &ctrl->circulant);
+        VL_LAUNCH_CHECK("circulant_graph_kernel");
+        int circulant = 0;
+        VL_HIP(hipMemcpyAsync(&circulant, &ctrl->circulant, sizeof(int), hipMemcpyDeviceToHost, st));
+        VL_HIP(hipStreamSynchronize(st));
+        table = circulant != 0;
+    }
+    if (!table) {
+        rc = make_ready();
+        if (rc < 0) return rc;
     }
 
     const int R = (int)p->speculative_readahead;
@@ -1026,11 +1121,6 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         VL_LAUNCH_CHECK("beam_status_kernel");
         return 0;
     }
-    bool prof;
-    {
-        std::lock_guard<std::mutex> hold(g_prof_mutex);
-        prof = g_prof.enabled != 0;
-    }
     step.count_evals = prof ? 1 : 0;
     EventSet events;
     hipEvent_t *ev = events.ev;
@@ -1057,8 +1147,30 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     ReportSlot<StreamOfCall> slot(StreamOfCall{st});
     const bool ahead = use_fused && !prof && slot.get() != nullptr;
     step.report = ahead ? slot.get() : nullptr;
+    TableStepArgs by_table;
+    by_table.beams = beams; by_table.n_vectors = p->n_vectors; by_table.width = step.width; by_table.width_magic = step.width_magic;
+    by_table.table = (uint32_t *)(ws + l.off_table); by_table.columns = l.table_columns; by_table.unordered = &ctrl->unordered;
+    by_table.enter = 1; by_table.window = R; by_table.count_wanted = step.count_evals; by_table.report = step.report;
     auto launch_next = [&]() -> int {  // the fused launch that follows iteration t; moves t on
-        const bool want_sketch = sketch_table && 2 * (int64_t)sketch_rows >= p->n_rows;
+        if (table && t % R == 0 && l.Vt * (t + R) <= l.E) {
+            if (by_table.enter) {
+                rc = vl_launch_pair_table(queries, p->n_rows, vectors, p->n_vectors, p->dim, (int)p->metric,
+                                          (uint8_t *)(ws + l.off_packed_queries), (uint8_t *)(ws + l.off_packed_vectors),
+                                          by_table.table, by_table.columns, &ctrl->unordered, st);
+                if (rc < 0) return rc;
+                step.memo = nullptr;  // the table lies over the cache
+            }
+            a.iter = (int)(t + 1);
+            by_table.m = a;
+            t += R;
+            by_table.raise_fill = l.Vt * (t + R) > l.E;
+            rc = vl_launch_table_step(by_table, st);
+            by_table.enter = 0;
+            g_step_launches.fetch_add(1, std::memory_order_relaxed);
+            return rc;
+        }
+        // (the iterations behind those of the table do without both)
+        const bool want_sketch = sketch_table && !table && 2 * (int64_t)sketch_rows >= p->n_rows;
         const bool windowed = window_fits(t + 1) && t % R == 0 && (!want_sketch || sketch_window);
         a.iter = (int)(t + 1);
         step.m = a;
@@ -1112,26 +1224,28 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
             }
             found = *slot.get();
             // the launch that has nothing left to do is waited for: the caller may use the workspace on another stream
-            if (!found.changed || found.error) {
+            if ((!found.changed && !found.refused_at) || found.error) {
                 VL_HIP(hipStreamSynchronize(st));
                 slot.drained();
             }
         } else {
-            // one copy brings the ring of progress flags and the two words behind it (they are neighbours in the
+            // one copy brings the ring of progress flags and the three words behind it (they are neighbours in the
             // control block): this check's flag, the rows still using the sketch, the error flag
             struct {
                 int changed[64];
-                int sketch_rows, error;
+                int sketch_rows, error, refused_at;
             } seen_by_host;
-            static_assert(offsetof(BeamCtrl, error) - offsetof(BeamCtrl, changed) == 65 * sizeof(int) &&
+            static_assert(offsetof(BeamCtrl, refused_at) - offsetof(BeamCtrl, changed) == 66 * sizeof(int) &&
+                              offsetof(BeamCtrl, error) - offsetof(BeamCtrl, changed) == 65 * sizeof(int) &&
                               offsetof(BeamCtrl, sketch_rows) - offsetof(BeamCtrl, changed) == 64 * sizeof(int),
-                          "changed[64], sketch_rows, error follow each other");
+                          "changed[64], sketch_rows, error, refused_at follow each other");
             VL_HIP(hipMemcpyAsync(&seen_by_host, &ctrl->changed[0], sizeof(seen_by_host), hipMemcpyDeviceToHost, st));
             VL_HIP(hipStreamSynchronize(st));
             slot.drained();
             found.changed = seen_by_host.changed[(checked / R) & 63];
             found.sketch_rows = seen_by_host.sketch_rows;
             found.error = seen_by_host.error;
+            found.refused_at = seen_by_host.refused_at;
         }
         if (sketch_table) sketch_rows = found.sketch_rows;
         if (found.error) {
@@ -1151,6 +1265,18 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
             }
             mine.expand_launches += launches;
             mine.merge_launches += launches;
+        }
+        if (table && found.refused_at) {
+            // the launches from iteration refused_at on did nothing: the loop goes on from there without the table
+            table = false;
+            step.memo = l.memo_slots > 0 ? memo : nullptr;
+            rc = make_ready();
+            if (rc < 0) return rc;
+            t = found.refused_at - 1;
+            if (ahead) slot.forget();  // (a check may be made again)
+            const bool checked_there = t == checked;
+            checked = t;
+            if (!checked_there) continue;
         }
         if (!found.changed) break;  // ann.py:90-91
         if (checked > t_limit) {

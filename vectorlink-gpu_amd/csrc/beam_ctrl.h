@@ -29,6 +29,9 @@ struct BeamCtrl {
     int sketch_rows;    // rows that currently look at their candidates through the 8-bit sketch first
     int error;          // set by a row whose visited-list fill is beyond what the iteration count allows: the
                         // workspace was overwritten while the loop ran (VL_ERR_STATE on the host)
+    int refused_at;     // iteration that found the call's table of distances of no use (beam_table.hip), or 0
+    int unordered;      // that table holds a distance that is not an ordinary number
+    int circulant;      // the graph is the one that builds start from (found out before the loop, where it matters)
     // profiling only, striped by workgroup so that the atomic adds do not queue up on one address:
     unsigned long long evals[kBeamStripes];   // candidate rows actually fetched
     unsigned long long wanted[kBeamStripes];  // candidate distances asked for (fetched or served by the cache)
@@ -39,6 +42,7 @@ __device__ inline void beam_report(const BeamCtrl *c, int t, int R, BeamReport *
     out->changed = c->changed[(t / R) & 63];
     out->sketch_rows = c->sketch_rows;
     out->error = c->error;
+    if (c->refused_at) out->refused_at = c->refused_at;  // (0 when the call took the slot; each word is a trip to the host's memory)
     __hip_atomic_store(&out->check, t, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

@@ -11,7 +11,7 @@
 #include <thread>
 
 struct BeamReport {
-    int changed, sketch_rows, error;  // as in BeamCtrl, after the checking iteration
+    int changed, sketch_rows, error, refused_at;  // as in BeamCtrl, after the checking iteration
     int check;                        // written last: iterations run up to that check
 };
 
@@ -30,7 +30,7 @@ public:
             if (!((lent_ >> i) & 1)) {
                 lent_ |= 1ull << i;
                 index_ = i;
-                page_[i].report.check = 0;
+                page_[i].report.check = page_[i].report.refused_at = 0;
                 break;
             }
     }
@@ -44,6 +44,7 @@ public:
     ReportSlot &operator=(const ReportSlot &) = delete;
 
     BeamReport *get() const { return index_ < 0 ? nullptr : &page_[index_].report; }
+    void forget() { __atomic_store_n(&page_[index_].report.check, 0, __ATOMIC_RELAXED); }  // the last report, with no launch left that reports
     void launching() { running_ = true; }  // before anything of the call goes to the stream
     void drained() { running_ = false; }   // the stream has been waited for
 

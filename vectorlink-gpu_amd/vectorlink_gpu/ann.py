@@ -30,6 +30,9 @@ BEAM_NO_CACHE = 8  # include/vlgpu.h: VL_BEAM_NO_CACHE (no per-row cache of eval
 BEAM_USES_SKETCH = 16  # include/vlgpu.h: VL_BEAM_USES_SKETCH (set by closest_vectors when it is given a sketch)
 BEAM_WINDOWS = 32  # include/vlgpu.h: VL_BEAM_WINDOWS (several iterations per launch wherever rows are independent; same result)
 BEAM_NO_WINDOWS = 64  # include/vlgpu.h: VL_BEAM_NO_WINDOWS (one iteration per launch; same result)
+BEAM_MANY_ITERATIONS = 128  # include/vlgpu.h: VL_BEAM_MANY_ITERATIONS (the loop is expected to be a long one; same result)
+BEAM_TABLE = 256  # include/vlgpu.h: VL_BEAM_TABLE (all distances ahead of the loop wherever that is built; same result)
+BEAM_NO_TABLE = 512  # include/vlgpu.h: VL_BEAM_NO_TABLE (never; same result)
 
 
 def _beam_params(batch: int, dim: int, n_vectors: int, width: int, queue: Queue, config: Dict,
@@ -174,7 +177,16 @@ def closest_vectors(query_vecs: Tensor, search_queue: Queue, vectors: Tensor, be
     need = nv.check(nv.lib().vl_beam_workspace_bytes(ctypes.byref(p)))
     workspace = _workspace(vectors.device)
     with workspace.lock:
-        ws = workspace.reserve(need, vectors.device)
+        try:
+            ws = workspace.reserve(need, vectors.device)
+        except torch.OutOfMemoryError:
+            # what the call takes without the distances of all its queries and vectors, which it runs without then
+            least = nv.check(nv.lib().vl_beam_workspace_bytes(ctypes.byref(
+                _beam_params(batch, dim, vectors.size(0), beams.size(1), search_queue, config, p.excl_cols,
+                             p.flags | BEAM_NO_TABLE))))
+            if least >= need:
+                raise
+            ws = workspace.reserve(least, vectors.device)
         if sketch is not None:
             assert sketch.dtype == torch.uint8 and sketch.is_contiguous() and sketch.is_cuda
             assert sketch.size() == (vectors.size(0), sketch_row_bytes(dim)), "not a sketch of these vectors"
@@ -266,6 +278,8 @@ class GraphBuild:
                 end = min(start + batch_size, self.num_vecs)
                 with torch.cuda.stream(stream):
                     exclude = excluding_self(start, end, ql, device)
+                    # (searches of the circulant graph, whose edges lead anywhere, are long ones)
+                    first = BEAM_MANY_ITERATIONS if loop == 0 and self.circulant_start and not self.stale else 0
                     queue = Queue(end - start, ql, ql + remaining_capacity, device=device)
                     queue.insert(self.beams.narrow(0, start, end - start), seed_distances.narrow(0, start, end - start))
                     if self.sketch is not None:
@@ -273,11 +287,13 @@ class GraphBuild:
                         # candidates twice (27 % at 1M x 768): with short sketch rows the cache's probes cost
                         # more than those repeats save, with long ones less (per launch, without and with the
                         # cache: 0.35 and 0.37 ms at 384 columns, 0.73 and 0.64 ms at 768, 1.54 and 1.24 ms at 1536)
-                        first = BEAM_NO_CACHE if (loop == 0 and self.circulant_start and vectors.size(1) <= 512) else 0
+                        if first and vectors.size(1) <= 512:
+                            first |= BEAM_NO_CACHE
                         t = search(vectors[start:end], queue, vectors, self.beams, config, exclude, flags=first,
                                    sketch=self.sketch)
                     else:
-                        t = search(vectors[start:end], queue, vectors, self.beams, config, exclude)
+                        t = search(vectors[start:end], queue, vectors, self.beams, config, exclude,
+                                   **({"flags": first} if first else {}))
                     next_beams.narrow(0, start, end - start).copy_(queue.indices.narrow(1, 0, ql))
                     next_beam_distances.narrow(0, start, end - start).copy_(queue.distances.narrow(1, 0, ql))
                     stream.synchronize()
@@ -716,8 +732,11 @@ class ANN:
                                               queue_size, self.dense_seeds)
         else:
             search_queue = initial_search_queue(self.vectors, query, self.configuration, queue_size)
-        closest_vectors(query, search_queue, self.vectors, self.beams, self.configuration, None,
-                        flags=BEAM_PER_QUERY_STOP if stop == "per_query" else 0, sketch=self._search_sketch(sketch))
+        flags = BEAM_PER_QUERY_STOP if stop == "per_query" else 0
+        if seeding == "circulant":  # seeds from anywhere
+            flags |= BEAM_MANY_ITERATIONS
+        closest_vectors(query, search_queue, self.vectors, self.beams, self.configuration, None, flags=flags,
+                        sketch=self._search_sketch(sketch))
         return search_queue
 
     def recall_at_k(self, query: Tensor, k: int = 10, queue_size: Optional[int] = None,
