@@ -676,18 +676,18 @@ inline bool meets_again(int64_t dim, int64_t n_vectors, int64_t asked, bool sket
 // are for the launches and for the first iterations, which fill the queues.  An iteration then takes some 11 ps for each candidate of a row (6.8 to 15 measured), 4.5 us at
 // least.  Without them it takes 7.5 us at least, and where the vectors are beyond the chip's L2s 30 ps and 0.08 for each column
 // (batches of 10,000 rows of a first loop at 200,000 x 50 40, x 128 50, x 384 66, x 768 111, 100,003 x 256 55, x 1,536 210), 30
-// otherwise (20,011 x 768 48).
-bool table_pays(const vl_beam_params *p, const BeamLayout &l, double iterations) {
+// otherwise (20,011 x 768 48); on a graph of near neighbours, where most distances are in the cache, 20 (20,011 x 768 22).
+bool table_pays(const vl_beam_params *p, const BeamLayout &l, double iterations, double candidate_ps) {
     const double rows = (double)p->n_rows, candidates = rows * (double)l.m, elements = (double)p->n_vectors * (double)p->dim;
     const double in_tiles = (double)(pair_tiles(p->n_rows) * kPairTile) * elements;
     const double made = 50.0 + 0.02 * (double)p->dim + 2e-6 * elements + in_tiles * (p->metric == VL_METRIC_L2 ? 5e-8 : 2e-8);  // us
-    const double with = candidates * 11e-6, without = candidates * (elements > (8 << 20) ? 30e-6 + 0.08e-6 * (double)p->dim : 30e-6);
+    const double with = candidates * 11e-6, without = candidates * candidate_ps * 1e-6;
     return made + iterations * (with > 4.5 ? with : 4.5) < 0.9 * iterations * (without > 7.5 ? without : 7.5);
 }
 // kTableAsk: if the graph is the one that builds start from.
 //   A batch of a build that says so (VL_BEAM_MANY_ITERATIONS) takes four fifths of the iterations that fill its visited lists and
-// more, a search 85 to 95 (37 to 300 queries), few queries 30; what a call that does not say takes is not known, and ten is
-// what the shortest do.  Batches of a build that come without a word
+// more, a search 85 to 95 (37 to 300 queries), few queries 30; what a call that does not say takes is not known: 15 to 125, and
+// 20 are counted on.  Batches of a build that come without a word
 // exclude their own ids; those of a first loop run as long as any, those of the later loops find most distances in the cache
 // (10,000 rows of 20,011 x 768 4.0 ms without and 5.6 with the table, of 100,000 x 128 6.0 and 8.5), so the graph itself is
 // looked at.  First loops without and with the table, ms: 10,000 rows of 20,011 x 768 60.2 and 12.6, 50,000 x 768 88.2 and 17.6,
@@ -703,9 +703,10 @@ TableUse table_use(const vl_beam_params *p, const BeamLayout &l) {
     if (p->n_vectors < kPairTile || p->n_rows * pair_columns(p->n_vectors) * 4 > kTableMostBytes) return kTableNo;
     if (p->flags & VL_BEAM_TABLE) return kTableYes;
     if ((p->flags & VL_BEAM_NO_CACHE) && !(p->flags & VL_BEAM_MANY_ITERATIONS)) return kTableNo;  // (asked for a small workspace)
-    if (table_pays(p, l, 10)) return kTableYes;
+    if (table_pays(p, l, 20, 20)) return kTableYes;
     const double all = 0.8 * (double)l.E / (double)l.Vt, search = p->n_rows >= 32 ? 30 : 20;
-    if (!table_pays(p, l, p->excl_cols > 0 || all < search ? all : search)) return kTableNo;
+    const double anywhere = p->n_vectors * p->dim > (8 << 20) ? 30 + 0.08 * (double)p->dim : 30;
+    if (!table_pays(p, l, p->excl_cols > 0 || all < search ? all : search, anywhere)) return kTableNo;
     if (p->flags & VL_BEAM_MANY_ITERATIONS) return kTableYes;
     return p->excl_cols > 0 && p->n_rows >= kComputeUnits ? kTableAsk : kTableNo;  // (asking waits for the stream: not for a few rows)
 }
