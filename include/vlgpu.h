@@ -148,6 +148,20 @@ int vl_queue_insert(int32_t *q_ids, float *q_dists, int64_t rows, int64_t capaci
                     int64_t m, const int32_t *excl, int64_t excl_cols,
                     uint8_t *changed, void *stream);
 
+/* The search queue that a search starts from (ann.py:217-232) in one launch: what
+ * vl_gather_distances_metric and vl_queue_insert make of a queue of empty pairs.
+ * seeds: ids [n_rows, n_seeds], or with names != NULL places in it (names[place]
+ * is the id; a place outside is an empty seed); circulant: n_seeds numbers, and
+ * the seeds of row r are (r + number) % n_vectors (utils.py:26-32).  Writes all
+ * `capacity` slots of a row.  length: the queue's .length, behind which the
+ * seeds have to fit. */
+int vl_seed_queue(const float *queries, int64_t n_rows, const float *vectors,
+                  int64_t n_vectors, int64_t dim, int metric,
+                  const int32_t *seeds, int64_t n_seeds, int circulant,
+                  const int32_t *names, int64_t n_names,
+                  int32_t *q_ids, float *q_dists, int64_t capacity,
+                  int64_t length, void *stream);
+
 /* Queue.pop_n_ids (queue.py:87-95): out[r, 0:take) = ids[r, 0:take); those
  * slots become the empty pair; nothing is re-sorted. */
 int vl_queue_pop(int32_t *q_ids, float *q_dists, int64_t rows, int64_t capacity,

@@ -22,6 +22,7 @@
 #include "pair_table.h"
 #include <stddef.h>
 #include <stdlib.h>
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -99,20 +100,21 @@ __device__ inline int lower_bound(const int32_t *a, int n, int32_t v) {
     return lo;
 }
 
+constexpr uint64_t kMemoEmpty = (uint64_t)(uint32_t)VL_MAXINT;  // id VL_MAXINT, which no probe asks for
 __global__ void beam_memo_clear_kernel(uint64_t *memo, int64_t n) {
-    // an empty slot holds id VL_MAXINT, which no probe asks for
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        memo[i] = (uint64_t)(uint32_t)VL_MAXINT;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) memo[i] = kMemoEmpty;
 }
 
-// row_word: what every row starts with in its word of the memo_rate array (StepArgs); sketch_rows: how many rows
+// memo: the cache, cleared here as well, or null (a launch of its own is some 10 us to one query).  row_word: what every row starts with in its word of the memo_rate array (StepArgs); sketch_rows: how many rows
 // that makes users of the sketch.
 __global__ __launch_bounds__(kQueueThreads) void beam_init_kernel(BeamCtrl *ctrl, int64_t n_rows, const int32_t *q_ids,
                                                                  const float *q_d, int cap, int head, int32_t *v_ids,
                                                                  float *v_d, int VL, int32_t *seen_count,
                                                                  int32_t *row_quiet, int32_t *memo_rate, int row_word,
-                                                                 int sketch_rows) {
+                                                                 int sketch_rows, uint64_t *memo, int64_t memo_slots) {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (memo)
+        for (int64_t i = t; i < memo_slots; i += (int64_t)gridDim.x * blockDim.x) memo[i] = kMemoEmpty;
     if (t == 0) {
         ctrl->stop = 0;
         ctrl->ended_after = 0;
@@ -1009,13 +1011,14 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     }
     // what is counted are the rows that are fetched: a profiled call has the table only where it is asked for
     if (prof && !(p->flags & (VL_BEAM_MANY_ITERATIONS | VL_BEAM_TABLE))) table = false;
-    auto make_ready = [&]() -> int {
+    const int64_t all_slots = p->n_rows * (int64_t)l.memo_slots;
+    auto make_ready = [&](bool clear) -> int {  // what a loop without the table needs
         if (sketch_from_start) {
             rc = vl_launch_sketch_queries(queries, p->n_rows, p->dim, (uint8_t *)(ws + l.off_rounded), st);
             if (rc < 0) return rc;
         }
-        if (l.memo_slots > 0) {
-            hipLaunchKernelGGL(beam_memo_clear_kernel, dim3(4096), dim3(256), 0, st, memo, p->n_rows * (int64_t)l.memo_slots);
+        if (clear && all_slots > 0) {
+            hipLaunchKernelGGL(beam_memo_clear_kernel, dim3(4096), dim3(256), 0, st, memo, all_slots);
             VL_LAUNCH_CHECK("beam_memo_clear_kernel");
         }
         return VL_OK;
@@ -1024,13 +1027,21 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         int64_t n = p->n_rows * l.VL;
         if (n < kBeamStripes) n = kBeamStripes;
         if (n < p->n_rows) n = p->n_rows;
-        hipLaunchKernelGGL(beam_init_kernel, dim3((unsigned)((n + kQueueThreads - 1) / kQueueThreads)),
+        int64_t blocks = (n + kQueueThreads - 1) / kQueueThreads;
+        const bool clear = !table && all_slots > 0;
+        if (clear) {  // eight slots a thread, up to 4,096 workgroups
+            const int64_t wanted = (all_slots + 8 * kQueueThreads - 1) / (8 * kQueueThreads);
+            blocks = std::max(blocks, std::min<int64_t>(wanted, 4096));
+        }
+        hipLaunchKernelGGL(beam_init_kernel, dim3((unsigned)blocks),
                            dim3(kQueueThreads), 0, st, ctrl, p->n_rows, q_ids, q_dists, (int)p->queue_capacity,
                            (int)l.head, v_ids, v_d, (int)l.VL, seen_count, row_quiet, (int32_t *)(ws + l.off_memo_rate),
-                           sketch_from_start ? (256 | (1 << 16)) : 256, sketch_from_start ? (int)p->n_rows : 0);
+                           sketch_from_start ? (256 | (1 << 16)) : 256, sketch_from_start ? (int)p->n_rows : 0,
+                           clear ? memo : nullptr, all_slots);
         VL_LAUNCH_CHECK("beam_init_kernel");
     }
-    if (table && l.use_table == kTableAsk) {
+    const bool asked = table && l.use_table == kTableAsk;
+    if (asked) {
         hipLaunchKernelGGL(circulant_graph_kernel, dim3(1), dim3(256), 0, st, beams, p->n_vectors, p->width, &ctrl->circulant);
         VL_LAUNCH_CHECK("circulant_graph_kernel");
         int circulant = 0;
@@ -1039,7 +1050,7 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         table = circulant != 0;
     }
     if (!table) {
-        rc = make_ready();
+        rc = make_ready(asked);
         if (rc < 0) return rc;
     }
 
@@ -1271,7 +1282,7 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
             // the launches from iteration refused_at on did nothing: the loop goes on from there without the table
             table = false;
             step.memo = l.memo_slots > 0 ? memo : nullptr;
-            rc = make_ready();
+            rc = make_ready(true);
             if (rc < 0) return rc;
             t = found.refused_at - 1;
             if (ahead) slot.forget();  // (a check may be made again)

@@ -51,6 +51,8 @@ _SIGNATURES = {
     "vl_punchout_duplicates": (C.c_int, [_ptr, _ptr, _i64, _i64, _ptr]),
     "vl_queue_sort": (C.c_int, [_ptr, _ptr, _i64, _i64, _ptr]),
     "vl_queue_insert": (C.c_int, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
+    "vl_seed_queue": (C.c_int, [_ptr, _i64, _ptr, _i64, _i64, C.c_int, _ptr, _i64, C.c_int, _ptr, _i64, _ptr, _ptr, _i64, _i64,
+                                _ptr]),
     "vl_queue_pop": (C.c_int, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr]),
     "vl_seen_add": (C.c_int, [_ptr, _i64, _i64, _ptr, _i64, _ptr, C.POINTER(C.c_int), _ptr]),
     "vl_beam_workspace_bytes": (C.c_int64, [C.POINTER(BeamParams)]),

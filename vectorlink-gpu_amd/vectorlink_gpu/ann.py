@@ -20,7 +20,8 @@ from .kernels import (build_sketch, calculate_distances, gather_distances, knn_e
 from . import log as _log
 from .log import log_time
 from .queue import Queue
-from .utils import add_new_to_seen_, generate_circulant_beams, generate_queue_circulants, primes
+from .utils import (add_new_to_seen_, generate_circulant_beams, generate_queue_circulants,  # noqa: F401
+                    primes)
 
 
 BEAM_TWO_LAUNCHES = 1  # include/vlgpu.h: VL_BEAM_TWO_LAUNCHES
@@ -406,15 +407,10 @@ def initial_search_queue(vectors: Tensor, query_vectors: Tensor, config: Dict,
     """reference ann.py:217-232; queue_size overrides recall_search_queue_factor * beam_size"""
     if queue_size is None:
         queue_size = config["recall_search_queue_factor"] * config["beam_size"]
-    (batch_size, _) = query_vectors.size()
     extra_capacity = max(queue_size, config["parallel_visit_count"] * config["beam_size"])
-    queue = Queue(batch_size, queue_size, queue_size + extra_capacity, device=vectors.device)
-    p = primes(queue_size, vectors.device)
-    (vector_count, _) = vectors.size()
-    initial_queue_indices = generate_queue_circulants(batch_size, vector_count, p)
-    d = query_cosine_distances(query_vectors, vectors, initial_queue_indices, config.get("metric", "cosine"))
-    queue.insert(initial_queue_indices, d)
-    return queue
+    # (seeds (b + p) % N, their distances and the insert in one launch)
+    return Queue.seeded(queue_size, queue_size + extra_capacity, query_vectors, vectors, primes(queue_size, vectors.device),
+                        config.get("metric", "cosine"))
 
 
 DENSE_SEEDS = 16  # seeds per query taken from the entry-point tiles (the exact-kNN kernel keeps 16 per lane)
@@ -440,17 +436,13 @@ def dense_search_queue(vectors: Tensor, query_vectors: Tensor, config: Dict, ent
     initial_search_queue (ann.py:217-232); slots beyond the seeds start empty."""
     if queue_size is None:
         queue_size = config["recall_search_queue_factor"] * config["beam_size"]
-    (batch_size, _) = query_vectors.size()
     extra_capacity = max(queue_size, config["parallel_visit_count"] * config["beam_size"])
-    queue = Queue(batch_size, queue_size, queue_size + extra_capacity, device=vectors.device)
     k = min(seeds or DENSE_SEEDS, DENSE_SEEDS, entry_ids.size(0), queue_size)
     cols = entry_vectors.size(1)
     ranked_by = query_vectors if cols == query_vectors.size(1) else query_vectors[:, :cols].contiguous()
     (local, _) = knn_exact(ranked_by, entry_vectors, k, config.get("metric", "cosine"))
-    seeds = entry_ids[local.long()].contiguous()
-    d = query_cosine_distances(query_vectors, vectors, seeds, config.get("metric", "cosine"))
-    queue.insert(seeds, d)
-    return queue
+    return Queue.seeded(queue_size, queue_size + extra_capacity, query_vectors, vectors, local, config.get("metric", "cosine"),
+                        names=entry_ids)
 
 
 def _flags_for_sample(sample: Tensor, vectors: Tensor) -> int:
