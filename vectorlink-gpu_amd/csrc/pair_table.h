@@ -53,7 +53,7 @@ static inline int64_t pair_columns(int64_t n_vectors) { return pair_tiles(PairCo
 
 // out[r * columns + PairColumns(n_vectors).of(v)] = distance of queries[r] and vectors[v] as bits (columns of no vector hold
 // values nobody asks for).  *unordered becomes 1 if a distance may not be a number below VL_MAXFLOAT.
-// packed_queries / packed_vectors: room for the copies (pair_packed_bytes of n_queries and of pair_columns), 1 KiB aligned.
+// packed_queries / packed_vectors: room for the copies (pair_packed_bytes of n_queries and of pair_columns), 16-byte aligned.
 // Nothing is allocated or waited for.
 int vl_launch_pair_table(const float *queries, int64_t n_queries, const float *vectors, int64_t n_vectors, int64_t dim,
                          int metric, uint8_t *packed_queries, uint8_t *packed_vectors, uint32_t *out, int64_t columns,

@@ -1,7 +1,7 @@
 // The search queue that a search starts from (ann.py:217-232), in one launch: a row's seeds, their distances, and the queue row
 // that Queue.insert (queue.py:37-61) makes of them when nothing is queued yet.  As single steps - two fills, seeds, distances, the
 // insert, for dense seeds also the translation of entry points to ids - each of them is some 5 us of work behind 10 to 30 us
-// of the host's, and a search of one query waits for all of them (FIXME).
+// of the host's, and a search of one query waits for all of them (one query at 100,000 x 768 222 us so, 167 in one launch).
 #include "dist_device.h"
 #include "rowsort.h"
 
