@@ -245,6 +245,10 @@ typedef struct vl_beam_params {
 #define VL_BEAM_MANY_ITERATIONS 128
 #define VL_BEAM_TABLE 256
 #define VL_BEAM_NO_TABLE 512
+/* Such a call with a sketch, too large for all distances, may be given bounds of
+ * all of them instead.  VL_BEAM_BOUNDS: always, where the call can use a sketch
+ * and has no such table; VL_BEAM_NO_TABLE: never. */
+#define VL_BEAM_BOUNDS 1024
 
 /* Bytes of workspace that serve a call with these parameters.  All but the last
  * part, the distance cache, follows from n_rows, width, beam_size, the queue and
@@ -255,8 +259,8 @@ typedef struct vl_beam_params {
  * accepted, and the cache then has the slots that fit; refused is one that could
  * not hold 1,024 per row.  Calls that are worth it (VL_BEAM_MANY_ITERATIONS) also
  * ask for the distances of all their queries and vectors, 4 bytes each and 16 GiB
- * at most, and copies of both, in the place of the cache; with less than that they
- * run without.  The result does not depend on it. */
+ * at most, and copies of both, in the place of the cache, or behind it for 2 bytes
+ * of bounds each and copies, 24 GiB at most; with less than that they run without.  The result does not depend on it. */
 int64_t vl_beam_workspace_bytes(const vl_beam_params *p);
 
 /* Runs the whole loop of closest_vectors on the search queue in place and

@@ -651,6 +651,10 @@ struct BeamLayout {
     // the table of all distances (beam_table.hip) and the copies it is made from, over the cache
     int use_table;  // TableUse
     int64_t table_columns, off_packed_queries, off_packed_vectors, off_table, table_end;
+    // or the bounds of all of them (near_products.h), behind the cache
+    int use_near;  // TableUse
+    NearPlan near_plan;
+    int64_t off_near, near_end;
 };
 
 inline int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
@@ -711,6 +715,27 @@ TableUse table_use(const vl_beam_params *p, const BeamLayout &l) {
     if (!table_pays(p, l, p->excl_cols > 0 || all < search ? all : search, anywhere)) return kTableNo;
     if (p->flags & VL_BEAM_MANY_ITERATIONS) return kTableYes;
     return p->excl_cols > 0 && p->n_rows >= kComputeUnits ? kTableAsk : kTableNo;  // (asking waits for the stream: not for a few rows)
+}
+
+// Whether a call whose table of distances would be too large or too much work is given the products of all its queries and vectors in
+// bfloat16 instead (near_products.h), where it would use the sketch: batches of a first loop, as above.  The products take 2 fs a
+// column, storing them 0.4 ps a pair, the copies 1.5 ps an element; an iteration then takes 24 + 0.016 ps a column for each
+// candidate, through the sketch 2 + 0.155.  Without and with, ms, 10,000 rows: 1M x 768 140 and 60, 500,000 x 1,024 200 and 61, x 1,536
+// 306 and 85, x 256 55.1 and 41.4, 1M x 384 (degree 48) 43.5 and 37.9, x 256 (degree 32: left alone) 14.3 and 20.5; 1,000 rows of 1M x
+// 768 15.9 and 8.8, 300 of 500,000 x 768 10.6 and 6.2.  The cache is left out: 62.8 ms for the first with it.
+constexpr int64_t kNearMostBytes = 24ll << 30;
+TableUse near_use(const vl_beam_params *p, const BeamLayout &l) {
+    if (!l.may_sketch || l.use_table != kTableNo || p->speculative_readahead < 2) return kTableNo;
+    if (p->flags & (VL_BEAM_NO_TABLE | VL_BEAM_NO_WINDOWS | VL_BEAM_WINDOWS)) return kTableNo;  // (it runs several iterations per launch)
+    if (l.near_plan.bytes > kNearMostBytes) return kTableNo;
+    if (p->flags & VL_BEAM_BOUNDS) return kTableYes;
+    const double rows = (double)p->n_rows, pairs = rows * (double)p->n_vectors, candidates = rows * (double)l.m;
+    const double made = 60.0 + pairs * (2.2e-9 * (double)p->dim + 4e-7) + 1.5e-6 * (double)p->n_vectors * (double)p->dim;  // us
+    const double iterations = 0.8 * (double)l.E / (double)l.Vt;
+    const double saved = iterations * candidates * (0.139 * (double)p->dim - 22.0) * 1e-6;
+    if (made > 0.8 * saved) return kTableNo;
+    if (p->flags & VL_BEAM_MANY_ITERATIONS) return p->excl_cols > 0 ? kTableYes : kTableNo;
+    return p->excl_cols > 0 && p->n_rows >= kComputeUnits ? kTableAsk : kTableNo;
 }
 
 // *circulant = 1 if the neighbours of node i + 1 are those of node i plus one, in a sample of the nodes.
@@ -810,6 +835,16 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
         l->off_table = l->off_packed_vectors + pair_packed_bytes(l->table_columns, p->dim);
         l->table_end = l->off_table + p->n_rows * l->table_columns * 4;
     }
+    l->use_near = kTableNo;
+    l->off_near = l->near_end = 0;
+    if (!lean && l->may_sketch) {
+        l->near_plan = vl_near_plan(p->n_rows, p->n_vectors, p->dim);
+        l->use_near = near_use(p, *l);
+        if (l->use_near != kTableNo) {
+            l->off_near = l->total;
+            l->near_end = l->off_near + l->near_plan.bytes;
+        }
+    }
     return VL_OK;
 }
 
@@ -818,7 +853,7 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
 VL_EXPORT int64_t vl_beam_workspace_bytes(const vl_beam_params *p) {
     BeamLayout l;
     int rc = beam_layout(p, &l);
-    return rc < 0 ? rc : l.total > l.table_end ? l.total : l.table_end;
+    return rc < 0 ? rc : std::max(l.total, std::max(l.table_end, l.near_end));
 }
 
 namespace {
@@ -988,6 +1023,7 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
                "a call with a sketch needs VL_BEAM_USES_SKETCH in flags (and a workspace sized with it)");
     step.rounded_queries = (const uint8_t *)(ws + l.off_rounded);
     step.rounded_query_bytes = sketch_query_bytes(p->dim);
+    step.near_values = nullptr;
     step.sketch_tails = sketch ? sketch + sketch_tails_offset(p->n_vectors, p->dim) : nullptr;
     step.sketch_chunks = (int)sketch_data_chunks(p->dim);
     step.window = 0;
@@ -1011,24 +1047,30 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     }
     // what is counted are the rows that are fetched: a profiled call has the table only where it is asked for
     if (prof && !(p->flags & (VL_BEAM_MANY_ITERATIONS | VL_BEAM_TABLE))) table = false;
+    bool near = step.sketch && !no_windows && l.use_near != kTableNo && l.near_end <= workspace_bytes;
+    if (prof && !(p->flags & (VL_BEAM_MANY_ITERATIONS | VL_BEAM_BOUNDS))) near = false;
     const int64_t all_slots = p->n_rows * (int64_t)l.memo_slots;
+    const bool cleared = !table && !near;  // the cache, with the loop's state
+    auto clear_cache = [&]() -> int {
+        if (all_slots > 0) {
+            hipLaunchKernelGGL(beam_memo_clear_kernel, dim3(4096), dim3(256), 0, st, memo, all_slots);
+            VL_LAUNCH_CHECK("beam_memo_clear_kernel");
+        }
+        return VL_OK;
+    };
     auto make_ready = [&](bool clear) -> int {  // what a loop without the table needs
         if (sketch_from_start) {
             rc = vl_launch_sketch_queries(queries, p->n_rows, p->dim, (uint8_t *)(ws + l.off_rounded), st);
             if (rc < 0) return rc;
         }
-        if (clear && all_slots > 0) {
-            hipLaunchKernelGGL(beam_memo_clear_kernel, dim3(4096), dim3(256), 0, st, memo, all_slots);
-            VL_LAUNCH_CHECK("beam_memo_clear_kernel");
-        }
-        return VL_OK;
+        return clear ? clear_cache() : VL_OK;
     };
     {
         int64_t n = p->n_rows * l.VL;
         if (n < kBeamStripes) n = kBeamStripes;
         if (n < p->n_rows) n = p->n_rows;
         int64_t blocks = (n + kQueueThreads - 1) / kQueueThreads;
-        const bool clear = !table && all_slots > 0;
+        const bool clear = cleared && all_slots > 0;
         if (clear) {  // eight slots a thread, up to 4,096 workgroups
             const int64_t wanted = (all_slots + 8 * kQueueThreads - 1) / (8 * kQueueThreads);
             blocks = std::max(blocks, std::min<int64_t>(wanted, 4096));
@@ -1040,18 +1082,19 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
                            clear ? memo : nullptr, all_slots);
         VL_LAUNCH_CHECK("beam_init_kernel");
     }
-    const bool asked = table && l.use_table == kTableAsk;
+    const bool asked = (table && l.use_table == kTableAsk) || (near && l.use_near == kTableAsk);
     if (asked) {
         hipLaunchKernelGGL(circulant_graph_kernel, dim3(1), dim3(256), 0, st, beams, p->n_vectors, p->width, &ctrl->circulant);
         VL_LAUNCH_CHECK("circulant_graph_kernel");
         int circulant = 0;
         VL_HIP(hipMemcpyAsync(&circulant, &ctrl->circulant, sizeof(int), hipMemcpyDeviceToHost, st));
         VL_HIP(hipStreamSynchronize(st));
-        table = circulant != 0;
+        if (!circulant) table = near = false;
     }
     if (!table) {
-        rc = make_ready(asked);
+        rc = make_ready(!cleared && !near);
         if (rc < 0) return rc;
+        if (near) step.memo = nullptr;
     }
 
     const int R = (int)p->speculative_readahead;
@@ -1163,6 +1206,7 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     by_table.beams = beams; by_table.n_vectors = p->n_vectors; by_table.width = step.width; by_table.width_magic = step.width_magic;
     by_table.table = (uint32_t *)(ws + l.off_table); by_table.columns = l.table_columns; by_table.unordered = &ctrl->unordered;
     by_table.enter = 1; by_table.window = R; by_table.count_wanted = step.count_evals; by_table.report = step.report;
+    bool near_made = false;
     auto launch_next = [&]() -> int {  // the fused launch that follows iteration t; moves t on
         if (table && t % R == 0 && l.Vt * (t + R) <= l.E) {
             if (by_table.enter) {
@@ -1183,7 +1227,27 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         }
         // (the iterations behind those of the table do without both)
         const bool want_sketch = sketch_table && !table && 2 * (int64_t)sketch_rows >= p->n_rows;
-        const bool windowed = window_fits(t + 1) && t % R == 0 && (!want_sketch || sketch_window);
+        const bool by_products = near && want_sketch && t % R == 0 && window_fits(t + 1);
+        const bool windowed = by_products || (window_fits(t + 1) && t % R == 0 && (!want_sketch || sketch_window));
+        step.near_values = nullptr;
+        // (the cache is worth less than its probes with them, and is there again for rows that gave the bounds up)
+        if (near && !by_products && !step.memo && l.memo_slots > 0 && !(near_made && want_sketch)) {
+            rc = clear_cache();
+            if (rc < 0) return rc;
+            step.memo = memo;
+        }
+        if (by_products) {
+            uint8_t *const at = (uint8_t *)ws + l.off_near;
+            if (!near_made) {
+                rc = vl_launch_near_products(l.near_plan, queries, p->n_rows, vectors, p->n_vectors, p->dim, at, st);
+                if (rc < 0) return rc;
+                near_made = true;
+            }
+            step.near_values = (const uint16_t *)(at + l.near_plan.off_values);
+            step.near_columns = (const uint32_t *)(at + l.near_plan.off_columns);
+            step.near_queries = (const NearQuery *)(at + l.near_plan.off_queries);
+            step.near_pitch = l.near_plan.columns;
+        }
         a.iter = (int)(t + 1);
         step.m = a;
         // (the sketch kernel also for a first window: its rows leave the sketch alone in iteration 1)

@@ -30,6 +30,14 @@ template <int CPL, int LPR, int U, int THREADS, int SCPL, int SLPR, int SU, int 
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void beam_window_sketch_kernel(StepArgs s) {
     beam_row<CPL, LPR, U, kRowAligned, THREADS, SCPL, SLPR, SU, true>(s);
 }
+// ... and with the products of all queries and vectors at hand (near_products.h); it keeps no query row for the sketch.  An
+// iteration of 10,000 rows at 1M x 768 takes 0.16 ms (through the sketch 0.58) and waits on round trips: neighbour lists, products,
+// rows.  Left room for eight wavefronts per SIMD instead of six it spills (first-loop batch at 1M x 768 59.9 -> 61.0 ms,
+// 500,000 x 1,536 84.7 -> 129.9); with 128 threads a row 76.0 and 96.6.
+template <int CPL, int LPR, int U, int THREADS, int SCPL, int WPE>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void beam_window_near_kernel(StepArgs s) {
+    beam_row<CPL, LPR, U, kRowAligned, THREADS, SCPL, 64, 1, true, true>(s);
+}
 
 // The same step for rows that may use the sketch.  WPE: wavefronts per SIMD the compiler is asked to leave room
 // for.  The sketch's copy of the query row takes 16 registers per chunk and lane, and a row's phases (sketch
@@ -55,7 +63,8 @@ template <int THREADS, int CPL, int LPR, int U, RowForm FORM, int SCPL, int SLPR
 void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
     if constexpr (SCPL > 0) {
         if (s.sketch) {
-            if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, (WPE < 6 ? WPE : 6)>, THREADS, s, smem, st);
+            if (s.window > 0 && s.near_values) launch_rows(beam_window_near_kernel<CPL, LPR, UX, THREADS, SCPL, 6>, THREADS, s, smem, st);
+            else if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, (WPE < 6 ? WPE : 6)>, THREADS, s, smem, st);
             else launch_rows(beam_step_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, WPE>, THREADS, s, smem, st);
             return;
         }

@@ -12,6 +12,7 @@
 #include "beam_ctrl.h"
 #include "rowsort.h"
 #include "dist_device.h"
+#include "near_products.h"
 #include "sketch_device.h"
 
 constexpr int kMaxVisit = 64;  // parallel_visit_count handled by one wavefront
@@ -57,6 +58,10 @@ struct StepArgs {
     int sketch_chunks;         // 16-byte chunks of data in a sketch row
     const uint8_t *rounded_queries;  // the call's query rows rounded for the sketch (sketch_device.h)
     int64_t rounded_query_bytes;
+    const uint16_t *near_values;    // products of the call's queries and vectors (near_products.h), instead of the sketch's rows; or null
+    const uint32_t *near_columns;   // what is known of the vector of a column
+    const NearQuery *near_queries;
+    int64_t near_pitch;
     int hash_slots;      // slots of the LDS hash set (row_hash_slots)
     int window;          // > 0: iterations m.iter ... m.iter + window - 1 in this launch
     BeamReport *report;  // pinned host memory that hears of the progress checks, or null
@@ -237,7 +242,10 @@ __device__ __forceinline__ void two_lower_bounds(const uint64_t *a, int na, int 
 // between two progress checks depends on another row of the batch; the only batch-wide facts, the progress flag of the
 // checking iteration (ann.py:90-91) and the largest fill after the last of them, are written once.  Such a launch starts
 // right after a progress check (m.iter = k * readahead + 1, window = readahead).
-template <int CPL, int LPR, int U, RowForm FORM, int THREADS, int SCPL = 0, int SLPR = 64, int SU = 1, bool WINDOW = false>
+//
+// NEAR: bounds come from the call's table of products (near_products.h), one look each.  They are not worth the cache, which
+// keeps exact distances only.
+template <int CPL, int LPR, int U, RowForm FORM, int THREADS, int SCPL = 0, int SLPR = 64, int SU = 1, bool WINDOW = false, bool NEAR = false>
 __device__ __forceinline__ void beam_row(const StepArgs &s) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kRows16 = THREADS / 16;
@@ -514,7 +522,9 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         if constexpr (SCPL > 0) {
             if (sketching) {
                 SketchQuery<SCPL> sq;
-                sketch_query_load<SCPL, SLPR>(sq, s.rounded_queries + row * s.rounded_query_bytes, s.sketch_chunks);
+                NearQuery nq;
+                if constexpr (NEAR) nq = s.near_queries[row];
+                else sketch_query_load<SCPL, SLPR>(sq, s.rounded_queries + row * s.rounded_query_bytes, s.sketch_chunks);
                 for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
                     const int slot = c0 + lane;
                     const bool has = slot < a.m;
@@ -524,6 +534,14 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                     // The cache serves two kinds of repeats: a candidate evaluated exactly before comes back with its
                     // distance, one that was only bounded comes back with its bounds (dist_device.h) - either way
                     // nothing is fetched for it now.
+                    uint32_t value = 0, of_column = 0;
+                    if constexpr (NEAR) {
+                        if (ok) {
+                            const uint32_t column = PairColumns(s.n_vectors).of((uint32_t)id);
+                            value = s.near_values[row * s.near_pitch + column];
+                            of_column = s.near_columns[column];
+                        }
+                    }
                     if (memo_row && ok) {
                         const uint64_t e = memo_load(memo_row, s.memo_shift, id);
                         if ((int32_t)((uint32_t)e & ~kMemoBounds) == id) {
@@ -540,8 +558,12 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                         }
                     }
                     if (s.count_evals || resample) n_sketched += __popcll(__ballot(ok));
-                    wave_sketch<SCPL, SLPR, SU>(sq, s.sketch, s.sketch_tails, s.sketch_chunks, id, ok, ld + c0, le + c0,
-                                                order, memo_row, s.memo_shift);
+                    if constexpr (NEAR) {
+                        if (ok) near_bounds(value, of_column, nq, ld + slot, le + slot);
+                    } else {
+                        wave_sketch<SCPL, SLPR, SU>(sq, s.sketch, s.sketch_tails, s.sketch_chunks, id, ok, ld + c0, le + c0,
+                                                    order, memo_row, s.memo_shift);
+                    }
                 }
                 n_fetched = n_sketched;  // for the share of cache hits: what the cache did not answer
             }
@@ -565,7 +587,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         if (s.count_evals && lane == 0) {
             if (n_wanted) atomicAdd(&c->wanted[stripe], (unsigned long long)n_wanted);
             if (n_fetched && !sketching) atomicAdd(&c->evals[stripe], (unsigned long long)n_fetched);
-            if (n_sketched) atomicAdd(&c->sketched[stripe], (unsigned long long)n_sketched);
+            if (n_sketched && !NEAR) atomicAdd(&c->sketched[stripe], (unsigned long long)n_sketched);
         }
         if (resample && lane == 0) {
             atomicAdd(&probe_asked_s, n_wanted);

@@ -29,6 +29,7 @@
 // candidates.
 #include "knn_device.h"
 #include "knn_filter.h"
+#include "near_products.h"
 
 #include <type_traits>
 
@@ -191,15 +192,18 @@ __device__ __forceinline__ void stage256(const float *const (&p)[4], int kt, flo
         __builtin_amdgcn_global_load_lds((glb_void *)(p[i] + kt), (lds_void *)(tile + 8 * (4 * wave + i) * KT), 16, 0, 0);
 }
 
-// EMIT = false: the sample pass, groups' maxima to gmax.  EMIT = true: the filter pass.
+// What a pass leaves of its values: the sample's groups' maxima in gmax, the filter's candidates in found, or all of them rounded to
+// 16 bits (kAllValues: query by query, id0 of them each and as many vectors, whole tiles; out).
+enum PassKind { kSampleMaxima, kCandidates, kAllValues };
 // Rows are bfloat16 of kp columns, addressed as floats (two columns each); a stage is KT floats = 64 columns.
-template <bool EMIT>
+template <PassKind KIND>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *__restrict__ v16, int64_t n_vectors,
                  int kp2, int64_t strip_len, int n_strips, int n_qblocks, int q_group, float *__restrict__ gmax,
                  const Sampled *__restrict__ bound, const RowStat *__restrict__ qstat, const uint32_t *__restrict__ vmax,
                  const uint32_t *__restrict__ sample_vmax, float most, int dim, int l2,
-                 int64_t id0, int32_t *__restrict__ count, uint64_t *__restrict__ found) {
+                 int64_t id0, int32_t *__restrict__ count, uint64_t *__restrict__ found, uint16_t *__restrict__ out) {
+    constexpr bool EMIT = KIND == kCandidates;
     extern __shared__ __align__(16) float smem[];
     constexpr int T = TR * KT;  // floats of a staged operand
     float *const sV0 = smem, *const sV1 = smem + T, *const sQ0 = smem + 2 * T, *const sQ1 = smem + 3 * T;
@@ -350,7 +354,30 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
     // accumulator register r of block rb: vector row 128 wr + 32 rb + 8 (r / 4) + 4 half + r % 4 of the tile, query l32
     auto fold = [&](int64_t vt) __attribute__((always_inline)) {
         const int64_t v_lane = vt + 128 * wr + 4 * half;
-        if constexpr (!EMIT) {
+        if constexpr (KIND == kAllValues) {
+            // The halves of the wavefront hold every other four vectors of a query; they change hands until a lane has eight that
+            // follow each other, 16 bytes a store, whole lines by the tile's end.  (Bound by the products: 10,000 x 1M x 768 with 20 GB
+            // stored 17.6 ms, 875 TFLOP/s.)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                const int64_t q = q0 + 64 * wc + 32 * cb + l32;
+                uint16_t *const to = out + (q < n_queries ? q : 0) * id0 + vt + 128 * wr + 8 * half;
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) {
+                    uint32_t w[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        w[j] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)acc[rb][cb][2 * j]) |
+                               (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)acc[rb][cb][2 * j + 1]) << 16;
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const auto a = __builtin_amdgcn_permlane32_swap(w[4 * p], w[4 * p + 2], false, false);
+                        const auto b = __builtin_amdgcn_permlane32_swap(w[4 * p + 1], w[4 * p + 3], false, false);
+                        if (q < n_queries) *reinterpret_cast<uint4 *>(to + 32 * rb + 16 * p) = make_uint4(a[0], b[0], a[1], b[1]);
+                    }
+                }
+            }
+        } else if constexpr (!EMIT) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -443,7 +470,7 @@ void pass_kernel(const float *__restrict__ q16, int64_t n_queries, const float *
             vt += TR;
         }
     }
-    if constexpr (!EMIT) {
+    if constexpr (KIND == kSampleMaxima) {
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
             const int64_t q = q0 + 64 * wc + 32 * cb + l32;
@@ -863,8 +890,8 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     const int64_t n_words = (slabs + 1) * kStripes * kStripeWords;
     const size_t smem = 4 * TR * KT * sizeof(float);
     auto allow = [&]() -> hipError_t {
-        const hipError_t e = vl_allow_lds(pass_kernel<false>, smem);
-        return e == hipSuccess ? vl_allow_lds(pass_kernel<true>, smem) : e;
+        const hipError_t e = vl_allow_lds(pass_kernel<kSampleMaxima>, smem);
+        return e == hipSuccess ? vl_allow_lds(pass_kernel<kCandidates>, smem) : e;
     };
     VL_HIP(allow());
     hipLaunchKernelGGL(filter_clear_kernel, dim3((unsigned)((n_words + 255) / 256)), dim3(256), 0, st, vmax,
@@ -885,10 +912,10 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), smem, st, (const float *)q16, n_queries,
                                (const float *)v16, rows, kp2, len, (int)strips, (int)q_blocks, (int)q_group, gmax, bound,
-                               qstat, top, vmax, (float)p.most, (int)dim, l2 ? 1 : 0, id0, count, found);
+                               qstat, top, vmax, (float)p.most, (int)dim, l2 ? 1 : 0, id0, count, found, nullptr);
         };
-        if (emit) go(pass_kernel<true>);
-        else go(pass_kernel<false>);
+        if (emit) go(pass_kernel<kCandidates>);
+        else go(pass_kernel<kSampleMaxima>);
     };
     prepare(prepare_kernel<false>, queries, n_queries, 1, q16, l2 ? q_norm : nullptr, qstat, nullptr);
     prepare(prepare_kernel<true>, vectors, p.sample_rows, 2, v16, nullptr, nullptr, vmax);
@@ -918,5 +945,89 @@ int vl_knn_filter(const KnnFilterPlan &p, const float *queries, int64_t n_querie
     VL_LAUNCH_CHECK("knn finish_kernel");
     hipLaunchKernelGGL(left_kernel, dim3(1), dim3(kLeftThreads), 0, st, count, (int)n_queries, (int)q_first, left, tile_bound);
     VL_LAUNCH_CHECK("knn left_kernel");
+    return VL_OK;
+}
+
+// ---- all products of a call's queries and vectors, for the beam step (near_products.h) ----
+
+namespace {
+
+// Rows rounded to bfloat16 and padded with zeros to kp columns and `padded` rows; a wavefront a row.  The queries in their order,
+// the vectors in the order of PairColumns.
+template <bool QUERIES>
+__global__ __launch_bounds__(256) void near_prepare_kernel(const float *__restrict__ rows, int64_t n, int64_t padded, int dim, int kp,
+                                                           __bf16 *__restrict__ out, NearQuery *__restrict__ queries,
+                                                           uint32_t *__restrict__ columns) {
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int64_t i = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave; i < padded; i += (int64_t)gridDim.x * 4) {
+        const int64_t row = QUERIES ? i : PairColumns(n).vector_at(i);
+        const bool real = row < n;
+        const float4 *src = reinterpret_cast<const float4 *>(rows + (real ? row : 0) * dim);
+        bf16x4 *dst = reinterpret_cast<bf16x4 *>(out + i * kp);
+        float s = 0.0f, e2 = 0.0f;
+        for (int c = lane; c < kp / 4; c += kWave) {
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (real && c < dim / 4) x = src[c];
+            const bf16x4 h = {(__bf16)x.x, (__bf16)x.y, (__bf16)x.z, (__bf16)x.w};
+            const float a = x.x - (float)h[0], b = x.y - (float)h[1], d = x.z - (float)h[2], e = x.w - (float)h[3];
+            s = fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, fmaf(x.w, x.w, s))));
+            e2 = fmaf(a, a, fmaf(b, b, fmaf(d, d, fmaf(e, e, e2))));
+            dst[c] = h;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            s += __shfl_xor(s, o);
+            e2 += __shfl_xor(e2, o);
+        }
+        float resid = up(sqrtf(e2)), norm = up(sqrtf(s));
+        if (!(resid < 1e18f)) resid = __builtin_inff();  // also NaN
+        if (!(norm < 1e18f)) norm = __builtin_inff();
+        if (lane != 0) continue;
+        if constexpr (QUERIES) {
+            // what near_bounds multiplies a vector's residual and norm with, the float32 roundings of both sums included
+            const float sums = (float)dim * 2.4e-7f * (norm + resid);
+            queries[i] = NearQuery{up(norm + resid) + sums, resid + sums};
+        } else {
+            columns[i] = half_bits_not_below(resid) | half_bits_not_below(norm) << 16;
+        }
+    }
+}
+
+}  // namespace
+
+NearPlan vl_near_plan(int64_t n_queries, int64_t n_vectors, int64_t dim) {
+    NearPlan p;
+    p.kp = (dim + 63) / 64 * 64;
+    p.columns = (PairColumns(n_vectors).count() + TR - 1) / TR * TR;
+    int64_t o = 0;
+    p.off_queries = o; o = align256(o + n_queries * (int64_t)sizeof(NearQuery));
+    p.off_columns = o; o = align256(o + p.columns * 4);
+    p.off_q16 = o; o = align256(o + n_queries * p.kp * 2);
+    p.off_v16 = o; o = align256(o + p.columns * p.kp * 2);
+    p.off_values = o; o = align256(o + n_queries * p.columns * 2);
+    p.bytes = o;
+    return p;
+}
+
+int vl_launch_near_products(const NearPlan &p, const float *queries, int64_t n_queries, const float *vectors, int64_t n_vectors,
+                            int64_t dim, uint8_t *ws, hipStream_t st) {
+    const size_t smem = 4 * TR * KT * sizeof(float);
+    VL_HIP(vl_allow_lds(pass_kernel<kAllValues>, smem));
+    __bf16 *const q16 = (__bf16 *)(ws + p.off_q16), *const v16 = (__bf16 *)(ws + p.off_v16);
+    auto blocks_for = [](int64_t rows) { return dim3((unsigned)((rows + 3) / 4 < 4096 ? (rows + 3) / 4 : 4096)); };
+    hipLaunchKernelGGL(near_prepare_kernel<true>, blocks_for(n_queries), dim3(256), 0, st, queries, n_queries, n_queries, (int)dim,
+                       (int)p.kp, q16, (NearQuery *)(ws + p.off_queries), (uint32_t *)nullptr);
+    hipLaunchKernelGGL(near_prepare_kernel<false>, blocks_for(p.columns), dim3(256), 0, st, vectors, n_vectors, p.columns, (int)dim,
+                       (int)p.kp, v16, (NearQuery *)nullptr, (uint32_t *)(ws + p.off_columns));
+    VL_LAUNCH_CHECK("near_prepare_kernel");
+    const int64_t q_blocks = (n_queries + TR - 1) / TR, tiles = p.columns / TR, strips = strips_for(q_blocks, tiles, 1024);
+    const int64_t len = (tiles + strips - 1) / strips * TR;
+    int64_t q_group = (2ll << 20) / (TR * p.kp * 2);
+    q_group = q_group < 1 ? 1 : (q_group > 8 ? 8 : q_group);
+    hipLaunchKernelGGL(pass_kernel<kAllValues>, dim3((unsigned)((q_blocks * strips + 7) / 8 * 8)), dim3(kThreads), smem, st,
+                       (const float *)q16, n_queries, (const float *)v16, p.columns, (int)p.kp / 2, len, (int)strips, (int)q_blocks,
+                       (int)q_group, nullptr, nullptr, nullptr, nullptr, nullptr, 0.0f, (int)dim, 0, p.columns, nullptr, nullptr,
+                       (uint16_t *)(ws + p.off_values));
+    VL_LAUNCH_CHECK("pass_kernel (all values)");
     return VL_OK;
 }
