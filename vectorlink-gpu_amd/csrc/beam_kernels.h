@@ -32,8 +32,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
 }
 // ... and with the products of all queries and vectors at hand (near_products.h); it keeps no query row for the sketch.  An
 // iteration of 10,000 rows at 1M x 768 takes 0.16 ms (through the sketch 0.58) and waits on round trips: neighbour lists, products,
-// rows.  Left room for eight wavefronts per SIMD instead of six it spills (first-loop batch at 1M x 768 59.9 -> 61.0 ms,
-// 500,000 x 1,536 84.7 -> 129.9); with 128 threads a row 76.0 and 96.6.
+// rows.  Rows in flight and room for wavefronts per SIMD are chosen by what spills.  First-loop batches of 10,000 (ms), 1M x 768 /
+// 500,000 x 1,024 / 500,000 x 1,536 / 1M x 384: one row and six wavefronts 59.2 / 57.6 / 93.3 / 35.9, two and six 57.8 / 66.5 / 93.1 / 36.0,
+// one and five 59.4 / 57.7 / 82.9 / 36.0, two and five 62.5 / 61.0 / 99.7 / 38.6, two and four 62.7 / 60.8 / 86.4 / 38.4, four and six 76.6 /
+// 135.6 / 305.9 / 47.7.  With 128 threads a row 76.0 and 96.6 instead of 59.9 and 84.7 (768 and 1,536 columns).
 template <int CPL, int LPR, int U, int THREADS, int SCPL, int WPE>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void beam_window_near_kernel(StepArgs s) {
     beam_row<CPL, LPR, U, kRowAligned, THREADS, SCPL, 64, 1, true, true>(s);
@@ -63,7 +65,7 @@ template <int THREADS, int CPL, int LPR, int U, RowForm FORM, int SCPL, int SLPR
 void launch_step_threads(const StepArgs &s, size_t smem, hipStream_t st) {
     if constexpr (SCPL > 0) {
         if (s.sketch) {
-            if (s.window > 0 && s.near_values) launch_rows(beam_window_near_kernel<CPL, LPR, UX, THREADS, SCPL, 6>, THREADS, s, smem, st);
+            if (s.window > 0 && s.near_values) launch_rows(beam_window_near_kernel<CPL, LPR, (CPL <= 3 ? 2 : 1), THREADS, SCPL, (CPL <= 3 ? 6 : 5)>, THREADS, s, smem, st);
             else if (s.window > 0) launch_rows(beam_window_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, (WPE < 6 ? WPE : 6)>, THREADS, s, smem, st);
             else launch_rows(beam_step_sketch_kernel<CPL, LPR, UX, THREADS, SCPL, SLPR, SU, WPE>, THREADS, s, smem, st);
             return;

@@ -262,11 +262,13 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
     // 20,000 x 200 2,950 -> 2,694, 3,194 -> 2,738 (degree 32) and 33,314 -> 32,890 us; clusters of 977 at 60,000 x 256 6,393 -> 6,508.
     constexpr bool kSums = FORM == kRowUnalignedSums || (FORM == kRowAligned && SCPL == 0 && CPL == 1 && LPR == 64);
     // Sets of 64 candidates of a wavefront whose neighbour ids and cache probes are on their way at a time.  (The kernels with
-    // the sketch, which wait on bytes, spill registers with two: a batch of the first loop at 1M x 768 141.0 and 143.1 ms.)
-    constexpr int kAhead = SCPL > 0 ? 1 : 2;
+    // the sketch, which wait on bytes, spill registers with two: a batch of the first loop at 1M x 768 141.0 and 143.1 ms.  With
+    // the table of products, whose looks are on their way along with them, two are the sooner: 59.9 -> 59.2, 500,000 x 1,024 61.0 ->
+    // 57.6, 1M x 384 37.8 -> 35.9.)
+    constexpr int kAhead = SCPL > 0 && !NEAR ? 1 : 2;
     // Where the ids to visit are read from: the heads of the visit queue, and in the kernels with the sketch a copy of their
     // own, which those need to be as fast (a batch of the first loop at 1M x 768 141.3 ms without it, 139.9 with it).
-    constexpr bool kOwnHeads = SCPL > 0;
+    constexpr bool kOwnHeads = SCPL > 0 && !NEAR;
     __shared__ int32_t visit_s[kOwnHeads ? kMaxVisit : 1];
     __shared__ uint32_t red[kRows16];
     __shared__ int n_ex_s;                  // exclusion ids before the row's first empty one
@@ -481,10 +483,15 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         // nodes visited in one iteration share ids; the reference evaluates every copy (kernels.py:238-255) and drops
         // all but one when the queues are sorted (kernels.py:314-349); copies carry the same distance.
         // A row without the sketch asks its cache for the others right away and lists the candidates to fetch.
+        // With the table of products it gets their bounds, all of a set's looks on their way at a time.
+        NearQuery nq;
+        if constexpr (NEAR)
+            if (sketching) nq = s.near_queries[row];
         for (int c0 = wave * kWave; c0 < a.m; c0 += kAhead * THREADS) {
             int32_t id[kAhead];
             bool ok[kAhead];
             uint64_t entry[kAhead];
+            uint32_t value[kAhead], of_column[kAhead];
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) {
                 const int slot = c0 + j * THREADS + lane;
@@ -501,6 +508,22 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                     if constexpr (WINDOW) set_slot[slot] = (uint16_t)(ok[j] ? h : 0xffffu);
                 }
                 if (!sketching && probing && ok[j]) entry[j] = memo_load(memo_row, s.memo_shift, id[j]);
+                if constexpr (NEAR) {
+                    if (sketching && ok[j]) {
+                        const uint32_t column = PairColumns(s.n_vectors).of((uint32_t)id[j]);
+                        value[j] = s.near_values[row * s.near_pitch + column];
+                        of_column[j] = s.near_columns[column];
+                    }
+                }
+            }
+            if constexpr (NEAR) {
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) {
+                    const int slot = c0 + j * THREADS + lane;
+                    if (!sketching || slot >= a.m) continue;
+                    flags[slot] = 0;
+                    if (ok[j]) near_bounds(value[j], of_column[j], nq, ld + slot, le + slot);
+                }
             }
             if (sketching) continue;
 #pragma unroll
@@ -519,12 +542,10 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                 if (ok[j]) missed[base + __popcll(all & ((1ull << lane) - 1))] = (uint16_t)slot;
             }
         }
-        if constexpr (SCPL > 0) {
+        if constexpr (SCPL > 0 && !NEAR) {
             if (sketching) {
                 SketchQuery<SCPL> sq;
-                NearQuery nq;
-                if constexpr (NEAR) nq = s.near_queries[row];
-                else sketch_query_load<SCPL, SLPR>(sq, s.rounded_queries + row * s.rounded_query_bytes, s.sketch_chunks);
+                sketch_query_load<SCPL, SLPR>(sq, s.rounded_queries + row * s.rounded_query_bytes, s.sketch_chunks);
                 for (int c0 = wave * kWave; c0 < a.m; c0 += THREADS) {
                     const int slot = c0 + lane;
                     const bool has = slot < a.m;
@@ -534,14 +555,6 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                     // The cache serves two kinds of repeats: a candidate evaluated exactly before comes back with its
                     // distance, one that was only bounded comes back with its bounds (dist_device.h) - either way
                     // nothing is fetched for it now.
-                    uint32_t value = 0, of_column = 0;
-                    if constexpr (NEAR) {
-                        if (ok) {
-                            const uint32_t column = PairColumns(s.n_vectors).of((uint32_t)id);
-                            value = s.near_values[row * s.near_pitch + column];
-                            of_column = s.near_columns[column];
-                        }
-                    }
                     if (memo_row && ok) {
                         const uint64_t e = memo_load(memo_row, s.memo_shift, id);
                         if ((int32_t)((uint32_t)e & ~kMemoBounds) == id) {
@@ -558,12 +571,8 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
                         }
                     }
                     if (s.count_evals || resample) n_sketched += __popcll(__ballot(ok));
-                    if constexpr (NEAR) {
-                        if (ok) near_bounds(value, of_column, nq, ld + slot, le + slot);
-                    } else {
-                        wave_sketch<SCPL, SLPR, SU>(sq, s.sketch, s.sketch_tails, s.sketch_chunks, id, ok, ld + c0, le + c0,
-                                                    order, memo_row, s.memo_shift);
-                    }
+                    wave_sketch<SCPL, SLPR, SU>(sq, s.sketch, s.sketch_tails, s.sketch_chunks, id, ok, ld + c0, le + c0,
+                                                order, memo_row, s.memo_shift);
                 }
                 n_fetched = n_sketched;  // for the share of cache hits: what the cache did not answer
             }
@@ -587,7 +596,7 @@ __device__ __forceinline__ void beam_row(const StepArgs &s) {
         if (s.count_evals && lane == 0) {
             if (n_wanted) atomicAdd(&c->wanted[stripe], (unsigned long long)n_wanted);
             if (n_fetched && !sketching) atomicAdd(&c->evals[stripe], (unsigned long long)n_fetched);
-            if (n_sketched && !NEAR) atomicAdd(&c->sketched[stripe], (unsigned long long)n_sketched);
+            if (n_sketched) atomicAdd(&c->sketched[stripe], (unsigned long long)n_sketched);
         }
         if (resample && lane == 0) {
             atomicAdd(&probe_asked_s, n_wanted);
