@@ -137,6 +137,42 @@ def test_distances_that_are_no_ordinary_numbers(metric, value):
         same(search(g, rows, beams, seeds, c, True, BEAM_TABLE, sketch=sketch), want)
 
 
+# The launch behind the refused one is an ordinary one: lists with room for one stretch between two progress checks and not for two
+# (24 ids of 4 a time in stretches of 5; 360 in stretches of 50).  Profiled calls wait for a check before they go on, others do not.
+@pytest.mark.parametrize("metric,value", [("cosine", np.nan), ("cosine", np.inf), ("l2", np.inf), ("l2", 1e19), ("l2", np.nan)])
+@pytest.mark.parametrize("beam,ef,ra", [(8, 1, 5), (24, 5, 50)])
+@pytest.mark.parametrize("per_query", [False, True])
+def test_refused_where_the_lists_fill_up_in_the_next_launch(beam, ef, ra, metric, value, per_query):
+    print(f"table refused beam={beam} ra={ra} {metric} {value} {per_query}", flush=True)
+    from vectorlink_gpu import _native as nv
+    from vectorlink_gpu.ann import BEAM_PER_QUERY_STOP, BEAM_TABLE
+    from vectorlink_gpu.kernels import build_sketch
+
+    (n, rows, dim) = (700, 130, 256)
+    v = vectors(n, dim, metric)
+    v[333, 5] = value
+    g = dev(v)
+    ids = orc.generate_circulant_beams(n, orc.primes(2 * beam))
+    c = config(beam_size=beam, exclude_factor=ef, speculative_readahead=ra, metric=metric)
+    flags = BEAM_TABLE | (BEAM_PER_QUERY_STOP if per_query else 0)
+    want = oracle(v, rows, ids, ids[:rows], c, True, per_query)
+    assert not np.array_equal(np.sort(want[1], axis=1), np.sort(ids[:rows], axis=1))  # (a call that does nothing is not right by chance)
+
+    def check(sketch=None):
+        got = search(g, rows, dev(ids), ids[:rows], c, True, flags, sketch=sketch)
+        assert got[0] == want[0] and np.array_equal(got[1], want[1])
+        assert np.array_equal(got[2].view(np.float32), want[2].view(np.float32), equal_nan=True)
+
+    check()
+    check(build_sketch(g))
+    if ra <= 64:
+        nv.lib().vl_beam_profile(1, 1, None)
+        try:
+            check()
+        finally:
+            nv.lib().vl_beam_profile(0, 1, None)
+
+
 def test_a_workspace_without_room_for_the_table():
     from vectorlink_gpu import Queue, _native as nv
     from vectorlink_gpu.ann import BEAM_NO_TABLE, BEAM_TABLE, _beam_params

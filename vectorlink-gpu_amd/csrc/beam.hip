@@ -876,6 +876,12 @@ __global__ void beam_status_kernel(const BeamCtrl *c, int iterations, int R, int
     status[1] = ended ? t : iterations;
 }
 
+// After a refused table: the launch that was enqueued behind the refused one may be an ordinary one, which takes the check that
+// nothing ran up to for one that found the batch quiet and ends the loop.  The loop begins again.
+__global__ void beam_resume_kernel(BeamCtrl *c) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) c->stop = c->ended_after = c->refused_at = 0;
+}
+
 // The loop itself.  fixed_iterations == 0: run until a progress check finds the batch quiet, reading the
 // flag on the host every speculative_readahead iterations; returns the iteration count.  fixed_iterations
 // > 0: enqueue exactly that many iterations and return 0 without ever waiting for the device - once a
@@ -1345,6 +1351,8 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
         if (table && found.refused_at) {
             // the launches from iteration refused_at on did nothing: the loop goes on from there without the table
             table = false;
+            hipLaunchKernelGGL(beam_resume_kernel, dim3(1), dim3(64), 0, st, ctrl);
+            VL_LAUNCH_CHECK("beam_resume_kernel");
             step.memo = l.memo_slots > 0 ? memo : nullptr;
             rc = make_ready(true);
             if (rc < 0) return rc;

@@ -44,7 +44,10 @@ public:
     ReportSlot &operator=(const ReportSlot &) = delete;
 
     BeamReport *get() const { return index_ < 0 ? nullptr : &page_[index_].report; }
-    void forget() { __atomic_store_n(&page_[index_].report.check, 0, __ATOMIC_RELAXED); }  // the last report, with no launch left that reports
+    void forget() {  // the last report, with no launch left that reports
+        page_[index_].report.refused_at = 0;
+        __atomic_store_n(&page_[index_].report.check, 0, __ATOMIC_RELAXED);
+    }
     void launching() { running_ = true; }  // before anything of the call goes to the stream
     void drained() { running_ = false; }   // the stream has been waited for
 
