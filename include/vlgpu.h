@@ -247,7 +247,8 @@ typedef struct vl_beam_params {
 #define VL_BEAM_NO_TABLE 512
 /* Such a call with a sketch, too large for all distances, may be given bounds of
  * all of them instead.  VL_BEAM_BOUNDS: always, where the call can use a sketch
- * and has no such table; VL_BEAM_NO_TABLE: never. */
+ * and has no such table; VL_BEAM_NO_TABLE: never.  Neither is made of fewer than
+ * 64 vectors. */
 #define VL_BEAM_BOUNDS 1024
 
 /* Bytes of workspace that serve a call with these parameters.  All but the last

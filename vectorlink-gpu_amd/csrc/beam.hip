@@ -727,7 +727,7 @@ constexpr int64_t kNearMostBytes = 24ll << 30;
 TableUse near_use(const vl_beam_params *p, const BeamLayout &l) {
     if (!l.may_sketch || l.use_table != kTableNo || p->speculative_readahead < 2) return kTableNo;
     if (p->flags & (VL_BEAM_NO_TABLE | VL_BEAM_NO_WINDOWS | VL_BEAM_WINDOWS)) return kTableNo;  // (it runs several iterations per launch)
-    if (l.near_plan.bytes > kNearMostBytes) return kTableNo;
+    if (p->n_vectors < kPairTile || l.near_plan.bytes > kNearMostBytes) return kTableNo;
     if (p->flags & VL_BEAM_BOUNDS) return kTableYes;
     const double rows = (double)p->n_rows, pairs = rows * (double)p->n_vectors, candidates = rows * (double)l.m;
     const double made = 60.0 + pairs * (2.2e-9 * (double)p->dim + 4e-7) + 1.5e-6 * (double)p->n_vectors * (double)p->dim;  // us
@@ -738,7 +738,7 @@ TableUse near_use(const vl_beam_params *p, const BeamLayout &l) {
     return p->excl_cols > 0 && p->n_rows >= kComputeUnits ? kTableAsk : kTableNo;
 }
 
-// *circulant = 1 if the neighbours of node i + 1 are those of node i plus one, in a sample of the nodes.
+// *circulant = 1 if the neighbours of node i + 1 are those of node i plus one, in a sample of the nodes (of two at least).
 constexpr int kCirculantNodes = 64;
 __global__ __launch_bounds__(256) void circulant_graph_kernel(const int32_t *__restrict__ beams, int64_t n, int64_t width, int *circulant) {
     __shared__ int other;
