@@ -24,3 +24,10 @@ def asks(flags, rows=10_000, n=1_000_000, dim=768, width=128, beam=64, visits=4,
 def test_a_few_vectors_have_neither(n, flags):
     """(The look at the graph reads the lists of a node and of the next one.)"""
     assert asks(flags, n=n) == 0
+
+
+@pytest.mark.parametrize("rows,n,dim", [(8, 70_000_000, 4), (1, 600_000_000, 4)])
+def test_sizes_beyond_the_grid_of_the_distances_do_without(rows, n, dim):
+    """(The kernels' launcher refuses them.)"""
+    assert asks(TABLE, rows=rows, n=n, dim=dim) == 0
+    assert asks(TABLE, rows=rows, n=60_000_000, dim=dim) > 0

@@ -706,7 +706,9 @@ TableUse table_use(const vl_beam_params *p, const BeamLayout &l) {
     if (l.Vt > kTableMaxVisit || l.VL <= l.Vt || l.VL > kTableMaxQueue || p->queue_length > kTableMaxQueue ||
         l.m > kTableMaxCandidates || p->excl_cols > kTableMaxExcluded || l.Vt * p->speculative_readahead > l.E || p->dim > 2048)
         return kTableNo;
-    if (p->n_vectors < kPairTile || p->n_rows * pair_columns(p->n_vectors) * 4 > kTableMostBytes) return kTableNo;
+    if (p->n_vectors < kPairTile || p->n_rows * pair_columns(p->n_vectors) * 4 > kTableMostBytes ||
+        !vl_pair_table_fits(p->n_rows, p->n_vectors, p->dim))
+        return kTableNo;
     if (p->flags & VL_BEAM_TABLE) return kTableYes;
     if ((p->flags & VL_BEAM_NO_CACHE) && !(p->flags & VL_BEAM_MANY_ITERATIONS)) return kTableNo;  // (asked for a small workspace)
     if (table_pays(p, l, 20, 20)) return kTableYes;

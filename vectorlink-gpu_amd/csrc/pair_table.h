@@ -51,6 +51,9 @@ static inline int64_t pair_packed_bytes(int64_t n, int64_t dim) {
 }
 static inline int64_t pair_columns(int64_t n_vectors) { return pair_tiles(PairColumns(n_vectors).count()) * kPairTile; }
 
+// Whether a launch takes tables of that size.
+bool vl_pair_table_fits(int64_t n_queries, int64_t n_vectors, int64_t dim);
+
 // out[r * columns + PairColumns(n_vectors).of(v)] = distance of queries[r] and vectors[v] as bits (columns of no vector hold
 // values nobody asks for).  *unordered becomes 1 if a distance may not be a number below VL_MAXFLOAT.
 // packed_queries / packed_vectors: room for the copies (pair_packed_bytes of n_queries and of pair_columns), 16-byte aligned.

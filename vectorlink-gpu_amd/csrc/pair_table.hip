@@ -310,21 +310,30 @@ void launch_tiles(const uint8_t *q, int64_t n_queries, const uint8_t *v, int64_t
     else go(pair_tile_kernel<L2, 5>);
 }
 
+int64_t pack_blocks(int64_t n_queries, int64_t n_vectors, int64_t dim) {
+    const int64_t strips = pair_tiles(n_queries) * (kPairTile / kPairStrip) + pair_columns(n_vectors) / kPairStrip;
+    return (strips * ((pair_units(dim).count + kPackUnits - 1) / kPackUnits) + 3) / 4;
+}
 }  // namespace
+
+bool vl_pair_table_fits(int64_t n_queries, int64_t n_vectors, int64_t dim) {
+    const int64_t n_columns = pair_columns(n_vectors);
+    return n_columns < (1 << 26) && pair_tiles(n_queries) * pair_tiles(n_columns) < 4 * kMaxBlocks &&
+           pack_blocks(n_queries, n_vectors, dim) < 4 * kMaxBlocks;
+}
 
 int vl_launch_pair_table(const float *queries, int64_t n_queries, const float *vectors, int64_t n_vectors, int64_t dim,
                          int metric, uint8_t *packed_queries, uint8_t *packed_vectors, uint32_t *out, int64_t columns,
                          int *unordered, hipStream_t st) {
     const PairUnits units = pair_units(dim);
-    const int64_t per_strip = (units.count + kPackUnits - 1) / kPackUnits, n_columns = pair_columns(n_vectors);
+    const int64_t n_columns = pair_columns(n_vectors);
     auto side = [&](const float *rows, int64_t n, int64_t padded, uint8_t *to, bool by_class) {
         return PackSide{rows, n, padded / kPairStrip, to, dim % 4 == 0 && (uintptr_t)rows % 16 == 0, by_class};
     };
     const PackSide q = side(queries, n_queries, pair_tiles(n_queries) * kPairTile, packed_queries, false);
     const PackSide v = side(vectors, n_vectors, n_columns, packed_vectors, true);
-    const int64_t blocks = ((q.strips + v.strips) * per_strip + 3) / 4;
-    VL_REQUIRE(columns >= n_columns && n_columns < (1 << 26) && pair_tiles(n_queries) * pair_tiles(n_columns) < 4 * kMaxBlocks &&
-                   blocks < 4 * kMaxBlocks,
+    const int64_t blocks = pack_blocks(n_queries, n_vectors, dim);
+    VL_REQUIRE(columns >= n_columns && vl_pair_table_fits(n_queries, n_vectors, dim),
                "a table of %lld x %lld distances is too large for one call", (long long)n_queries, (long long)n_vectors);
     hipLaunchKernelGGL(pair_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, q, v, (int)dim, units);
     VL_LAUNCH_CHECK("pair_pack_kernel");
