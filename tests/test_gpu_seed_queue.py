@@ -69,3 +69,17 @@ def test_what_does_not_fit_is_refused():
     with pytest.raises(ValueError, match="do not fit"):
         Queue.seeded(6, 10, v, v, torch.zeros((10, 5), dtype=torch.int32, device="cuda:0"))
     assert Queue.seeded(4, 9, v[:0], v, torch.zeros((0, 4), dtype=torch.int32, device="cuda:0")).indices.size() == (0, 9)
+
+
+def test_entry_points_from_every_other_id_of_a_list():
+    from vectorlink_gpu.ann import dense_search_queue
+
+    rng = np.random.default_rng(3)
+    v = rng.standard_normal((400, 32)).astype(np.float32)
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    ids = rng.permutation(400)[:200].astype(np.int32)
+    c = dict(orc.DEFAULT_CONFIG, beam_size=8)
+    entry = dev(v[ids[::2]])
+    want = dense_search_queue(dev(v), dev(v[:9]), c, dev(ids[::2]), entry)
+    got = dense_search_queue(dev(v), dev(v[:9]), c, dev(ids)[::2], entry)
+    assert torch.equal(got.indices, want.indices) and torch.equal(got.distances, want.distances)

@@ -443,7 +443,7 @@ def dense_search_queue(vectors: Tensor, query_vectors: Tensor, config: Dict, ent
     ranked_by = query_vectors if cols == query_vectors.size(1) else query_vectors[:, :cols].contiguous()
     (local, _) = knn_exact(ranked_by, entry_vectors, k, config.get("metric", "cosine"))
     return Queue.seeded(queue_size, queue_size + extra_capacity, query_vectors, vectors, local, config.get("metric", "cosine"),
-                        names=entry_ids)
+                        names=entry_ids.contiguous())
 
 
 def _flags_for_sample(sample: Tensor, vectors: Tensor) -> int:
