@@ -238,18 +238,23 @@ typedef struct vl_beam_params {
 #define VL_BEAM_WINDOWS 32
 #define VL_BEAM_NO_WINDOWS 64
 /* The caller expects many iterations (same loop, same result): a search that
- * starts anywhere, or a batch of a build.  Such a call is the more likely to be
- * given the distances of all its queries and vectors ahead of the loop, which
- * iterations then look up.  VL_BEAM_TABLE: always, where the kernels are built
- * for the call's sizes, VL_BEAM_NO_TABLE: never. */
+ * starts anywhere, or a batch of a build's first loop, whose graph's edges lead
+ * anywhere.  Such a call is the more likely to be given the distances of all its
+ * queries and vectors ahead of the loop, which iterations then look up; one that
+ * does not say so is if twenty iterations on a graph of near neighbours pay for
+ * it.  VL_BEAM_TABLE: always, where the kernels are built for the call's sizes,
+ * VL_BEAM_NO_TABLE: never. */
 #define VL_BEAM_MANY_ITERATIONS 128
 #define VL_BEAM_TABLE 256
 #define VL_BEAM_NO_TABLE 512
-/* Such a call with a sketch, too large for all distances, may be given bounds of
- * all of them instead.  VL_BEAM_BOUNDS: always, where the call can use a sketch
+/* A call that says so, with a sketch and with exclusions, and too large for all
+ * distances, may be given bounds of all of them instead.  VL_BEAM_BOUNDS: always, where the call can use a sketch
  * and has no such table; VL_BEAM_NO_TABLE: never.  Neither is made of fewer than
  * 64 vectors. */
 #define VL_BEAM_BOUNDS 1024
+/* The caller knows that its graph is not the one that builds start from
+ * (vl_circulant_graph): vl_beam_ahead proposes no look at it. */
+#define VL_BEAM_KNOWN_GRAPH 2048
 
 /* Bytes of workspace that serve a call with these parameters.  All but the last
  * part, the distance cache, follows from n_rows, width, beam_size, the queue and
@@ -258,11 +263,26 @@ typedef struct vl_beam_params {
  * n_vectors and dim as well, not always upwards: a larger table may need a
  * smaller cache.  A workspace that was sized with another n_vectors or dim is
  * accepted, and the cache then has the slots that fit; refused is one that could
- * not hold 1,024 per row.  Calls that are worth it (VL_BEAM_MANY_ITERATIONS) also
- * ask for the distances of all their queries and vectors, 4 bytes each and 16 GiB
- * at most, and copies of both, in the place of the cache, or behind it for 2 bytes
- * of bounds each and copies, 24 GiB at most; with less than that they run without.  The result does not depend on it. */
+ * not hold 1,024 per row.  Calls that are given distances ahead of the loop
+ * (vl_beam_ahead) ask for 4 bytes for each, 16 GiB at most, and copies of queries
+ * and vectors, in the place of the cache; those that are given bounds for 2 bytes
+ * each and copies, 24 GiB at most, behind it.  With less than that they run
+ * without: what they take with VL_BEAM_NO_TABLE is enough.  The result does not depend on it. */
 int64_t vl_beam_workspace_bytes(const vl_beam_params *p);
+
+/* What a call with these parameters is given ahead of its loop if its workspace
+ * has room for it: VL_BEAM_TABLE (distances), VL_BEAM_BOUNDS or 0.  Or
+ * VL_BEAM_MANY_ITERATIONS: nothing as it stands, but one of them with that flag,
+ * which suits a call with exclusions on the graph that builds start from, and no
+ * other; vl_circulant_graph tells.  That is said of 256 rows and more (the answer
+ * has to be waited for), not with VL_BEAM_NO_CACHE, which asks for a small
+ * workspace, and not while launches are profiled.  Negative: an error. */
+int vl_beam_ahead(const vl_beam_params *p);
+
+/* *circulant (on the device) = 1 if the neighbour list of node i + 1 is that of
+ * node i plus one, modulo n_vectors, in a sample of 64 nodes, else 0. */
+int vl_circulant_graph(const int32_t *beams, int64_t n_vectors, int64_t width,
+                       int32_t *circulant, void *stream);
 
 /* Runs the whole loop of closest_vectors on the search queue in place and
  * returns the number of iterations (a multiple of speculative_readahead) or

@@ -1,29 +1,43 @@
-"""Which calls of the beam loop ask for the distances or bounds of all their queries and vectors, by the bytes of workspace that
-they ask for (include/vlgpu.h); nothing is launched."""
+"""Which calls of the beam loop are given the distances or bounds of all their queries and vectors, by the bytes of workspace that
+they ask for and by vl_beam_ahead (include/vlgpu.h); nothing is launched."""
 import ctypes as C
 
 import pytest
 
-NO_CACHE, SKETCH, MANY, TABLE, NO_TABLE, BOUNDS = 8, 16, 128, 256, 512, 1024  # VL_BEAM_*
+NO_CACHE, SKETCH, MANY, TABLE, NO_TABLE, BOUNDS, KNOWN = 8, 16, 128, 256, 512, 1024, 2048  # VL_BEAM_*
 
 
-def asks(flags, rows=10_000, n=1_000_000, dim=768, width=128, beam=64, visits=4, ef=5, readahead=5, excl=1, metric=0):
-    """Bytes beyond those of the same call without distances and bounds (and without the cache, which they may lie over)."""
+def params(flags, rows=10_000, n=1_000_000, dim=768, width=128, beam=64, visits=4, ef=5, readahead=5, excl=1, metric=0):
     from vectorlink_gpu import _native as nv
 
-    def need(f):
-        p = nv.BeamParams(n_rows=rows, dim=dim, n_vectors=n, width=width, queue_capacity=128 + visits * width, queue_length=128,
-                          beam_size=beam, parallel_visit_count=visits, visit_queue_factor=3, exclude_factor=ef,
-                          speculative_readahead=readahead, excl_cols=excl, flags=f | NO_CACHE, metric=metric)
-        return nv.check(nv.lib().vl_beam_workspace_bytes(C.byref(p)))
-    return need(flags) - need((flags | NO_TABLE) & ~(TABLE | BOUNDS))
+    return nv.BeamParams(n_rows=rows, dim=dim, n_vectors=n, width=width, queue_capacity=128 + visits * width, queue_length=128,
+                         beam_size=beam, parallel_visit_count=visits, visit_queue_factor=3, exclude_factor=ef,
+                         speculative_readahead=readahead, excl_cols=excl, flags=flags, metric=metric)
+
+
+def need(flags, **kw):
+    from vectorlink_gpu import _native as nv
+
+    return nv.check(nv.lib().vl_beam_workspace_bytes(C.byref(params(flags, **kw))))
+
+
+def asks(flags, **kw):
+    """Bytes beyond those of the same call without distances and bounds (and without the cache, which they may lie over)."""
+    flags |= NO_CACHE
+    return need(flags, **kw) - need((flags | NO_TABLE) & ~(TABLE | BOUNDS), **kw)
+
+
+def ahead(flags, **kw):
+    from vectorlink_gpu import _native as nv
+
+    return nv.check(nv.lib().vl_beam_ahead(C.byref(params(flags, **kw))))
 
 
 @pytest.mark.parametrize("n", [1, 2, 63])
 @pytest.mark.parametrize("flags", [SKETCH, SKETCH | MANY, SKETCH | BOUNDS, TABLE])
 def test_a_few_vectors_have_neither(n, flags):
     """(The look at the graph reads the lists of a node and of the next one.)"""
-    assert asks(flags, n=n) == 0
+    assert asks(flags, n=n) == 0 == ahead(flags, n=n)
 
 
 @pytest.mark.parametrize("rows,n,dim", [(8, 70_000_000, 4), (1, 600_000_000, 4)])
@@ -31,3 +45,26 @@ def test_sizes_beyond_the_grid_of_the_distances_do_without(rows, n, dim):
     """(The kernels' launcher refuses them.)"""
     assert asks(TABLE, rows=rows, n=n, dim=dim) == 0
     assert asks(TABLE, rows=rows, n=60_000_000, dim=dim) > 0
+
+
+def test_a_call_that_does_not_say_that_it_is_long_asks_for_no_more_than_without():
+    """Rows that exclude their own ids, 10,000 of 1M x 768 (bounds, 20 GiB) and of 150,000 x 768 (distances, 6 GiB)."""
+    for (sketch, n, given) in ((SKETCH, 1_000_000, BOUNDS), (0, 150_000, TABLE)):
+        assert need(sketch, n=n) == need(sketch | NO_TABLE, n=n)
+        assert need(sketch | MANY, n=n) > need(sketch | NO_TABLE, n=n)
+        assert ahead(sketch | MANY, n=n) == given
+        assert ahead(sketch, n=n) == MANY                                            # the graph is worth a look
+        assert ahead(sketch | KNOWN, n=n) == 0 == ahead(sketch | NO_TABLE, n=n)
+        assert ahead(sketch | NO_CACHE, n=n) == 0 == ahead(sketch, n=n, excl=0)      # a small workspace; a search
+        assert ahead(sketch, n=n, rows=255) == 0
+
+
+def test_a_small_table_needs_no_word():
+    small = dict(rows=4096, n=4096, dim=128, width=64, beam=32)
+    assert ahead(0, **small) == TABLE == ahead(KNOWN, **small) and asks(TABLE, **small) > 0
+
+
+def test_bounds_that_no_launch_could_use_are_not_asked_for():
+    """Lists that fill up before the first progress check run one iteration per launch, which the bounds are not built for."""
+    assert ahead(SKETCH | MANY, readahead=200) == BOUNDS                  # 960 ids, 800 of them
+    assert ahead(SKETCH | MANY, readahead=241) == 0 == asks(SKETCH | BOUNDS, readahead=241)

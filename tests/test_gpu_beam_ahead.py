@@ -1,0 +1,52 @@
+"""What closest_vectors gives a call ahead of its loop: the look at the graph, the workspace, and builds that say what their loops
+are (vectorlink_gpu/ann.py)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from test_gpu_beam_table import config, dev, same, search, vectors
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,width", [(2, 1), (3, 2), (64, 5), (65, 24), (1000, 64), (5003, 128)])
+def test_the_graph_that_builds_start_from(n, width):
+    from vectorlink_gpu.ann import _circulant_graph
+
+    ids = orc.generate_circulant_beams(n, orc.primes(width))
+    assert _circulant_graph(dev(ids))
+    for (node, k) in ((0, 0), ((63 * (n - 1)) // 64 + 1, width - 1)):  # the first and the last list that are read
+        other = ids.copy()
+        other[node, k] = (other[node, k] + 1) % n if n > 2 else 7
+        assert not _circulant_graph(dev(other))
+    empty = ids.copy()
+    empty[:, 0] = 0x7FFFFFFF
+    assert not _circulant_graph(dev(empty)) and not _circulant_graph(dev(ids[:1]))
+
+
+def test_only_the_graph_of_a_first_loop_is_given_the_large_workspace(monkeypatch):
+    from vectorlink_gpu import ann
+
+    (n, rows) = (70_001, 400)
+    v = dev(vectors(n, 64))
+    c = config(beam_size=32)
+    ids = orc.generate_circulant_beams(n, orc.primes(64))
+    other = np.random.default_rng(5).integers(0, n, ids.shape).astype(np.int32)
+    (asked, reserve) = ([], ann._Workspace.reserve)
+    monkeypatch.setattr(ann._Workspace, "reserve", lambda self, nbytes, device: asked.append(nbytes) or reserve(self, nbytes, device))
+    for beams in (ids, other):
+        same(search(v, rows, dev(beams), ids[:rows], c, True, 0), search(v, rows, dev(beams), ids[:rows], c, True, ann.BEAM_NO_TABLE))
+    assert asked[0] > asked[1] == asked[2] == asked[3]
+
+
+def test_later_loops_of_a_build_are_not_looked_at(monkeypatch):
+    from vectorlink_gpu import ann
+
+    (looked, flags, search_) = ([], [], ann.closest_vectors)
+    monkeypatch.setattr(ann, "_circulant_graph", lambda beams: looked.append(1))
+    monkeypatch.setattr(ann, "ann_calculate_recall", lambda *a, **k: (0, 0.0))  # (a recall of 1 ends a build)
+    monkeypatch.setattr(ann, "closest_vectors", lambda *a, **k: flags.append(k["flags"]) or search_(*a, **k))
+    ann.ANN(dev(vectors(6007, 384)), beam_size=48, beam_queue_factor=2)
+    assert flags == [ann.BEAM_MANY_ITERATIONS | ann.BEAM_NO_CACHE, ann.BEAM_KNOWN_GRAPH, ann.BEAM_KNOWN_GRAPH]
+    assert not looked

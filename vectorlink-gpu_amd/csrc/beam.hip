@@ -649,10 +649,10 @@ struct BeamLayout {
     bool may_sketch;     // the call may bring a sketch and use it (as far as its parameters tell: not the rows' addresses)
     bool rows_meet_again;  // what meets_again says
     // the table of all distances (beam_table.hip) and the copies it is made from, over the cache
-    int use_table;  // TableUse
+    bool use_table;
     int64_t table_columns, off_packed_queries, off_packed_vectors, off_table, table_end;
     // or the bounds of all of them (near_products.h), behind the cache
-    int use_near;  // TableUse
+    bool use_near;
     NearPlan near_plan;
     int64_t off_near, near_end;
 };
@@ -690,33 +690,27 @@ bool table_pays(const vl_beam_params *p, const BeamLayout &l, double iterations,
     const double with = candidates * 11e-6, without = candidates * candidate_ps * 1e-6;
     return made + iterations * (with > 4.5 ? with : 4.5) < 0.9 * iterations * (without > 7.5 ? without : 7.5);
 }
-// kTableAsk: if the graph is the one that builds start from.
-//   A batch of a build that says so (VL_BEAM_MANY_ITERATIONS) takes four fifths of the iterations that fill its visited lists and
-// more, a search 85 to 95 (37 to 300 queries), few queries 30; what a call that does not say takes is not known: 15 to 125, and
-// 20 are counted on.  Batches of a build that come without a word
-// exclude their own ids; those of a first loop run as long as any, those of the later loops find most distances in the cache
-// (10,000 rows of 20,011 x 768 4.0 ms without and 5.6 with the table, of 100,000 x 128 6.0 and 8.5), so the graph itself is
-// looked at.  First loops without and with the table, ms: 10,000 rows of 20,011 x 768 60.2 and 12.6, 50,000 x 768 88.2 and 17.6,
+//   A batch of a first loop of a build takes four fifths of the iterations that fill its visited lists and more, a search 85 to
+// 95 (37 to 300 queries), few queries 30 (VL_BEAM_MANY_ITERATIONS); what a call that does not say takes is not known: 15 to 125, and
+// 20 are counted on.  Batches of later loops find most distances in the cache (10,000 rows of 20,011 x 768 4.0 ms without and 5.6
+// with the table, of 100,000 x 128 6.0 and 8.5).  First loops without and with the table, ms: 10,000 rows of 20,011 x 768 60.2 and 12.6, 50,000 x 768 88.2 and 17.6,
 // 200,000 x 768 138.9 and 39.2, 100,003 x 1,536 263 and 40, 100,000 x 128 15.7 and 6.1, 200,000 x 50 10.8 and 6.1, 60,000 x 200 (L2)
 // 72.9 and 12.5, 1,000 rows of 200,000 x 768 15.8 and 7.0, of 50,000 x 100 1.75 and 1.03.
-enum TableUse { kTableNo, kTableYes, kTableAsk };
 constexpr int64_t kTableMostBytes = 16ll << 30;
-TableUse table_use(const vl_beam_params *p, const BeamLayout &l) {
-    if (p->flags & (VL_BEAM_NO_TABLE | VL_BEAM_TWO_LAUNCHES | VL_BEAM_SORT_MERGE | VL_BEAM_NO_WINDOWS | VL_BEAM_WINDOWS)) return kTableNo;
+bool table_use(const vl_beam_params *p, const BeamLayout &l) {
+    if (p->flags & (VL_BEAM_NO_TABLE | VL_BEAM_TWO_LAUNCHES | VL_BEAM_SORT_MERGE | VL_BEAM_NO_WINDOWS | VL_BEAM_WINDOWS)) return false;
     if (l.Vt > kTableMaxVisit || l.VL <= l.Vt || l.VL > kTableMaxQueue || p->queue_length > kTableMaxQueue ||
         l.m > kTableMaxCandidates || p->excl_cols > kTableMaxExcluded || l.Vt * p->speculative_readahead > l.E || p->dim > 2048)
-        return kTableNo;
+        return false;
     if (p->n_vectors < kPairTile || p->n_rows * pair_columns(p->n_vectors) * 4 > kTableMostBytes ||
         !vl_pair_table_fits(p->n_rows, p->n_vectors, p->dim))
-        return kTableNo;
-    if (p->flags & VL_BEAM_TABLE) return kTableYes;
-    if ((p->flags & VL_BEAM_NO_CACHE) && !(p->flags & VL_BEAM_MANY_ITERATIONS)) return kTableNo;  // (asked for a small workspace)
-    if (table_pays(p, l, 20, 20)) return kTableYes;
+        return false;
+    if (p->flags & VL_BEAM_TABLE) return true;
+    if ((p->flags & VL_BEAM_NO_CACHE) && !(p->flags & VL_BEAM_MANY_ITERATIONS)) return false;  // (asked for a small workspace)
+    if (table_pays(p, l, 20, 20)) return true;
     const double all = 0.8 * (double)l.E / (double)l.Vt, search = p->n_rows >= 32 ? 30 : 20;
     const double anywhere = p->n_vectors * p->dim > (8 << 20) ? 30 + 0.08 * (double)p->dim : 30;
-    if (!table_pays(p, l, p->excl_cols > 0 || all < search ? all : search, anywhere)) return kTableNo;
-    if (p->flags & VL_BEAM_MANY_ITERATIONS) return kTableYes;
-    return p->excl_cols > 0 && p->n_rows >= kComputeUnits ? kTableAsk : kTableNo;  // (asking waits for the stream: not for a few rows)
+    return (p->flags & VL_BEAM_MANY_ITERATIONS) && table_pays(p, l, p->excl_cols > 0 || all < search ? all : search, anywhere);
 }
 
 // Whether a call whose table of distances would be too large or too much work is given the products of all its queries and vectors in
@@ -726,27 +720,26 @@ TableUse table_use(const vl_beam_params *p, const BeamLayout &l) {
 // 306 and 85, x 256 55.1 and 41.4, 1M x 384 (degree 48) 43.5 and 37.9, x 256 (degree 32: left alone) 14.3 and 20.5; 1,000 rows of 1M x
 // 768 15.9 and 8.8, 300 of 500,000 x 768 10.6 and 6.2.  The cache is left out: 62.8 ms for the first with it.
 constexpr int64_t kNearMostBytes = 24ll << 30;
-TableUse near_use(const vl_beam_params *p, const BeamLayout &l) {
-    if (!l.may_sketch || l.use_table != kTableNo || p->speculative_readahead < 2) return kTableNo;
-    if (p->flags & (VL_BEAM_NO_TABLE | VL_BEAM_NO_WINDOWS | VL_BEAM_WINDOWS)) return kTableNo;  // (it runs several iterations per launch)
-    if (p->n_vectors < kPairTile || l.near_plan.bytes > kNearMostBytes) return kTableNo;
-    if (p->flags & VL_BEAM_BOUNDS) return kTableYes;
+bool near_use(const vl_beam_params *p, const BeamLayout &l) {
+    // (several iterations to a launch, as long as no list fills up in one)
+    if (!l.may_sketch || l.use_table || p->speculative_readahead < 2 || l.Vt * p->speculative_readahead > l.E) return false;
+    if (p->flags & (VL_BEAM_NO_TABLE | VL_BEAM_NO_WINDOWS | VL_BEAM_WINDOWS)) return false;  // (it runs several iterations per launch)
+    if (p->n_vectors < kPairTile || l.near_plan.bytes > kNearMostBytes) return false;
+    if (p->flags & VL_BEAM_BOUNDS) return true;
     const double rows = (double)p->n_rows, pairs = rows * (double)p->n_vectors, candidates = rows * (double)l.m;
     const double made = 60.0 + pairs * (2.2e-9 * (double)p->dim + 4e-7) + 1.5e-6 * (double)p->n_vectors * (double)p->dim;  // us
     const double iterations = 0.8 * (double)l.E / (double)l.Vt;
     const double saved = iterations * candidates * (0.139 * (double)p->dim - 22.0) * 1e-6;
-    if (made > 0.8 * saved) return kTableNo;
-    if (p->flags & VL_BEAM_MANY_ITERATIONS) return p->excl_cols > 0 ? kTableYes : kTableNo;
-    return p->excl_cols > 0 && p->n_rows >= kComputeUnits ? kTableAsk : kTableNo;
+    return (p->flags & VL_BEAM_MANY_ITERATIONS) && p->excl_cols > 0 && made <= 0.8 * saved;
 }
 
-// *circulant = 1 if the neighbours of node i + 1 are those of node i plus one, in a sample of the nodes (of two at least).
+// *circulant = 1 if the neighbours of node i + 1 are those of node i plus one, in a sample of the nodes (there are two at least).
 constexpr int kCirculantNodes = 64;
-__global__ __launch_bounds__(256) void circulant_graph_kernel(const int32_t *__restrict__ beams, int64_t n, int64_t width, int *circulant) {
+__global__ __launch_bounds__(256) void circulant_graph_kernel(const int32_t *__restrict__ beams, int64_t n, int64_t width, int32_t *circulant) {
     __shared__ int other;
-    if (threadIdx.x == 0) other = 0;
+    if (threadIdx.x == 0) other = n < 2;
     __syncthreads();
-    for (int64_t i = threadIdx.x; i < kCirculantNodes * width; i += 256) {
+    for (int64_t i = threadIdx.x; n >= 2 && i < kCirculantNodes * width; i += 256) {
         const int64_t node = i / width * (n - 1) / kCirculantNodes, k = i % width;
         const int32_t here = beams[node * width + k], next = beams[(node + 1) * width + k];
         if (here < 0 || here >= n || next != (here + 1 == n ? 0 : here + 1)) other = 1;
@@ -828,21 +821,21 @@ int beam_layout(const vl_beam_params *p, BeamLayout *l, bool lean = false) {
     l->memo_slots = slots;
     l->off_memo = o; o = align256(o + p->n_rows * (int64_t)slots * 8);
     l->total = o;
-    l->use_table = lean ? kTableNo : table_use(p, *l);
+    l->use_table = !lean && table_use(p, *l);
     l->table_columns = l->off_packed_queries = l->off_packed_vectors = l->off_table = l->table_end = 0;
-    if (l->use_table != kTableNo) {
+    if (l->use_table) {
         l->table_columns = pair_columns(p->n_vectors);
         l->off_packed_queries = l->off_memo;
         l->off_packed_vectors = l->off_packed_queries + pair_packed_bytes(p->n_rows, p->dim);
         l->off_table = l->off_packed_vectors + pair_packed_bytes(l->table_columns, p->dim);
         l->table_end = l->off_table + p->n_rows * l->table_columns * 4;
     }
-    l->use_near = kTableNo;
+    l->use_near = false;
     l->off_near = l->near_end = 0;
     if (!lean && l->may_sketch) {
         l->near_plan = vl_near_plan(p->n_rows, p->n_vectors, p->dim);
         l->use_near = near_use(p, *l);
-        if (l->use_near != kTableNo) {
+        if (l->use_near) {
             l->off_near = l->total;
             l->near_end = l->off_near + l->near_plan.bytes;
         }
@@ -856,6 +849,36 @@ VL_EXPORT int64_t vl_beam_workspace_bytes(const vl_beam_params *p) {
     BeamLayout l;
     int rc = beam_layout(p, &l);
     return rc < 0 ? rc : std::max(l.total, std::max(l.table_end, l.near_end));
+}
+
+namespace {
+bool profiling() {
+    std::lock_guard<std::mutex> hold(g_prof_mutex);
+    return g_prof.enabled != 0;
+}
+}  // namespace
+
+VL_EXPORT int vl_beam_ahead(const vl_beam_params *p) {
+    BeamLayout l;
+    int rc = beam_layout(p, &l);
+    if (rc < 0) return rc;
+    const bool said = (p->flags & VL_BEAM_MANY_ITERATIONS) != 0, prof = profiling();
+    if (l.use_table) return prof && !said && !(p->flags & VL_BEAM_TABLE) ? 0 : VL_BEAM_TABLE;
+    if (l.use_near) return VL_BEAM_BOUNDS;
+    // (a look at the graph waits for the stream: not for a few rows)
+    if (prof || said || (p->flags & (VL_BEAM_NO_CACHE | VL_BEAM_KNOWN_GRAPH)) || p->excl_cols == 0 || p->n_rows < kComputeUnits) return 0;
+    vl_beam_params of_first_loop = *p;
+    of_first_loop.flags |= VL_BEAM_MANY_ITERATIONS;
+    rc = beam_layout(&of_first_loop, &l);
+    return rc < 0 ? rc : l.use_table || l.use_near ? VL_BEAM_MANY_ITERATIONS : 0;
+}
+
+VL_EXPORT int vl_circulant_graph(const int32_t *beams, int64_t n_vectors, int64_t width, int32_t *circulant, void *stream) {
+    VL_REQUIRE(n_vectors > 0 && width > 0, "bad sizes");
+    VL_REQUIRE(beams && circulant, "null pointer");
+    hipLaunchKernelGGL(circulant_graph_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, beams, n_vectors, width, circulant);
+    VL_LAUNCH_CHECK("circulant_graph_kernel");
+    return VL_OK;
 }
 
 namespace {
@@ -1047,16 +1070,11 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
     // with a sketch every row starts out using it (and the cache, when there is one)
     const bool sketch_from_start = step.sketch != nullptr;
     // (neither with the table of all distances)
-    bool table = use_fused && !no_windows && l.use_table != kTableNo && l.table_end <= workspace_bytes;
-    bool prof;
-    {
-        std::lock_guard<std::mutex> hold(g_prof_mutex);
-        prof = g_prof.enabled != 0 && fixed_iterations == 0;
-    }
+    const bool prof = fixed_iterations == 0 && profiling();
+    bool table = use_fused && !no_windows && l.use_table && l.table_end <= workspace_bytes;
     // what is counted are the rows that are fetched: a profiled call has the table only where it is asked for
     if (prof && !(p->flags & (VL_BEAM_MANY_ITERATIONS | VL_BEAM_TABLE))) table = false;
-    bool near = step.sketch && !no_windows && l.use_near != kTableNo && l.near_end <= workspace_bytes;
-    if (prof && !(p->flags & (VL_BEAM_MANY_ITERATIONS | VL_BEAM_BOUNDS))) near = false;
+    const bool near = step.sketch && !no_windows && l.use_near && l.near_end <= workspace_bytes;
     const int64_t all_slots = p->n_rows * (int64_t)l.memo_slots;
     const bool cleared = !table && !near;  // the cache, with the loop's state
     auto clear_cache = [&]() -> int {
@@ -1089,15 +1107,6 @@ int64_t beam_loop(const vl_beam_params *p, BeamLayout l, const float *queries, c
                            sketch_from_start ? (256 | (1 << 16)) : 256, sketch_from_start ? (int)p->n_rows : 0,
                            clear ? memo : nullptr, all_slots);
         VL_LAUNCH_CHECK("beam_init_kernel");
-    }
-    const bool asked = (table && l.use_table == kTableAsk) || (near && l.use_near == kTableAsk);
-    if (asked) {
-        hipLaunchKernelGGL(circulant_graph_kernel, dim3(1), dim3(256), 0, st, beams, p->n_vectors, p->width, &ctrl->circulant);
-        VL_LAUNCH_CHECK("circulant_graph_kernel");
-        int circulant = 0;
-        VL_HIP(hipMemcpyAsync(&circulant, &ctrl->circulant, sizeof(int), hipMemcpyDeviceToHost, st));
-        VL_HIP(hipStreamSynchronize(st));
-        if (!circulant) table = near = false;
     }
     if (!table) {
         rc = make_ready(!cleared && !near);

@@ -31,7 +31,6 @@ struct BeamCtrl {
                         // workspace was overwritten while the loop ran (VL_ERR_STATE on the host)
     int refused_at;     // iteration that found the call's table of distances of no use (beam_table.hip), or 0
     int unordered;      // that table holds a distance that is not an ordinary number
-    int circulant;      // the graph is the one that builds start from (found out before the loop, where it matters)
     // profiling only, striped by workgroup so that the atomic adds do not queue up on one address:
     unsigned long long evals[kBeamStripes];   // candidate rows actually fetched
     unsigned long long wanted[kBeamStripes];  // candidate distances asked for (fetched or served by the cache)

@@ -56,6 +56,8 @@ _SIGNATURES = {
     "vl_queue_pop": (C.c_int, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr]),
     "vl_seen_add": (C.c_int, [_ptr, _i64, _i64, _ptr, _i64, _ptr, C.POINTER(C.c_int), _ptr]),
     "vl_beam_workspace_bytes": (C.c_int64, [C.POINTER(BeamParams)]),
+    "vl_beam_ahead": (C.c_int, [C.POINTER(BeamParams)]),
+    "vl_circulant_graph": (C.c_int, [_ptr, _i64, _i64, _ptr, _ptr]),
     "vl_closest_vectors": (C.c_int64, [C.POINTER(BeamParams), _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
     "vl_closest_vectors_noalloc": (C.c_int, [C.POINTER(BeamParams), _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr]),
     "vl_closest_vectors_with_sketch": (C.c_int64, [C.POINTER(BeamParams), _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,

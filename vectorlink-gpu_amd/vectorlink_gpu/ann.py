@@ -35,6 +35,7 @@ BEAM_MANY_ITERATIONS = 128  # include/vlgpu.h: VL_BEAM_MANY_ITERATIONS (the loop
 BEAM_TABLE = 256  # include/vlgpu.h: VL_BEAM_TABLE (all distances ahead of the loop wherever that is built; same result)
 BEAM_NO_TABLE = 512  # include/vlgpu.h: VL_BEAM_NO_TABLE (never; same result)
 BEAM_BOUNDS = 1024  # include/vlgpu.h: VL_BEAM_BOUNDS (bounds of all distances wherever a call has a sketch and no such table; same result)
+BEAM_KNOWN_GRAPH = 2048  # include/vlgpu.h: VL_BEAM_KNOWN_GRAPH (the graph is not the one that builds start from: it is not looked at)
 
 
 def _beam_params(batch: int, dim: int, n_vectors: int, width: int, queue: Queue, config: Dict,
@@ -143,6 +144,13 @@ def closest_vectors_stepwise(query_vecs: Tensor, search_queue: Queue, vectors: T
     return count
 
 
+def _circulant_graph(beams: Tensor) -> bool:
+    """Whether a graph is the one that builds start from; waits for the stream."""
+    found = torch.empty(1, dtype=torch.int32, device=beams.device)
+    nv.check(nv.lib().vl_circulant_graph(nv.ptr(beams), beams.size(0), beams.size(1), nv.ptr(found), nv.stream()))
+    return bool(found.item())
+
+
 @log_time
 def closest_vectors(query_vecs: Tensor, search_queue: Queue, vectors: Tensor, beams: Tensor, config: Dict,
                     exclude: Optional[Tensor] = None, flags: int = 0, sketch: Optional[Tensor] = None) -> int:
@@ -176,6 +184,8 @@ def closest_vectors(query_vecs: Tensor, search_queue: Queue, vectors: Tensor, be
         excl = exclude.contiguous()
     p = _beam_params(batch, dim, vectors.size(0), beams.size(1), search_queue, config,
                      0 if excl is None else excl.size(1), flags | (BEAM_USES_SKETCH if sketch is not None else 0))
+    if nv.check(nv.lib().vl_beam_ahead(ctypes.byref(p))) == BEAM_MANY_ITERATIONS and _circulant_graph(beams):
+        p.flags |= BEAM_MANY_ITERATIONS  # a batch of a first loop that comes without a word
     need = nv.check(nv.lib().vl_beam_workspace_bytes(ctypes.byref(p)))
     workspace = _workspace(vectors.device)
     with workspace.lock:
@@ -281,7 +291,8 @@ class GraphBuild:
                 with torch.cuda.stream(stream):
                     exclude = excluding_self(start, end, ql, device)
                     # (searches of the circulant graph, whose edges lead anywhere, are long ones)
-                    first = BEAM_MANY_ITERATIONS if loop == 0 and self.circulant_start and not self.stale else 0
+                    first = loop == 0 and self.circulant_start
+                    flags = BEAM_MANY_ITERATIONS if first else BEAM_KNOWN_GRAPH if loop > 0 else 0
                     queue = Queue(end - start, ql, ql + remaining_capacity, device=device)
                     queue.insert(self.beams.narrow(0, start, end - start), seed_distances.narrow(0, start, end - start))
                     if self.sketch is not None:
@@ -290,12 +301,12 @@ class GraphBuild:
                         # more than those repeats save, with long ones less (per launch, without and with the
                         # cache: 0.35 and 0.37 ms at 384 columns, 0.73 and 0.64 ms at 768, 1.54 and 1.24 ms at 1536)
                         if first and vectors.size(1) <= 512:
-                            first |= BEAM_NO_CACHE
-                        t = search(vectors[start:end], queue, vectors, self.beams, config, exclude, flags=first,
+                            flags |= BEAM_NO_CACHE
+                        t = search(vectors[start:end], queue, vectors, self.beams, config, exclude, flags=flags,
                                    sketch=self.sketch)
                     else:
                         t = search(vectors[start:end], queue, vectors, self.beams, config, exclude,
-                                   **({"flags": first} if first else {}))
+                                   **({} if self.stale else {"flags": flags}))
                     next_beams.narrow(0, start, end - start).copy_(queue.indices.narrow(1, 0, ql))
                     next_beam_distances.narrow(0, start, end - start).copy_(queue.distances.narrow(1, 0, ql))
                     stream.synchronize()
