@@ -50,3 +50,33 @@ def test_later_loops_of_a_build_are_not_looked_at(monkeypatch):
     ann.ANN(dev(vectors(6007, 384)), beam_size=48, beam_queue_factor=2)
     assert flags == [ann.BEAM_MANY_ITERATIONS | ann.BEAM_NO_CACHE, ann.BEAM_KNOWN_GRAPH, ann.BEAM_KNOWN_GRAPH]
     assert not looked
+
+
+def test_a_size_that_cannot_be_had_is_asked_for_once(monkeypatch):
+    """... until the workspaces are let go; the smaller block stays where it is meanwhile."""
+    from vectorlink_gpu import ann
+
+    (n, rows) = (3000, 200)
+    v = dev(vectors(n, 24))
+    beams = dev(orc.generate_circulant_beams(n, orc.primes(32)))
+    seeds = orc.generate_circulant_beams(n, orc.primes(32))[:rows]
+    c = config(beam_size=16, exclude_factor=2)
+    want = search(v, rows, beams, seeds, c, True, ann.BEAM_NO_TABLE | ann.BEAM_NO_CACHE)
+    (made, most, empty) = ([], 1 << 21, torch.empty)
+    ann.release_workspaces()
+
+    def no_room(size, *a, **k):
+        if k.get("dtype") == torch.uint8:
+            made.append(size)
+            if size > most:
+                raise torch.OutOfMemoryError("no room")
+        return empty(size, *a, **k)
+
+    monkeypatch.setattr(ann.torch, "empty", no_room)
+    for _ in range(3):
+        same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE), want)
+    assert len(made) == 2 and made[1] <= most < made[0]
+    ann.release_workspaces()
+    same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE), want)
+    assert made[2:] == made[:2]
+    ann.release_workspaces()

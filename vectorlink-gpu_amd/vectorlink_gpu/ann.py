@@ -57,9 +57,13 @@ class _Workspace:
     def __init__(self):
         self.lock = threading.Lock()
         self.tensor: Optional[Tensor] = None
+        self.too_large: Optional[int] = None  # a size that could not be had
+
+    def has(self, nbytes: int) -> bool:
+        return self.tensor is not None and self.tensor.numel() >= nbytes
 
     def reserve(self, nbytes: int, device) -> Tensor:
-        if self.tensor is None or self.tensor.numel() < nbytes:
+        if not self.has(nbytes):
             self.tensor = None  # let the old block go before the larger one is asked for
             self.tensor = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         return self.tensor
@@ -91,7 +95,7 @@ def release_workspaces(streams=None) -> None:
             if only is not None and stream not in only:
                 continue
             with ws.lock:
-                ws.tensor = None
+                (ws.tensor, ws.too_large) = (None, None)
 
 
 _BUILD_STREAMS: Dict[str, list] = {}
@@ -189,15 +193,20 @@ def closest_vectors(query_vecs: Tensor, search_queue: Queue, vectors: Tensor, be
     need = nv.check(nv.lib().vl_beam_workspace_bytes(ctypes.byref(p)))
     workspace = _workspace(vectors.device)
     with workspace.lock:
-        try:
-            ws = workspace.reserve(need, vectors.device)
-        except torch.OutOfMemoryError:
-            # what the call takes without the distances of all its queries and vectors, which it runs without then
+        least = need
+        if not workspace.has(need):
+            # what the call takes without distances or bounds of all its queries and vectors, which it can run without
             least = nv.check(nv.lib().vl_beam_workspace_bytes(ctypes.byref(
                 _beam_params(batch, dim, vectors.size(0), beams.size(1), search_queue, config, p.excl_cols,
                              p.flags | BEAM_NO_TABLE))))
+            if workspace.too_large is not None and need >= workspace.too_large:
+                need = min(need, least)  # (asking again would cost the block that is there and torch's cache)
+        try:
+            ws = workspace.reserve(need, vectors.device)
+        except torch.OutOfMemoryError:
             if least >= need:
                 raise
+            workspace.too_large = need
             ws = workspace.reserve(least, vectors.device)
         if sketch is not None:
             assert sketch.dtype == torch.uint8 and sketch.is_contiguous() and sketch.is_cuda
