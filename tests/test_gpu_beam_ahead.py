@@ -80,3 +80,44 @@ def test_a_size_that_cannot_be_had_is_asked_for_once(monkeypatch):
     same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE), want)
     assert made[2:] == made[:2]
     ann.release_workspaces()
+
+
+def test_as_much_again_is_left_for_others(monkeypatch):
+    """10,000 of 100,000 x 64: 4 GiB of distances."""
+    from vectorlink_gpu import ann
+
+    (n, rows) = (100_000, 10_000)
+    v = dev(vectors(n, 64))
+    c = config(beam_size=8, beam_queue_factor=2, exclude_factor=1)
+    beams = dev(orc.generate_circulant_beams(n, orc.primes(16)))
+    seeds = orc.generate_circulant_beams(n, orc.primes(16))[:rows]
+    want = search(v, rows, beams, seeds, c, True, ann.BEAM_NO_TABLE)
+    stream = torch.cuda.current_stream()
+
+    def block(room):
+        ann.release_workspaces()
+        monkeypatch.setattr(ann, "_room", lambda device: room)
+        same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE), want)
+        return ann._WORKSPACES[("cuda:0", int(stream.cuda_stream))].tensor.numel()
+
+    large = block(1 << 40)
+    small = block(0)
+    assert large - small > 3 << 30
+    assert block(small + 2 * (large - small)) == large and block(small + 2 * (large - small) - 1) == small
+    # a block that is there counts: it goes before a larger one is asked for
+    monkeypatch.setattr(ann, "_room", lambda device: 2 * (large - small))
+    same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE), want)
+    assert ann._WORKSPACES[("cuda:0", int(stream.cuda_stream))].tensor.numel() == large
+    ann.release_workspaces()
+
+
+def test_room_is_what_is_free_and_what_torch_keeps():
+    from vectorlink_gpu import ann
+
+    device = torch.device("cuda:0")
+    torch.cuda.synchronize()
+    before = ann._room(device)
+    x = torch.empty(3 << 30, dtype=torch.uint8, device=device)
+    assert abs(before - (3 << 30) - ann._room(device)) < 64 << 20
+    del x
+    assert abs(before - ann._room(device)) < 64 << 20  # (torch keeps the block)

@@ -68,6 +68,36 @@ class _Workspace:
             self.tensor = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         return self.tensor
 
+    def reserve_up_to(self, most: int, least: int, device) -> Tensor:
+        """A block of `most` bytes where there is room for it, else of `least`."""
+        if most > least:
+            if self.too_large is not None and most >= self.too_large:
+                most = least  # (asking again would cost the block that is there and torch's cache)
+            elif most - least > _ALWAYS_TAKEN:
+                own = 0 if self.tensor is None else self.tensor.numel()
+                if 2 * (most - least) > _room(device) + own - least:
+                    most = least
+        try:
+            return self.reserve(most, device)
+        except torch.OutOfMemoryError:
+            if least >= most:
+                raise
+            self.too_large = most
+            return self.reserve(least, device)
+
+
+# Distances and bounds of all vectors are an option of tens of GiB per batch in flight: what a call takes beyond what it cannot
+# do without leaves as much again for whatever is allocated next (the other batches, the tables of a build).  Parts below
+# _ALWAYS_TAKEN are not worth the question.  The lock: the batches in flight must not all be told of the same room.
+_ALWAYS_TAKEN = 256 << 20
+_ROOM_LOCK = threading.Lock()
+
+
+def _room(device) -> int:
+    """Bytes that allocations on the device can still have: what is free and what torch keeps of what was given back."""
+    (free, _) = torch.cuda.mem_get_info(device)
+    return free + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+
 
 _WORKSPACES: Dict[Tuple[str, int], _Workspace] = {}
 _WORKSPACES_LOCK = threading.Lock()
@@ -193,21 +223,15 @@ def closest_vectors(query_vecs: Tensor, search_queue: Queue, vectors: Tensor, be
     need = nv.check(nv.lib().vl_beam_workspace_bytes(ctypes.byref(p)))
     workspace = _workspace(vectors.device)
     with workspace.lock:
-        least = need
-        if not workspace.has(need):
+        if workspace.has(need):
+            ws = workspace.reserve(need, vectors.device)
+        else:
             # what the call takes without distances or bounds of all its queries and vectors, which it can run without
             least = nv.check(nv.lib().vl_beam_workspace_bytes(ctypes.byref(
                 _beam_params(batch, dim, vectors.size(0), beams.size(1), search_queue, config, p.excl_cols,
                              p.flags | BEAM_NO_TABLE))))
-            if workspace.too_large is not None and need >= workspace.too_large:
-                need = min(need, least)  # (asking again would cost the block that is there and torch's cache)
-        try:
-            ws = workspace.reserve(need, vectors.device)
-        except torch.OutOfMemoryError:
-            if least >= need:
-                raise
-            workspace.too_large = need
-            ws = workspace.reserve(least, vectors.device)
+            with _ROOM_LOCK:
+                ws = workspace.reserve_up_to(need, least, vectors.device)
         if sketch is not None:
             assert sketch.dtype == torch.uint8 and sketch.is_contiguous() and sketch.is_cuda
             assert sketch.size() == (vectors.size(0), sketch_row_bytes(dim)), "not a sketch of these vectors"
