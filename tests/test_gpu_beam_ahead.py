@@ -25,6 +25,17 @@ def test_the_graph_that_builds_start_from(n, width):
     assert not _circulant_graph(dev(empty)) and not _circulant_graph(dev(ids[:1]))
 
 
+def test_a_captured_call_is_not_looked_at(monkeypatch):
+    """It is refused by the loop, which says why; waiting for the stream would end the capture."""
+    from vectorlink_gpu import _native as nv
+    from vectorlink_gpu.ann import _circulant_graph
+
+    beams = dev(orc.generate_circulant_beams(100, orc.primes(8)))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(nv, "lib", None)  # (no launch)
+    assert not _circulant_graph(beams)
+
+
 def test_only_the_graph_of_a_first_loop_is_given_the_large_workspace(monkeypatch):
     from vectorlink_gpu import ann
 

@@ -180,6 +180,8 @@ def closest_vectors_stepwise(query_vecs: Tensor, search_queue: Queue, vectors: T
 
 def _circulant_graph(beams: Tensor) -> bool:
     """Whether a graph is the one that builds start from; waits for the stream."""
+    if torch.cuda.is_current_stream_capturing():  # (the loop will refuse the call and leave the capture as it is)
+        return False
     found = torch.empty(1, dtype=torch.int32, device=beams.device)
     nv.check(nv.lib().vl_circulant_graph(nv.ptr(beams), beams.size(0), beams.size(1), nv.ptr(found), nv.stream()))
     return bool(found.item())
