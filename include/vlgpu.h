@@ -248,9 +248,10 @@ typedef struct vl_beam_params {
 #define VL_BEAM_TABLE 256
 #define VL_BEAM_NO_TABLE 512
 /* A call that says so, with a sketch and with exclusions, and too large for all
- * distances, may be given bounds of all of them instead.  VL_BEAM_BOUNDS: always, where the call can use a sketch
- * and has no such table; VL_BEAM_NO_TABLE: never.  Neither is made of fewer than
- * 64 vectors. */
+ * distances, may be given bounds of all of them instead.  VL_BEAM_BOUNDS: always,
+ * where the call can use a sketch, and no distances (unless VL_BEAM_TABLE asks
+ * for those); VL_BEAM_NO_TABLE: never.  Neither is made of fewer than 64 vectors,
+ * nor where the visited lists fill up before the first progress check. */
 #define VL_BEAM_BOUNDS 1024
 /* The caller knows that its graph is not the one that builds start from
  * (vl_circulant_graph): vl_beam_ahead proposes no look at it. */

@@ -64,6 +64,16 @@ def test_a_small_table_needs_no_word():
     assert ahead(0, **small) == TABLE == ahead(KNOWN, **small) and asks(TABLE, **small) > 0
 
 
+def test_bounds_where_they_are_asked_for():
+    """... and the sizes would have the distances: of rows that exclude their own ids and of a small table."""
+    for kw in (dict(rows=300, n=2500, dim=256, width=32, beam=16), dict(rows=257, n=1530, dim=128, width=48, beam=24),
+               dict(rows=4096, n=4096, dim=128, width=64, beam=32)):
+        for said in (0, MANY):
+            assert ahead(SKETCH | BOUNDS | said, **kw) == BOUNDS
+            assert ahead(SKETCH | BOUNDS | TABLE | said, **kw) == TABLE
+            assert ahead(BOUNDS | said, **kw) == ahead(said, **kw)  # brings no sketch
+
+
 def test_bounds_that_no_launch_could_use_are_not_asked_for():
     """Lists that fill up before the first progress check run one iteration per launch, which the bounds are not built for."""
     assert ahead(SKETCH | MANY, readahead=200) == BOUNDS                  # 960 ids, 800 of them

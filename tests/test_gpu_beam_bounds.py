@@ -13,12 +13,16 @@ pytestmark = pytest.mark.gpu
 
 
 def both(v, rows, beams, seeds, c, exclude=True, flags=0):
-    """Results with the bounds and without bounds and sketch; the first ones' rows looked at through the sketch are none."""
-    from vectorlink_gpu import _native as nv
-    from vectorlink_gpu.ann import BEAM_BOUNDS, BEAM_NO_TABLE
+    """Results with the bounds and without bounds and sketch, and what was counted in a third run, with the bounds."""
+    from vectorlink_gpu import Queue, _native as nv
+    from vectorlink_gpu.ann import BEAM_BOUNDS, BEAM_NO_TABLE, BEAM_USES_SKETCH, _beam_params
     from vectorlink_gpu.kernels import build_sketch
 
     g = dev(v)
+    length = seeds.shape[1]
+    q = Queue(rows, length, length + max(length, beams.size(1) * c["parallel_visit_count"]))
+    p = _beam_params(rows, v.shape[1], v.shape[0], beams.size(1), q, c, int(exclude), BEAM_BOUNDS | BEAM_USES_SKETCH | flags)
+    assert nv.lib().vl_beam_ahead(C.byref(p)) == BEAM_BOUNDS  # (a call that took the distances would show nothing)
     sketch = build_sketch(g)
     want = search(g, rows, beams, seeds, c, exclude, BEAM_NO_TABLE | flags)
     got = search(g, rows, beams, seeds, c, exclude, BEAM_NO_TABLE | flags, sketch=sketch)

@@ -706,6 +706,7 @@ bool table_use(const vl_beam_params *p, const BeamLayout &l) {
         !vl_pair_table_fits(p->n_rows, p->n_vectors, p->dim))
         return false;
     if (p->flags & VL_BEAM_TABLE) return true;
+    if ((p->flags & VL_BEAM_BOUNDS) && l.may_sketch) return false;  // (wants those)
     if ((p->flags & VL_BEAM_NO_CACHE) && !(p->flags & VL_BEAM_MANY_ITERATIONS)) return false;  // (asked for a small workspace)
     if (table_pays(p, l, 20, 20)) return true;
     const double all = 0.8 * (double)l.E / (double)l.Vt, search = p->n_rows >= 32 ? 30 : 20;

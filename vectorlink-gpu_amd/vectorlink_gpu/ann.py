@@ -34,7 +34,7 @@ BEAM_NO_WINDOWS = 64  # include/vlgpu.h: VL_BEAM_NO_WINDOWS (one iteration per l
 BEAM_MANY_ITERATIONS = 128  # include/vlgpu.h: VL_BEAM_MANY_ITERATIONS (the loop is expected to be a long one; same result)
 BEAM_TABLE = 256  # include/vlgpu.h: VL_BEAM_TABLE (all distances ahead of the loop wherever that is built; same result)
 BEAM_NO_TABLE = 512  # include/vlgpu.h: VL_BEAM_NO_TABLE (never; same result)
-BEAM_BOUNDS = 1024  # include/vlgpu.h: VL_BEAM_BOUNDS (bounds of all distances wherever a call has a sketch and no such table; same result)
+BEAM_BOUNDS = 1024  # include/vlgpu.h: VL_BEAM_BOUNDS (bounds of all distances, not the distances, wherever a call has a sketch; same result)
 BEAM_KNOWN_GRAPH = 2048  # include/vlgpu.h: VL_BEAM_KNOWN_GRAPH (the graph is not the one that builds start from: it is not looked at)
 
 
