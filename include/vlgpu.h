@@ -241,8 +241,8 @@ typedef struct vl_beam_params {
  * starts anywhere, or a batch of a build's first loop, whose graph's edges lead
  * anywhere.  Such a call is the more likely to be given the distances of all its
  * queries and vectors ahead of the loop, which iterations then look up; one that
- * does not say so is if twenty iterations on a graph of near neighbours pay for
- * it.  VL_BEAM_TABLE: always, where the kernels are built for the call's sizes,
+ * does not say so is if the few iterations that a graph of near neighbours takes
+ * pay for it.  VL_BEAM_TABLE: always, where the kernels are built for the call's sizes,
  * VL_BEAM_NO_TABLE: never. */
 #define VL_BEAM_MANY_ITERATIONS 128
 #define VL_BEAM_TABLE 256

@@ -7,10 +7,11 @@ import pytest
 NO_CACHE, SKETCH, MANY, TABLE, NO_TABLE, BOUNDS, KNOWN = 8, 16, 128, 256, 512, 1024, 2048  # VL_BEAM_*
 
 
-def params(flags, rows=10_000, n=1_000_000, dim=768, width=128, beam=64, visits=4, ef=5, readahead=5, excl=1, metric=0):
+def params(flags, rows=10_000, n=1_000_000, dim=768, width=128, beam=64, visits=4, ef=5, readahead=5, excl=1, metric=0,
+           length=128):
     from vectorlink_gpu import _native as nv
 
-    return nv.BeamParams(n_rows=rows, dim=dim, n_vectors=n, width=width, queue_capacity=128 + visits * width, queue_length=128,
+    return nv.BeamParams(n_rows=rows, dim=dim, n_vectors=n, width=width, queue_capacity=length + max(length, visits * width), queue_length=length,
                          beam_size=beam, parallel_visit_count=visits, visit_queue_factor=3, exclude_factor=ef,
                          speculative_readahead=readahead, excl_cols=excl, flags=flags, metric=metric)
 
@@ -62,6 +63,26 @@ def test_a_call_that_does_not_say_that_it_is_long_asks_for_no_more_than_without(
 def test_a_small_table_needs_no_word():
     small = dict(rows=4096, n=4096, dim=128, width=64, beam=32)
     assert ahead(0, **small) == TABLE == ahead(KNOWN, **small) and asks(TABLE, **small) > 0
+
+
+# (rows, vectors, columns, degree, queue): where storing the distances takes longer than looking at them saves, and where it does not
+@pytest.mark.parametrize("given,sizes", [
+    (0, (10_000, 100_000, 4, 64, 10)), (0, (10_000, 60_000, 24, 64, 10)), (0, (10_000, 60_000, 25, 64, 128)), (0, (10_000, 20_011, 64, 64, 10)),
+    (TABLE, (10_000, 4_096, 24, 64, 10)), (TABLE, (10_000, 20_011, 24, 64, 10)), (TABLE, (10_000, 20_011, 64, 64, 128)),
+    (TABLE, (2_000, 10_000, 24, 64, 10))])
+def test_searches_that_say_nothing_pay_for_the_stores(given, sizes):
+    (rows, n, dim, degree, length) = sizes
+    assert ahead(0, rows=rows, n=n, dim=dim, width=degree, beam=degree, excl=0, length=length) == given
+
+
+@pytest.mark.parametrize("given,sizes", [
+    (0, (10_000, 400_000, 4, 24, 0)), (0, (10_000, 150_000, 4, 24, 0)), (0, (300, 400_000, 4, 32, 0)),
+    (TABLE, (10_000, 60_000, 16, 24, 0)), (TABLE, (10_000, 60_000, 64, 64, 0)), (TABLE, (37, 20_011, 50, 24, 0)),
+    (0, (10_000, 400_000, 16, 24, 1)), (TABLE, (10_000, 150_000, 50, 24, 1)), (TABLE, (10_000, 100_000, 128, 32, 1)),
+    (TABLE, (10_000, 20_011, 768, 64, 1))])
+def test_long_calls_pay_for_the_stores(given, sizes):
+    (rows, n, dim, degree, first_loop) = sizes
+    assert ahead(MANY, rows=rows, n=n, dim=dim, width=degree * (1 + first_loop), beam=degree, excl=first_loop, length=2 * degree) == given
 
 
 def test_bounds_where_they_are_asked_for():

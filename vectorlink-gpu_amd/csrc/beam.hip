@@ -690,6 +690,40 @@ bool table_pays(const vl_beam_params *p, const BeamLayout &l, double iterations,
     const double with = candidates * 11e-6, without = candidates * candidate_ps * 1e-6;
     return made + iterations * (with > 4.5 ? with : 4.5) < 0.9 * iterations * (without > 7.5 ? without : 7.5);
 }
+// And whether it still is when the stores count: a pair is 1.1 ps to store (the partial sums that short rows leave empty included) and
+// 0.0175 ps a column as products, 1.2 and 0.045 as squared differences (10,000 queries of 100,000 x 4 1.27 ms, x 32 1.65, x 128 3.2, of
+// 20,011 x 256 1.14, x 768 2.9; squared differences of 100,000 x 4 1.69, x 128 6.9).  Above, which rows of some 60 columns and more
+// decide, they are left out against iterations that are counted low; here these are what was measured.
+//   First loops fill their visited lists (where there are no more than some thousand vectors, before).  Searches that say that they are
+// long take the longer the more queries wait for each other: 10 to 60 iterations with 40, 15 to 125 with 300, 45 to 220 with 2,000 and
+// more.  Searches with dense seeds, which say nothing, took 5 to 15 with queues of 10, 15 and more with longer ones (half the queue's
+// length is counted on, 25 at most), and 40 ps and 0.08 a column for a candidate in the first five iterations, which fetch what they look at.
+//   Without and with the distances, us.  10,000 queries with dense seeds and queues of 10, degree 64, at 4,096 x 24 569 and 270, 20,011 x 24 567
+// and 542; left alone: 20,011 x 64 601 and 673, 60,000 x 24 2,567 and 2,787, 100,000 x 4 947 and 2,000; queues of 128 at 20,011 x 64 3,231
+// and 2,587.  Searches that say that they are long, 10,000 queries: degree 24 at 60,000 x 16 3,014 and 2,420, degree 64 at 60,000 x 64 7,094
+// and 5,498; left alone: degree 24 at 150,000 x 4 2,865 and 3,477, 400,000 x 4 2,383 and 6,697.  First loops, degree 24: 150,000 x 50 7,670
+// and 4,436; left alone: 400,000 x 16 5,727 and 7,300.
+struct ExpectedLoop {
+    double iterations;
+    double candidate_ps, first_ps;  // a candidate without the distances: in all iterations but the first five, in those
+    double lookup_ps;               // with them
+};
+bool stores_pay(const vl_beam_params *p, const BeamLayout &l, const ExpectedLoop &e) {
+    const double candidates = (double)p->n_rows * (double)l.m, elements = (double)p->n_vectors * (double)p->dim, dim = (double)p->dim;
+    const double pairs = (double)(pair_tiles(p->n_rows) * kPairTile) * (double)p->n_vectors;
+    const double made = 40.0 + 0.02 * dim + 2e-6 * elements + pairs * (p->metric == VL_METRIC_L2 ? 1.2e-6 + 4.5e-8 * dim : 1.1e-6 + 1.75e-8 * dim);  // us
+    const double with = e.iterations * std::max(4.5, candidates * e.lookup_ps * 1e-6);
+    const double without = e.iterations * std::max(7.5, candidates * e.candidate_ps * 1e-6) +
+                           std::min(5.0, e.iterations) * candidates * (e.first_ps - e.candidate_ps) * 1e-6;
+    return made + with < 0.95 * without;
+}
+ExpectedLoop expected_loop(const vl_beam_params *p, const BeamLayout &l, bool said) {
+    const double most = (double)l.E / (double)l.Vt, anywhere = 30.0 + 0.08 * (double)p->dim;
+    const double search = p->n_rows < 32 ? 20.0 : p->n_rows < 200 ? 30.0 : p->n_rows < 1000 ? 45.0 : 60.0;
+    if (!said) return {std::min(25.0, 0.5 * (double)p->queue_length), 20.0, 40.0 + 0.08 * (double)p->dim, 11.0};
+    if (p->excl_cols > 0) return {most, anywhere, anywhere, 10.0};
+    return {std::min(most, search), anywhere, anywhere, 11.0};
+}
 //   A batch of a first loop of a build takes four fifths of the iterations that fill its visited lists and more, a search 85 to
 // 95 (37 to 300 queries), few queries 30 (VL_BEAM_MANY_ITERATIONS); what a call that does not say takes is not known: 15 to 125, and
 // 20 are counted on.  Batches of later loops find most distances in the cache (10,000 rows of 20,011 x 768 4.0 ms without and 5.6
@@ -708,10 +742,11 @@ bool table_use(const vl_beam_params *p, const BeamLayout &l) {
     if (p->flags & VL_BEAM_TABLE) return true;
     if ((p->flags & VL_BEAM_BOUNDS) && l.may_sketch) return false;  // (wants those)
     if ((p->flags & VL_BEAM_NO_CACHE) && !(p->flags & VL_BEAM_MANY_ITERATIONS)) return false;  // (asked for a small workspace)
-    if (table_pays(p, l, 20, 20)) return true;
     const double all = 0.8 * (double)l.E / (double)l.Vt, search = p->n_rows >= 32 ? 30 : 20;
     const double anywhere = p->n_vectors * p->dim > (8 << 20) ? 30 + 0.08 * (double)p->dim : 30;
-    return (p->flags & VL_BEAM_MANY_ITERATIONS) && table_pays(p, l, p->excl_cols > 0 || all < search ? all : search, anywhere);
+    if (table_pays(p, l, 20, 20) && stores_pay(p, l, expected_loop(p, l, false))) return true;
+    return (p->flags & VL_BEAM_MANY_ITERATIONS) && table_pays(p, l, p->excl_cols > 0 || all < search ? all : search, anywhere) &&
+           stores_pay(p, l, expected_loop(p, l, true));
 }
 
 // Whether a call whose table of distances would be too large or too much work is given the products of all its queries and vectors in
