@@ -13,8 +13,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "vectorlink-gpu_amd")
 OPT = "/opt/rocm/llvm/bin/opt"
 
-# a kernel of each kind: one iteration and several, without and with the sketch, 16-byte loads and single elements, sums that
-# become distances right away and together
+# a kernel of each kind: one iteration and several, without and with the sketch, with the bounds of all vectors, 16-byte loads and
+# single elements, sums that become distances right away and together
 KERNELS = """#include "beam_kernels.h"
 namespace {
 template __global__ void beam_step_kernel_w<2, 16, 4, 128, 8>(StepArgs);
@@ -25,6 +25,8 @@ template __global__ void beam_window_kernel<2, 16, 2, kRowUnalignedSums, 128, 1>
 template __global__ void beam_window_kernel<1, 64, 8, kRowAligned, 256, 6>(StepArgs);
 template __global__ void beam_step_sketch_kernel<3, 64, 1, 256, 3, 16, 1, 8>(StepArgs);
 template __global__ void beam_window_sketch_kernel<3, 64, 1, 256, 3, 16, 1, 6>(StepArgs);
+template __global__ void beam_window_near_kernel<3, 64, 2, 256, 3, 6>(StepArgs);
+template __global__ void beam_window_near_kernel<6, 64, 1, 256, 6, 5>(StepArgs);
 }
 """
 
@@ -83,7 +85,7 @@ def test_no_barrier_of_the_step_lies_behind_a_branch_of_lanes(tmp_path):
                     str(src), "-o", str(ir)], check=True, capture_output=True)
     told = subprocess.run([OPT, "-disable-output", "-passes=print<uniformity>", str(ir)], check=True, capture_output=True, text=True)
     kernels = dict(_kernels(told.stderr))
-    assert len(kernels) == 8 and all(sum(b[2] for b in k.values()) >= 8 for k in kernels.values())
+    assert len(kernels) == 10 and all(sum(b[2] for b in k.values()) >= 8 for k in kernels.values())
     assert all(any(b[1] for b in k.values()) for k in kernels.values())  # (the printer does tell them apart)
     for name, blocks in kernels.items():
         assert not _barriers_behind_lanes(blocks), name
