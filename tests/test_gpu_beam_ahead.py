@@ -85,10 +85,10 @@ def test_a_size_that_cannot_be_had_is_asked_for_once(monkeypatch):
 
     monkeypatch.setattr(ann.torch, "empty", no_room)
     for _ in range(3):
-        same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE), want)
+        same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE, table=False), want)
     assert len(made) == 2 and made[1] <= most < made[0]
     ann.release_workspaces()
-    same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE), want)
+    same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE, table=False), want)
     assert made[2:] == made[:2]
     ann.release_workspaces()
 
@@ -105,16 +105,16 @@ def test_as_much_again_is_left_for_others(monkeypatch):
     want = search(v, rows, beams, seeds, c, True, ann.BEAM_NO_TABLE)
     stream = torch.cuda.current_stream()
 
-    def block(room):
+    def block(room, table=False):
         ann.release_workspaces()
         monkeypatch.setattr(ann, "_room", lambda device: room)
-        same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE), want)
+        same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE, table=table), want)
         return ann._WORKSPACES[("cuda:0", int(stream.cuda_stream))].tensor.numel()
 
-    large = block(1 << 40)
+    large = block(1 << 40, True)
     small = block(0)
     assert large - small > 3 << 30
-    assert block(small + 2 * (large - small)) == large and block(small + 2 * (large - small) - 1) == small
+    assert block(small + 2 * (large - small), True) == large and block(small + 2 * (large - small) - 1) == small
     # a block that is there counts: it goes before a larger one is asked for
     monkeypatch.setattr(ann, "_room", lambda device: 2 * (large - small))
     same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE), want)

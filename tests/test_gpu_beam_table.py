@@ -31,10 +31,20 @@ def config(**kw):
     return c
 
 
-def search(v, rows, beams, seeds, c, exclude, flags, sketch=None, workspace=None):
-    """(iterations, ids, distance bits) of rows 0 .. rows - 1 searched from seeds (ids)."""
+def ahead(rows, n, dim, beams, queue, c, exclude, flags):
+    """What the sizes and the flags give a call ahead of its loop (include/vlgpu.h: vl_beam_ahead)."""
+    from vectorlink_gpu import _native as nv
+    from vectorlink_gpu.ann import _beam_params
+
+    p = _beam_params(rows, dim, n, beams.size(1), queue, c, int(exclude), flags)
+    return nv.check(nv.lib().vl_beam_ahead(C.byref(p))), nv.check(nv.lib().vl_beam_workspace_bytes(C.byref(p)))
+
+
+def search(v, rows, beams, seeds, c, exclude, flags, sketch=None, table=True):
+    """(iterations, ids, distance bits) of rows 0 .. rows - 1 searched from seeds (ids).  A call that asks for the table is given
+    it, and finds the room (table=False: is expected not to find it)."""
     from vectorlink_gpu import Queue
-    from vectorlink_gpu.ann import closest_vectors, excluding_self
+    from vectorlink_gpu.ann import BEAM_TABLE, BEAM_USES_SKETCH, _workspace, closest_vectors, excluding_self
     from vectorlink_gpu.kernels import gather_distances
 
     length = seeds.shape[1]
@@ -42,6 +52,10 @@ def search(v, rows, beams, seeds, c, exclude, flags, sketch=None, workspace=None
     ids = dev(seeds)
     q.insert(ids, gather_distances(v[:rows], v, ids, metric=c.get("metric", "cosine")))
     t = closest_vectors(v[:rows], q, v, beams, c, excluding_self(0, rows) if exclude else None, flags=flags, sketch=sketch)
+    if flags & BEAM_TABLE:
+        (given, need) = ahead(rows, v.size(0), v.size(1), beams, q, c, exclude, flags | (BEAM_USES_SKETCH if sketch is not None else 0))
+        assert given == BEAM_TABLE
+        assert _workspace(v.device).has(need) == table
     return t, q.indices.cpu().numpy()[:, :length], bits(q.distances)[:, :length]
 
 
@@ -101,6 +115,27 @@ def test_queues_around_the_sets_of_64(beam, length, width, visits, ef, per_query
     for exclude in (False, True):
         got = search(dev(v), rows, dev(beams), seeds, c, exclude, flags)
         same(got, oracle(v, rows, beams, seeds, c, exclude, per_query))
+
+
+@pytest.mark.parametrize("sketched", [False, True])
+def test_distances_are_looked_up_and_not_fetched(sketched):
+    """What a profiled call counts: candidates, and none of them a row that was read."""
+    from vectorlink_gpu import _native as nv
+    from vectorlink_gpu.ann import BEAM_TABLE
+    from vectorlink_gpu.kernels import build_sketch
+
+    (n, rows) = (900, 300)
+    v = dev(vectors(n, 256))
+    ids = orc.generate_circulant_beams(n, orc.primes(32))
+    out = (C.c_double * 9)()
+    nv.lib().vl_beam_profile(1, 1, out)
+    try:
+        search(v, rows, dev(ids), ids[:rows], config(beam_size=16, exclude_factor=30), True, BEAM_TABLE,
+               sketch=build_sketch(v) if sketched else None)
+    finally:
+        nv.lib().vl_beam_profile(0, 1, out)
+    (evals, wanted, through_sketch) = (out[4], out[7], out[8])
+    assert evals == through_sketch == 0 and wanted > 4 * 32 * rows
 
 
 def test_many_rows_and_the_sketch():
@@ -241,7 +276,7 @@ def test_no_memory_for_the_table(monkeypatch):
 
     ann.release_workspaces()
     monkeypatch.setattr(ann._Workspace, "reserve", refuse_first)
-    same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE), want)
+    same(search(v, rows, beams, seeds, c, True, ann.BEAM_TABLE | ann.BEAM_NO_CACHE, table=False), want)
     assert len(asked) == 2 and asked[1] < asked[0]
 
 
@@ -255,6 +290,10 @@ def test_a_batch_of_a_build_that_comes_without_a_word(circulant):
         ids = np.random.default_rng(5).integers(0, n, ids.shape).astype(np.int32)
     seeds = orc.generate_circulant_beams(n, orc.primes(64))[:rows]
     c = config(beam_size=32)
-    from vectorlink_gpu.ann import BEAM_NO_TABLE
+    from vectorlink_gpu import Queue
+    from vectorlink_gpu.ann import BEAM_MANY_ITERATIONS, BEAM_NO_TABLE, BEAM_TABLE, _circulant_graph
 
+    q = Queue(rows, 64, 64 + 256)
+    assert ahead(rows, n, 64, dev(ids), q, c, True, 0)[0] == BEAM_MANY_ITERATIONS and _circulant_graph(dev(ids)) == circulant
+    assert ahead(rows, n, 64, dev(ids), q, c, True, BEAM_MANY_ITERATIONS)[0] == BEAM_TABLE
     same(search(v, rows, dev(ids), seeds, c, True, 0), search(v, rows, dev(ids), seeds, c, True, BEAM_NO_TABLE))
