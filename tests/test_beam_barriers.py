@@ -26,7 +26,7 @@ template __global__ void beam_window_kernel<1, 64, 8, kRowAligned, 256, 6>(StepA
 template __global__ void beam_step_sketch_kernel<3, 64, 1, 256, 3, 16, 1, 8>(StepArgs);
 template __global__ void beam_window_sketch_kernel<3, 64, 1, 256, 3, 16, 1, 6>(StepArgs);
 template __global__ void beam_window_near_kernel<3, 64, 2, 256, 3, 6>(StepArgs);
-template __global__ void beam_window_near_kernel<6, 64, 1, 256, 6, 5>(StepArgs);
+template __global__ void beam_window_near_kernel<8, 64, 1, 256, 4, 5>(StepArgs);
 }
 """
 
