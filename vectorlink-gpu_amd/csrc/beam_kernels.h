@@ -31,8 +31,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
     beam_row<CPL, LPR, U, kRowAligned, THREADS, SCPL, SLPR, SU, true>(s);
 }
 // ... and with the products of all queries and vectors at hand (near_products.h); it keeps no query row for the sketch.  An
-// iteration of 10,000 rows at 1M x 768 takes 0.16 ms (through the sketch 0.58) and waits on round trips: neighbour lists, products,
-// rows.  Rows in flight and room for wavefronts per SIMD are chosen by what spills.  First-loop batches of 10,000 (ms), 1M x 768 /
+// iteration of 10,000 rows at 1M x 768 takes 0.16 ms (through the sketch 0.58): a launch of five moves 3.9 GB past L2, most of it rows
+// that the bounds leave, 4.9 TB/s of the 6.0 that gathered rows reach, with vector instructions issuing in 62 % of cycles.  Rows in
+// flight and room for wavefronts per SIMD are the fastest of those tried (of the chosen ones those for 384, 768 and 1,536 columns keep
+// three or four vector registers in scratch memory, for 1,792 25, for 2,048 57, the others none).  First-loop batches of 10,000 (ms), 1M x 768 /
 // 500,000 x 1,024 / 500,000 x 1,536 / 1M x 384: one row and six wavefronts 59.2 / 57.6 / 93.3 / 35.9, two and six 57.8 / 66.5 / 93.1 / 36.0,
 // one and five 59.4 / 57.7 / 82.9 / 36.0, two and five 62.5 / 61.0 / 99.7 / 38.6, two and four 62.7 / 60.8 / 86.4 / 38.4, four and six 76.6 /
 // 135.6 / 305.9 / 47.7.  With 128 threads a row 76.0 and 96.6 instead of 59.9 and 84.7 (768 and 1,536 columns).

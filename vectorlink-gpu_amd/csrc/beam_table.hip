@@ -5,7 +5,8 @@
 // them.  (One after the other, with the queues in registers and two instructions for each 64 slots of them, a candidate took
 // 560 cycles: 12 of them 6,970 of a lone wavefront's 10,350 an iteration, 60 of them 31,300 in the first ones.  256 queries at
 // 4,096 x 128 564 -> 514 us, 37 at 20,011 x 50 682 -> 575, first-loop batches at 4,096 x 128 1.31 -> 1.17 ms, 6,007 x 384 2.85 ->
-// 2.52, 20,011 x 768 12.5 -> 11.8, where an iteration waits for the table's cache lines, 5 TB/s of them.)
+// 2.52, 20,011 x 768 12.5 -> 11.8, where a launch of five iterations moves 0.53 GB past L2 in 118 us, 4.5 TB/s, most of it the
+// table's cache lines.)
 //
 // An entry of the row's table is taken while its id sits in the visit queue and from the moment it was visited.  Such a
 // candidate can change neither queue (beam_row.h says why for visited ones; one in the visit queue was offered to the search
@@ -24,11 +25,6 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-__device__ __forceinline__ uint64_t lane_key(uint64_t k, int lane) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, lane);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(k >> 32), lane);
-    return ((uint64_t)hi << 32) | lo;
 }
 __device__ __forceinline__ int below(uint64_t mask) {  // lanes of the mask before this one
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));

@@ -7,7 +7,8 @@
 // What bounds it: these products run on the vector unit's multipliers (157 TFLOP/s either way), so the additions of the folds,
 // one per partial sum and pair, take their time from them: at most 135 TFLOP/s at 768 columns, 105 at 128.  Measured with what
 // packs the operands: 10,000 x 20,011 x 768 2.95 ms (104 TFLOP/s), x 1,536 5.65 (109), 10,000 x 100,000 x 128 3.0 (85), 10,000 x
-// 40,000 x 130 1.50 (69), 256 x 4,096 x 128 17 us; squared differences 6,007 x 6,007 x 384 0.69 ms (40).  Tried and left out:
+// 40,000 x 130 1.50 (69), 256 x 4,096 x 128 17 us; squared differences 6,007 x 6,007 x 384 0.69 ms (40; beyond 128 columns that kernel keeps 34 registers in
+// scratch memory).  Tried and left out:
 // tiles of 128 x 64 and 128 x 128 (half the operands from L2: 3,060 and 3,030 us for the first), three and four stages in
 // flight (3,000 to 3,060), the operands of the next unit read ahead (3,010), partial sums one at a time (3,600).
 #include "pair_table.h"
